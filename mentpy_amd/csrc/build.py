@@ -1,7 +1,7 @@
 """Build the native library ``mentpy_amd/lib/libmbqc_hip.so`` for gfx950.
 
-One ``hipcc`` invocation compiles the HIP kernels and the host plan compiler
-into a shared library with a plain C ABI (declared in ``include/mbqc_hip.h``).
+``hipcc`` compiles the HIP kernels and the host plan compiler into a shared
+library with a plain C ABI (declared in ``include/mbqc_hip.h``).
 Packed FP32 instructions are disabled for all device code.
 
 ``--sanitize`` builds ``mentpy_amd/lib/libmbqc_hip_sanitize.so`` instead: the
@@ -17,6 +17,8 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import tempfile
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
@@ -25,7 +27,7 @@ ROOT = PKG.parent
 LIB_DIR = PKG / "lib"
 LIB = LIB_DIR / "libmbqc_hip.so"
 SANITIZE_LIB = LIB_DIR / "libmbqc_hip_sanitize.so"
-SOURCES = [HERE / "kernels.hip", HERE / "plan.cpp", HERE / "flow.cpp"]
+SOURCES = [HERE / "kernels.hip", HERE / "wide.hip", HERE / "plan.cpp", HERE / "flow.cpp"]
 ARCH = os.environ.get("MBQC_OFFLOAD_ARCH", "gfx950")
 SANITIZE_FLAGS = ["-Xarch_host", "-fsanitize=address", "-Xarch_host", "-fsanitize=undefined",
                   "-Xarch_host", "-fno-omit-frame-pointer", "-Xarch_host",
@@ -39,22 +41,30 @@ def hipcc() -> str:
     return "hipcc"
 
 
-def _compile(target: Path, extra, opt: str, verbose: bool) -> Path:
-    LIB_DIR.mkdir(parents=True, exist_ok=True)
-    tmp = target.with_suffix(".so.tmp")
-    cmd = [
-        hipcc(), f"--offload-arch={ARCH}", opt, "-std=c++17", "-shared", "-fPIC",
-        "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-        "-Wno-unused-command-line-argument", *extra,
-        "-I", str(ROOT / "include"),
-        *[str(s) for s in SOURCES], "-o", str(tmp),
-    ]
+def _run(cmd, verbose: bool):
     if verbose:
         print(" ".join(cmd), flush=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         sys.stderr.write(res.stdout + res.stderr)
         raise RuntimeError(f"hipcc failed with status {res.returncode}")
+
+
+def _compile(target: Path, extra, opt: str, verbose: bool) -> Path:
+    """Compile every source (concurrently: the kernel files take about a minute
+    each) and link them into ``target``."""
+    LIB_DIR.mkdir(parents=True, exist_ok=True)
+    tmp = target.with_suffix(".so.tmp")
+    flags = [
+        f"--offload-arch={ARCH}", opt, "-std=c++17", "-fPIC",
+        "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+        "-Wno-unused-command-line-argument", *extra,
+    ]
+    with tempfile.TemporaryDirectory() as obj_dir, ThreadPoolExecutor(len(SOURCES)) as pool:
+        objs = [str(Path(obj_dir) / f"{src.stem}.o") for src in SOURCES]
+        list(pool.map(lambda so: _run([hipcc(), *flags, "-I", str(ROOT / "include"), "-c",
+                                       str(so[0]), "-o", so[1]], verbose), zip(SOURCES, objs)))
+        _run([hipcc(), *flags, "-shared", *objs, "-o", str(tmp)], verbose)
     os.replace(tmp, target)
     return target
 

@@ -19,111 +19,11 @@
 #include <cstring>
 #include <utility>
 
+#include "device.h"
 #include "plan.h"
+#include "wide.h"
 
 namespace mbqc {
-
-// ------------------------------------------------------------------ helpers
-__device__ __forceinline__ float2 cmul(float2 a, float2 b) {
-  return make_float2(fmaf(a.x, b.x, -a.y * b.y), fmaf(a.x, b.y, a.y * b.x));
-}
-__device__ __forceinline__ float2 cconj(float2 a) { return make_float2(a.x, -a.y); }
-__device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
-__device__ __forceinline__ float2 cscale(float2 a, float s) { return make_float2(a.x * s, a.y * s); }
-// flip the sign of both components when sbit == 0x80000000
-__device__ __forceinline__ float2 flip(float2 v, uint32_t sbit) {
-  return make_float2(__uint_as_float(__float_as_uint(v.x) ^ sbit),
-                     __uint_as_float(__float_as_uint(v.y) ^ sbit));
-}
-// CZ sign of slot-index j against the neighbour mask: parity(j & mask) << 31
-__device__ __forceinline__ uint32_t czbit(uint32_t j, uint32_t mask) {
-  return uint32_t(__builtin_popcount(j & mask) & 1) << 31;
-}
-
-// Round-to-nearest-even integer of v (|v| < 2^22) by the 1.5 * 2^23 shifter:
-// fl(v + 1.5 * 2^23) has a unit last mantissa bit, so its lowest bit is the
-// parity of rint(v).  With the shifter added in an FMA, v = a * c is rounded
-// once (no rounding of a * c first).
-constexpr float kShifter = 12582912.0f;      // 1.5 * 2^23
-
-// sin and cos of x for |x| up to a few thousand: x = k pi + r with a two-term
-// Cody-Waite split of pi (hi part the nearest float), |r| <= pi/2, then
-// polynomials fitted for minimum maximum error on [-pi/2, pi/2] (odd degree 9
-// for sin, even degree 10 for cos; fitted in double by linear programming on
-// 4,000 Chebyshev points, approximation error below 5e-10, float evaluation
-// error about 1e-7), and the sign (-1)^k on both.
-__device__ __forceinline__ void sincos_poly(float x, float* sn, float* cs) {
-  const float kb = fmaf(x, 0.318309886183790671538f, kShifter);
-  const float k = kb - kShifter;
-  float r = fmaf(-k, 3.14159274101257324219f, x);
-  r = fmaf(-k, -8.74227800037248e-8f, r);
-  const float r2 = r * r;
-  float ps = fmaf(r2, 2.601407004e-6f, -1.980598900e-4f);
-  ps = fmaf(r2, ps, 8.332983591e-3f);
-  ps = fmaf(r2, ps, -1.666665375e-1f);
-  const float sr = fmaf(r * r2, ps, r);
-  float pc = fmaf(r2, -2.650938882e-7f, 2.479057366e-5f);
-  pc = fmaf(r2, pc, -1.388906501e-3f);
-  pc = fmaf(r2, pc, 4.166670144e-2f);
-  pc = fmaf(r2, pc, -0.5f);
-  const float cr = fmaf(r2, pc, 1.0f);
-  const uint32_t sgn = __float_as_uint(kb) << 31;
-  *sn = __uint_as_float(__float_as_uint(sr) ^ sgn);
-  *cs = __uint_as_float(__float_as_uint(cr) ^ sgn);
-}
-
-// The reference's global phase, prod_k sgn(cos(theta_k/2)) e^{i theta_k/2}
-// (the factor its amplitude-sum partial trace introduces,
-// mentpy/calculator/state_ops.py:68-73).  With m_k = rint(theta_k / 2 pi),
-// theta_k/2 - pi m_k lies in [-pi/2, pi/2], so sgn(cos(theta_k/2)) = (-1)^m_k
-// and the product is exp(i (sum_k theta_k / 2 - pi sum_k m_k)).  The angles
-// are summed in double (full-rate on this GPU) and the integers m_k in int32,
-// and the phase is formed once at the end.
-// m_k must be exact for every float32 angle, also the ones next to an odd
-// multiple of pi where cos(theta/2) changes sign (float32(pi) itself lies
-// 8.7e-8 above pi: m = 1, phase -i).  A float32 product with fl32(1/2pi),
-// 4e-8 too small relative to 1/2pi, rounds those down, so m_k is rounded in
-// double: fma(theta, fl64(1/2pi), 1.5 * 2^52) rounds the exact product to an
-// integer (ties to even) held in the low word of its bits, with a relative
-// error of 1.1e-16 that can only matter within 1e-13 of a half-integer;
-// no float32 angle below 2^12 comes that close (the nearest lies more than
-// 1e-9 away, checked exhaustively on the CPU).
-constexpr double kShifter64 = 6755399441055744.0;   // 1.5 * 2^52
-struct RefPhase {
-  double th_sum = 0.0;
-  int32_t m_sum = 0;
-  __device__ __forceinline__ void add(float th) {
-    const double d = double(th);
-    const double mb = fma(d, 0.15915494309189533577, kShifter64);
-    m_sum += int32_t(uint32_t(__double_as_longlong(mb)));
-    th_sum += d;
-  }
-  // add(th) where `on`, nothing elsewhere
-  __device__ __forceinline__ void add_if(float th, bool on) {
-    const double d = on ? double(th) : 0.0;
-    const double mb = fma(d, 0.15915494309189533577, kShifter64);
-    m_sum += int32_t(uint32_t(__double_as_longlong(mb)));
-    th_sum += d;
-  }
-  __device__ __forceinline__ float2 value() const {
-    constexpr double kPi = 3.14159265358979323846;
-    double a = 0.5 * th_sum - kPi * double(m_sum);
-    a -= 2.0 * kPi * rint(a * (0.5 / kPi));
-    double sd, cd;
-    sincos(a, &sd, &cd);
-    return make_float2(float(cd), float(sd));
-  }
-};
-
-// b = e^{-i theta}; with REF the step's reference phase is accumulated too.
-template <bool REF>
-__device__ __forceinline__ float2 step_coeff(float th, RefPhase* ph) {
-  if constexpr (REF) ph->add(th);
-  float s, c;
-  sincos_poly(th, &s, &c);
-  return make_float2(c, -s);
-}
 
 // ---------------------------------------------------------------- SV step
 // Measure slot Q at XY angle theta (b = e^{-i theta}) and put the next
@@ -176,31 +76,6 @@ __device__ __forceinline__ void sv_step_periodic(float2 (&t)[1 << NS], float2 b)
       t[j | QB] = make_float2(fmaf(2.0f, x.x, -u0.x), fmaf(2.0f, x.y, -u0.y));
   }
 }
-
-// Job description shared by the SV / DM / adjoint kernels (passed by value
-// or read from global memory by the persistent kernel).
-struct Job {
-  const int32_t* tab;       // packed device tables of the plan
-  int32_t off_in, off_sign, off_out, off_svres, off_dmres, e_sv, e_dm;
-  int32_t ns, n_steps, n_out, live_mask, off_coef;
-  int32_t off_aidx, off_run;  // contiguous angle indices, stretch ends
-  // 1: no step has a fixed angle and every angle offset angle_index *
-  // angle_stride_a fits in 32 bits (the statevector kernels' short fetch)
-  int32_t fast_fetch;
-  const float* angles;
-  int64_t angle_stride;     // elements between angle vectors (0: shared)
-  int64_t angle_stride_a;   // elements between the angles of one vector
-  const float2* psi;
-  int64_t in_stride;
-  float2* out;
-  float2* phase_out;
-  int64_t S, total;
-};
-
-// Identity modifier of the per-step projection coefficient b = e^{-i theta}.
-struct NoModify {
-  __device__ __forceinline__ float2 operator()(int, float2 b) const { return b; }
-};
 
 // Pair coefficients of step k: row (steps[k].flags >> 16) of the plan's
 // coefficient table.  Long patterns store each distinct row once (a grid has
@@ -525,11 +400,6 @@ __device__ __forceinline__ void sv_load_input(const Job& J, const float2* psi, f
     const float2 v = psi[in_index[j]];
     t[j] = flip(v, sign[j] ? 0x80000000u : 0u);
   }
-}
-
-__device__ __forceinline__ float sv_final_scale(int e) {
-  float s = ldexpf(1.0f, -(e >> 1));
-  return (e & 1) ? s * 0.70710678118654752440f : s;
 }
 
 // Makes this wave's LDS writes visible to its own later LDS reads: waits for
@@ -873,51 +743,6 @@ __global__ __launch_bounds__(256) void k_dm_forward(Job J, DmNoise nz, uint32_t 
 }
 
 // ------------------------------------------------------- sampled outcomes
-// 32 pseudo-random bits per (seed, simulation, block of 32 steps): the
-// splitmix64 finaliser (Steele, Lea, Flood, "Fast splittable pseudorandom
-// number generators", OOPSLA 2014) applied to a Weyl-sequence key.
-__device__ __forceinline__ uint32_t draw32(uint64_t seed, uint64_t sim, uint64_t block) {
-  uint64_t z = seed + sim * 0x9E3779B97F4A7C15ull + (block + 1) * 0xD1B54A32D192ED03ull;
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-  return uint32_t(z ^ (z >> 31));
-}
-
-// Per-lane Pauli frame and outcome draw of the sampled mode.  Before step k,
-// bit 0 of fx / fz is the X / Z frame of schedule[k]: the node is measured at
-// (-1)^x theta, the drawn projection m' (probability 1/2 each) is onto
-// |+/- theta'>, and the physical outcome is m' xor z.  An outcome 1 flips the
-// frames of the flow successor and of its later neighbours (xmask/zmask).
-// Frames are 32-bit: a plan that samples applies every CZ edge within its
-// window of at most 7 positions, so every offset is below 14 (the host
-// checks < 32).
-struct SampleMod {
-  uint32_t fx = 0, fz = 0;
-  uint64_t seed = 0, sim = 0;
-  const uint64_t* xm;
-  const uint64_t* zm;
-  int32_t* out_words;   // this simulation's outcome words (null for inactive lanes)
-  int n;
-  uint32_t rbits = 0, word = 0;
-  __device__ __forceinline__ float2 operator()(int k, float2 b) {
-    const int kb = k & 31;
-    if (kb == 0) rbits = draw32(seed, sim, uint64_t(k >> 5));
-    const uint32_t mprime = (rbits >> kb) & 1u;
-    const uint32_t xk = fx & 1u, zk = fz & 1u;
-    const uint32_t mk = mprime ^ zk;
-    word |= mk << kb;
-    if (kb == 31 || k == n - 1) {
-      if (out_words) out_words[k >> 5] = int32_t(word);
-      word = 0;
-    }
-    const uint32_t sel = 0u - mk;
-    fx = (fx ^ (uint32_t(xm[k]) & sel)) >> 1;
-    fz = (fz ^ (uint32_t(zm[k]) & sel)) >> 1;
-    float2 bb = xk ? cconj(b) : b;
-    return mprime ? make_float2(-bb.x, -bb.y) : bb;
-  }
-};
-
 template <int NS, bool PERIODIC>
 __global__ __launch_bounds__(256) void k_sv_sample(Job J, const uint64_t* __restrict__ xm,
                                                    const uint64_t* __restrict__ zm,
@@ -1003,43 +828,11 @@ __global__ __launch_bounds__(256) void k_sv_sample(Job J, const uint64_t* __rest
 }
 
 // ------------------------------------------------------- LDS-resident kernels
-// Larger live windows (SV with 7..12 slots, DM with 4..6 slots): one
-// workgroup per simulation keeps the state in LDS; the measured slot is a
-// runtime value, each thread updates a strided subset of the amplitude pairs
-// (DM: quartets) and the workgroup synchronises between steps.
-// Workgroups are dealt to the chip's kXcds XCDs round-robin (workgroup b runs
-// on XCD b % kXcds), each XCD with its own L2.  xcd_block maps workgroup b of
-// n to a logical block so that every XCD takes a contiguous run of logical
-// blocks (a bijection of [0, n)): neighbouring simulations, which share cache
-// lines of the angle table, then meet in one L2 instead of each XCD fetching
-// the line.
-constexpr unsigned kXcds = 8;
-__device__ __forceinline__ unsigned xcd_block(unsigned b, unsigned n) {
-  const unsigned q = n / kXcds, r = n % kXcds, x = b % kXcds;
-  return x * q + (x < r ? x : r) + b / kXcds;
-}
-
-__device__ __forceinline__ int insert_zero(int v, int q) {
-  return ((v >> q) << (q + 1)) | (v & ((1 << q) - 1));
-}
-
-// Sum over the T threads of a workgroup (T a power of two); a workgroup of
-// fewer than 64 threads only exchanges among its own lanes.
-template <int T>
-__device__ __forceinline__ float block_sum(float v, float* red) {
-  constexpr int first = T >= 64 ? 32 : T / 2;
-  for (int m = first; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-  if constexpr (T > 64) {
-    const int w = threadIdx.x >> 6;
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[w] = v;
-    __syncthreads();
-    v = 0.0f;
-#pragma unroll
-    for (int i = 0; i < T / 64; ++i) v += red[i];
-  }
-  return v;
-}
+// One workgroup per simulation keeps the state in LDS (DM with 3..7 slots; SV
+// for plans whose measured slots leave the rotation, up to 14 slots, the
+// others of 7 slots and more run in wide.hip): the measured slot is a runtime
+// value, each thread updates a strided subset of the amplitude pairs (DM:
+// quartets) and the workgroup synchronises between steps.
 
 // Angles of the workgroup's simulation for steps [k0, k0 + kAngleChunk), read
 // by all threads into LDS at once, so a step does not wait on its own global
@@ -1210,11 +1003,11 @@ __global__ __launch_bounds__(256) void k_sv_forward_global(Job J, uint32_t flags
   sv_lds_run<NS, 256>(J, g0 + l, flags, ws + (l << NS), red, th_s, threadIdx.x);
 }
 
-// Sampled outcomes for windows of 7..14 slots: k_sv_sample's frame and draw
+// Sampled outcomes for windows above the LDS: k_sv_sample's frame and draw
 // arithmetic (SampleMod, evaluated identically by every thread of the
-// workgroup, so the frame is uniform) on the LDS-resident state of
-// k_sv_forward_lds.  Raw phase; the output is renormalised and leaves with the
-// output frame applied, as in k_sv_sample.
+// workgroup, so the frame is uniform) on a state in a global workspace.  Raw
+// phase; the output is renormalised and leaves with the output frame applied,
+// as in k_sv_sample.
 template <int NS, int T>
 __device__ __forceinline__ void sample_run(const Job& J, const uint64_t* __restrict__ xm,
                                            const uint64_t* __restrict__ zm,
@@ -1281,20 +1074,6 @@ __device__ __forceinline__ void sample_run(const Job& J, const uint64_t* __restr
   }
 }
 
-template <int NS, int T>
-__global__ __launch_bounds__(T) void k_sv_sample_lds(Job J, const uint64_t* __restrict__ xm,
-                                                     const uint64_t* __restrict__ zm,
-                                                     const int32_t* __restrict__ out_off,
-                                                     int32_t* __restrict__ outcomes, int32_t words,
-                                                     uint64_t seed) {
-  __shared__ float2 st[1 << NS];
-  __shared__ float red[4];
-  __shared__ float th_s[kAngleChunk];
-  sample_run<NS, T>(J, xm, zm, out_off, outcomes, words, seed, st, red, th_s,
-                    xcd_block(blockIdx.x, gridDim.x), threadIdx.x);
-}
-
-// Windows above the LDS: the same with the state in a global workspace.
 template <int NS>
 __global__ __launch_bounds__(256) void k_sv_sample_global(Job J, const uint64_t* __restrict__ xm,
                                                           const uint64_t* __restrict__ zm,
@@ -1941,11 +1720,6 @@ __global__ __launch_bounds__(256) void k_sv_adj_forward_global(Job J, float2* __
   __shared__ float th_s[kAngleChunk];
   const int64_t l = xcd_block(blockIdx.x, gridDim.x);
   adj_forward_run<NS, 256>(J, ckpt, ck, ws + (l << NS), th_s, g0 + l, threadIdx.x);
-}
-
-// The angle of step k of this simulation (its angle-vector entry or its fixed angle).
-__device__ __forceinline__ float step_angle(const mbqc_step& st, const float* ang, int64_t sa) {
-  return st.angle_index >= 0 ? ang[int64_t(st.angle_index) * sa] : st.fixed_angle;
 }
 
 // Block [k0, k0 + NS) of the LDS adjoint: recompute the block forward from
@@ -3216,78 +2990,17 @@ __global__ __launch_bounds__(256) void k_dm_general_global(Job J, const float* _
 
 
 // ---------------------------------------------------------------- batched
-struct BatchItem {
-  int32_t job;
-  int32_t count;   // simulations in this item
-  int64_t first;   // first simulation index within the job
-};
-
-// Persistent kernel over the work items of one live-window size NS: every
-// wave pulls items (runs of simulations of one job) from its group's device
-// counter until none are left.  Items are sorted by decreasing cost on the
-// host, so long patterns start first.  One kernel per NS keeps each group at
-// the register footprint (and so the occupancy) of its own window size.
-// A Job read from device memory (rather than passed as a kernel argument)
-// holds generic pointers: loads and stores through them compile to flat
-// instructions, and the plan-table loads could not be proven free of the
-// kernel's own stores, so they would all be per-lane vector loads.  The same
-// layout with the pointers typed as global memory, and the read-only plan
-// tables as constant memory, restores global vector instructions and scalar
-// table loads.
-struct GlobalJob {
-  const __attribute__((address_space(4))) int32_t* tab;
-  int32_t off_in, off_sign, off_out, off_svres, off_dmres, e_sv, e_dm;
-  int32_t ns, n_steps, n_out, live_mask, off_coef;
-  int32_t off_aidx, off_run;
-  int32_t fast_fetch;
-  const __attribute__((address_space(1))) float* angles;
-  int64_t angle_stride;
-  int64_t angle_stride_a;
-  const __attribute__((address_space(1))) float2* psi;
-  int64_t in_stride;
-  __attribute__((address_space(1))) float2* out;
-  __attribute__((address_space(1))) float2* phase_out;
-  int64_t S, total;
-};
-static_assert(sizeof(GlobalJob) == sizeof(Job), "GlobalJob mirrors Job");
-
-__device__ __forceinline__ Job load_job(const Job* jobs, int i) {
-  const GlobalJob g = reinterpret_cast<const GlobalJob*>(jobs)[i];
-  Job j;
-  j.tab = (const int32_t*)g.tab;
-  j.off_in = g.off_in;
-  j.off_sign = g.off_sign;
-  j.off_out = g.off_out;
-  j.off_svres = g.off_svres;
-  j.off_dmres = g.off_dmres;
-  j.e_sv = g.e_sv;
-  j.e_dm = g.e_dm;
-  j.ns = g.ns;
-  j.n_steps = g.n_steps;
-  j.n_out = g.n_out;
-  j.live_mask = g.live_mask;
-  j.off_coef = g.off_coef;
-  j.off_aidx = g.off_aidx;
-  j.off_run = g.off_run;
-  j.fast_fetch = g.fast_fetch;
-  j.angles = (const float*)g.angles;
-  j.angle_stride = g.angle_stride;
-  j.angle_stride_a = g.angle_stride_a;
-  j.psi = (const float2*)g.psi;
-  j.in_stride = g.in_stride;
-  j.out = (float2*)g.out;
-  j.phase_out = (float2*)g.phase_out;
-  j.S = g.S;
-  j.total = g.total;
-  return j;
-}
-
 // Output stores of the batched kernel: direct (staging the 32-amplitude rows
 // through LDS tiles measured slower here: 3.54e9 -> 3.27e9 sims/s on the
 // 64-grid batch, whose window-size groups run concurrently).
 template <int NS>
 constexpr int kBatchStore = kStoreDirect;
 
+// Persistent kernel over the work items of one live-window size NS: every
+// wave pulls items (runs of simulations of one job) from its group's device
+// counter until none are left.  Items are sorted by decreasing cost on the
+// host, so long patterns start first.  One kernel per NS keeps each group at
+// the register footprint (and so the occupancy) of its own window size.
 template <bool REF, int NS, bool SH, bool PERIODIC>
 __global__ __launch_bounds__(256) void k_batch(const Job* __restrict__ jobs,
                                                const BatchItem* __restrict__ items, int64_t n_items,
@@ -3312,39 +3025,11 @@ __global__ __launch_bounds__(256) void k_batch(const Job* __restrict__ jobs,
   }
 }
 
-// Batched groups of 7..14 live slots: a persistent workgroup per resident
-// slot pulls items from the group's counter and runs their simulations one
-// after the other with the state in LDS (sv_lds_run, as k_sv_forward_lds).
-// Every thread reads the item index from LDS, so all leave the loop together
-// once the counter passes n_items.
-template <int NS, int T>
-__global__ __launch_bounds__(T) void k_batch_lds(const Job* __restrict__ jobs,
-                                                 const BatchItem* __restrict__ items,
-                                                 int64_t n_items, int* counter, uint32_t flags) {
-  __shared__ float2 st[1 << NS];
-  __shared__ float red[4];
-  __shared__ float th_s[kAngleChunk];
-  __shared__ int item_s;
-  const int tid = threadIdx.x;
-  for (;;) {
-    __syncthreads();   // the previous item's last reads of item_s and st are done
-    if (tid == 0) item_s = atomicAdd(counter, 1);
-    __syncthreads();
-    const int it = item_s;
-    if (it >= n_items) break;
-    const BatchItem I = items[it];
-    const Job J = load_job(jobs, I.job);
-    const int64_t end = std::min<int64_t>(I.first + I.count, J.total);
-    for (int64_t g = I.first; g < end; ++g) {
-      __syncthreads();
-      sv_lds_run<NS, T>(J, g, flags, st, red, th_s, tid);
-    }
-  }
-}
-
-// Groups above the LDS (15..20 slots): the same with each persistent
-// workgroup's state in its own slice of a global workspace,
-// ws[blockIdx * 2^NS + j].
+// Groups above the LDS (15..20 slots): a persistent workgroup per resident slot
+// pulls items from the group's counter and runs their simulations one after the
+// other (sv_lds_run) with the state in its own slice of a global workspace,
+// ws[blockIdx * 2^NS + j].  Every thread reads the item index from LDS, so all
+// leave the loop together once the counter passes n_items.
 template <int NS>
 __global__ __launch_bounds__(256) void k_batch_global(const Job* __restrict__ jobs,
                                                       const BatchItem* __restrict__ items,
@@ -3370,9 +3055,6 @@ __global__ __launch_bounds__(256) void k_batch_global(const Job* __restrict__ jo
     }
   }
 }
-
-// group counters live kCounterStride ints apart (separate cache lines)
-constexpr int kCounterStride = 64;
 
 __global__ void k_reset_counters(int* counter, int n) {
   const int i = threadIdx.x;
@@ -3438,8 +3120,8 @@ int global_fail(hipError_t e, const char* what) {
   return hip_fail(e, what);
 }
 
-// Launch `kernel_chunk(ws, g0, n)` over the job's simulations in chunks whose
-// states (state_bytes each) fit the workspace.
+// Launch `kernel_chunk(ws, g0, n)` (which returns its launch status) over the
+// job's simulations in chunks whose states (state_bytes each) fit the workspace.
 template <typename F>
 hipError_t run_global_chunks(const Job& J, size_t state_bytes, hipStream_t st, F&& kernel_chunk) {
   const int64_t per = std::max<int64_t>(
@@ -3449,8 +3131,7 @@ hipError_t run_global_chunks(const Job& J, size_t state_bytes, hipStream_t st, F
   hipError_t e = global_ws_alloc(&ws, size_t(n0) * state_bytes, st);
   if (e != hipSuccess) return e;
   for (int64_t g0 = 0; g0 < J.total && e == hipSuccess; g0 += n0) {
-    kernel_chunk(static_cast<float2*>(ws), g0, std::min<int64_t>(n0, J.total - g0));
-    e = hipGetLastError();
+    e = kernel_chunk(static_cast<float2*>(ws), g0, std::min<int64_t>(n0, J.total - g0));
   }
   const hipError_t ef = hipFreeAsync(ws, st);
   return e != hipSuccess ? e : ef;
@@ -3461,6 +3142,7 @@ hipError_t launch_sv_global(const Job& J, uint32_t flags, hipStream_t st) {
   return run_global_chunks(J, sizeof(float2) << NS, st, [&](float2* ws, int64_t g0, int64_t n) {
     hipLaunchKernelGGL((k_sv_forward_global<NS>), dim3(unsigned(n)), dim3(256), 0, st, J, flags, ws,
                        g0);
+    return hipGetLastError();
   });
 }
 
@@ -3472,6 +3154,7 @@ hipError_t launch_dm_global(const Job& J, const DmNoise& nz, uint32_t flags, flo
     hipLaunchKernelGGL(k_dm_general_global, dim3(unsigned(n)), dim3(256), 0, st, J,
                        static_cast<const float*>(nullptr), int64_t(0), int32_t(J.n_steps), none, 0,
                        nz, flags, outcomes, ws, g0);
+    return hipGetLastError();
   });
 }
 constexpr int kMaxAdjSlots = 5;
@@ -3732,6 +3415,7 @@ hipError_t launch_adj_fwd_global(const Job& J, float2* ckpt, int ck, hipStream_t
   return run_global_chunks(J, sizeof(float2) << NS, st, [&](float2* ws, int64_t g0, int64_t n) {
     hipLaunchKernelGGL((k_sv_adj_forward_global<NS>), dim3(unsigned(n)), dim3(256), 0, st, J, ckpt,
                        ck, ws, g0);
+    return hipGetLastError();
   });
 }
 
@@ -3938,18 +3622,8 @@ hipError_t launch_sample_global(const Job& J, const int32_t* tab, const TableOff
   return run_global_chunks(J, sizeof(float2) << NS, st, [&](float2* ws, int64_t g0, int64_t n) {
     hipLaunchKernelGGL((k_sv_sample_global<NS>), dim3(unsigned(n)), dim3(256), 0, st, J, xm, zm,
                        tab + o.out_offset, outcomes, words, seed, ws, g0);
+    return hipGetLastError();
   });
-}
-
-template <int NS>
-hipError_t launch_sample_lds(const Job& J, const int32_t* tab, const TableOffsets& o,
-                             int32_t* outcomes, int32_t words, uint64_t seed, hipStream_t st) {
-  constexpr int T = (1 << (NS - 1)) < 256 ? (1 << (NS - 1)) : 256;
-  const uint64_t* xm = reinterpret_cast<const uint64_t*>(tab + o.xmask);
-  const uint64_t* zm = reinterpret_cast<const uint64_t*>(tab + o.zmask);
-  hipLaunchKernelGGL((k_sv_sample_lds<NS, T>), dim3(unsigned(J.total)), dim3(T), 0, st, J, xm, zm,
-                     tab + o.out_offset, outcomes, words, seed);
-  return hipGetLastError();
 }
 
 template <int NS>
@@ -4131,17 +3805,6 @@ int scratch_ptr(float** out) {
   return MBQC_OK;
 }
 
-// Groups above kMaxSvSlots: one persistent workgroup of T threads (T / 64
-// waves) per resident slot, `waves` / (T / 64) of them, at least one and at
-// most one per item.
-template <int NS>
-void launch_batch_lds_group(int64_t waves, const BatchGroupLaunch& L) {
-  constexpr int T = (1 << (NS - 1)) < 256 ? (1 << (NS - 1)) : 256;
-  const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(waves / (T / 64), L.n_items));
-  hipLaunchKernelGGL((k_batch_lds<NS, T>), dim3(unsigned(wgs)), dim3(T), 0, L.stream, L.jobs,
-                     L.items, L.n_items, L.counter, L.flags);
-}
-
 // Groups above the LDS: `waves` / 4 persistent 256-thread workgroups (at least
 // one, at most one per item, at most kGlobalWorkspaceBytes of states), each
 // with its slice of a workspace allocated and freed in stream order.
@@ -4237,14 +3900,9 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
       case 4: launch_batch_group<4>(L, ref, sh, pe); break;
       case 5: launch_batch_group<5>(L, ref, sh, pe); break;
       case 6: launch_batch_group<6>(L, ref, sh, pe); break;
-      case 7: launch_batch_lds_group<7>(group_waves[ns], L); break;
-      case 8: launch_batch_lds_group<8>(group_waves[ns], L); break;
-      case 9: launch_batch_lds_group<9>(group_waves[ns], L); break;
-      case 10: launch_batch_lds_group<10>(group_waves[ns], L); break;
-      case 11: launch_batch_lds_group<11>(group_waves[ns], L); break;
-      case 12: launch_batch_lds_group<12>(group_waves[ns], L); break;
-      case 13: launch_batch_lds_group<13>(group_waves[ns], L); break;
-      case 14: launch_batch_lds_group<14>(group_waves[ns], L); break;
+      case 7: case 8: case 9: case 10: case 11: case 12: case 13: case 14:
+        e = launch_wide_batch(ns, pe, group_waves[ns], bt->d_jobs, items, n, counter, flags, gs);
+        break;
       case 15: e = launch_batch_global_group<15>(group_waves[ns], L, bt->gws[ns], bt->gws_wgs[ns]); break;
       case 16: e = launch_batch_global_group<16>(group_waves[ns], L, bt->gws[ns], bt->gws_wgs[ns]); break;
       case 17: e = launch_batch_global_group<17>(group_waves[ns], L, bt->gws[ns], bt->gws_wgs[ns]); break;
@@ -4298,14 +3956,22 @@ int mbqc_sv_forward_c64(const mbqc_plan* plan, const float* angles, int64_t angl
   hipError_t e = hipSuccess;
   const bool periodic = p->periodic && !(flags & MBQC_FLAG_TABLE_STEPS);
   if (p->ns > kMaxSvLdsSlots) {
-    // statevectors beyond the LDS: the LDS kernel's simulation on a global workspace
-    switch (p->ns) {
-      case 15: e = launch_sv_global<15>(J, flags, st); break;
-      case 16: e = launch_sv_global<16>(J, flags, st); break;
-      case 17: e = launch_sv_global<17>(J, flags, st); break;
-      case 18: e = launch_sv_global<18>(J, flags, st); break;
-      case 19: e = launch_sv_global<19>(J, flags, st); break;
-      case 20: e = launch_sv_global<20>(J, flags, st); break;
+    // statevectors beyond the LDS: passes over tiles of the state, or for
+    // plans off the slot rotation the LDS kernel's simulation on a workspace
+    if (p->rotating) {
+      const bool column = p->column_steps && !(flags & MBQC_FLAG_TABLE_STEPS);
+      e = run_global_chunks(J, wide_tile_bytes(p->ns), st, [&](float2* ws, int64_t g0, int64_t n) {
+        return launch_wide_tiles(J, column, flags, ws, g0, n, st);
+      });
+    } else {
+      switch (p->ns) {
+        case 15: e = launch_sv_global<15>(J, flags, st); break;
+        case 16: e = launch_sv_global<16>(J, flags, st); break;
+        case 17: e = launch_sv_global<17>(J, flags, st); break;
+        case 18: e = launch_sv_global<18>(J, flags, st); break;
+        case 19: e = launch_sv_global<19>(J, flags, st); break;
+        case 20: e = launch_sv_global<20>(J, flags, st); break;
+      }
     }
     return e == hipSuccess ? MBQC_OK : global_fail(e, "sv_forward launch (global workspace)");
   }
@@ -4336,14 +4002,7 @@ int mbqc_sv_forward_c64(const mbqc_plan* plan, const float* angles, int64_t angl
     case 4: e = launch_sv<4>(J, p->coef_per_step, periodic, flags, st); break;
     case 5: e = launch_sv<5>(J, p->coef_per_step, periodic, flags, st); break;
     case 6: e = launch_sv<6>(J, p->coef_per_step, periodic, flags, st); break;
-    case 7: e = launch_sv_lds<7>(J, flags, st); break;
-    case 8: e = launch_sv_lds<8>(J, flags, st); break;
-    case 9: e = launch_sv_lds<9>(J, flags, st); break;
-    case 10: e = launch_sv_lds<10>(J, flags, st); break;
-    case 11: e = launch_sv_lds<11>(J, flags, st); break;
-    case 12: e = launch_sv_lds<12>(J, flags, st); break;
-    case 13: e = launch_sv_lds<13>(J, flags, st); break;
-    case 14: e = launch_sv_lds<14>(J, flags, st); break;
+    default: e = launch_wide_sv(J, p->column_steps && !(flags & MBQC_FLAG_TABLE_STEPS), flags, st); break;
   }
   return e == hipSuccess ? MBQC_OK : hip_fail(e, "sv_forward launch");
 }
@@ -4374,14 +4033,11 @@ int mbqc_sv_sample_c64(const mbqc_plan* plan, const float* angles, int64_t angle
     case 4: e = launch_sample<4>(J, tab, o, outcomes, words, seed, p->periodic, st); break;
     case 5: e = launch_sample<5>(J, tab, o, outcomes, words, seed, p->periodic, st); break;
     case 6: e = launch_sample<6>(J, tab, o, outcomes, words, seed, p->periodic, st); break;
-    case 7: e = launch_sample_lds<7>(J, tab, o, outcomes, words, seed, st); break;
-    case 8: e = launch_sample_lds<8>(J, tab, o, outcomes, words, seed, st); break;
-    case 9: e = launch_sample_lds<9>(J, tab, o, outcomes, words, seed, st); break;
-    case 10: e = launch_sample_lds<10>(J, tab, o, outcomes, words, seed, st); break;
-    case 11: e = launch_sample_lds<11>(J, tab, o, outcomes, words, seed, st); break;
-    case 12: e = launch_sample_lds<12>(J, tab, o, outcomes, words, seed, st); break;
-    case 13: e = launch_sample_lds<13>(J, tab, o, outcomes, words, seed, st); break;
-    case 14: e = launch_sample_lds<14>(J, tab, o, outcomes, words, seed, st); break;
+    case 7: case 8: case 9: case 10: case 11: case 12: case 13: case 14:
+      e = launch_wide_sample(J, p->column_steps, reinterpret_cast<const uint64_t*>(tab + o.xmask),
+                             reinterpret_cast<const uint64_t*>(tab + o.zmask), tab + o.out_offset,
+                             outcomes, words, seed, st);
+      break;
     case 15: e = launch_sample_global<15>(J, tab, o, outcomes, words, seed, st); break;
     case 16: e = launch_sample_global<16>(J, tab, o, outcomes, words, seed, st); break;
     case 17: e = launch_sample_global<17>(J, tab, o, outcomes, words, seed, st); break;
@@ -4432,6 +4088,7 @@ int mbqc_sv_window_c64(const mbqc_plan* plan, const float* step_angles, int64_t 
                                      [&](float2* ws, int64_t g0, int64_t n) {
       hipLaunchKernelGGL(k_sv_window_global, dim3(unsigned(n)), dim3(256), 0, gst, J, step_angles,
                          step_stride, k, map, flags, ws, g0);
+      return hipGetLastError();
     });
     return e == hipSuccess ? MBQC_OK : global_fail(e, "sv_window launch (global workspace)");
   }
@@ -4467,6 +4124,7 @@ int mbqc_dm_window_c64(const mbqc_plan* plan, const float* step_angles, int64_t 
       else
         hipLaunchKernelGGL(k_dm_window_global, dim3(unsigned(n)), dim3(256), 0, gst, J,
                            step_angles, step_stride, k, map, nz, ws, g0);
+      return hipGetLastError();
     });
     return e == hipSuccess ? MBQC_OK : global_fail(e, "dm_window launch (global workspace)");
   }
@@ -4726,7 +4384,7 @@ int mbqc_batch_create(const mbqc_batch_job* jobs, int32_t n_jobs, int32_t sims_p
     bt->jobs.push_back(J);
     bt->max_ns = std::max(bt->max_ns, p->ns);
     if (p->ns < 2 || J.S % share_group(p->ns) != 0) bt->share[p->ns] = false;
-    if (!p->periodic) bt->periodic[p->ns] = false;
+    if (!p->column_steps) bt->periodic[p->ns] = false;
     const int64_t cost = int64_t(p->n_steps) << p->ns;
     for (int64_t f = 0; f < J.total; f += sims_per_item) {
       BatchItem it{};

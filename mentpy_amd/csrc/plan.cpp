@@ -301,11 +301,12 @@ int compile_plan(const mbqc_pattern_desc* d, Plan* p) {
       st.flags = (st.flags & 0xffffu) | (r << 16);
     }
   }
-  p->periodic = p->rotating && ns <= kMaxCoefSlots && nm > 0 && nm % ns == 0;
-  for (int k = 0; k < nm && p->periodic; ++k) {
+  p->column_steps = p->rotating && nm > 0 && nm % ns == 0;
+  for (int k = 0; k < nm && p->column_steps; ++k) {
     const mbqc_step& st = p->steps[k];
-    p->periodic = (st.flags & 3u) == 3u && st.nmask == periodic_nmask(ns, k % ns);
+    p->column_steps = (st.flags & 3u) == 3u && st.nmask == periodic_nmask(ns, k % ns);
   }
+  p->periodic = p->column_steps && ns <= kMaxCoefSlots;
   // Pauli-frame tables for sampled outcomes (PennyLane backend order,
   // pennylane_simulator.py:146-153): outcome 1 on schedule[k] flips the X
   // frame of its flow successor and the Z frame of the successor's neighbours

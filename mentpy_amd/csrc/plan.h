@@ -53,6 +53,9 @@ struct Plan {
   // neighbours periodic_nmask(ns, k % ns), and n_steps % ns == 0: the forward
   // kernel can take its coefficients at compile time
   bool periodic = false;
+  // the same step structure at any window size (the register-blocked kernels
+  // of wider windows take their CZ signs at compile time)
+  bool column_steps = false;
   // some angle-vector entry is used by more than one measured node: the
   // forward kernels allow it, the adjoint entry points reject it (each writes
   // one gradient entry per step)

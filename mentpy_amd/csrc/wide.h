@@ -1,0 +1,26 @@
+// Launchers of the register-blocked kernels for live windows of 7..20 slots
+// (wide.hip).  They need a plan whose
+// measured slots follow the rotation (Plan::rotating).
+#pragma once
+#include "device.h"
+
+namespace mbqc {
+
+// `column`: every step is that of a grid in column order (Plan::column_steps),
+// so the CZ signs are compile-time constants.
+hipError_t launch_wide_sv(const Job& J, bool column, uint32_t flags, hipStream_t st);
+// Windows of 15..20 slots: simulations [g0, g0 + n) in passes over tiles of
+// their states, in a workspace of n * wide_tile_bytes(ns) bytes.
+size_t wide_tile_bytes(int ns);
+hipError_t launch_wide_tiles(const Job& J, bool column, uint32_t flags, void* ws, int64_t g0,
+                             int64_t n, hipStream_t st);
+hipError_t launch_wide_sample(const Job& J, bool column, const uint64_t* xm, const uint64_t* zm,
+                              const int32_t* out_off, int32_t* outcomes, int32_t words,
+                              uint64_t seed, hipStream_t st);
+// One persistent launch over a batch's work items of window size ns with
+// `waves` resident wavefronts.
+hipError_t launch_wide_batch(int ns, bool column, int64_t waves, const Job* jobs,
+                             const BatchItem* items, int64_t n_items, int* counter, uint32_t flags,
+                             hipStream_t st);
+
+}  // namespace mbqc

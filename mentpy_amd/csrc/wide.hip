@@ -1,0 +1,660 @@
+// Statevector kernels for live windows of 7..14 slots (gfx950).
+//
+// The state of one simulation is spread over TL = 2^(NS - R) lanes with 2^R
+// amplitudes each in registers: amplitude v = r * TL + lane, r the register.
+// A block of NS steps measures the slots from the most significant to the
+// least, so the first steps of a block pair amplitudes of one lane: they are
+// register-only butterflies.  After M <= R of them the lanes exchange through
+// LDS so that the M slots just measured become the least significant bits
+// (v -> rotate-left(v, M)) and the next slots to measure are register bits
+// again.  A block is ceil(NS / R) such phases; after it the rotation is back
+// at slot order.  The LDS then carries every amplitude once per phase instead
+// of once per step, and a barrier (only where a simulation spans more than
+// one wave) stands between phases, not between steps.
+//
+// Sine, cosine and the reference phase are evaluated once per step, one step
+// per lane, for a chunk of whole blocks at a time, and read back as LDS
+// broadcasts.
+//
+// Bound by LDS bandwidth and VALU issue about equally: a block of the 9-slot
+// loop is 232 VALU and 41 LDS instructions per wave.  9x10 grid, 4,099
+// simulations: 103.6 us with one LDS pass and one barrier per step, 28.4 us so.
+#include "wide.h"
+
+#include <algorithm>
+#include <utility>
+
+namespace mbqc {
+
+namespace {
+
+// Register bits R by window size.  More of them mean fewer exchanges, fewer
+// mean more lanes per simulation and more waves in flight.  Measured (us per
+// call of 4,096 simulations of a 10-column grid, R = 2 / 3 / 4 / 5): 9 slots
+// 43 / 31 / 33 / 40, 10 slots 79 / 62 / 53 / 54, 11 slots (6 columns) 112 / 75 /
+// 63 / 74; from 12 slots on 4 is at least as good as 5.
+constexpr int wide_reg_bits(int ns) { return ns <= 9 ? 3 : 4; }
+
+// NS amplitude bits over lanes and registers, M of them measured per block
+// (all of them except in a pass over tiles of a larger state).
+template <int NS, int R, int M = NS>
+struct Wide {
+  static constexpr int TL = 1 << (NS - R);        // lanes per simulation
+  static constexpr int T = TL > 64 ? TL : 64;     // threads per workgroup
+  static constexpr int G = T / TL;                // simulations per workgroup
+  static constexpr int NR = 1 << R;               // amplitudes per lane
+  static constexpr int P = (M + R - 1) / R;       // phases per block
+  static constexpr int CS = M == NS ? (64 / NS) * NS : M;   // steps per coefficient chunk
+  static constexpr int BUF = (1 << NS) + (1 << NS) / 16;   // padded exchange buffer
+  static constexpr int SIM = BUF + CS;            // float2 of LDS per simulation
+  static constexpr int len(int p) { return M / P + (p < M % P ? 1 : 0); }
+  static constexpr int first(int p) {
+    int f = 0;
+    for (int i = 0; i < p; ++i) f += len(i);
+    return f;
+  }
+};
+
+// Makes the LDS writes of a simulation's lanes visible to all of them: a
+// barrier where it spans several waves, else only an order within the wave.
+template <int T>
+__device__ __forceinline__ void lanes_sync() {
+  if constexpr (T > 64) {
+    __syncthreads();
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+__device__ __forceinline__ int padded(int a) { return a + (a >> 4); }
+
+// CZ neighbours of the qubit appended by a step, as a mask over the amplitude
+// bits at the block's start, and the sign (bit 31) that amplitude bits outside
+// the workgroup's tile contribute.
+struct StepSigns {
+  uint32_t mask, outer;
+};
+struct SlotSigns {
+  __device__ __forceinline__ StepSigns operator()(const mbqc_step& st) const { return {st.nmask, 0u}; }
+};
+
+// Step FIRST + S of a block on its phase's register bit R - 1 - S.
+template <int NS, int R, int FIRST, int S, bool COLUMN, typename Signs>
+__device__ __forceinline__ void wide_step(float2 (&t)[1 << R], float2 b, const mbqc_step* steps,
+                                          int k, int lane, bool top, const Signs& signs) {
+  constexpr int NR = 1 << R, QB = 1 << (R - 1 - S);
+  constexpr int TL = 1 << (NS - R);
+  if constexpr (COLUMN) {
+    // the appended qubit's other neighbour is the one appended a step
+    // earlier: no one at the column's first step (`top`), lane bit 0 at the
+    // first step of a later phase, else the register bit above the measured one
+    const float sg = (S == 0 && !top && (lane & 1)) ? -1.0f : 1.0f;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if (r & QB) continue;
+      const float2 x = t[r], y = t[r | QB];
+      float2 u0;
+      u0.x = fmaf(-b.y, y.y, fmaf(b.x, y.x, x.x));
+      u0.y = fmaf(b.x, y.y, fmaf(b.y, y.x, x.y));
+      t[r] = u0;
+      if constexpr (S == 0) {
+        const float be = 2.0f * sg;
+        t[r | QB] = make_float2(fmaf(be, x.x, -sg * u0.x), fmaf(be, x.y, -sg * u0.y));
+      } else if (r & (QB << 1)) {
+        t[r | QB] = make_float2(fmaf(-2.0f, x.x, u0.x), fmaf(-2.0f, x.y, u0.y));
+      } else {
+        t[r | QB] = make_float2(fmaf(2.0f, x.x, -u0.x), fmaf(2.0f, x.y, -u0.y));
+      }
+    }
+  } else {
+    const mbqc_step st = steps[k];
+    const float s = (st.flags & 2u) ? -1.0f : 1.0f;
+    const float app = (st.flags & 1u) ? 1.0f : 0.0f;
+    // the neighbour mask in the phase's amplitude order (rotated by FIRST)
+    const StepSigns z = signs(st);
+    const uint32_t m = ((z.mask << FIRST) | (z.mask >> (NS - FIRST))) & ((1u << NS) - 1);
+    const uint32_t lane_sign = czbit(uint32_t(lane), m & uint32_t(TL - 1)) ^ z.outer;
+    const uint32_t mr = m >> (NS - R);
+#pragma unroll
+    for (int r = 0; r < NR; ++r) {
+      if (r & QB) continue;
+      const float c = __uint_as_float(__float_as_uint(app) ^ lane_sign ^ czbit(uint32_t(r), mr));
+      const float al = c * s, be = c * (1.0f - s);
+      const float2 x = t[r], y = t[r | QB];
+      float2 u0;
+      u0.x = fmaf(-b.y, y.y, fmaf(b.x, y.x, x.x));
+      u0.y = fmaf(b.x, y.y, fmaf(b.y, y.x, x.y));
+      t[r] = u0;
+      t[r | QB] = make_float2(fmaf(al, u0.x, be * x.x), fmaf(al, u0.y, be * x.y));
+    }
+  }
+}
+
+// v -> rotate-left(v, M): the top M bits of v (register bits) become the lowest.
+template <int NS, int R, int M, int T>
+__device__ __forceinline__ void wide_rotate(float2 (&t)[1 << R], float2* buf, int lane) {
+  constexpr int NR = 1 << R;
+  lanes_sync<T>();   // earlier reads of the buffer are done
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const int top = r >> (R - M), low = r & ((1 << (R - M)) - 1);
+    buf[padded((low << (NS - R + M)) | (lane << M) | top)] = t[r];
+  }
+  lanes_sync<T>();
+#pragma unroll
+  for (int r = 0; r < NR; ++r) t[r] = buf[padded((r << (NS - R)) | lane)];
+}
+
+// `top`: the block starts a column (a compile-time fact except in tile passes).
+template <int NS, int R, int M, int P, bool COLUMN, typename Mod, typename Signs, int... SS>
+__device__ __forceinline__ void wide_phase(float2 (&t)[1 << R], float2* buf, const float2* bs,
+                                           const mbqc_step* steps, int k0, int n, int lane, bool top,
+                                           Mod& mod, const Signs& signs,
+                                           std::integer_sequence<int, SS...>) {
+  using W = Wide<NS, R, M>;
+  constexpr int F = W::first(P);
+  // a column plan has only full blocks
+  ((COLUMN || k0 + F + SS < n
+        ? wide_step<NS, R, F, SS, COLUMN>(t, mod(k0 + F + SS, bs[F + SS]), steps, k0 + F + SS, lane,
+                                          F == 0 && top, signs)
+        : void()),
+   ...);
+  wide_rotate<NS, R, W::len(P), W::T>(t, buf, lane);
+}
+
+template <int NS, int R, int M, bool COLUMN, typename Mod, typename Signs, int... PS>
+__device__ __forceinline__ void wide_block(float2 (&t)[1 << R], float2* buf, const float2* bs,
+                                           const mbqc_step* steps, int k0, int n, int lane, bool top,
+                                           Mod& mod, const Signs& signs,
+                                           std::integer_sequence<int, PS...>) {
+  (wide_phase<NS, R, M, PS, COLUMN>(t, buf, bs, steps, k0, n, lane, top, mod, signs,
+                                    std::make_integer_sequence<int, Wide<NS, R, M>::len(PS)>{}),
+   ...);
+}
+
+// e^{-i theta} of the chunk of steps [k0, k0 + CS), one step per lane.
+template <int NS, int R, bool REF, int M = NS>
+__device__ __forceinline__ void wide_coeffs(float2* bs, const mbqc_step* steps, const float* ang,
+                                            int64_t sa, int k0, int n, int lane, RefPhase* ph) {
+  using W = Wide<NS, R, M>;
+#pragma unroll 1
+  for (int i = lane; i < W::CS; i += W::TL) {
+    const int k = k0 + i;
+    if (k < n) bs[i] = step_coeff<REF>(step_angle(steps[k], ang, sa), ph);
+  }
+}
+
+// All steps of one simulation; `on_block(blk, t)` runs at the start of every
+// block (after its rescale).
+template <int NS, int R, bool REF, bool COLUMN, typename OnBlock, typename Mod>
+__device__ __forceinline__ void wide_run(float2 (&t)[1 << R], const Job& J, const float* ang,
+                                         float2* buf, float2* bs, int lane, RefPhase* ph,
+                                         OnBlock on_block, Mod&& mod) {
+  using W = Wide<NS, R>;
+  const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
+  const int32_t* resc = J.tab + J.off_svres;
+  const int n = J.n_steps;
+  for (int kc = 0; kc < n; kc += W::CS) {
+    // the previous chunk's last read came before its last exchange
+    wide_coeffs<NS, R, REF>(bs, steps, ang, J.angle_stride_a, kc, n, lane, ph);
+    lanes_sync<W::T>();
+    const int ke = kc + W::CS < n ? kc + W::CS : n;
+    for (int k0 = kc; k0 < ke; k0 += NS) {
+      if (resc[k0 / NS]) {
+#pragma unroll
+        for (int r = 0; r < W::NR; ++r) t[r] = cscale(t[r], 0x1p-32f);
+      }
+      on_block(k0 / NS, t);
+      wide_block<NS, R, NS, COLUMN>(t, buf, bs + (k0 - kc), steps, k0, n, lane, true, mod,
+                                    SlotSigns(), std::make_integer_sequence<int, W::P>{});
+    }
+  }
+}
+
+template <int NS, int R>
+__device__ __forceinline__ void wide_load(float2 (&t)[1 << R], const Job& J, int64_t si, int lane) {
+  const int32_t* in_index = J.tab + J.off_in;
+  const int32_t* sign = J.tab + J.off_sign;
+  const float2* psi = J.psi + si * J.in_stride;
+#pragma unroll
+  for (int r = 0; r < (1 << R); ++r) {
+    const int j = (r << (NS - R)) | lane;
+    t[r] = flip(psi[in_index[j]], sign[j] ? 0x80000000u : 0u);
+  }
+}
+
+// Sum over a simulation's lanes; `red`: LDS of T / 64 values, used where it
+// spans several waves.
+template <int NS, int R, typename V>
+__device__ __forceinline__ V lanes_sum(V v, V* red) {
+  using W = Wide<NS, R>;
+#pragma unroll
+  for (int m = (W::TL < 64 ? W::TL : 64) / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+  if constexpr (W::T > 64) {
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = red[0];
+#pragma unroll
+    for (int i = 1; i < W::T / 64; ++i) v += red[i];
+  }
+  return v;
+}
+
+// 1 / norm of the state over the output amplitudes (those with out_pos >= 0).
+template <int NS, int R>
+__device__ __forceinline__ float wide_inv_norm(const float2 (&t)[1 << R], const int32_t* out_pos,
+                                               int lane, void* red) {
+  float n2 = 0.0f;
+#pragma unroll
+  for (int r = 0; r < (1 << R); ++r)
+    if (out_pos[(r << (NS - R)) | lane] >= 0) n2 = fmaf(t[r].x, t[r].x, fmaf(t[r].y, t[r].y, n2));
+  return 1.0f / sqrtf(lanes_sum<NS, R>(n2, static_cast<float*>(red)));
+}
+
+// Simulation g of job J on the lanes of one group (inactive groups run the
+// last simulation and store nothing).
+template <int NS, int R, bool REF, bool COLUMN>
+__device__ __forceinline__ void wide_sim(const Job& J, int64_t g, bool active, uint32_t flags,
+                                         float2* buf, float2* bs, int lane) {
+  using W = Wide<NS, R>;
+  const int64_t gg = active ? g : J.total - 1;
+  int64_t bi, si;
+  split_sim(J, gg, &bi, &si);
+  float2 t[W::NR];
+  wide_load<NS, R>(t, J, si, lane);
+  RefPhase rp;
+  wide_run<NS, R, REF, COLUMN>(t, J, J.angles + bi * J.angle_stride, buf, bs, lane, &rp,
+                               [](int, const float2 (&)[W::NR]) {}, NoModify());
+  if constexpr (REF) {
+    rp.m_sum = lanes_sum<NS, R>(rp.m_sum, reinterpret_cast<int32_t*>(bs));
+    rp.th_sum = lanes_sum<NS, R>(rp.th_sum, reinterpret_cast<double*>(bs));
+  }
+  const float2 ph = REF ? rp.value() : make_float2(1.0f, 0.0f);
+  const int32_t* out_pos = J.tab + J.off_out;
+  const float scale = (flags & MBQC_FLAG_RENORMALIZE) ? wide_inv_norm<NS, R>(t, out_pos, lane, bs)
+                                                      : sv_final_scale(J.e_sv);
+  const float2 f = cscale(ph, scale);
+  if (active) {
+    float2* o = J.out + g * (int64_t(1) << J.n_out);
+#pragma unroll
+    for (int r = 0; r < W::NR; ++r) {
+      const int p = out_pos[(r << (NS - R)) | lane];
+      if (p >= 0) o[p] = cmul(t[r], f);
+    }
+    if (lane == 0 && (flags & MBQC_FLAG_WRITE_PHASE) && J.phase_out) J.phase_out[g] = ph;
+  }
+}
+
+template <int NS, int R, bool REF, bool COLUMN>
+__global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_sv(Job J, uint32_t flags) {
+  using W = Wide<NS, R>;
+  __shared__ float2 lds[W::G * W::SIM];
+  const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
+  float2* buf = lds + sub * W::SIM;
+  const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
+  wide_sim<NS, R, REF, COLUMN>(J, g, g < J.total, flags, buf, buf + W::BUF, lane);
+}
+
+// Sampled outcomes: the frame and draws of SampleMod, evaluated identically by
+// every lane of a simulation; one lane writes the outcome words.
+template <int NS, int R, bool COLUMN>
+__global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_sample(
+    Job J, const uint64_t* __restrict__ xm, const uint64_t* __restrict__ zm,
+    const int32_t* __restrict__ out_off, int32_t* __restrict__ outcomes, int32_t words,
+    uint64_t seed) {
+  using W = Wide<NS, R>;
+  __shared__ float2 lds[W::G * W::SIM];
+  const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
+  float2* buf = lds + sub * W::SIM;
+  float2* bs = buf + W::BUF;
+  const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
+  const bool active = g < J.total;
+  const int64_t gg = active ? g : J.total - 1;
+  int64_t bi, si;
+  split_sim(J, gg, &bi, &si);
+  float2 t[W::NR];
+  wide_load<NS, R>(t, J, si, lane);
+  int32_t* row = outcomes + gg * (words + 2);
+  SampleMod mod;
+  mod.seed = seed;
+  mod.sim = uint64_t(gg);
+  mod.xm = xm;
+  mod.zm = zm;
+  mod.n = J.n_steps;
+  mod.out_words = active && lane == 0 ? row : nullptr;
+  RefPhase ph;
+  wide_run<NS, R, false, COLUMN>(t, J, J.angles + bi * J.angle_stride, buf, bs, lane, &ph,
+                                 [](int, const float2 (&)[W::NR]) {}, mod);
+  uint32_t xo = 0, zo = 0;
+  for (int m = 0; m < J.n_out; ++m) {
+    const int off = out_off[m];
+    xo |= ((mod.fx >> off) & 1u) << (J.n_out - 1 - m);
+    zo |= ((mod.fz >> off) & 1u) << (J.n_out - 1 - m);
+  }
+  const int32_t* out_pos = J.tab + J.off_out;
+  const float scale = wide_inv_norm<NS, R>(t, out_pos, lane, bs);
+  if (!active) return;
+  float2* o = J.out + g * (int64_t(1) << J.n_out);
+#pragma unroll
+  for (int r = 0; r < W::NR; ++r) {
+    const int p = out_pos[(r << (NS - R)) | lane];
+    if (p >= 0) {
+      const uint32_t q = uint32_t(p) ^ xo;
+      o[q] = flip(cscale(t[r], scale), czbit(q, zo));
+    }
+  }
+  if (lane == 0) {
+    row[words] = int32_t(xo);
+    row[words + 1] = int32_t(zo);
+  }
+}
+
+// Batched groups: a persistent workgroup pulls items from the group's counter
+// and runs their simulations, G at a time.  Every thread reads the item index
+// from LDS, so all leave the loop together once the counter passes n_items.
+template <int NS, int R, bool REF, bool COLUMN>
+__global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_batch(
+    const Job* __restrict__ jobs, const BatchItem* __restrict__ items, int64_t n_items, int* counter,
+    uint32_t flags) {
+  using W = Wide<NS, R>;
+  __shared__ float2 lds[W::G * W::SIM];
+  __shared__ int item_s;
+  const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
+  float2* buf = lds + sub * W::SIM;
+  for (;;) {
+    __syncthreads();   // the previous item's last reads of item_s and the buffers are done
+    if (threadIdx.x == 0) item_s = atomicAdd(counter, 1);
+    __syncthreads();
+    const int it = item_s;
+    if (it >= n_items) break;
+    const BatchItem I = items[it];
+    const Job J = load_job(jobs, I.job);
+    const int64_t end = std::min<int64_t>(I.first + I.count, J.total);
+    for (int64_t g = I.first; g < end; g += W::G) {
+      __syncthreads();
+      wide_sim<NS, R, REF, COLUMN>(J, g + sub, g + sub < end, flags, buf, buf + W::BUF, lane);
+    }
+  }
+}
+
+// ---------------------------------------------------------------- tile passes
+// Windows of 15..20 slots: the state is cut into tiles of 2^kTileBits
+// amplitudes and a pass runs M steps on every tile, one workgroup each, so
+// that a single simulation already spreads over 2^(ns - kTileBits) workgroups
+// (one workgroup walking the whole state is bound by its own memory latency).
+// With v the amplitude in the current rotation (the next slots to measure are
+// its top bits) a tile holds all values of the top M bits and of the lowest
+// kTileBits - M bits; the other bits (`mid`) name the tile.  It reads runs of
+// 2^(kTileBits - M) amplitudes and, as rotate-left(v, M) puts the measured
+// bits lowest, writes one contiguous run.  The passes alternate between two
+// buffers; the first reads the input, the last leaves the output unscaled and
+// one partial norm per tile, which k_tile_finish applies.  With few simulations
+// the passes are bound by their own launch and memory latency (5-9 us each, six
+// of them for three columns of 16 slots): 16x4 grid, 4 simulations, 1,470 us
+// with one workgroup per simulation, 61 us so.
+constexpr int kTileBits = 12;
+constexpr int kTileRegBits = 4;
+
+struct TileSigns {
+  int ns, m, sub;
+  uint32_t mid;
+  __device__ __forceinline__ StepSigns operator()(const mbqc_step& st) const {
+    const int c = kTileBits - m;
+    const uint32_t all = (1u << ns) - 1;
+    const uint32_t v = sub ? ((st.nmask << sub) | (st.nmask >> (ns - sub))) & all : st.nmask;
+    const uint32_t low = v & ((1u << c) - 1), top = v >> (ns - m);
+    const uint32_t outer = (v >> c) & ((1u << (ns - kTileBits)) - 1);
+    return {(top << c) | low, czbit(mid, outer)};
+  }
+};
+
+// One pass: steps [k0, k0 + M) of simulations g0 + blockIdx / tiles; `sub`: the
+// rotation before it (k0 % ns).  in == nullptr: the first pass (the input
+// state); `last`: the output and its partial norms.
+template <int M, bool COLUMN>
+__global__ __launch_bounds__((Wide<kTileBits, kTileRegBits>::T)) void k_tile_pass(
+    Job J, const float2* __restrict__ in, float2* __restrict__ out, float* __restrict__ norms,
+    int64_t g0, int k0, int sub, int last) {
+  using W = Wide<kTileBits, kTileRegBits, M>;
+  constexpr int C = kTileBits - M;
+  __shared__ float2 buf[W::BUF];
+  __shared__ float2 bs[M];
+  __shared__ float red[W::T / 64];
+  const int lane = threadIdx.x;
+  const int tile_bits = J.ns - kTileBits;
+  const int64_t l = int64_t(blockIdx.x) >> tile_bits;          // simulation of this launch
+  const uint32_t mid = blockIdx.x & ((1u << tile_bits) - 1);
+  const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
+  const int32_t* resc = J.tab + J.off_svres;
+  int64_t bi, si;
+  split_sim(J, g0 + l, &bi, &si);
+  float2 t[W::NR];
+  const int64_t state = l << J.ns;
+#pragma unroll
+  for (int r = 0; r < W::NR; ++r) {
+    const int u = r * W::TL + lane;
+    const int v = ((u >> C) << (J.ns - M)) | int(mid << C) | (u & ((1 << C) - 1));
+    if (in) {
+      t[r] = in[state + v];
+    } else {
+      const int32_t* in_index = J.tab + J.off_in;
+      const int32_t* sign = J.tab + J.off_sign;
+      t[r] = flip(J.psi[si * J.in_stride + in_index[v]], sign[v] ? 0x80000000u : 0u);
+    }
+  }
+  wide_coeffs<kTileBits, kTileRegBits, false, M>(bs, steps, J.angles + bi * J.angle_stride,
+                                                 J.angle_stride_a, k0, J.n_steps, lane, nullptr);
+  __syncthreads();
+  if (sub == 0 && resc[k0 / J.ns]) {
+#pragma unroll
+    for (int r = 0; r < W::NR; ++r) t[r] = cscale(t[r], 0x1p-32f);
+  }
+  NoModify mod;
+  wide_block<kTileBits, kTileRegBits, M, COLUMN>(t, buf, bs, steps, k0, J.n_steps, lane, sub == 0,
+                                                 mod, TileSigns{J.ns, M, sub, mid},
+                                                 std::make_integer_sequence<int, W::P>{});
+  const int base = int(mid << kTileBits);
+  if (!last) {
+#pragma unroll
+    for (int r = 0; r < W::NR; ++r) out[state + base + r * W::TL + lane] = t[r];
+    return;
+  }
+  const int32_t* out_pos = J.tab + J.off_out;
+  float2* o = J.out + (g0 + l) * (int64_t(1) << J.n_out);
+  float n2 = 0.0f;
+#pragma unroll
+  for (int r = 0; r < W::NR; ++r) {
+    const int p = out_pos[base + r * W::TL + lane];
+    if (p >= 0) {
+      o[p] = t[r];
+      n2 = fmaf(t[r].x, t[r].x, fmaf(t[r].y, t[r].y, n2));
+    }
+  }
+  n2 = lanes_sum<kTileBits, kTileRegBits>(n2, red);
+  if (lane == 0) norms[blockIdx.x] = n2;
+}
+
+// Phase and scale of the outputs a last pass left: workgroup (x, y) takes
+// 1,024 amplitudes of simulation g0 + y.
+__global__ __launch_bounds__(256) void k_tile_finish(Job J, const float* __restrict__ norms,
+                                                     int64_t g0, uint32_t flags) {
+  __shared__ float red_f[4];
+  __shared__ double red_d[4];
+  __shared__ int32_t red_i[4];
+  const int tid = threadIdx.x;
+  const int tiles = 1 << (J.ns - kTileBits);
+  const int64_t l = blockIdx.y, g = g0 + l;
+  const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
+  float2 ph = make_float2(1.0f, 0.0f);
+  if (flags & MBQC_FLAG_REF_PHASE) {
+    int64_t bi, si;
+    split_sim(J, g, &bi, &si);
+    const float* ang = J.angles + bi * J.angle_stride;
+    RefPhase rp;
+    for (int k = tid; k < J.n_steps; k += 256) rp.add(step_angle(steps[k], ang, J.angle_stride_a));
+    rp.m_sum = lanes_sum<kTileBits, kTileRegBits>(rp.m_sum, red_i);
+    rp.th_sum = lanes_sum<kTileBits, kTileRegBits>(rp.th_sum, red_d);
+    ph = rp.value();
+  }
+  float scale = sv_final_scale(J.e_sv);
+  if (flags & MBQC_FLAG_RENORMALIZE) {
+    float n2 = 0.0f;
+    for (int i = tid; i < tiles; i += 256) n2 += norms[l * tiles + i];
+    scale = 1.0f / sqrtf(lanes_sum<kTileBits, kTileRegBits>(n2, red_f));
+  }
+  const float2 f = cscale(ph, scale);
+  const int64_t dout = int64_t(1) << J.n_out;
+  float2* o = J.out + g * dout;
+  const int64_t e0 = int64_t(blockIdx.x) * 1024;
+  for (int64_t e = e0 + tid; e < e0 + 1024 && e < dout; e += 256) o[e] = cmul(o[e], f);
+  if (blockIdx.x == 0 && tid == 0 && (flags & MBQC_FLAG_WRITE_PHASE) && J.phase_out)
+    J.phase_out[g] = ph;
+}
+
+template <int M>
+void tile_pass(const Job& J, bool column, const float2* in, float2* out, float* norms, int64_t g0,
+               int64_t n, int k0, int sub, int last, hipStream_t st) {
+  const dim3 grid(unsigned(n << (J.ns - kTileBits)));
+  const dim3 block(Wide<kTileBits, kTileRegBits>::T);
+  if (column)
+    hipLaunchKernelGGL((k_tile_pass<M, true>), grid, block, 0, st, J, in, out, norms, g0, k0, sub,
+                       last);
+  else
+    hipLaunchKernelGGL((k_tile_pass<M, false>), grid, block, 0, st, J, in, out, norms, g0, k0, sub,
+                       last);
+}
+
+template <int NS>
+hipError_t sv_launch(const Job& J, bool column, uint32_t flags, hipStream_t st) {
+  constexpr int R = wide_reg_bits(NS);
+  using W = Wide<NS, R>;
+  const dim3 grid(unsigned((J.total + W::G - 1) / W::G)), block(W::T);
+  const bool ref = flags & MBQC_FLAG_REF_PHASE;
+  if (column) {
+    if (ref) hipLaunchKernelGGL((k_wide_sv<NS, R, true, true>), grid, block, 0, st, J, flags);
+    else hipLaunchKernelGGL((k_wide_sv<NS, R, false, true>), grid, block, 0, st, J, flags);
+  } else {
+    if (ref) hipLaunchKernelGGL((k_wide_sv<NS, R, true, false>), grid, block, 0, st, J, flags);
+    else hipLaunchKernelGGL((k_wide_sv<NS, R, false, false>), grid, block, 0, st, J, flags);
+  }
+  return hipGetLastError();
+}
+
+template <int NS>
+hipError_t sample_launch(const Job& J, bool column, const uint64_t* xm, const uint64_t* zm,
+                         const int32_t* out_off, int32_t* outcomes, int32_t words, uint64_t seed,
+                         hipStream_t st) {
+  constexpr int R = wide_reg_bits(NS);
+  using W = Wide<NS, R>;
+  const dim3 grid(unsigned((J.total + W::G - 1) / W::G)), block(W::T);
+  if (column)
+    hipLaunchKernelGGL((k_wide_sample<NS, R, true>), grid, block, 0, st, J, xm, zm, out_off, outcomes,
+                       words, seed);
+  else
+    hipLaunchKernelGGL((k_wide_sample<NS, R, false>), grid, block, 0, st, J, xm, zm, out_off,
+                       outcomes, words, seed);
+  return hipGetLastError();
+}
+
+template <int NS>
+hipError_t batch_launch(bool column, int64_t waves, const Job* jobs, const BatchItem* items,
+                        int64_t n_items, int* counter, uint32_t flags, hipStream_t st) {
+  constexpr int R = wide_reg_bits(NS);
+  using W = Wide<NS, R>;
+  const int64_t wgs = std::max<int64_t>(1, std::min<int64_t>(waves / (W::T / 64), n_items));
+  const dim3 grid{unsigned(wgs)}, block(W::T);
+  const bool ref = flags & MBQC_FLAG_REF_PHASE;
+#define MBQC_WIDE_BATCH(REF, COL)                                                                \
+  hipLaunchKernelGGL((k_wide_batch<NS, R, REF, COL>), grid, block, 0, st, jobs, items, n_items, \
+                     counter, flags)
+  if (column) {
+    if (ref) MBQC_WIDE_BATCH(true, true);
+    else MBQC_WIDE_BATCH(false, true);
+  } else {
+    if (ref) MBQC_WIDE_BATCH(true, false);
+    else MBQC_WIDE_BATCH(false, false);
+  }
+#undef MBQC_WIDE_BATCH
+  return hipGetLastError();
+}
+
+}  // namespace
+
+#define MBQC_WIDE_SWITCH(ns, CALL)        \
+  switch (ns) {                           \
+    case 7: return CALL(7);               \
+    case 8: return CALL(8);               \
+    case 9: return CALL(9);               \
+    case 10: return CALL(10);             \
+    case 11: return CALL(11);             \
+    case 12: return CALL(12);             \
+    case 13: return CALL(13);             \
+    case 14: return CALL(14);             \
+    default: return hipErrorInvalidValue; \
+  }
+
+hipError_t launch_wide_sv(const Job& J, bool column, uint32_t flags, hipStream_t st) {
+#define MBQC_CALL(NS) sv_launch<NS>(J, column, flags, st)
+  MBQC_WIDE_SWITCH(J.ns, MBQC_CALL)
+#undef MBQC_CALL
+}
+
+size_t wide_tile_bytes(int ns) {
+  return 2 * (sizeof(float2) << ns) + (sizeof(float) << (ns - kTileBits));
+}
+
+hipError_t launch_wide_tiles(const Job& J, bool column, uint32_t flags, void* ws, int64_t g0,
+                             int64_t n, hipStream_t st) {
+  float2* a = static_cast<float2*>(ws);
+  float2* b = a + (n << J.ns);
+  float* norms = reinterpret_cast<float*>(b + (n << J.ns));
+  // passes of at most 8 steps, of near equal length within a block
+  const int per = (J.ns + 7) / 8;
+  const float2* in = nullptr;
+  for (int blk = 0; blk * J.ns < J.n_steps; ++blk) {
+    int sub = 0;
+    for (int p = 0; p < per; ++p) {
+      const int m = J.ns / per + (p < J.ns % per ? 1 : 0);
+      const int k0 = blk * J.ns + sub;
+      // after the last block's last pass the rotation is back at slot order
+      const int last = p + 1 == per && (blk + 1) * J.ns >= J.n_steps;
+      float2* out = in == a ? b : a;
+      switch (m) {
+        case 5: tile_pass<5>(J, column, in, out, norms, g0, n, k0, sub, last, st); break;
+        case 6: tile_pass<6>(J, column, in, out, norms, g0, n, k0, sub, last, st); break;
+        case 7: tile_pass<7>(J, column, in, out, norms, g0, n, k0, sub, last, st); break;
+        case 8: tile_pass<8>(J, column, in, out, norms, g0, n, k0, sub, last, st); break;
+        default: return hipErrorInvalidValue;
+      }
+      in = out;
+      sub += m;
+    }
+  }
+  const unsigned chunks = unsigned(((int64_t(1) << J.n_out) + 1023) / 1024);
+  for (int64_t y = 0; y < n; y += 65535) {   // grid rows are limited to 65,535
+    const unsigned ny = unsigned(std::min<int64_t>(n - y, 65535));
+    hipLaunchKernelGGL(k_tile_finish, dim3(chunks, ny), dim3(256), 0, st, J,
+                       norms + (y << (J.ns - kTileBits)), g0 + y, flags);
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_wide_sample(const Job& J, bool column, const uint64_t* xm, const uint64_t* zm,
+                              const int32_t* out_off, int32_t* outcomes, int32_t words,
+                              uint64_t seed, hipStream_t st) {
+#define MBQC_CALL(NS) sample_launch<NS>(J, column, xm, zm, out_off, outcomes, words, seed, st)
+  MBQC_WIDE_SWITCH(J.ns, MBQC_CALL)
+#undef MBQC_CALL
+}
+
+hipError_t launch_wide_batch(int ns, bool column, int64_t waves, const Job* jobs,
+                             const BatchItem* items, int64_t n_items, int* counter, uint32_t flags,
+                             hipStream_t st) {
+#define MBQC_CALL(NS) batch_launch<NS>(column, waves, jobs, items, n_items, counter, flags, st)
+  MBQC_WIDE_SWITCH(ns, MBQC_CALL)
+#undef MBQC_CALL
+}
+
+}  // namespace mbqc

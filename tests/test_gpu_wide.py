@@ -1,0 +1,54 @@
+"""Register-blocked statevector kernels of 7..20-slot windows: every window
+size (its own split over lanes, registers and LDS exchanges), plans off the
+grid's column structure, partly filled last workgroups, against the
+complex128 oracle; compile-time and table step forms bit-identical."""
+import numpy as np
+import pytest
+
+from conftest import haar_state
+
+pytestmark = pytest.mark.gpu
+
+
+def _torch():
+    import torch
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    return torch
+
+
+# (rows, cols, window, angle vectors, inputs): the default window is rows + 1;
+# a wider one gives a plan with rows + 1 live slots whose steps are not a
+# column's.  Batches leave a partly filled last workgroup where several
+# simulations share one; 7x12 crosses a coefficient chunk and a rescale.
+CASES = [(7, 12, None, 5, 3), (8, 4, None, 3, 1), (9, 5, None, 1, 1), (9, 4, None, 7, 2),
+         (10, 3, None, 2, 1), (11, 3, None, 1, 2), (12, 3, None, 1, 1), (13, 3, None, 1, 1),
+         (14, 3, None, 1, 1), (15, 3, None, 2, 1), (16, 3, None, 1, 2), (17, 3, None, 1, 1), (19, 3, None, 1, 1),
+         (6, 5, 8, 5, 1), (7, 4, 9, 3, 3), (8, 4, 10, 2, 1), (9, 3, 11, 1, 2), (14, 3, 16, 1, 1),
+         (15, 3, 17, 1, 1)]
+
+
+@pytest.mark.parametrize("rows,cols,window,B,S", CASES)
+def test_wide_windows_match_oracle(rows, cols, window, B, S, rng):
+    torch = _torch()
+    import mentpy_amd as mp
+    from mentpy_amd.simulators.hip_simulator import sv_forward, _as_angles, _as_states
+    from oracle.vectorized import sv_batch
+    g = mp.templates.grid_cluster(rows, cols)
+    sim = mp.PatternSimulator(g, backend="hip-sv", **({"window_size": window} if window else {}))
+    plan = sim.simulator.plan
+    assert plan.info["n_slots"] == (window - 1 if window else rows)
+    th = rng.uniform(-7, 7, (B, len(g.trainable_nodes))).astype(np.float32)
+    psi = np.stack([haar_state(rows, rng) for _ in range(S)])
+    dev = torch.device("cuda")
+    a, s = _as_angles(th, plan.info["n_angles"], dev), _as_states(psi, plan.info["n_inputs"], dev)
+    guard = torch.full((B + 1, S, 1 << rows), 7.0, dtype=torch.complex64, device=dev)
+    out = sv_forward(plan, a, s, out=guard[:B])
+    table = sv_forward(plan, a, s, table_steps=True)
+    torch.cuda.synchronize()
+    assert torch.equal(out, table), "compile-time and table steps differ"
+    assert (guard[B] == 7.0).all(), "a store past the last simulation"
+    ref = sv_batch(g, th.astype(np.float64), psi)
+    err = np.abs(out.cpu().numpy() - ref).max()
+    # complex64 butterflies: each step adds about one rounding (6e-8) to amplitudes below 1
+    assert err < 2e-5, f"amplitude error {err}"
