@@ -1652,8 +1652,9 @@ __global__ __launch_bounds__(64) void k_sv_adj_backward(Job J, const float2* __r
 }
 
 // ---------------------------------------------------- adjoint, LDS-resident
-// Windows of 6..kMaxAdjLdsSlots live slots: one workgroup per simulation in
-// the forward, the state in LDS (as k_sv_forward_lds, raw phase), a
+// Windows of 6..kMaxAdjLdsSlots live slots of plans that are no column plans
+// (those run the register-blocked sweeps of wide.hip): one workgroup per
+// simulation in the forward, the state in LDS (as k_sv_forward_lds, raw phase), a
 // checkpoint of the state at the start of every ck-th block (after the
 // block's rescale) stored contiguously per simulation:
 // ckpt[(c * total + g) * 2^NS + j].
@@ -3025,37 +3026,6 @@ __global__ __launch_bounds__(256) void k_batch(const Job* __restrict__ jobs,
   }
 }
 
-// Groups above the LDS (15..20 slots): a persistent workgroup per resident slot
-// pulls items from the group's counter and runs their simulations one after the
-// other (sv_lds_run) with the state in its own slice of a global workspace,
-// ws[blockIdx * 2^NS + j].  Every thread reads the item index from LDS, so all
-// leave the loop together once the counter passes n_items.
-template <int NS>
-__global__ __launch_bounds__(256) void k_batch_global(const Job* __restrict__ jobs,
-                                                      const BatchItem* __restrict__ items,
-                                                      int64_t n_items, int* counter, uint32_t flags,
-                                                      float2* __restrict__ ws) {
-  __shared__ float red[4];
-  __shared__ float th_s[kAngleChunk];
-  __shared__ int item_s;
-  const int tid = threadIdx.x;
-  float2* st = ws + (int64_t(blockIdx.x) << NS);
-  for (;;) {
-    __syncthreads();   // the previous item's last reads of item_s and st are done
-    if (tid == 0) item_s = atomicAdd(counter, 1);
-    __syncthreads();
-    const int it = item_s;
-    if (it >= n_items) break;
-    const BatchItem I = items[it];
-    const Job J = load_job(jobs, I.job);
-    const int64_t end = std::min<int64_t>(I.first + I.count, J.total);
-    for (int64_t g = I.first; g < end; ++g) {
-      __syncthreads();
-      sv_lds_run<NS, 256>(J, g, flags, st, red, th_s, tid);
-    }
-  }
-}
-
 __global__ void k_reset_counters(int* counter, int n) {
   const int i = threadIdx.x;
   if (blockIdx.x == 0 && i < n) counter[i * kCounterStride] = 0;
@@ -3373,6 +3343,29 @@ hipError_t launch_dm(const Job& J, const DmNoise& nz, uint32_t flags, bool perio
 // column and block, written once and read once), so every second block is
 // kept and the backward sweep recomputes the other from it.
 inline int adj_ckpt_blocks(int64_t n_columns) { return n_columns >= 65536 ? 2 : 1; }
+
+// Columns whose contributions to an angle are summed on the device: a row of
+// partial sums (mbqc_sv_adjoint_partials(C) rows per set).
+inline int32_t adj_reduced_columns(int64_t C) {
+  return (C <= 64 && (C & (C - 1)) == 0) ? int32_t(C) : (C % 64 == 0 ? 64 : 1);
+}
+
+// Column plans of 6..14 slots run the register-blocked sweeps (the checkpoints
+// of the two kinds differ, so the choice depends on the plan and C only).
+bool wide_adjoint(const Plan* p, int64_t C) {
+  return p->ns > kMaxAdjSlots && p->column_steps &&
+         wide_adjoint_fits(p->ns, adj_reduced_columns(C), p->n_angles);
+}
+
+// Adjoint sweeps above kMaxAdjLdsSlots slots refuse stream capture whichever
+// kernels run them (those on a workspace allocate it per call).
+hipError_t refuse_capture(const Plan* p, hipStream_t st) {
+  if (p->ns <= kMaxAdjLdsSlots) return hipSuccess;
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  hipError_t e = hipStreamIsCapturing(st, &cs);
+  if (e != hipSuccess) return e;
+  return cs == hipStreamCaptureStatusNone ? hipSuccess : hipErrorStreamCaptureUnsupported;
+}
 
 template <int NS>
 hipError_t launch_adj_fwd(const Job& J, float2* ckpt, int ck, bool periodic, hipStream_t st) {
@@ -3805,25 +3798,10 @@ int scratch_ptr(float** out) {
   return MBQC_OK;
 }
 
-// Groups above the LDS: `waves` / 4 persistent 256-thread workgroups (at least
-// one, at most one per item, at most kGlobalWorkspaceBytes of states), each
-// with its slice of a workspace allocated and freed in stream order.
-template <int NS>
-hipError_t launch_batch_global_group(int64_t waves, const BatchGroupLaunch& L, void* ws,
-                                     int64_t ws_wgs) {
-  // the batch's own workspace (allocated with the batch, so that a launch
-  // allocates nothing and can be captured in a HIP graph): one state per
-  // resident workgroup
-  const int64_t wgs =
-      std::max<int64_t>(1, std::min<int64_t>(std::min<int64_t>(waves / 4, L.n_items), ws_wgs));
-  hipLaunchKernelGGL((k_batch_global<NS>), dim3(unsigned(wgs)), dim3(256), 0, L.stream, L.jobs,
-                     L.items, L.n_items, L.counter, L.flags, static_cast<float2*>(ws));
-  return hipGetLastError();
-}
-
-// Resident workgroups of a batch group of 15..20 slots (one per CU); the batch
-// allocates its workspace for this many states per group at creation.
-constexpr int64_t kBatchGlobalWgs = 256;
+// Simulations of a batch group of 15..20 slots run at a time: the batch holds
+// a workspace for this many (2 GiB for a 20-slot group), so that a launch
+// allocates nothing and can be captured in a HIP graph.
+constexpr int64_t kBatchGlobalSims = 128;
 
 }  // namespace
 
@@ -3847,9 +3825,11 @@ struct mbqc_batch {
   bool share[kMaxBatchSlots + 1] = {};
   // every plan of the group is periodic (Plan::periodic)
   bool periodic[kMaxBatchSlots + 1] = {};
-  // groups of 15..20 slots: the states of up to gws_wgs[ns] resident workgroups
+  // jobs whose plans are column plans (Plan::column_steps)
+  std::vector<char> column;
+  // groups of 15..20 slots: a workspace for gws_sims[ns] simulations
   void* gws[kMaxBatchSlots + 1] = {};
-  int64_t gws_wgs[kMaxBatchSlots + 1] = {};
+  int64_t gws_sims[kMaxBatchSlots + 1] = {};
 };
 
 // One launch of a batch: the counter reset, then one persistent kernel per
@@ -3903,12 +3883,18 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
       case 7: case 8: case 9: case 10: case 11: case 12: case 13: case 14:
         e = launch_wide_batch(ns, pe, group_waves[ns], bt->d_jobs, items, n, counter, flags, gs);
         break;
-      case 15: e = launch_batch_global_group<15>(group_waves[ns], L, bt->gws[ns], bt->gws_wgs[ns]); break;
-      case 16: e = launch_batch_global_group<16>(group_waves[ns], L, bt->gws[ns], bt->gws_wgs[ns]); break;
-      case 17: e = launch_batch_global_group<17>(group_waves[ns], L, bt->gws[ns], bt->gws_wgs[ns]); break;
-      case 18: e = launch_batch_global_group<18>(group_waves[ns], L, bt->gws[ns], bt->gws_wgs[ns]); break;
-      case 19: e = launch_batch_global_group<19>(group_waves[ns], L, bt->gws[ns], bt->gws_wgs[ns]); break;
-      default: e = launch_batch_global_group<20>(group_waves[ns], L, bt->gws[ns], bt->gws_wgs[ns]); break;
+      default:
+        // above the LDS: every job of the group in passes over tiles, as its
+        // own launch runs them
+        for (size_t i = 0; i < bt->jobs.size() && e == hipSuccess; ++i) {
+          const Job& J = bt->jobs[i];
+          if (J.ns != ns) continue;
+          const bool column = bt->column[i] && !(flags & MBQC_FLAG_TABLE_STEPS);
+          for (int64_t g0 = 0; g0 < J.total && e == hipSuccess; g0 += bt->gws_sims[ns])
+            e = launch_wide_tiles(J, column, flags, bt->gws[ns], g0,
+                                  std::min<int64_t>(bt->gws_sims[ns], J.total - g0), gs);
+        }
+        break;
     }
     if (e == hipSuccess) e = hipGetLastError();
     if (e == hipSuccess && concurrent) {
@@ -4261,6 +4247,11 @@ int mbqc_sv_adjoint_forward_c64(const mbqc_plan* plan, const float* angles, int6
   hipStream_t st = static_cast<hipStream_t>(stream);
   float2* ck = static_cast<float2*>(ckpt);
   hipError_t e = hipSuccess;
+  if (wide_adjoint(p, C)) {
+    e = refuse_capture(p, st);
+    if (e == hipSuccess) e = launch_wide_adj_forward(J, ck, adj_ckpt_blocks(B * C), st);
+    return e == hipSuccess ? MBQC_OK : global_fail(e, "adjoint forward launch");
+  }
   switch (p->ns) {
     case 1: e = launch_adj_fwd<1>(J, ck, adj_ckpt_blocks(B * C), p->periodic, st); break;
     case 2: e = launch_adj_fwd<2>(J, ck, adj_ckpt_blocks(B * C), p->periodic, st); break;
@@ -4303,7 +4294,7 @@ int mbqc_sv_adjoint_backward_c64(const mbqc_plan* plan, const float* angles, int
   A.gpart = grad_partial;
   A.C = C;
   A.P = mbqc_sv_adjoint_partials(C);
-  A.red = (C <= 64 && (C & (C - 1)) == 0) ? int32_t(C) : (C % 64 == 0 ? 64 : 1);
+  A.red = adj_reduced_columns(C);
   A.n_angles = p->n_angles;
   A.ck = adj_ckpt_blocks(B * C);
   if (p->ns > kMaxAdjSlots &&
@@ -4316,6 +4307,13 @@ int mbqc_sv_adjoint_backward_c64(const mbqc_plan* plan, const float* angles, int
   const float2* ck = static_cast<const float2*>(ckpt);
   const float2* sd = static_cast<const float2*>(seed);
   hipError_t e = hipSuccess;
+  if (wide_adjoint(p, C)) {
+    e = refuse_capture(p, st);
+    if (e == hipSuccess)
+      e = launch_wide_adj_backward(J, ck, sd, WideAdjoint{A.C, A.P, A.red, A.ck, A.n_angles}, A.gpart,
+                                   st);
+    return e == hipSuccess ? MBQC_OK : global_fail(e, "adjoint backward launch");
+  }
   switch (p->ns) {
     case 1: e = launch_adj_bwd<1>(J, ck, sd, A, p->periodic, st); break;
     case 2: e = launch_adj_bwd<2>(J, ck, sd, A, p->periodic, st); break;
@@ -4385,6 +4383,9 @@ int mbqc_batch_create(const mbqc_batch_job* jobs, int32_t n_jobs, int32_t sims_p
     bt->max_ns = std::max(bt->max_ns, p->ns);
     if (p->ns < 2 || J.S % share_group(p->ns) != 0) bt->share[p->ns] = false;
     if (!p->column_steps) bt->periodic[p->ns] = false;
+    bt->column.push_back(p->column_steps);
+    if (p->ns > kMaxSvLdsSlots)
+      bt->gws_sims[p->ns] = std::min(kBatchGlobalSims, std::max(bt->gws_sims[p->ns], J.total));
     const int64_t cost = int64_t(p->n_steps) << p->ns;
     for (int64_t f = 0; f < J.total; f += sims_per_item) {
       BatchItem it{};
@@ -4416,10 +4417,7 @@ int mbqc_batch_create(const mbqc_batch_job* jobs, int32_t n_jobs, int32_t sims_p
   if (e == hipSuccess) e = hipMalloc(&bt->d_counter, sizeof(int) * kCounterStride * (kMaxBatchSlots + 1));
   for (int ns = kMaxSvLdsSlots + 1; ns <= kMaxBatchSlots && e == hipSuccess; ++ns) {
     if (bt->group_count[ns] == 0) continue;
-    const size_t state_bytes = sizeof(float2) << ns;
-    bt->gws_wgs[ns] = std::min<int64_t>(std::min<int64_t>(bt->group_count[ns], kBatchGlobalWgs),
-                                        int64_t(kGlobalWorkspaceBytes / state_bytes));
-    e = hipMalloc(&bt->gws[ns], size_t(bt->gws_wgs[ns]) * state_bytes);
+    e = hipMalloc(&bt->gws[ns], size_t(bt->gws_sims[ns]) * wide_tile_bytes(ns));
   }
   int n_groups = 0;
   for (int ns = 1; ns <= kMaxBatchSlots; ++ns) n_groups += bt->group_count[ns] > 0;

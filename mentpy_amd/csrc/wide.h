@@ -23,4 +23,19 @@ hipError_t launch_wide_batch(int ns, bool column, int64_t waves, const Job* jobs
                              const BatchItem* items, int64_t n_items, int* counter, uint32_t flags,
                              hipStream_t st);
 
+// Adjoint sweeps of column plans with 6..14 slots.  Checkpoints: the state after
+// every ck-th block and after the last, ckpt[(block / ck) * total + g] each
+// 2^ns amplitudes.
+struct WideAdjoint {
+  int64_t C;          // columns per parameter set
+  int32_t P, red;     // partial-sum rows per set, columns per row
+  int32_t ck;         // blocks per checkpoint
+  int32_t n_angles;
+};
+constexpr size_t kWideMaxLds = 160 * 1024 - 256;   // gfx950: 160 KiB per workgroup
+bool wide_adjoint_fits(int ns, int red, int n_angles);
+hipError_t launch_wide_adj_forward(const Job& J, float2* ckpt, int ck, hipStream_t st);
+hipError_t launch_wide_adj_backward(const Job& J, const float2* ckpt, const float2* seed,
+                                    const WideAdjoint& A, float* gpart, hipStream_t st);
+
 }  // namespace mbqc

@@ -181,16 +181,19 @@ __device__ __forceinline__ void wide_coeffs(float2* bs, const mbqc_step* steps, 
 #pragma unroll 1
   for (int i = lane; i < W::CS; i += W::TL) {
     const int k = k0 + i;
-    if (k < n) bs[i] = step_coeff<REF>(step_angle(steps[k], ang, sa), ph);
+    if (k < n) {
+      const float th = step_angle(steps[k], ang, sa);
+      if constexpr (REF) ph->add(th);
+      bs[i] = exp_minus_i(th);
+    }
   }
 }
 
-// All steps of one simulation; `on_block(blk, t)` runs at the start of every
-// block (after its rescale).
-template <int NS, int R, bool REF, bool COLUMN, typename OnBlock, typename Mod>
+// All steps of one simulation; `on_end(blk, t)` runs after every block.
+template <int NS, int R, bool REF, bool COLUMN, typename OnEnd, typename Mod>
 __device__ __forceinline__ void wide_run(float2 (&t)[1 << R], const Job& J, const float* ang,
                                          float2* buf, float2* bs, int lane, RefPhase* ph,
-                                         OnBlock on_block, Mod&& mod) {
+                                         OnEnd on_end, Mod&& mod) {
   using W = Wide<NS, R>;
   const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
   const int32_t* resc = J.tab + J.off_svres;
@@ -205,9 +208,9 @@ __device__ __forceinline__ void wide_run(float2 (&t)[1 << R], const Job& J, cons
 #pragma unroll
         for (int r = 0; r < W::NR; ++r) t[r] = cscale(t[r], 0x1p-32f);
       }
-      on_block(k0 / NS, t);
       wide_block<NS, R, NS, COLUMN>(t, buf, bs + (k0 - kc), steps, k0, n, lane, true, mod,
                                     SlotSigns(), std::make_integer_sequence<int, W::P>{});
+      on_end(k0 / NS, t);
     }
   }
 }
@@ -377,6 +380,287 @@ __global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_batch(
       wide_sim<NS, R, REF, COLUMN>(J, g + sub, g + sub < end, flags, buf, buf + W::BUF, lane);
     }
   }
+}
+
+// ---------------------------------------------------------------- adjoint
+// Adjoint sweeps of column plans.  Every step of a column plan is invertible:
+// new0 = x + b y, new1 = c (x - b y) with c the CZ sign, so
+//   2x = new0 + c new1,   2 b y = new0 - c new1,
+// and the backward sweep runs the state back from a checkpoint at the end of a
+// group of ck blocks instead of recomputing it forward from the group's start
+// and keeping every step's measured half.  With h = lam0 - c lam1 the cotangent of
+// new0 (L real, dL = Re sum conj(lam) d(new)):
+//   lam_x = lam0 + c lam1,   lam_y = conj(b) h,
+//   dL/dtheta += Im(sum b y conj(h)).
+// The factors 2 of the state are powers of two carried per block, so they round
+// nothing; a state is at most ck blocks of steps away from its checkpoint.
+// Bound by VALU issue (18 FMA-rate instructions per pair and step, two states
+// in registers) and the two exchanges per phase.  8x6 grid, 509 sets x 4
+// columns: backward 172 -> 20 us against one workgroup per row with the states
+// and the measured halves in LDS and a barrier per step, forward 22.7 -> 14.2.
+// Gradient error against 64 bits 3.6e-7 -> 3.0e-7 (the running back costs
+// about 8%, the correctly rounded coefficients gain more).
+template <int NS, int R>
+__global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_adj_forward(Job J,
+                                                                       float2* __restrict__ ckpt,
+                                                                       int ck) {
+  using W = Wide<NS, R>;
+  __shared__ float2 lds[W::G * W::SIM];
+  const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
+  float2* buf = lds + sub * W::SIM;
+  const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
+  const bool active = g < J.total;
+  const int64_t gg = active ? g : J.total - 1;
+  int64_t bi, si;
+  split_sim(J, gg, &bi, &si);
+  float2 t[W::NR];
+  wide_load<NS, R>(t, J, si, lane);
+  const int nblk = (J.n_steps + NS - 1) / NS;
+  RefPhase ph;
+  wide_run<NS, R, false, true>(
+      t, J, J.angles + bi * J.angle_stride, buf, buf + W::BUF, lane, &ph,
+      [&](int blk, const float2 (&tt)[W::NR]) {
+        if ((blk + 1) % ck != 0 && blk + 1 != nblk) return;
+        // inactive groups repeat the last simulation's stores
+        float2* cp = ckpt + ((int64_t(blk / ck) * J.total + gg) << NS) + lane;
+#pragma unroll
+        for (int r = 0; r < W::NR; ++r) cp[r << (NS - R)] = tt[r];
+      },
+      NoModify());
+  if (!active) return;
+  const int32_t* out_pos = J.tab + J.off_out;
+  const float scale = sv_final_scale(J.e_sv);
+  float2* o = J.out + g * (int64_t(1) << J.n_out);
+#pragma unroll
+  for (int r = 0; r < W::NR; ++r) {
+    const int p = out_pos[(r << (NS - R)) | lane];
+    if (p >= 0) o[p] = cscale(t[r], scale);
+  }
+}
+
+// The inverse exchange: v -> rotate-right(v, M).
+template <int NS, int R, int M, int TL>
+__device__ __forceinline__ void wide_unrotate(float2 (&t)[1 << R], float2* buf, int lane) {
+  constexpr int NR = 1 << R;
+  lanes_sync<TL>();
+#pragma unroll
+  for (int r = 0; r < NR; ++r) buf[padded((r << (NS - R)) | lane)] = t[r];
+  lanes_sync<TL>();
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    const int top = r >> (R - M), low = r & ((1 << (R - M)) - 1);
+    t[r] = buf[padded((low << (NS - R + M)) | (lane << M) | top)];
+  }
+}
+
+// Step FIRST + S backwards on state t (scaled by a power of two: doubled by
+// each step) and cotangent lam; returns this lane's Im(sum 2 b y conj(h)).
+template <int NS, int R, int FIRST, int S>
+__device__ __forceinline__ float wide_unstep(float2 (&t)[1 << R], float2 (&lam)[1 << R], float2 b,
+                                             int lane) {
+  constexpr int NR = 1 << R, QB = 1 << (R - 1 - S);
+  const float2 bc = cconj(b);
+  const float lc = (S == 0 && FIRST > 0 && (lane & 1)) ? -1.0f : 1.0f;
+  float d = 0.0f;
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    if (r & QB) continue;
+    const float c = S == 0 ? lc : ((r & (QB << 1)) ? -1.0f : 1.0f);
+    const float2 u0 = t[r], u1 = t[r | QB], l0 = lam[r], l1 = lam[r | QB];
+    const float2 y = make_float2(fmaf(-c, u1.x, u0.x), fmaf(-c, u1.y, u0.y));
+    const float2 h = make_float2(fmaf(-c, l1.x, l0.x), fmaf(-c, l1.y, l0.y));
+    d = fmaf(y.y, h.x, fmaf(-y.x, h.y, d));
+    t[r] = make_float2(fmaf(c, u1.x, u0.x), fmaf(c, u1.y, u0.y));
+    lam[r] = make_float2(fmaf(c, l1.x, l0.x), fmaf(c, l1.y, l0.y));
+    t[r | QB] = cmul(bc, y);
+    lam[r | QB] = cmul(bc, h);
+  }
+  return d;
+}
+
+// Sum over the TL lanes of a group, in its last lane at least.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float add_dpp(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+}
+template <int TL>
+__device__ __forceinline__ float last_lane_sum(float v) {
+  if constexpr (TL > 1) v = add_dpp<0xB1, 0xf>(v);     // quad_perm [1,0,3,2]
+  if constexpr (TL > 2) v = add_dpp<0x4E, 0xf>(v);     // quad_perm [2,3,0,1]
+  if constexpr (TL > 4) v = add_dpp<0x141, 0xf>(v);    // row_half_mirror
+  if constexpr (TL > 8) v = add_dpp<0x140, 0xf>(v);    // row_mirror
+  if constexpr (TL > 16) v = add_dpp<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+  if constexpr (TL > 32) v = add_dpp<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+// Where a lane puts the gradient entries of its simulation: acc[angle index]
+// in LDS, one writer per simulation and wave (waves: entry stride n_angles).
+struct GradSlot {
+  float* acc;
+  bool writer, first;
+};
+
+template <int NS, int R, int P, int... SS>
+__device__ __forceinline__ void wide_unphase(float2 (&t)[1 << R], float2 (&lam)[1 << R], float2* buf,
+                                             const float2* bs, const mbqc_step* steps, int k0,
+                                             int lane, const GradSlot& slot,
+                                             std::integer_sequence<int, SS...>) {
+  using W = Wide<NS, R>;
+  constexpr int F = W::first(P), M = W::len(P);
+  wide_unrotate<NS, R, M, W::TL>(t, buf, lane);
+  wide_unrotate<NS, R, M, W::TL>(lam, buf, lane);
+  auto one = [&](auto sc) {
+    constexpr int S = M - 1 - decltype(sc)::value, SUB = F + S;
+    float d = wide_unstep<NS, R, F, S>(t, lam, bs[SUB], lane);
+    const int ai = steps[k0 + SUB].angle_index;
+    if (ai >= 0) {
+      d = last_lane_sum<(W::TL < 64 ? W::TL : 64)>(d);
+      // the state has been doubled by the NS - 1 - SUB steps after this one
+      d *= 1.0f / float(1 << (NS - SUB));
+      if (slot.writer) slot.acc[ai] = slot.first ? d : slot.acc[ai] + d;
+    }
+  };
+  (one(std::integral_constant<int, SS>{}), ...);
+}
+
+template <int NS, int R, int... PS>
+__device__ __forceinline__ void wide_unblock(float2 (&t)[1 << R], float2 (&lam)[1 << R], float2* buf,
+                                             const float2* bs, const mbqc_step* steps, int k0,
+                                             int lane, const GradSlot& slot,
+                                             std::integer_sequence<int, PS...>) {
+  using W = Wide<NS, R>;
+  (wide_unphase<NS, R, W::P - 1 - PS>(t, lam, buf, bs, steps, k0, lane, slot,
+                                      std::make_integer_sequence<int, W::len(W::P - 1 - PS)>{}),
+   ...);
+}
+
+// Backward sweep of a column plan: a workgroup holds N = blockDim / TL
+// simulations at a time.  Rows of `red` <= N columns that are reduced together
+// take `red` neighbouring groups (N / red rows per workgroup), longer ones
+// run in red / N rounds.  Per-angle sums stay in LDS (one row of n_angles per
+// group and wave of it) and are added up once at the end.
+template <int NS, int R>
+__global__ __launch_bounds__((Wide<NS, R>::TL > 256 ? Wide<NS, R>::TL : 256)) void k_wide_adj_backward(
+    Job J, const float2* __restrict__ ckpt, const float2* __restrict__ seed, WideAdjoint A,
+    float* __restrict__ gpart) {
+  using W = Wide<NS, R>;
+  constexpr int TL = W::TL;
+  constexpr int WV = TL > 64 ? TL / 64 : 1;       // waves of one simulation
+  extern __shared__ float2 dyn[];
+  const int N = blockDim.x / TL;
+  const int sub = threadIdx.x / TL, lane = threadIdx.x % TL;
+  float2* buf = dyn + sub * (W::BUF + NS);
+  float2* bs = buf + W::BUF;
+  float* accs = reinterpret_cast<float*>(dyn + N * (W::BUF + NS));
+  const int wave = TL > 64 ? lane >> 6 : 0;
+  const int per = A.red < N ? A.red : N;          // columns of a row held at once
+  const int rows = N / per;                       // rows of this workgroup
+  const int64_t n_rows = (J.total / A.C) * A.P;
+  const int64_t row0 = int64_t(xcd_block(blockIdx.x, gridDim.x)) * rows;
+  const int64_t row = row0 + sub / per;
+  const bool active = row < n_rows;
+  const int64_t rr = active ? row : n_rows - 1;
+  const int64_t bi = rr / A.P, r0 = rr - bi * A.P;
+  const float* ang = J.angles + bi * J.angle_stride;
+  const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
+  const int32_t* resc = J.tab + J.off_svres;
+  const int32_t* out_pos = J.tab + J.off_out;
+  const float scale = sv_final_scale(J.e_sv);
+  const int nblk = J.n_steps / NS;
+  for (int a = threadIdx.x; a < N * WV * A.n_angles; a += blockDim.x) accs[a] = 0.0f;
+  __syncthreads();
+  GradSlot slot;
+  slot.acc = accs + (sub * WV + wave) * A.n_angles;
+  slot.writer = (threadIdx.x & ((TL < 64 ? TL : 64) - 1)) == (TL < 64 ? TL : 64) - 1;
+  for (int c0 = 0; c0 < A.red; c0 += per) {
+    slot.first = c0 == 0;
+    const int64_t g = bi * A.C + r0 * A.red + c0 + sub % per;
+    const float2* sd = seed + g * (int64_t(1) << J.n_out);
+    float2 t[W::NR], lam[W::NR];
+#pragma unroll
+    for (int r = 0; r < W::NR; ++r) {
+      const int p = out_pos[(r << (NS - R)) | lane];
+      lam[r] = cscale(sd[p >= 0 ? p : 0], p >= 0 ? scale : 0.0f);
+    }
+    // the angle of the next block this lane evaluates, one block ahead
+    float th = 0.0f;
+    if (lane < NS) th = step_angle(steps[(nblk - 1) * NS + lane], ang, J.angle_stride_a);
+    for (int blk = nblk - 1; blk >= 0; --blk) {
+      if (blk + 1 == nblk || (blk + 1) % A.ck == 0) {
+        const float2* cp = ckpt + ((int64_t(blk / A.ck) * J.total + g) << NS) + lane;
+#pragma unroll
+        for (int r = 0; r < W::NR; ++r) t[r] = cp[r << (NS - R)];
+      }
+      lanes_sync<TL>();
+      if (lane < NS) bs[lane] = exp_minus_i(th);
+      if (lane < NS && blk > 0) th = step_angle(steps[(blk - 1) * NS + lane], ang, J.angle_stride_a);
+      lanes_sync<TL>();
+      wide_unblock<NS, R>(t, lam, buf, bs, steps, blk * NS, lane, slot,
+                          std::make_integer_sequence<int, W::P>{});
+      // the block's doublings and rescale undone; the cotangent takes the rescale
+      const bool rs = resc[blk] != 0;
+      const float f = (rs ? 0x1p32f : 1.0f) / float(1 << NS);
+#pragma unroll
+      for (int r = 0; r < W::NR; ++r) t[r] = cscale(t[r], f);
+      if (rs) {
+#pragma unroll
+        for (int r = 0; r < W::NR; ++r) lam[r] = cscale(lam[r], 0x1p-32f);
+      }
+    }
+  }
+  __syncthreads();
+  for (int i = threadIdx.x; i < rows * A.n_angles; i += blockDim.x) {
+    const int q = i / A.n_angles, a = i - q * A.n_angles;
+    float v = 0.0f;
+    for (int c = 0; c < per * WV; ++c) v += accs[(q * per * WV + c) * A.n_angles + a];
+    if (row0 + q < n_rows) gpart[(row0 + q) * A.n_angles + a] = v;
+  }
+}
+
+template <int NS>
+size_t adj_backward_lds(int N, int n_angles) {
+  using W = Wide<NS, wide_reg_bits(NS)>;
+  const int WV = W::TL > 64 ? W::TL / 64 : 1;
+  return size_t(N) * (W::BUF + NS) * sizeof(float2) + size_t(N) * WV * n_angles * sizeof(float);
+}
+
+template <int NS>
+hipError_t adj_forward_launch(const Job& J, float2* ckpt, int ck, hipStream_t st) {
+  constexpr int R = wide_reg_bits(NS);
+  using W = Wide<NS, R>;
+  hipLaunchKernelGGL((k_wide_adj_forward<NS, R>), dim3(unsigned((J.total + W::G - 1) / W::G)),
+                     dim3(W::T), 0, st, J, ckpt, ck);
+  return hipGetLastError();
+}
+
+// Threads per workgroup of the backward sweep: a row's columns together, up to
+// 256 threads, in whole waves, as far as the LDS allows.
+template <int NS>
+int adj_backward_groups(int red, int n_angles) {
+  constexpr int TL = Wide<NS, wide_reg_bits(NS)>::TL;
+  int N = TL >= 256 ? 1 : std::min(256 / TL, red);
+  if (N * TL < 64) N = 64 / TL;
+  while (N > 1 && N * TL > 64 && adj_backward_lds<NS>(N, n_angles) > kWideMaxLds / 2) N /= 2;
+  return N;
+}
+
+template <int NS>
+hipError_t adj_backward_launch(const Job& J, const float2* ckpt, const float2* seed,
+                               const WideAdjoint& A, float* gpart, hipStream_t st) {
+  constexpr int R = wide_reg_bits(NS);
+  const int N = adj_backward_groups<NS>(A.red, A.n_angles);
+  const size_t lds = adj_backward_lds<NS>(N, A.n_angles);
+  if (lds > 65536) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_wide_adj_backward<NS, R>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    if (e != hipSuccess) return e;
+  }
+  const int rows = N / std::min(A.red, N);
+  const int64_t n_rows = (J.total / A.C) * A.P;
+  hipLaunchKernelGGL((k_wide_adj_backward<NS, R>), dim3(unsigned((n_rows + rows - 1) / rows)),
+                     dim3(unsigned(N * Wide<NS, R>::TL)), lds, st, J, ckpt, seed, A, gpart);
+  return hipGetLastError();
 }
 
 // ---------------------------------------------------------------- tile passes
@@ -584,6 +868,7 @@ hipError_t batch_launch(bool column, int64_t waves, const Job* jobs, const Batch
 
 #define MBQC_WIDE_SWITCH(ns, CALL)        \
   switch (ns) {                           \
+    case 6: return CALL(6);               \
     case 7: return CALL(7);               \
     case 8: return CALL(8);               \
     case 9: return CALL(9);               \
@@ -654,6 +939,36 @@ hipError_t launch_wide_batch(int ns, bool column, int64_t waves, const Job* jobs
                              hipStream_t st) {
 #define MBQC_CALL(NS) batch_launch<NS>(column, waves, jobs, items, n_items, counter, flags, st)
   MBQC_WIDE_SWITCH(ns, MBQC_CALL)
+#undef MBQC_CALL
+}
+
+bool wide_adjoint_fits(int ns, int red, int n_angles) {
+#define MBQC_CALL(NS) adj_backward_lds<NS>(adj_backward_groups<NS>(red, n_angles), n_angles) <= kWideMaxLds
+  switch (ns) {
+    case 6: return MBQC_CALL(6);
+    case 7: return MBQC_CALL(7);
+    case 8: return MBQC_CALL(8);
+    case 9: return MBQC_CALL(9);
+    case 10: return MBQC_CALL(10);
+    case 11: return MBQC_CALL(11);
+    case 12: return MBQC_CALL(12);
+    case 13: return MBQC_CALL(13);
+    case 14: return MBQC_CALL(14);
+    default: return false;
+  }
+#undef MBQC_CALL
+}
+
+hipError_t launch_wide_adj_forward(const Job& J, float2* ckpt, int ck, hipStream_t st) {
+#define MBQC_CALL(NS) adj_forward_launch<NS>(J, ckpt, ck, st)
+  MBQC_WIDE_SWITCH(J.ns, MBQC_CALL)
+#undef MBQC_CALL
+}
+
+hipError_t launch_wide_adj_backward(const Job& J, const float2* ckpt, const float2* seed,
+                                    const WideAdjoint& A, float* gpart, hipStream_t st) {
+#define MBQC_CALL(NS) adj_backward_launch<NS>(J, ckpt, seed, A, gpart, st)
+  MBQC_WIDE_SWITCH(J.ns, MBQC_CALL)
 #undef MBQC_CALL
 }
 

@@ -52,3 +52,50 @@ def test_wide_windows_match_oracle(rows, cols, window, B, S, rng):
     err = np.abs(out.cpu().numpy() - ref).max()
     # complex64 butterflies: each step adds about one rounding (6e-8) to amplitudes below 1
     assert err < 2e-5, f"amplitude error {err}"
+
+
+@pytest.mark.parametrize("rows,cols,C,B", [(6, 14, 4, 5), (6, 14, 128, 512), (7, 12, 3, 2), (8, 4, 16, 3),
+                                           (9, 4, 1, 3), (10, 4, 2, 1), (11, 3, 4, 1), (12, 3, 2, 1),
+                                           (13, 3, 2, 1), (14, 3, 1, 1)])
+def test_wide_adjoint_matches_complex128(rows, cols, C, B, rng):
+    """Outputs and angle gradients of the register-blocked adjoint sweeps
+    against torch autograd on the complex128 grid steps: one and several
+    simulations per wave and per row, rows of 64 columns, checkpoint pairs
+    (65,536 columns), a rescale (more than 64 steps)."""
+    torch = _torch()
+    import mentpy_amd as mp
+    from mentpy_amd.gradients.adjoint import pattern_sv
+    g = mp.templates.grid_cluster(rows, cols)
+    sim = mp.PatternSimulator(g, backend="hip-sv")
+    n, d = len(g.trainable_nodes), 1 << rows
+    gen = torch.Generator().manual_seed(rows)
+    th = (torch.rand((B, n), generator=gen) * 6.2).cuda().requires_grad_(True)
+    x = torch.randn((C, d), generator=gen, dtype=torch.complex64).cuda()
+    x = x / torch.linalg.vector_norm(x, dim=1, keepdim=True)
+    cot = torch.randn((B, C, d), generator=gen, dtype=torch.complex64).cuda() / d ** 0.5
+    out = pattern_sv(sim, th, x)
+    grad, = torch.autograd.grad(out, th, cot)
+    bs = list(range(B)) if B < 8 else [0, B // 2, B - 1]
+    a = th.detach()[bs].double().requires_grad_(True)
+    j = torch.arange(d, device="cuda")
+    bit = [((j >> (rows - 1 - i)) & 1).double() for i in range(rows)]
+    t = x.to(torch.complex128)
+    for i in range(rows - 1):
+        t = t * (1 - 2 * bit[i] * bit[i + 1])
+    t = t[None].expand(len(bs), -1, -1)
+    for k in range(rows * (cols - 1)):
+        i, col = k % rows, k // rows
+        ph = torch.polar(torch.ones_like(a[:, 0]), -a[:, i * (cols - 1) + col])
+        v = t.reshape(len(bs), C, 1 << i, 2, -1)
+        p, q = v[:, :, :, 0], v[:, :, :, 1] * ph[:, None, None, None]
+        t = (torch.stack([p + q, p - q], 3) * 0.5 ** 0.5).reshape(len(bs), C, d)
+        if i:
+            t = t * (1 - 2 * bit[i - 1] * bit[i])
+    want, = torch.autograd.grad(t, a, cot[bs].to(torch.complex128))
+    oerr = (out.detach()[bs] - t.detach()).abs().max().item()
+    scale = want.abs().max().item()
+    gerr = (grad[bs] - want).abs().max().item()
+    # one rounding (6e-8) per step on unit-norm states and cotangents of norm about
+    # sqrt(2 C): far below 2e-5 of the largest entry
+    assert oerr < 2e-5, f"output error {oerr}"
+    assert gerr < 2e-5 * max(scale, 1.0), f"gradient error {gerr} of {scale}"
