@@ -61,33 +61,37 @@ __device__ __forceinline__ void sincos_poly(float x, float* sn, float* cs) {
   *cs = __uint_as_float(__float_as_uint(cr) ^ sgn);
 }
 
-// e^{-i x} from double arithmetic, correctly rounded but for rare near-ties: for
-// kernels that evaluate a step's coefficient once per simulation, where it
-// costs nothing next to the amplitudes.  (The float polynomials above leave
-// about 1e-7 in every coefficient, an error that all amplitudes share and
-// that adds up over the steps.)  x = k pi/2 + r, |r| <= pi/4, Taylor series to
-// r^11 and r^12 (remainders below 1e-11).
-__device__ __forceinline__ float2 exp_minus_i(float x) {
-  const double xd = double(x);
-  const double k = rint(xd * 0.63661977236758134308);
-  double r = fma(-k, 1.57079632679489661923, xd);
+// (cos a, sin a) rounded from double arithmetic, |a| up to a few thousand:
+// a = k pi/2 + r, |r| <= pi/4, Taylor series to r^13 and r^14 (remainders below
+// 3e-14, so the floats are the nearest ones but for very rare near-ties).
+__device__ __forceinline__ float2 cis_f64(double a) {
+  const double k = rint(a * 0.63661977236758134308);
+  double r = fma(-k, 1.57079632679489661923, a);
   r = fma(-k, 6.12323399573676603587e-17, r);
   const double r2 = r * r;
-  double ps = fma(r2, -1.0 / 39916800.0, 1.0 / 362880.0);
+  double ps = fma(r2, 1.0 / 6227020800.0, -1.0 / 39916800.0);
+  ps = fma(r2, ps, 1.0 / 362880.0);
   ps = fma(r2, ps, -1.0 / 5040.0);
   ps = fma(r2, ps, 1.0 / 120.0);
   ps = fma(r2, ps, -1.0 / 6.0);
   const float s = float(fma(r * r2, ps, r));
-  double pc = fma(r2, 1.0 / 479001600.0, -1.0 / 3628800.0);
+  double pc = fma(r2, -1.0 / 87178291200.0, 1.0 / 479001600.0);
+  pc = fma(r2, pc, -1.0 / 3628800.0);
   pc = fma(r2, pc, 1.0 / 40320.0);
   pc = fma(r2, pc, -1.0 / 720.0);
   pc = fma(r2, pc, 1.0 / 24.0);
   pc = fma(r2, pc, -0.5);
   const float c = float(fma(r2, pc, 1.0));
-  const int q = int(k) & 3;   // cos, sin of r + q pi/2
+  const int q = int(k) & 3;
   const float cs = (q & 1) ? s : c, sn = (q & 1) ? c : s;
-  return make_float2(((q + 1) & 2) ? -cs : cs, (q & 2) ? sn : -sn);
+  return make_float2(((q + 1) & 2) ? -cs : cs, (q & 2) ? -sn : sn);
 }
+
+// e^{-i x} for kernels that evaluate a step's coefficient once per simulation,
+// where double arithmetic costs nothing next to the amplitudes.  (The float
+// polynomials above leave about 1e-7 in every coefficient, an error that all
+// amplitudes share and that adds up over the steps.)
+__device__ __forceinline__ float2 exp_minus_i(float x) { return cis_f64(-double(x)); }
 
 // The reference's global phase, prod_k sgn(cos(theta_k/2)) e^{i theta_k/2}
 // (the factor its amplitude-sum partial trace introduces,
@@ -123,12 +127,8 @@ struct RefPhase {
     th_sum += d;
   }
   __device__ __forceinline__ float2 value() const {
-    constexpr double kPi = 3.14159265358979323846;
-    double a = 0.5 * th_sum - kPi * double(m_sum);
-    a -= 2.0 * kPi * rint(a * (0.5 / kPi));
-    double sd, cd;
-    sincos(a, &sd, &cd);
-    return make_float2(float(cd), float(sd));
+    // at most pi/2 per step: small enough for cis_f64's reduction
+    return cis_f64(fma(-3.14159265358979323846, double(m_sum), 0.5 * th_sum));
   }
 };
 

@@ -3981,6 +3981,10 @@ int mbqc_sv_forward_c64(const mbqc_plan* plan, const float* angles, int64_t angl
     }
     return e == hipSuccess ? MBQC_OK : hip_fail(e, "sv_forward launch");
   }
+  if (narrow_sv(J)) {
+    e = launch_narrow_sv(J, periodic, flags, st);
+    return e == hipSuccess ? MBQC_OK : hip_fail(e, "sv_forward launch");
+  }
   switch (p->ns) {
     case 1: e = launch_sv<1>(J, p->coef_per_step, periodic, flags, st); break;
     case 2: e = launch_sv<2>(J, p->coef_per_step, periodic, flags, st); break;

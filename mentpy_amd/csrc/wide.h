@@ -1,5 +1,5 @@
-// Launchers of the register-blocked kernels for live windows of 7..20 slots
-// (wide.hip).  They need a plan whose
+// Launchers of the register-blocked kernels (wide.hip): live windows of 7..20
+// slots, small batches of narrower ones, adjoint sweeps.  They need a plan whose
 // measured slots follow the rotation (Plan::rotating).
 #pragma once
 #include "device.h"
@@ -9,6 +9,10 @@ namespace mbqc {
 // `column`: every step is that of a grid in column order (Plan::column_steps),
 // so the CZ signs are compile-time constants.
 hipError_t launch_wide_sv(const Job& J, bool column, uint32_t flags, hipStream_t st);
+// The same for windows of 2..6 slots, where narrow_sv says that the batch is
+// too small for one simulation per lane.
+bool narrow_sv(const Job& J);
+hipError_t launch_narrow_sv(const Job& J, bool column, uint32_t flags, hipStream_t st);
 // Windows of 15..20 slots: simulations [g0, g0 + n) in passes over tiles of
 // their states, in a workspace of n * wide_tile_bytes(ns) bytes.
 size_t wide_tile_bytes(int ns);

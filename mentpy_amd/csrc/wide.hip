@@ -1,4 +1,5 @@
-// Statevector kernels for live windows of 7..14 slots (gfx950).
+// Statevector kernels that spread one simulation over several lanes (gfx950):
+// live windows of 7 slots and more, and small batches of narrower ones.
 //
 // The state of one simulation is spread over TL = 2^(NS - R) lanes with 2^R
 // amplitudes each in registers: amplitude v = r * TL + lane, r the register.
@@ -36,12 +37,15 @@ namespace {
 constexpr int wide_reg_bits(int ns) { return ns <= 9 ? 3 : 4; }
 
 // NS amplitude bits over lanes and registers, M of them measured per block
-// (all of them except in a pass over tiles of a larger state).
-template <int NS, int R, int M = NS>
+// (all of them except in a pass over tiles of a larger state).  SPARE: log2 of
+// the lanes per amplitude lane; the spare ones share the coefficient work and
+// repeat the state's.
+template <int NS, int R, int M = NS, int SPARE = 0>
 struct Wide {
   static constexpr int TL = 1 << (NS - R);        // lanes per simulation
-  static constexpr int T = TL > 64 ? TL : 64;     // threads per workgroup
-  static constexpr int G = T / TL;                // simulations per workgroup
+  static constexpr int CL = TL << SPARE;          // lanes that evaluate its coefficients
+  static constexpr int T = CL > 64 ? CL : 64;     // threads per workgroup
+  static constexpr int G = T / CL;                // simulations per workgroup
   static constexpr int NR = 1 << R;               // amplitudes per lane
   static constexpr int P = (M + R - 1) / R;       // phases per block
   static constexpr int CS = M == NS ? (64 / NS) * NS : M;   // steps per coefficient chunk
@@ -135,6 +139,7 @@ __device__ __forceinline__ void wide_step(float2 (&t)[1 << R], float2 b, const m
 template <int NS, int R, int M, int T>
 __device__ __forceinline__ void wide_rotate(float2 (&t)[1 << R], float2* buf, int lane) {
   constexpr int NR = 1 << R;
+  if constexpr (R == NS) return;   // one lane: rotated by all its bits, back in place
   lanes_sync<T>();   // earlier reads of the buffer are done
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
@@ -174,33 +179,37 @@ __device__ __forceinline__ void wide_block(float2 (&t)[1 << R], float2* buf, con
 }
 
 // e^{-i theta} of the chunk of steps [k0, k0 + CS), one step per lane.
-template <int NS, int R, bool REF, int M = NS>
+// (cl: the lane's place among the CL coefficient lanes.)  POLY: from the float
+// polynomials of the one-simulation-per-lane kernels, bit for bit.
+template <int NS, int R, bool REF, int M = NS, int SPARE = 0, bool POLY = false>
 __device__ __forceinline__ void wide_coeffs(float2* bs, const mbqc_step* steps, const float* ang,
-                                            int64_t sa, int k0, int n, int lane, RefPhase* ph) {
-  using W = Wide<NS, R, M>;
+                                            int64_t sa, int k0, int n, int cl, RefPhase* ph) {
+  using W = Wide<NS, R, M, SPARE>;
 #pragma unroll 1
-  for (int i = lane; i < W::CS; i += W::TL) {
+  for (int i = cl; i < W::CS; i += W::CL) {
     const int k = k0 + i;
     if (k < n) {
       const float th = step_angle(steps[k], ang, sa);
       if constexpr (REF) ph->add(th);
-      bs[i] = exp_minus_i(th);
+      bs[i] = POLY ? step_coeff<false>(th, nullptr) : exp_minus_i(th);
     }
   }
 }
 
 // All steps of one simulation; `on_end(blk, t)` runs after every block.
-template <int NS, int R, bool REF, bool COLUMN, typename OnEnd, typename Mod>
+template <int NS, int R, bool REF, bool COLUMN, int SPARE = 0, bool POLY = false, typename OnEnd,
+          typename Mod>
 __device__ __forceinline__ void wide_run(float2 (&t)[1 << R], const Job& J, const float* ang,
-                                         float2* buf, float2* bs, int lane, RefPhase* ph,
+                                         float2* buf, float2* bs, int cl, RefPhase* ph,
                                          OnEnd on_end, Mod&& mod) {
-  using W = Wide<NS, R>;
+  using W = Wide<NS, R, NS, SPARE>;
+  const int lane = cl & (W::TL - 1);
   const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
   const int32_t* resc = J.tab + J.off_svres;
   const int n = J.n_steps;
   for (int kc = 0; kc < n; kc += W::CS) {
     // the previous chunk's last read came before its last exchange
-    wide_coeffs<NS, R, REF>(bs, steps, ang, J.angle_stride_a, kc, n, lane, ph);
+    wide_coeffs<NS, R, REF, NS, SPARE, POLY>(bs, steps, ang, J.angle_stride_a, kc, n, cl, ph);
     lanes_sync<W::T>();
     const int ke = kc + W::CS < n ? kc + W::CS : n;
     for (int k0 = kc; k0 < ke; k0 += NS) {
@@ -227,20 +236,19 @@ __device__ __forceinline__ void wide_load(float2 (&t)[1 << R], const Job& J, int
   }
 }
 
-// Sum over a simulation's lanes; `red`: LDS of T / 64 values, used where it
-// spans several waves.
-template <int NS, int R, typename V>
+// Sum over L neighbouring lanes; `red`: LDS of L / 64 values, used where they
+// span several waves (then the whole workgroup).
+template <int L, typename V>
 __device__ __forceinline__ V lanes_sum(V v, V* red) {
-  using W = Wide<NS, R>;
 #pragma unroll
-  for (int m = (W::TL < 64 ? W::TL : 64) / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-  if constexpr (W::T > 64) {
+  for (int m = (L < 64 ? L : 64) / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+  if constexpr (L > 64) {
     __syncthreads();
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     v = red[0];
 #pragma unroll
-    for (int i = 1; i < W::T / 64; ++i) v += red[i];
+    for (int i = 1; i < L / 64; ++i) v += red[i];
   }
   return v;
 }
@@ -253,33 +261,63 @@ __device__ __forceinline__ float wide_inv_norm(const float2 (&t)[1 << R], const 
 #pragma unroll
   for (int r = 0; r < (1 << R); ++r)
     if (out_pos[(r << (NS - R)) | lane] >= 0) n2 = fmaf(t[r].x, t[r].x, fmaf(t[r].y, t[r].y, n2));
-  return 1.0f / sqrtf(lanes_sum<NS, R>(n2, static_cast<float*>(red)));
+  return 1.0f / sqrtf(lanes_sum<Wide<NS, R>::TL>(n2, static_cast<float*>(red)));
+}
+
+// The same with the squares added in amplitude order on every lane, as the
+// one-simulation-per-lane kernels add them (small states only).
+template <int NS, int R>
+__device__ __forceinline__ float wide_inv_norm_in_order(const float2 (&t)[1 << R],
+                                                        const int32_t* out_pos, float2* buf,
+                                                        int lane) {
+  float n2 = 0.0f;
+  if constexpr (R == NS) {
+#pragma unroll
+    for (int j = 0; j < (1 << NS); ++j)
+      if (out_pos[j] >= 0) n2 = fmaf(t[j].x, t[j].x, fmaf(t[j].y, t[j].y, n2));
+  } else {
+    lanes_sync<Wide<NS, R>::TL>();
+#pragma unroll
+    for (int r = 0; r < (1 << R); ++r) buf[padded((r << (NS - R)) | lane)] = t[r];
+    lanes_sync<Wide<NS, R>::TL>();
+#pragma unroll
+    for (int j = 0; j < (1 << NS); ++j) {
+      const float2 v = buf[padded(j)];
+      if (out_pos[j] >= 0) n2 = fmaf(v.x, v.x, fmaf(v.y, v.y, n2));
+    }
+  }
+  return 1.0f / sqrtf(n2);
 }
 
 // Simulation g of job J on the lanes of one group (inactive groups run the
 // last simulation and store nothing).
-template <int NS, int R, bool REF, bool COLUMN>
+template <int NS, int R, bool REF, bool COLUMN, int SPARE = 0>
 __device__ __forceinline__ void wide_sim(const Job& J, int64_t g, bool active, uint32_t flags,
-                                         float2* buf, float2* bs, int lane) {
-  using W = Wide<NS, R>;
+                                         float2* buf, float2* bs, int cl) {
+  using W = Wide<NS, R, NS, SPARE>;
+  const int lane = cl & (W::TL - 1);
   const int64_t gg = active ? g : J.total - 1;
   int64_t bi, si;
   split_sim(J, gg, &bi, &si);
   float2 t[W::NR];
   wide_load<NS, R>(t, J, si, lane);
   RefPhase rp;
-  wide_run<NS, R, REF, COLUMN>(t, J, J.angles + bi * J.angle_stride, buf, bs, lane, &rp,
-                               [](int, const float2 (&)[W::NR]) {}, NoModify());
+  constexpr bool kLaneKernelToo = NS <= 6;   // then equal to it bit for bit
+  wide_run<NS, R, REF, COLUMN, SPARE, kLaneKernelToo>(
+      t, J, J.angles + bi * J.angle_stride, buf, bs, cl, &rp, [](int, const float2 (&)[W::NR]) {},
+      NoModify());
   if constexpr (REF) {
-    rp.m_sum = lanes_sum<NS, R>(rp.m_sum, reinterpret_cast<int32_t*>(bs));
-    rp.th_sum = lanes_sum<NS, R>(rp.th_sum, reinterpret_cast<double*>(bs));
+    rp.m_sum = lanes_sum<W::CL>(rp.m_sum, reinterpret_cast<int32_t*>(bs));
+    rp.th_sum = lanes_sum<W::CL>(rp.th_sum, reinterpret_cast<double*>(bs));
   }
   const float2 ph = REF ? rp.value() : make_float2(1.0f, 0.0f);
   const int32_t* out_pos = J.tab + J.off_out;
-  const float scale = (flags & MBQC_FLAG_RENORMALIZE) ? wide_inv_norm<NS, R>(t, out_pos, lane, bs)
-                                                      : sv_final_scale(J.e_sv);
+  float scale;
+  if (!(flags & MBQC_FLAG_RENORMALIZE)) scale = sv_final_scale(J.e_sv);
+  else if constexpr (kLaneKernelToo) scale = wide_inv_norm_in_order<NS, R>(t, out_pos, buf, lane);
+  else scale = wide_inv_norm<NS, R>(t, out_pos, lane, bs);
   const float2 f = cscale(ph, scale);
-  if (active) {
+  if (active && cl < W::TL) {
     float2* o = J.out + g * (int64_t(1) << J.n_out);
 #pragma unroll
     for (int r = 0; r < W::NR; ++r) {
@@ -290,14 +328,14 @@ __device__ __forceinline__ void wide_sim(const Job& J, int64_t g, bool active, u
   }
 }
 
-template <int NS, int R, bool REF, bool COLUMN>
-__global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_sv(Job J, uint32_t flags) {
-  using W = Wide<NS, R>;
+template <int NS, int R, bool REF, bool COLUMN, int SPARE = 0>
+__global__ __launch_bounds__((Wide<NS, R, NS, SPARE>::T)) void k_wide_sv(Job J, uint32_t flags) {
+  using W = Wide<NS, R, NS, SPARE>;
   __shared__ float2 lds[W::G * W::SIM];
-  const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
+  const int sub = threadIdx.x / W::CL, cl = threadIdx.x % W::CL;
   float2* buf = lds + sub * W::SIM;
   const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
-  wide_sim<NS, R, REF, COLUMN>(J, g, g < J.total, flags, buf, buf + W::BUF, lane);
+  wide_sim<NS, R, REF, COLUMN, SPARE>(J, g, g < J.total, flags, buf, buf + W::BUF, cl);
 }
 
 // Sampled outcomes: the frame and draws of SampleMod, evaluated identically by
@@ -756,7 +794,7 @@ __global__ __launch_bounds__((Wide<kTileBits, kTileRegBits>::T)) void k_tile_pas
       n2 = fmaf(t[r].x, t[r].x, fmaf(t[r].y, t[r].y, n2));
     }
   }
-  n2 = lanes_sum<kTileBits, kTileRegBits>(n2, red);
+  n2 = lanes_sum<256>(n2, red);
   if (lane == 0) norms[blockIdx.x] = n2;
 }
 
@@ -778,15 +816,15 @@ __global__ __launch_bounds__(256) void k_tile_finish(Job J, const float* __restr
     const float* ang = J.angles + bi * J.angle_stride;
     RefPhase rp;
     for (int k = tid; k < J.n_steps; k += 256) rp.add(step_angle(steps[k], ang, J.angle_stride_a));
-    rp.m_sum = lanes_sum<kTileBits, kTileRegBits>(rp.m_sum, red_i);
-    rp.th_sum = lanes_sum<kTileBits, kTileRegBits>(rp.th_sum, red_d);
+    rp.m_sum = lanes_sum<256>(rp.m_sum, red_i);
+    rp.th_sum = lanes_sum<256>(rp.th_sum, red_d);
     ph = rp.value();
   }
   float scale = sv_final_scale(J.e_sv);
   if (flags & MBQC_FLAG_RENORMALIZE) {
     float n2 = 0.0f;
     for (int i = tid; i < tiles; i += 256) n2 += norms[l * tiles + i];
-    scale = 1.0f / sqrtf(lanes_sum<kTileBits, kTileRegBits>(n2, red_f));
+    scale = 1.0f / sqrtf(lanes_sum<256>(n2, red_f));
   }
   const float2 f = cscale(ph, scale);
   const int64_t dout = int64_t(1) << J.n_out;
@@ -824,6 +862,47 @@ hipError_t sv_launch(const Job& J, bool column, uint32_t flags, hipStream_t st) 
     else hipLaunchKernelGGL((k_wide_sv<NS, R, false, false>), grid, block, 0, st, J, flags);
   }
   return hipGetLastError();
+}
+
+// Windows of 1..6 slots with too few simulations to fill the chip at one per
+// lane, where a launch takes as long as one lane's chain of steps: here the
+// lanes of a group share a simulation's coefficients (one step per lane) and,
+// from 4 slots on, its amplitudes, 4 per lane.  A group is a whole wave up to
+// 1,024 simulations (one wave per SIMD), else at least 8 lanes.
+constexpr int narrow_reg_bits(int ns) { return ns <= 3 ? ns : 2; }
+
+// Most simulations that run so.  Measured in replayed graphs, 30-column grids,
+// us per launch (one lane per simulation / this): 2 slots 64 sims 8.1 / 6.4,
+// 4,096 9.7 / 9.4, 8,192 9.9 / 10.0; 3 slots 64 13.3 / 9.8, 1,024 14.0 / 11.9,
+// 4,096 14.3 / 14.6; 4 slots 64 22.4 / 11.2, 8,192 23.6 / 20.4, 16,384
+// 24.0 / 23.8, 32,768 24.8 / 38.5; 5 slots 64 45.5 / 14.1, 16,384 48.0 / 32.4,
+// 32,768 49.9 / 54.2; 6 slots 64 86 / 14.7, 32,768 94.7 / 75.6.  One slot: no gain.
+constexpr int64_t kNarrowMaxSims[7] = {0, 0, 4096, 2048, 16384, 16384, 32768};
+
+template <int NS, int SPARE>
+hipError_t narrow_launch(const Job& J, bool column, uint32_t flags, hipStream_t st) {
+  constexpr int R = narrow_reg_bits(NS);
+  using W = Wide<NS, R, NS, SPARE>;
+  const dim3 grid(unsigned((J.total + W::G - 1) / W::G)), block(W::T);
+  const bool ref = flags & MBQC_FLAG_REF_PHASE;
+#define MBQC_NARROW(REF, COL) \
+  hipLaunchKernelGGL((k_wide_sv<NS, R, REF, COL, SPARE>), grid, block, 0, st, J, flags)
+  if (column) {
+    if (ref) MBQC_NARROW(true, true);
+    else MBQC_NARROW(false, true);
+  } else {
+    if (ref) MBQC_NARROW(true, false);
+    else MBQC_NARROW(false, false);
+  }
+#undef MBQC_NARROW
+  return hipGetLastError();
+}
+
+template <int NS>
+hipError_t narrow_launch(const Job& J, bool column, uint32_t flags, hipStream_t st) {
+  constexpr int lane_bits = NS - narrow_reg_bits(NS);
+  if (J.total <= 1024) return narrow_launch<NS, 6 - lane_bits>(J, column, flags, st);
+  return narrow_launch<NS, (lane_bits < 3 ? 3 - lane_bits : 0)>(J, column, flags, st);
 }
 
 template <int NS>
@@ -879,6 +958,19 @@ hipError_t batch_launch(bool column, int64_t waves, const Job* jobs, const Batch
     case 14: return CALL(14);             \
     default: return hipErrorInvalidValue; \
   }
+
+bool narrow_sv(const Job& J) { return J.ns <= 6 && J.total <= kNarrowMaxSims[J.ns]; }
+
+hipError_t launch_narrow_sv(const Job& J, bool column, uint32_t flags, hipStream_t st) {
+  switch (J.ns) {
+    case 2: return narrow_launch<2>(J, column, flags, st);
+    case 3: return narrow_launch<3>(J, column, flags, st);
+    case 4: return narrow_launch<4>(J, column, flags, st);
+    case 5: return narrow_launch<5>(J, column, flags, st);
+    case 6: return narrow_launch<6>(J, column, flags, st);
+    default: return hipErrorInvalidValue;
+  }
+}
 
 hipError_t launch_wide_sv(const Job& J, bool column, uint32_t flags, hipStream_t st) {
 #define MBQC_CALL(NS) sv_launch<NS>(J, column, flags, st)

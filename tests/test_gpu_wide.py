@@ -99,3 +99,55 @@ def test_wide_adjoint_matches_complex128(rows, cols, C, B, rng):
     # sqrt(2 C): far below 2e-5 of the largest entry
     assert oerr < 2e-5, f"output error {oerr}"
     assert gerr < 2e-5 * max(scale, 1.0), f"gradient error {gerr} of {scale}"
+
+
+@pytest.mark.parametrize("rows,cols,window,B,S", [
+    (2, 5, None, 1, 1), (2, 40, None, 2050, 1), (3, 5, None, 1, 1), (3, 30, None, 7, 3),
+    (4, 20, None, 1, 1), (4, 20, None, 1023, 2), (4, 5, None, 4, 4096), (5, 14, None, 9, 1),
+    (5, 6, None, 2049, 1), (6, 13, None, 3, 1), (6, 5, None, 1100, 3), (3, 6, 5, 5, 3),
+    (4, 6, 6, 5, 300), (5, 5, 7, 11, 1), (2, 6, 7, 3, 2)])
+def test_narrow_windows_small_batches(rows, cols, window, B, S, rng):
+    """Batches below the one-simulation-per-lane kernel's share of the chip: a
+    whole wave or a few lanes per simulation, partly filled last workgroups,
+    several coefficient chunks, column and general plans."""
+    torch = _torch()
+    import mentpy_amd as mp
+    from mentpy_amd.simulators.hip_simulator import sv_forward, _as_angles, _as_states
+    from oracle.vectorized import sv_batch
+    g = mp.templates.grid_cluster(rows, cols)
+    sim = mp.PatternSimulator(g, backend="hip-sv", **({"window_size": window} if window else {}))
+    plan = sim.simulator.plan
+    th = rng.uniform(-7, 7, (B, len(g.trainable_nodes))).astype(np.float32)
+    psi = np.stack([haar_state(rows, rng) for _ in range(S)])
+    dev = torch.device("cuda")
+    a, s = _as_angles(th, plan.info["n_angles"], dev), _as_states(psi, plan.info["n_inputs"], dev)
+    guard = torch.full((B + 1, S, 1 << rows), 7.0, dtype=torch.complex64, device=dev)
+    out, phase = sv_forward(plan, a, s, out=guard[:B], want_phase=True)
+    table = sv_forward(plan, a, s, table_steps=True)
+    raw = sv_forward(plan, a, s, ref_phase=False, renormalize=False)
+    torch.cuda.synchronize()
+    assert torch.equal(out, table), "compile-time and table steps differ"
+    assert (guard[B] == 7.0).all(), "a store past the last simulation"
+    rows_b = sorted({0, B // 2, B - 1})
+    ref = sv_batch(g, th[rows_b].astype(np.float64), psi)
+    assert np.abs(out[rows_b].cpu().numpy() - ref).max() < 2e-5
+    assert (raw * phase[..., None] - out).abs().max().item() < 2e-5
+
+
+@pytest.mark.parametrize("rows,B", [(2, 4097), (3, 2049), (4, 16385), (5, 16385), (6, 32769)])
+def test_narrow_windows_lane_kernel_above_the_threshold(rows, B, rng):
+    """The first batch above the threshold (one simulation per lane) against
+    the oracle and, row by row, against the small-batch kernel."""
+    torch = _torch()
+    import mentpy_amd as mp
+    from oracle.vectorized import sv_batch
+    g = mp.templates.grid_cluster(rows, 9)
+    sim = mp.PatternSimulator(g, backend="hip-sv")
+    gen = torch.Generator().manual_seed(rows)
+    th = (torch.rand((B, len(g.trainable_nodes)), generator=gen) * 6.2).cuda()
+    psi = haar_state(rows, rng)
+    full = sim.run_batch(th, psi)
+    small = sim.run_batch(th[-40:].contiguous(), psi)
+    assert torch.equal(full[-40:], small), "the two kernels differ"
+    ref = sv_batch(g, th[:8].double().cpu().numpy(), psi[None])
+    assert np.abs(full[:8].cpu().numpy() - ref).max() < 2e-5
