@@ -191,13 +191,24 @@ int mbqc_plan_get_rescale(const mbqc_plan* plan, int32_t* sv_flags, int32_t* dm_
  * angle_stride_a = B, gives coalesced loads) and input s at
  * psi_in + s*in_stride amplitudes (in_stride 0 = shared).  out is
  * [B*S][2^n_outputs]; phase_out (optional, MBQC_FLAG_WRITE_PHASE) is [B*S].
- * Live windows up to 20 slots: up to 6 with the state in registers, 7..14 in
- * LDS, 15..20 in a workspace of 2^n_slots complex64 per simulation that the
+ * Live windows up to 20 slots: up to 14 with the state in registers and LDS,
+ * 15..20 in a workspace of about 2 x 2^n_slots complex64 per simulation that the
  * call allocates and frees in stream order (hipMallocAsync / hipFreeAsync on
  * `stream`, at most 4 GiB per launch, larger batches in chunks). */
 int mbqc_sv_forward_c64(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
                         int64_t angle_stride_a, const void* psi_in, int64_t in_stride, void* out,
                         void* phase_out, int64_t B, int64_t S, uint32_t flags, void* stream);
+
+/* One post-selected simulation from and to host memory, done when the call
+ * returns (NumpySimulatorSV.run, np_simulator_sv.py:227-297): angles[n_angles]
+ * and psi_in[2^n_inputs] are ordinary host memory, out[2^n_outputs] is pinned
+ * host memory that the device can write (hipHostMalloc).  One launch that takes
+ * the inputs by value, no copies; waits for `stream`.  Results equal
+ * mbqc_sv_forward_c64's bit for bit.  Live windows of at most 6 slots in
+ * schedule order and 2 x 2^n_inputs + n_angles <= 896, else
+ * MBQC_ERR_NOT_IMPLEMENTED; not under graph capture (MBQC_ERR_RUNTIME). */
+int mbqc_sv_run_host_c64(const mbqc_plan* plan, const float* angles, const void* psi_in, void* out,
+                         uint32_t flags, void* stream);
 
 /* Sampled outcomes with flow corrections (force0=False), complex64: the
  * semantics of the PennyLane backend (mentpy/simulators/pennylane_simulator.py:138-153):

@@ -39,7 +39,7 @@ PLANE_Z = 3
 
 EXPORTED_SYMBOLS = (
     "mbqc_causal_flow", "mbqc_plan_create", "mbqc_plan_upload", "mbqc_plan_destroy", "mbqc_plan_get_info", "mbqc_plan_get_tables",
-    "mbqc_plan_get_rescale", "mbqc_sv_forward_c64", "mbqc_sv_sample_c64", "mbqc_dm_forward_c64",
+    "mbqc_plan_get_rescale", "mbqc_sv_forward_c64", "mbqc_sv_run_host_c64", "mbqc_sv_sample_c64", "mbqc_dm_forward_c64",
     "mbqc_dm_forward_outcomes_c64",
     "mbqc_plan_window_qubits", "mbqc_sv_window_c64", "mbqc_dm_window_c64",
     "mbqc_gram_workspace_bytes", "mbqc_gram_loss_seed_c64", "mbqc_gram_loss_seed_c64_noalloc",
@@ -125,6 +125,8 @@ def lib() -> C.CDLL:
     L.mbqc_plan_get_rescale.restype = C.c_int
     L.mbqc_sv_forward_c64.argtypes = [vp, vp, i64, i64, vp, i64, vp, vp, i64, i64, u32, vp]
     L.mbqc_sv_forward_c64.restype = C.c_int
+    L.mbqc_sv_run_host_c64.argtypes = [vp, vp, vp, vp, u32, vp]
+    L.mbqc_sv_run_host_c64.restype = C.c_int
     L.mbqc_gram_workspace_bytes.argtypes = [i64, i32]
     L.mbqc_gram_workspace_bytes.restype = sz
     L.mbqc_gram_loss_seed_c64.argtypes = [vp, vp, i64, i32, i32, vp, vp, vp, vp]
@@ -206,6 +208,37 @@ def check(rc: int) -> None:
     raise RuntimeError(msg)
 
 
+def launch(device, fn, *args) -> None:
+    """``fn(*args, stream)`` on the current stream of ``device`` (where the
+    operands live), with that device current; raises on a failed launch."""
+    import torch
+    cur = torch._C._cuda_getDevice()
+    idx = device.index
+    if idx is None or idx == cur:
+        rc = fn(*args, torch._C._cuda_getCurrentRawStream(cur))
+    else:
+        with torch.cuda.device(device):
+            rc = fn(*args, torch._C._cuda_getCurrentRawStream(idx))
+    if rc != MBQC_OK:
+        check(rc)
+
+
+# Pinned host buffer of each thread (and device) that host runs write their
+# output to: a call fills it and copies it out before it returns.
+_pinned = threading.local()
+
+
+def pinned_output(device_index: int, n: int):
+    """``n`` complex64 in this thread's pinned buffer: ``(address, array)``."""
+    import torch
+    bufs = _pinned.__dict__
+    buf = bufs.get(device_index)
+    if buf is None or buf[1].shape[0] < n:
+        t = torch.empty(max(n, 64), dtype=torch.complex64, pin_memory=True)
+        buf = bufs[device_index] = (t, t.numpy(), t.data_ptr())
+    return buf[2], buf[1][:n]
+
+
 def _i32(a) -> np.ndarray:
     return np.ascontiguousarray(np.asarray(a, dtype=np.int32))
 
@@ -241,6 +274,8 @@ def release_pending() -> int:
 
 class NativePlan:
     """Owner of an ``mbqc_plan*`` compiled from flat pattern arrays."""
+
+    all_angles_used = False   # set by the compiler of a pattern whose angles all are
 
     def __init__(self, n_nodes: int, edges, schedule, n_measure: int, window: int,
                  input_nodes, output_nodes, angle_index, fixed_angle, n_angles: int,

@@ -144,18 +144,16 @@ class BatchedForward:
             group_waves = cfg.get("group_waves")
         flags = ((nat.FLAG_REF_PHASE if ref_phase else 0) | (nat.FLAG_RENORMALIZE if renormalize else 0)
                  | (nat.FLAG_TABLE_STEPS if table_steps else 0))
-        stream = C.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
-        with torch.cuda.device(self.device):
-            if group_waves is not None:
-                gw = [int(x) for x in group_waves]
-                if len(gw) > MAX_GROUPS:
-                    raise ValueError(f"group_waves has at most {MAX_GROUPS} entries")
-                arr = (C.c_int32 * len(gw))(*gw)
-                nat.check(nat.lib().mbqc_batch_launch_groups(self._handle, arr, len(gw), wg, flags,
-                                                             stream))
-            else:
-                waves = int(waves or cfg["waves"])
-                nat.check(nat.lib().mbqc_batch_launch(self._handle, waves, wg, flags, stream))
+        if group_waves is not None:
+            gw = [int(x) for x in group_waves]
+            if len(gw) > MAX_GROUPS:
+                raise ValueError(f"group_waves has at most {MAX_GROUPS} entries")
+            arr = (C.c_int32 * len(gw))(*gw)
+            nat.launch(self.device, nat.lib().mbqc_batch_launch_groups, self._handle, arr, len(gw),
+                       wg, flags)
+        else:
+            waves = int(waves or cfg["waves"])
+            nat.launch(self.device, nat.lib().mbqc_batch_launch, self._handle, waves, wg, flags)
         return self.outputs
 
     def capture_graph(self, **launch_kwargs):

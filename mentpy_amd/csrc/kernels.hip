@@ -3997,6 +3997,39 @@ int mbqc_sv_forward_c64(const mbqc_plan* plan, const float* angles, int64_t angl
   return e == hipSuccess ? MBQC_OK : hip_fail(e, "sv_forward launch");
 }
 
+int mbqc_sv_run_host_c64(const mbqc_plan* plan, const float* angles, const void* psi_in, void* out,
+                         uint32_t flags, void* stream) {
+  if (!plan) return fail(MBQC_ERR_VALUE, "null plan");
+  Plan* p = const_cast<Plan*>(reinterpret_cast<const Plan*>(plan));
+  int rc = check_xy_plan(p);
+  if (rc != MBQC_OK) return rc;
+  const int first_angle = 2 << p->n_in, words = first_angle + p->n_angles;
+  if (p->ns > kMaxSvSlots || !p->rotating || words > kHostInputWords)
+    return fail(MBQC_ERR_NOT_IMPLEMENTED,
+                "host runs support live windows of at most " + std::to_string(kMaxSvSlots) +
+                    " qubits in schedule order and " + std::to_string(kHostInputWords) +
+                    " input words");
+  Job J;
+  rc = make_job(p, angles, 0, 1, psi_in, 0, out, 1, 1, &J);
+  if (rc != MBQC_OK) return rc;
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  hipError_t e = hipStreamIsCapturing(st, &cs);
+  if (e == hipSuccess && cs != hipStreamCaptureStatusNone)
+    return fail(MBQC_ERR_RUNTIME, "a run that returns to the host cannot be captured in a HIP graph");
+  if (e == hipSuccess) {
+    HostInputs in{};
+    in.n_words = words;
+    in.first_angle = first_angle;
+    std::memcpy(in.word, psi_in, sizeof(float2) << p->n_in);
+    if (p->n_angles > 0) std::memcpy(in.word + first_angle, angles, sizeof(float) * p->n_angles);
+    e = launch_run_one(J, in, p->column_steps && !(flags & MBQC_FLAG_TABLE_STEPS),
+                       flags & ~uint32_t(MBQC_FLAG_WRITE_PHASE), st);
+  }
+  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  return e == hipSuccess ? MBQC_OK : hip_fail(e, "host run");
+}
+
 int mbqc_sv_sample_c64(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
                        int64_t angle_stride_a, const void* psi_in, int64_t in_stride, void* out,
                        int32_t* outcomes, int64_t B, int64_t S, uint64_t seed, void* stream) {

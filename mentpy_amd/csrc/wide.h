@@ -13,6 +13,15 @@ hipError_t launch_wide_sv(const Job& J, bool column, uint32_t flags, hipStream_t
 // too small for one simulation per lane.
 bool narrow_sv(const Job& J);
 hipError_t launch_narrow_sv(const Job& J, bool column, uint32_t flags, hipStream_t st);
+// One simulation of a window of 1..6 slots, its input state (2^n_in amplitudes,
+// from word 0) and angles (from word first_angle) passed by value.
+constexpr int kHostInputWords = 896;   // with the Job within the 4 KiB of kernel arguments
+struct HostInputs {
+  int32_t n_words, first_angle;
+  uint32_t word[kHostInputWords];
+};
+hipError_t launch_run_one(const Job& J, const HostInputs& in, bool column, uint32_t flags,
+                          hipStream_t st);
 // Windows of 15..20 slots: simulations [g0, g0 + n) in passes over tiles of
 // their states, in a workspace of n * wide_tile_bytes(ns) bytes.
 size_t wide_tile_bytes(int ns);

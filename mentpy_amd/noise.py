@@ -63,6 +63,14 @@ class NoiseModel:
         raise ValueError(f"Unrecognized circuit noise: {circuit_noise}")
 
     def native(self):
+        """The C struct of these (immutable) parameters, built once."""
+        struct = self.__dict__.get("_struct")
+        if struct is None:
+            struct = self._native()
+            object.__setattr__(self, "_struct", struct)
+        return struct
+
+    def _native(self):
         from . import _native as nat
         return nat.Noise(p_depol=self.depolarizing, p_readout=self.readout_flip,
                          amp_damping=self.amplitude_damping, phase_damping=self.phase_damping,

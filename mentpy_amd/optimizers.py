@@ -126,15 +126,12 @@ class DeviceAdam:
         self.t = torch.zeros(1, dtype=torch.int32, device=params.device)
 
     def step(self, grad):
-        import ctypes as C
         import torch
         from . import _native as nat
         g = grad.to(torch.float32).contiguous()
-        stream = C.c_void_p(torch.cuda.current_stream(self.params.device).cuda_stream)
-        nat.check(nat.lib().mbqc_adam_step_f32(
-            C.c_void_p(self.params.data_ptr()), C.c_void_p(g.data_ptr()), C.c_void_p(self.m.data_ptr()),
-            C.c_void_p(self.v.data_ptr()), self.params.numel(), self.step_size, self.b1, self.b2,
-            self.eps, C.c_void_p(self.t.data_ptr()), stream))
+        nat.launch(self.params.device, nat.lib().mbqc_adam_step_f32, self.params.data_ptr(),
+                   g.data_ptr(), self.m.data_ptr(), self.v.data_ptr(), self.params.numel(),
+                   self.step_size, self.b1, self.b2, self.eps, self.t.data_ptr())
 
 
 class DeviceSGD:
@@ -149,14 +146,12 @@ class DeviceSGD:
         self.v = torch.zeros_like(params)
 
     def step(self, grad):
-        import ctypes as C
         import torch
         from . import _native as nat
         g = grad.to(torch.float32).contiguous()
-        stream = C.c_void_p(torch.cuda.current_stream(self.params.device).cuda_stream)
-        nat.check(nat.lib().mbqc_sgd_step_f32(
-            C.c_void_p(self.params.data_ptr()), C.c_void_p(g.data_ptr()), C.c_void_p(self.v.data_ptr()),
-            self.params.numel(), self.step_size, self.momentum, int(self.nesterov), stream))
+        nat.launch(self.params.device, nat.lib().mbqc_sgd_step_f32, self.params.data_ptr(),
+                   g.data_ptr(), self.v.data_ptr(), self.params.numel(), self.step_size,
+                   self.momentum, int(self.nesterov))
 
 
 class MBQMLTrainer:

@@ -170,6 +170,8 @@ def compile_pattern(mbqcircuit, schedule=None, window_size: int = 1, exclude: st
         n_angles=len(trainable), flow=flow, plane=plane if plane.any() else None,
         measure_order=None if order == sched_meas else [idx[v] for v in order])
     plan.measure_order = order
+    # every entry of an angle vector belongs to some measured node
+    plan.all_angles_used = len(set(angle_index[angle_index >= 0].tolist())) == len(trainable)
     return plan, schedule, sched_meas, int(window_size)
 
 
@@ -184,6 +186,8 @@ def _as_angles(angles, n_angles: int, device):
     ``[n, B]`` tensor passed as ``.t()`` gives coalesced loads)."""
     torch = _torch()
     a = torch.as_tensor(angles, dtype=torch.float32, device=device)
+    if a.dim() == 2 and a.shape[1] == n_angles and a.stride(1) != 0:
+        return a
     if a.dim() == 1:
         a = a.unsqueeze(0)
     if a.dim() != 2 or a.shape[1] != n_angles:
@@ -200,6 +204,9 @@ def _angle_strides(a):
 def _as_states(states, n_qubits: int, device):
     torch = _torch()
     s = torch.as_tensor(states, device=device)
+    if (s.dtype == torch.complex64 and s.dim() == 2 and s.shape[1] == (1 << n_qubits)
+            and s.is_contiguous()):
+        return s
     if not torch.is_complex(s):
         s = s.to(torch.float32)
     s = s.to(torch.complex64)
@@ -210,8 +217,11 @@ def _as_states(states, n_qubits: int, device):
     return s.contiguous()
 
 
-def _require_gpu(device):
+def _require_gpu(device, *operands):
+    """Raise without a GPU; operands already on one show that there is."""
     torch = _torch()
+    if device.type == "cuda" and any(isinstance(x, torch.Tensor) and x.is_cuda for x in operands):
+        return
     if device.type != "cuda" or not torch.cuda.is_available():
         raise RuntimeError("hip backends need a ROCm GPU device (device='cuda')")
 
@@ -226,7 +236,7 @@ def sv_forward(plan: nat.NativePlan, angles, states, *, ref_phase: bool = True,
     other plan; both give identical results."""
     torch = _torch()
     device = states.device
-    _require_gpu(device)
+    _require_gpu(device, states)
     info = plan.info
     B, S = angles.shape[0], states.shape[0]
     if out is None:
@@ -236,12 +246,9 @@ def sv_forward(plan: nat.NativePlan, angles, states, *, ref_phase: bool = True,
              | (nat.FLAG_WRITE_PHASE if want_phase else 0)
              | (nat.FLAG_TABLE_STEPS if table_steps else 0))
     sb, sa = _angle_strides(angles)
-    with torch.cuda.device(device):
-        nat.check(nat.lib().mbqc_sv_forward_c64(
-            plan.handle, C.c_void_p(angles.data_ptr()), sb, sa,
-            C.c_void_p(states.data_ptr()), states.shape[1], C.c_void_p(out.data_ptr()),
-            C.c_void_p(phase.data_ptr() if phase is not None else 0), B, S, flags,
-            _stream_ptr(device)))
+    nat.launch(device, nat.lib().mbqc_sv_forward_c64, plan.handle, angles.data_ptr(), sb, sa,
+               states.data_ptr(), states.shape[1], out.data_ptr(),
+               phase.data_ptr() if phase is not None else 0, B, S, flags)
     return (out, phase) if want_phase else out
 
 
@@ -256,7 +263,7 @@ def sv_sample(plan: nat.NativePlan, angles, states, seed: int, *, out=None, outc
     """
     torch = _torch()
     device = states.device
-    _require_gpu(device)
+    _require_gpu(device, states)
     info = plan.info
     B, S = angles.shape[0], states.shape[0]
     W = (info["n_steps"] + 31) // 32
@@ -265,12 +272,9 @@ def sv_sample(plan: nat.NativePlan, angles, states, seed: int, *, out=None, outc
     if outcomes is None:
         outcomes = torch.empty((B, S, W + 2), dtype=torch.int32, device=device)
     sb, sa = _angle_strides(angles)
-    with torch.cuda.device(device):
-        nat.check(nat.lib().mbqc_sv_sample_c64(
-            plan.handle, C.c_void_p(angles.data_ptr()), sb, sa,
-            C.c_void_p(states.data_ptr()), states.shape[1], C.c_void_p(out.data_ptr()),
-            C.c_void_p(outcomes.data_ptr()), B, S, C.c_uint64(int(seed) & (2 ** 64 - 1)),
-            _stream_ptr(device)))
+    nat.launch(device, nat.lib().mbqc_sv_sample_c64, plan.handle, angles.data_ptr(), sb, sa,
+               states.data_ptr(), states.shape[1], out.data_ptr(), outcomes.data_ptr(), B, S,
+               int(seed) & (2 ** 64 - 1))
     return out, outcomes
 
 
@@ -293,7 +297,7 @@ def dm_forward(plan: nat.NativePlan, angles, states, *, p_depol: float = 0.0,
     (a float32 ``[B, S, n_steps]`` device tensor) also receives the outcomes."""
     torch = _torch()
     device = states.device
-    _require_gpu(device)
+    _require_gpu(device, states)
     info = plan.info
     B, S = angles.shape[0], states.shape[0]
     d = 1 << info["n_outputs"]
@@ -307,19 +311,15 @@ def dm_forward(plan: nat.NativePlan, angles, states, *, p_depol: float = 0.0,
              | (nat.FLAG_TABLE_STEPS if table_steps else 0)
              | (nat.FLAG_STEP_PROBS if step_probs else 0))
     sb, sa = _angle_strides(angles)
-    with torch.cuda.device(device):
-        if outcomes is not None:
-            if tuple(outcomes.shape) != (B, S, info["n_steps"]) or outcomes.dtype != torch.float32:
-                raise ValueError(f"outcomes must be a float32 tensor of shape {(B, S, info['n_steps'])}")
-            nat.check(nat.lib().mbqc_dm_forward_outcomes_c64(
-                plan.handle, C.c_void_p(angles.data_ptr()), sb, sa,
-                C.c_void_p(states.data_ptr()), states.shape[1], C.c_void_p(out.data_ptr()),
-                C.c_void_p(outcomes.data_ptr()), B, S, C.byref(noise), flags, _stream_ptr(device)))
-        else:
-            nat.check(nat.lib().mbqc_dm_forward_c64(
-                plan.handle, C.c_void_p(angles.data_ptr()), sb, sa,
-                C.c_void_p(states.data_ptr()), states.shape[1], C.c_void_p(out.data_ptr()), B, S,
-                C.byref(noise), flags, _stream_ptr(device)))
+    if outcomes is not None:
+        if tuple(outcomes.shape) != (B, S, info["n_steps"]) or outcomes.dtype != torch.float32:
+            raise ValueError(f"outcomes must be a float32 tensor of shape {(B, S, info['n_steps'])}")
+        nat.launch(device, nat.lib().mbqc_dm_forward_outcomes_c64, plan.handle, angles.data_ptr(), sb,
+                   sa, states.data_ptr(), states.shape[1], out.data_ptr(), outcomes.data_ptr(), B, S,
+                   C.byref(noise), flags)
+    else:
+        nat.launch(device, nat.lib().mbqc_dm_forward_c64, plan.handle, angles.data_ptr(), sb, sa,
+                   states.data_ptr(), states.shape[1], out.data_ptr(), B, S, C.byref(noise), flags)
     return out
 
 
@@ -387,7 +387,8 @@ class _HipBackend(BaseSimulator):
     @property
     def device(self):
         torch = _torch()
-        return torch.device(self._device_arg)
+        dev = self._device_arg
+        return dev if isinstance(dev, torch.device) else torch.device(dev)
 
     def _set_input(self, state):
         n_in = len(self.mbqcircuit.input_nodes)
@@ -465,7 +466,7 @@ class _HipBackend(BaseSimulator):
     def _finish_run(self, bits=None):
         self.current_measurement = len(self.schedule_measure)
         if bits is None:
-            self.outcomes = {v: 0 for v in self.measure_order}
+            self.outcomes = dict.fromkeys(self.measure_order, 0)
         else:
             self.outcomes = {v: int(b) for v, b in zip(self.measure_order, bits)}
 
@@ -524,21 +525,51 @@ class HipSimulatorSV(_HipBackend):
         if mbqcircuit.classical_output_nodes:
             raise NotImplementedError("measured output nodes are not supported by hip-sv")
 
+    @property
+    def _host_run(self) -> bool:
+        """Whether ``run`` is one native call on host memory: windows of at most 6
+        slots whose input and angles fit a launch's arguments (896 words)."""
+        i = self.plan.info
+        return bool(i["n_slots"] <= 6 and i["rotating"]
+                    and (2 << i["n_inputs"]) + i["n_angles"] <= 896)
+
+    def _run_host(self, angles):
+        torch = _torch()
+        dev = self.device
+        _require_gpu(dev)
+        info = self.plan.info
+        a = np.asarray(angles, dtype=np.float64).reshape(-1).astype(np.float32)
+        if a.shape[0] != info["n_angles"]:
+            raise ValueError(f"angles must have shape [B, {info['n_angles']}], got {(1, a.shape[0])}")
+        s = self._input_np.astype(np.complex64)
+        idx = torch.cuda.current_device() if dev.index is None else dev.index
+        flags = ((nat.FLAG_REF_PHASE if self.phase == "reference" else 0)
+                 | (nat.FLAG_RENORMALIZE if self.renormalize else 0))
+        with torch.cuda.device(idx):
+            ptr, out = nat.pinned_output(idx, 1 << info["n_outputs"])
+            nat.check(nat.lib().mbqc_sv_run_host_c64(
+                self.plan.handle, a.ctypes.data, s.ctypes.data, ptr, flags,
+                torch._C._cuda_getCurrentRawStream(idx)))
+        return out.astype(np.complex128)
+
     def run(self, angles, output_form: str = "dm", **kwargs):
         self._check_run(angles, kwargs.get("input_state"))
         form = output_form.lower()
         if form not in ("dm", "densitymatrix", "sv", "statevector"):
             raise ValueError(f"Output form {output_form} is not supported.")
-        a, s = self._device_inputs(angles)
-        if self.force0:
-            out = sv_forward(self.plan, a, s, ref_phase=self.phase == "reference",
-                             renormalize=self.renormalize)
-            bits = None
+        if self.force0 and self._host_run:
+            psi, bits = self._run_host(angles), None
         else:
-            out, rows = sv_sample(self.plan, a, s, self._next_seed())
-            self.last_outcomes = rows
-            bits = decode_outcomes(rows[0, 0], self.plan.info["n_steps"])
-        psi = out[0, 0].cpu().numpy().astype(np.complex128)
+            a, s = self._device_inputs(angles)
+            if self.force0:
+                out = sv_forward(self.plan, a, s, ref_phase=self.phase == "reference",
+                                 renormalize=self.renormalize)
+                bits = None
+            else:
+                out, rows = sv_sample(self.plan, a, s, self._next_seed())
+                self.last_outcomes = rows
+                bits = decode_outcomes(rows[0, 0], self.plan.info["n_steps"])
+            psi = out[0, 0].cpu().numpy().astype(np.complex128)
         self._finish_run(bits)
         self.qstate = psi
         if form in ("dm", "densitymatrix"):
@@ -563,7 +594,7 @@ class HipSimulatorSV(_HipBackend):
         With ``force0=False`` the outcomes are sampled (``last_outcomes`` holds
         the ``[B, S, W + 2]`` outcome words and output frame)."""
         dev = self.device
-        _require_gpu(dev)
+        _require_gpu(dev, angles)
         a = _as_angles(angles, self.plan.info["n_angles"], dev)
         st = self._input_np if input_states is None else input_states
         s = _as_states(st, self.plan.info["n_inputs"], dev)
@@ -617,7 +648,8 @@ class HipSimulatorDM(_HipBackend):
 
     @property
     def _has_z(self):
-        return any(self.mbqcircuit[v].plane == "Z" for v in self.schedule_measure)
+        # a Z node makes the plan a general one (decided when it is compiled)
+        return bool(self.plan.info["general_planes"]) and any(self.mbqcircuit[v].plane == "Z" for v in self.schedule_measure)
 
     @property
     def _exact_probs(self):
@@ -685,7 +717,7 @@ class HipSimulatorDM(_HipBackend):
         receives every simulation's outcomes."""
         self._check_mode(mode)
         dev = self.device
-        _require_gpu(dev)
+        _require_gpu(dev, angles)
         a = _as_angles(angles, self.plan.info["n_angles"], dev)
         st = self._input_np if input_states is None else input_states
         s = _as_states(st, self.plan.info["n_inputs"], dev)

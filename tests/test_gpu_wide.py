@@ -151,3 +151,44 @@ def test_narrow_windows_lane_kernel_above_the_threshold(rows, B, rng):
     assert torch.equal(full[-40:], small), "the two kernels differ"
     ref = sv_batch(g, th[:8].double().cpu().numpy(), psi[None])
     assert np.abs(full[:8].cpu().numpy() - ref).max() < 2e-5
+
+
+@pytest.mark.parametrize("rows,cols,window", [(1, 7, None), (2, 5, None), (3, 4, 5), (4, 20, None),
+                                              (5, 14, None), (6, 30, None), (4, 6, 7)])
+def test_host_runs_equal_batched_runs(rows, cols, window, rng):
+    """run() as one native call on host memory against run_batch on device
+    tensors, bit for bit; raw phase and no renormalisation too; calls from
+    several threads and on a side stream."""
+    import threading
+    torch = _torch()
+    import mentpy_amd as mp
+    g = mp.templates.linear_cluster(cols) if rows == 1 else mp.templates.grid_cluster(rows, cols)
+    n = len(g.trainable_nodes)
+    psi = [haar_state(rows, rng) for _ in range(3)]
+    th = rng.uniform(-7, 7, (3, n))
+    kw = {"window_size": window} if window else {}
+    for extra in ({}, {"phase": "raw"}, {"renormalize": False}):
+        sim = mp.PatternSimulator(g, backend="hip-sv", **kw, **extra)
+        assert sim.simulator._host_run
+        for t, x in zip(th, psi):
+            sim.reset(x)
+            got = sim.run(t, output_form="sv")
+            want = sim.run_batch(t, x)[0, 0].cpu().numpy().astype(np.complex128)
+            assert got.dtype == np.complex128 and np.array_equal(got, want)
+    want = [sim.run_batch(t, x)[0, 0].cpu().numpy() for t, x in zip(th, psi)]
+    bad = []
+
+    def work(i):
+        s = mp.PatternSimulator(g, backend="hip-sv", renormalize=False, **kw)
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(50):
+                s.reset(psi[i])
+                if not np.array_equal(s.run(th[i], output_form="sv"), want[i]):
+                    bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
