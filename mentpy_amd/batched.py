@@ -34,7 +34,7 @@ __all__ = ["BatchedForward", "autotune", "default_cache_path"]
 # global workspace above)
 MAX_GROUPS = 21
 # tag of the cached tuning results (entries timed another way are not reused)
-_TUNE_VERSION = "graph-replay"
+_TUNE_VERSION = "graph-replay, one launch over the register groups"
 
 
 def _torch():
@@ -133,7 +133,8 @@ class BatchedForward:
                group_waves: Optional[Sequence[int]] = None, ref_phase: bool = True,
                renormalize: bool = True, table_steps: bool = False):
         """One persistent launch over every job.  ``waves`` resident
-        wavefronts per live-window group, or ``group_waves[ns]`` for the group
+        wavefronts per live-window group (the groups up to 6 slots then share
+        one kernel), or ``group_waves[ns]`` for a kernel of its own for the group
         of size ns (0 skips that group); without either, the tuned (or
         default) configuration.  ``table_steps`` makes groups of periodic plans
         read the pair coefficients from the tables (same results)."""

@@ -2997,38 +2997,108 @@ __global__ __launch_bounds__(256) void k_dm_general_global(Job J, const float* _
 template <int NS>
 constexpr int kBatchStore = kStoreDirect;
 
+// The simulations of item I of job J, 64 at a time on the wave's lanes.
+template <bool REF, int NS, bool SH, bool PERIODIC>
+__device__ __forceinline__ void batch_item(const Job& J, const BatchItem& I, int lane,
+                                           uint32_t flags) {
+  for (int off = 0; off < I.count; off += 64) {
+    const int64_t g = I.first + off + lane;
+    const int64_t left = J.total - (I.first + off);
+    const int rows = int(std::min<int64_t>(std::min<int64_t>(I.count - off, left), 64));
+    // direct stores: staging tiles would cost the concurrently running
+    // window-size groups LDS occupancy (measured slower)
+    sv_sim<NS, REF, kBatchStore<NS>, false, SH, PERIODIC, false>(
+        J, g, (off + lane) < I.count && g < J.total, rows, flags);
+  }
+}
+
+// The items of a launch, dealt round-robin to `lists` lists with a device counter
+// each; a wave pulls from its own list.  One counter for all is a serial chain:
+// it hands out an item every 20-25 ns, which bounds a batch of short items (64
+// grids of 2..5 rows x 1,024 x 16, 16,384 items of 64 simulations, all window sizes
+// in one launch: 440 us with one counter, 192 with 32).  Items are
+// sorted by decreasing cost, so the lists carry the same work and long items
+// start first.  The host gives every list at least one wave.
+// (The item list stays a __restrict__ kernel argument: from a struct its loads, and
+// with them the whole job, would be per-lane vector loads.)
+struct ItemLists {
+  int64_t n;
+  int* counter;   // of list 0; the others follow kCounterStride ints apart
+  int32_t lists;
+};
+// This wave's list.
+__device__ __forceinline__ int my_list(const ItemLists& Q) {
+  return __builtin_amdgcn_readfirstlane(
+      int(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) % Q.lists);
+}
+// The index of the wave's next item (at least Q.n when its list is done).
+__device__ __forceinline__ int64_t pull_item(const ItemLists& Q, int list) {
+  int k = 0;
+  if ((threadIdx.x & 63) == 0) k = atomicAdd(Q.counter + list * kCounterStride, 1);
+  return list + int64_t(Q.lists) * __builtin_amdgcn_readfirstlane(k);
+}
+
 // Persistent kernel over the work items of one live-window size NS: every
-// wave pulls items (runs of simulations of one job) from its group's device
-// counter until none are left.  Items are sorted by decreasing cost on the
-// host, so long patterns start first.  One kernel per NS keeps each group at
-// the register footprint (and so the occupancy) of its own window size.
+// wave pulls items (runs of simulations of one job) until its list is done (one
+// by one: a wave that pulled ahead would hold items that idle waves could
+// take).  One kernel per NS keeps each group at the register footprint (and so
+// the occupancy) of its own window size.
 template <bool REF, int NS, bool SH, bool PERIODIC>
 __global__ __launch_bounds__(256) void k_batch(const Job* __restrict__ jobs,
-                                               const BatchItem* __restrict__ items, int64_t n_items,
-                                               int* counter, uint32_t flags) {
-  const int lane = threadIdx.x & 63;
+                                               const BatchItem* __restrict__ items, ItemLists Q,
+                                               uint32_t flags) {
+  const int list = my_list(Q);
   for (;;) {
-    int it = 0;
-    if (lane == 0) it = atomicAdd(counter, 1);
-    it = __builtin_amdgcn_readfirstlane(it);
-    if (it >= n_items) break;
+    const int64_t it = pull_item(Q, list);
+    if (it >= Q.n) break;
+    const BatchItem I = items[it];
+    batch_item<REF, NS, SH, PERIODIC>(load_job(jobs, I.job), I, threadIdx.x & 63, flags);
+  }
+}
+
+// The same over the items of all window sizes up to MAXNS, longest first: one
+// launch instead of a kernel per size forked to and joined from side streams.
+// The chip's few hardware queues run some of those one after the other, and each
+// fork and join costs the host and the device several us.  It runs at the
+// register footprint of the largest window size, which costs less than that
+// (call by call, us per launch, a kernel per size / this: 64 grids x 1,024 x 16
+// 221 / 192, 405 before with one counter and every kernel on a side stream;
+// 40 grids x 100 x 3 90 / 48; 8 grids x 16 76 / 24).
+// share: bit ns set where the lanes of that group share coefficients.
+template <bool REF, bool PERIODIC, int MAXNS>
+__global__ __launch_bounds__(256) void k_batch_mixed(const Job* __restrict__ jobs,
+                                                     const BatchItem* __restrict__ items,
+                                                     ItemLists Q, uint32_t flags, uint32_t share) {
+  const int lane = threadIdx.x & 63;
+  const int list = my_list(Q);
+  for (;;) {
+    const int64_t it = pull_item(Q, list);
+    if (it >= Q.n) break;
     const BatchItem I = items[it];
     const Job J = load_job(jobs, I.job);
-    for (int off = 0; off < I.count; off += 64) {
-      const int64_t g = I.first + off + lane;
-      const int64_t left = J.total - (I.first + off);
-      const int rows = int(std::min<int64_t>(std::min<int64_t>(I.count - off, left), 64));
-      // direct stores: staging tiles would cost the concurrently running
-      // window-size groups LDS occupancy (measured slower)
-      sv_sim<NS, REF, kBatchStore<NS>, false, SH, PERIODIC, false>(
-          J, g, (off + lane) < I.count && g < J.total, rows, flags);
+    const bool sh = (share >> J.ns) & 1u;
+#define MBQC_MIXED_CASE(NS)                                                  \
+  case NS:                                                                   \
+    if constexpr (NS <= MAXNS) {                                             \
+      if (NS >= 2 && sh) batch_item<REF, (NS <= MAXNS ? NS : 2), (NS >= 2), PERIODIC>(J, I, lane, flags); \
+      else batch_item<REF, (NS <= MAXNS ? NS : 2), false, PERIODIC>(J, I, lane, flags);                 \
+    }                                                                        \
+    break;
+    switch (J.ns) {
+      MBQC_MIXED_CASE(1)
+      MBQC_MIXED_CASE(2)
+      MBQC_MIXED_CASE(3)
+      MBQC_MIXED_CASE(4)
+      MBQC_MIXED_CASE(5)
+      MBQC_MIXED_CASE(6)
     }
+#undef MBQC_MIXED_CASE
   }
 }
 
 __global__ void k_reset_counters(int* counter, int n) {
-  const int i = threadIdx.x;
-  if (blockIdx.x == 0 && i < n) counter[i * kCounterStride] = 0;
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) counter[i * kCounterStride] = 0;
 }
 
 }  // namespace mbqc
@@ -3550,8 +3620,7 @@ struct BatchGroupLaunch {
   hipStream_t stream;
   const Job* jobs;
   const BatchItem* items;
-  int64_t n_items;
-  int* counter;
+  ItemLists lists;
   uint32_t flags;
 };
 
@@ -3565,7 +3634,7 @@ void launch_batch_group_p(const BatchGroupLaunch& L, bool ref, bool share) {
       kBatchStore<NS> == kStoreColumns ? (L.block.x / 64) * kColumnTile * sizeof(float2) : 0;
 #define MBQC_BATCH_LAUNCH(R, SH)                                                                     \
   hipLaunchKernelGGL((k_batch<R, NS, SH, PER>), L.grid, L.block, lds, L.stream, L.jobs, L.items, \
-                     L.n_items, L.counter, L.flags)
+                     L.lists, L.flags)
   if constexpr (NS >= 2) {
     if (share) {
       if (ref) MBQC_BATCH_LAUNCH(true, true);
@@ -3582,6 +3651,21 @@ template <int NS>
 void launch_batch_group(const BatchGroupLaunch& L, bool ref, bool share, bool periodic) {
   if (periodic) launch_batch_group_p<NS, true>(L, ref, share);
   else launch_batch_group_p<NS, false>(L, ref, share);
+}
+
+template <int MAXNS>
+void launch_batch_mixed(const BatchGroupLaunch& L, bool ref, bool periodic, uint32_t share) {
+#define MBQC_MIXED(R, PER)                                                                         \
+  hipLaunchKernelGGL((k_batch_mixed<R, PER, MAXNS>), L.grid, L.block, 0, L.stream, L.jobs, L.items, \
+                     L.lists, L.flags, share)
+  if (periodic) {
+    if (ref) MBQC_MIXED(true, true);
+    else MBQC_MIXED(false, true);
+  } else {
+    if (ref) MBQC_MIXED(true, false);
+    else MBQC_MIXED(false, false);
+  }
+#undef MBQC_MIXED
 }
 
 template <int NS>
@@ -3805,6 +3889,11 @@ constexpr int64_t kBatchGlobalSims = 128;
 
 }  // namespace
 
+// Item lists of a register group's launch, and the counters of a batch: one set
+// per window size, set 0 for the launch over all register groups.
+constexpr int kItemLists = 32;
+constexpr int kBatchCounters = (kMaxBatchSlots + 1) * kItemLists;
+
 struct mbqc_batch {
   int max_ns = 1;
   int64_t group_begin[kMaxBatchSlots + 1] = {};  // items of live-window size ns
@@ -3813,6 +3902,10 @@ struct mbqc_batch {
   std::vector<BatchItem> items;
   Job* d_jobs = nullptr;
   BatchItem* d_items = nullptr;
+  // the items of the register groups (up to kMaxSvSlots) once more, longest first
+  // whatever their window size, after the grouped ones in d_items
+  int64_t n_mixed = 0;
+  int mixed_groups = 0, mixed_max = 0;
   int* d_counter = nullptr;
   int device = -1;
   // side streams and events that run the window-size groups concurrently
@@ -3834,11 +3927,13 @@ struct mbqc_batch {
 
 // One launch of a batch: the counter reset, then one persistent kernel per
 // live-window size ns with group_waves[ns] > 0 resident wavefronts (capped at
-// the group's item count); with several groups each runs on its own stream,
-// forked from and joined into `stream`.  Groups given no waves are skipped
+// the group's item count); with several groups all but one run on side streams
+// forked from and joined into `stream`.  mixed: the register groups together as
+// one kernel with the sum of their waves.  Groups given no waves are skipped
 // (their outputs are not written).
 static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_waves,
-                        uint32_t flags, void* stream) {
+                        uint32_t flags, bool mixed, void* stream) {
+  bool joined[kMaxBatchSlots + 1] = {};
   if (wg_waves < 1 || wg_waves > 4) return fail(MBQC_ERR_VALUE, "wg_waves must be 1..4");
   int launched = 0;
   for (int ns = 1; ns <= kMaxBatchSlots; ++ns) {
@@ -3848,18 +3943,25 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
   }
   if (bt->items.empty() || launched == 0) return MBQC_OK;
   hipStream_t st = static_cast<hipStream_t>(stream);
-  hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(64), 0, st, bt->d_counter, kMaxBatchSlots + 1);
+  hipLaunchKernelGGL(k_reset_counters, dim3((kBatchCounters + 255) / 256), dim3(256), 0, st,
+                     bt->d_counter, kBatchCounters);
   const int threads = 64 * wg_waves;
   const bool ref = flags & MBQC_FLAG_REF_PHASE;
+  // several register groups with the same resident waves run as one launch
+  mixed = mixed && bt->mixed_groups > 1;
+  const int first_single = mixed ? kMaxSvSlots + 1 : 1;
+  if (mixed) launched -= bt->mixed_groups - 1;
   const bool concurrent = bt->fork != nullptr && launched > 1;
   hipError_t e = hipGetLastError();
   if (e == hipSuccess && concurrent) e = hipEventRecord(bt->fork, st);
-  // largest windows first
-  for (int ns = kMaxBatchSlots; ns >= 1 && e == hipSuccess; --ns) {
+  // largest windows first; the last launch stays on the caller's stream
+  int left = launched;
+  for (int ns = kMaxBatchSlots; ns >= first_single && e == hipSuccess; --ns) {
     const int64_t n = bt->group_count[ns];
     if (n == 0 || group_waves[ns] == 0) continue;
     hipStream_t gs = st;
-    if (concurrent) {
+    const bool side = concurrent && --left > 0;
+    if (side) {
       gs = bt->side[ns];
       e = hipStreamWaitEvent(gs, bt->fork, 0);
       if (e != hipSuccess) break;
@@ -3869,8 +3971,9 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
         std::min<int64_t>(group_waves[ns], ((n + wg_waves - 1) / wg_waves) * wg_waves);
     const int blocks = int(wv / wg_waves);
     const BatchItem* items = bt->d_items + bt->group_begin[ns];
-    int* counter = bt->d_counter + ns * kCounterStride;
-    const BatchGroupLaunch L{dim3(blocks), dim3(threads), gs, bt->d_jobs, items, n, counter, flags};
+    int* counter = bt->d_counter + ns * kItemLists * kCounterStride;
+    const BatchGroupLaunch L{dim3(blocks), dim3(threads), gs, bt->d_jobs,
+                             items, {n, counter, int32_t(std::min<int64_t>(wv, kItemLists))}, flags};
     const bool sh = bt->share[ns];
     const bool pe = bt->periodic[ns] && !(flags & MBQC_FLAG_TABLE_STEPS);
     switch (ns) {
@@ -3897,11 +4000,31 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
         break;
     }
     if (e == hipSuccess) e = hipGetLastError();
-    if (e == hipSuccess && concurrent) {
-      e = hipEventRecord(bt->join[ns], gs);
-      if (e == hipSuccess) e = hipStreamWaitEvent(st, bt->join[ns], 0);
-    }
+    if (e == hipSuccess && side) e = hipEventRecord(bt->join[ns], gs);
+    joined[ns] = side;
   }
+  if (e == hipSuccess && mixed) {
+    int64_t waves = 0;
+    uint32_t share = 0;
+    bool periodic = !(flags & MBQC_FLAG_TABLE_STEPS);
+    for (int ns = 1; ns <= kMaxSvSlots; ++ns) {
+      if (bt->group_count[ns] == 0) continue;
+      waves += group_waves[ns];
+      share |= uint32_t(bt->share[ns] && ns >= 2) << ns;
+      periodic = periodic && bt->periodic[ns];
+    }
+    waves = std::min<int64_t>(waves, ((bt->n_mixed + wg_waves - 1) / wg_waves) * wg_waves);
+    const BatchGroupLaunch L{dim3(unsigned(waves / wg_waves)), dim3(threads), st, bt->d_jobs,
+                             bt->d_items + bt->items.size(),
+                             {bt->n_mixed, bt->d_counter,
+                              int32_t(std::min<int64_t>(waves, kItemLists))},
+                             flags};
+    if (bt->mixed_max == 6) launch_batch_mixed<6>(L, ref, periodic, share);
+    else launch_batch_mixed<5>(L, ref, periodic, share);
+    e = hipGetLastError();
+  }
+  for (int ns = 1; ns <= kMaxBatchSlots && e == hipSuccess; ++ns)
+    if (joined[ns]) e = hipStreamWaitEvent(st, bt->join[ns], 0);
   return e == hipSuccess ? MBQC_OK : hip_fail(e, "batch launch");
 }
 
@@ -4447,11 +4570,22 @@ int mbqc_batch_create(const mbqc_batch_job* jobs, int32_t n_jobs, int32_t sims_p
     sorted.push_back(bt->items[order[k].index]);
   }
   bt->items.swap(sorted);
+  std::vector<BatchItem> mixed;
+  std::stable_sort(order.begin(), order.end(),
+                   [](const Key& a, const Key& b) { return a.cost > b.cost; });
+  for (const Key& k : order)
+    if (k.ns <= kMaxSvSlots) mixed.push_back(sorted[k.index]);   // (sorted: the items as created)
+  bt->n_mixed = int64_t(mixed.size());
+  for (int ns = 1; ns <= kMaxSvSlots; ++ns) {
+    if (bt->group_count[ns] == 0) continue;
+    ++bt->mixed_groups;
+    bt->mixed_max = ns;
+  }
   hipError_t e = hipGetDevice(&bt->device);
   if (e == hipSuccess) e = hipMalloc(&bt->d_jobs, sizeof(Job) * bt->jobs.size());
   if (e == hipSuccess && !bt->items.empty())
-    e = hipMalloc(&bt->d_items, sizeof(BatchItem) * bt->items.size());
-  if (e == hipSuccess) e = hipMalloc(&bt->d_counter, sizeof(int) * kCounterStride * (kMaxBatchSlots + 1));
+    e = hipMalloc(&bt->d_items, sizeof(BatchItem) * (bt->items.size() + mixed.size()));
+  if (e == hipSuccess) e = hipMalloc(&bt->d_counter, sizeof(int) * kCounterStride * kBatchCounters);
   for (int ns = kMaxSvLdsSlots + 1; ns <= kMaxBatchSlots && e == hipSuccess; ++ns) {
     if (bt->group_count[ns] == 0) continue;
     e = hipMalloc(&bt->gws[ns], size_t(bt->gws_sims[ns]) * wide_tile_bytes(ns));
@@ -4470,6 +4604,9 @@ int mbqc_batch_create(const mbqc_batch_job* jobs, int32_t n_jobs, int32_t sims_p
     e = hipMemcpy(bt->d_jobs, bt->jobs.data(), sizeof(Job) * bt->jobs.size(), hipMemcpyHostToDevice);
   if (e == hipSuccess && !bt->items.empty())
     e = hipMemcpy(bt->d_items, bt->items.data(), sizeof(BatchItem) * bt->items.size(),
+                  hipMemcpyHostToDevice);
+  if (e == hipSuccess && !mixed.empty())
+    e = hipMemcpy(bt->d_items + bt->items.size(), mixed.data(), sizeof(BatchItem) * mixed.size(),
                   hipMemcpyHostToDevice);
   if (e != hipSuccess) {
     mbqc_batch_destroy(bt);
@@ -4578,7 +4715,7 @@ int mbqc_batch_launch(mbqc_batch* bt, int32_t waves, int32_t wg_waves, uint32_t 
   if (!bt) return fail(MBQC_ERR_VALUE, "null batch");
   int32_t gw[kMaxBatchSlots + 1];
   for (int ns = 0; ns <= kMaxBatchSlots; ++ns) gw[ns] = bt->group_count[ns] > 0 ? waves : 0;
-  return batch_launch(bt, gw, wg_waves, flags, stream);
+  return batch_launch(bt, gw, wg_waves, flags, true, stream);
 }
 
 int mbqc_batch_launch_groups(mbqc_batch* bt, const int32_t* group_waves, int32_t n_entries,
@@ -4593,7 +4730,7 @@ int mbqc_batch_launch_groups(mbqc_batch* bt, const int32_t* group_waves, int32_t
     if (group_waves[ns] < 0) return fail(MBQC_ERR_VALUE, "negative wave count");
     gw[ns] = bt->group_count[ns] > 0 ? group_waves[ns] : 0;
   }
-  return batch_launch(bt, gw, wg_waves, flags, stream);
+  return batch_launch(bt, gw, wg_waves, flags, false, stream);
 }
 
 int64_t mbqc_batch_group_items(const mbqc_batch* bt, int32_t n_slots) {

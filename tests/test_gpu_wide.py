@@ -192,3 +192,33 @@ def test_host_runs_equal_batched_runs(rows, cols, window, rng):
     for t in threads:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("waves,wg_waves,max_rows", [(1, 1, 5), (4, 4, 6), (33, 3, 5), (4096, 4, 6)])
+def test_batched_register_groups_in_one_launch(waves, wg_waves, max_rows, rng):
+    """Every register group of a batch in one kernel, its items dealt to lists:
+    fewer waves than lists, a ragged last workgroup, more waves than items; the
+    outputs equal the launch with a kernel per group bit for bit."""
+    torch = _torch()
+    import mentpy_amd as mp
+    from mentpy_amd.batched import BatchedForward
+    jobs = []
+    for i in range(23):
+        r = 1 + i % max_rows
+        g = mp.templates.linear_cluster(5 + i) if r == 1 else mp.templates.grid_cluster(r, 4 + i % 7)
+        sim = mp.PatternSimulator(g, backend="hip-sv")
+        S = (16, 3, 1)[i % 3]
+        th = rng.uniform(0, 6, (7 + 11 * i, len(g.trainable_nodes))).astype(np.float32)
+        jobs.append((sim, th, np.stack([haar_state(r, rng) for _ in range(S)])))
+    bf = BatchedForward(jobs)
+    sizes = [64 if ns in bf.groups() else 0 for ns in range(max_rows + 1)]
+    want = [o.clone() for o in bf.launch(wg_waves=1, group_waves=sizes)]
+    for _ in range(2):
+        for o in bf.outputs:
+            o.zero_()
+        got = bf.launch(waves=max(waves, wg_waves), wg_waves=wg_waves)
+        torch.cuda.synchronize()
+        for x, y in zip(got, want):
+            assert torch.equal(x, y)
+    for (sim, th, st), o in zip(jobs, want):
+        assert (sim.run_batch(th, st) - o).abs().max().item() < 1e-6
