@@ -42,9 +42,10 @@ extern "C" {
 #define MBQC_FLAG_REF_PHASE 1u    /* reference global phase: prod_k sgn(cos(t_k/2)) e^{i t_k/2} */
 #define MBQC_FLAG_RENORMALIZE 2u  /* divide the output by its norm (SV) / trace (DM) */
 #define MBQC_FLAG_WRITE_PHASE 4u  /* also write the per-sim global phase (SV forward) */
-#define MBQC_FLAG_TABLE_STEPS 8u  /* SV / DM forward and batched launch: read the step
+#define MBQC_FLAG_TABLE_STEPS 8u  /* SV forward and batched launch: read the step
                                      coefficients and CZ masks from the plan's tables
-                                     also for a periodic plan (same results) */
+                                     also for a periodic plan (same results; density
+                                     matrices of such plans have one form only) */
 #define MBQC_FLAG_STEP_PROBS 16u  /* DM forward / window: evaluate every step's outcome
                                      probability (outcome 1 where outcome 0 has
                                      probability below 1e-4, division by the outcome

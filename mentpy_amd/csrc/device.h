@@ -177,6 +177,20 @@ __device__ __forceinline__ void split_sim(const Job& J, int64_t g, int64_t* bi, 
   }
 }
 
+// Single-qubit noise of the density-matrix path.  Every supported channel is
+// phase covariant: on a qubit's 2x2 blocks it maps the diagonal pair
+// (r00, r11) -> (d00 r00 + d01 r11, d10 r00 + d11 r11) and scales both
+// off-diagonal blocks by the real factor coh.  A measured qubit only shows
+// the trace (preserved) and coh to its XY projection, so its noise (and the
+// readout flip) folds into gamma = coh (1 - 2 p_readout); output qubits get the
+// full map at the end.
+struct DmNoise {
+  float gamma;
+  float d00, d01, d10, d11, coh;
+  int32_t out_noise;  // 0: the output map is the identity
+  float flip;         // 1 - 2 p_readout
+};
+
 // Identity modifier of the per-step projection coefficient b = e^{-i theta}.
 struct NoModify {
   __device__ __forceinline__ float2 operator()(int, float2 b) const { return b; }
@@ -262,6 +276,35 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     v = 0.0f;
 #pragma unroll
     for (int i = 0; i < T / 64; ++i) v += red[i];
+  }
+  return v;
+}
+
+// Makes the LDS writes of a simulation's lanes visible to all of them: a
+// barrier where it spans several waves, else only an order within the wave.
+template <int T>
+__device__ __forceinline__ void lanes_sync() {
+  if constexpr (T > 64) {
+    __syncthreads();
+  } else {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// Sum over L neighbouring lanes; `red`: LDS of L / 64 values, used where they
+// span several waves (then the whole workgroup).
+template <int L, typename V>
+__device__ __forceinline__ V lanes_sum(V v, V* red) {
+#pragma unroll
+  for (int m = (L < 64 ? L : 64) / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
+  if constexpr (L > 64) {
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = red[0];
+#pragma unroll
+    for (int i = 1; i < L / 64; ++i) v += red[i];
   }
   return v;
 }

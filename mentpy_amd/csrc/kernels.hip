@@ -623,20 +623,6 @@ __device__ __forceinline__ void dm_step(HermReg<1 << NS>& r, float2 gb, uint32_t
   }
 }
 
-// Single-qubit noise of the density-matrix path.  Every supported channel is
-// phase covariant: on a qubit's 2x2 blocks it maps the diagonal pair
-// (r00, r11) -> (d00 r00 + d01 r11, d10 r00 + d11 r11) and scales both
-// off-diagonal blocks by the real factor coh.  A measured qubit only shows
-// the trace (preserved) and coh to its XY projection, so its noise (and the
-// readout flip) folds into gamma = coh (1 - 2 p_readout); output qubits get the
-// full map at the end.
-struct DmNoise {
-  float gamma;
-  float d00, d01, d10, d11, coh;
-  int32_t out_noise;  // 0: the output map is the identity
-  float flip;         // 1 - 2 p_readout
-};
-
 template <int NS, int M>
 __device__ __forceinline__ void dm_channel(HermReg<1 << NS>& r, const DmNoise& nz) {
   constexpr int H = 1 << NS;
@@ -1090,35 +1076,30 @@ __global__ __launch_bounds__(256) void k_sv_sample_global(Job J, const uint64_t*
 
 // Sub-step SUB of the block starting at step k0 (measured slot NS - 1 - SUB);
 // c0 = k0's position in the staged coefficient chunk.
-template <int NS, int T, bool PERIODIC, int SUB>
+template <int NS, int T, int SUB>
 __device__ __forceinline__ void dm_lds_sub(float2* r, const mbqc_step* steps, const float2* gb_s,
                                            int k0, int c0, int n, int tid) {
   const int k = k0 + SUB;
   if (k < n) {
     const float2 gb = gb_s[c0 + SUB];
-    if constexpr (PERIODIC) {
-      __syncthreads();
-      dm_lds_step<T>(r, 1 << NS, NS - 1 - SUB, 3u, periodic_nmask(NS, SUB), gb, tid);
-    } else {
-      const mbqc_step st = steps[k];
-      __syncthreads();
-      dm_lds_step<T>(r, 1 << NS, NS - 1 - SUB, st.flags, st.nmask, gb, tid);
-    }
+    const mbqc_step st = steps[k];
+    __syncthreads();
+    dm_lds_step<T>(r, 1 << NS, NS - 1 - SUB, st.flags, st.nmask, gb, tid);
   }
 }
 
-template <int NS, int T, bool PERIODIC, int... SUBS>
+template <int NS, int T, int... SUBS>
 __device__ __forceinline__ void dm_lds_block(float2* r, const mbqc_step* steps, const float2* gb_s,
                                              int k0, int c0, int n, int tid,
                                              std::integer_sequence<int, SUBS...>) {
-  (dm_lds_sub<NS, T, PERIODIC, SUBS>(r, steps, gb_s, k0, c0, n, tid), ...);
+  (dm_lds_sub<NS, T, SUBS>(r, steps, gb_s, k0, c0, n, tid), ...);
 }
 
 // Density matrix in LDS: T threads per simulation (one quartet each per step)
 // and G simulations per workgroup, so that small windows (T < 64) still fill
 // whole waves.  Steps run in blocks of NS with the measured slot fixed per
 // sub-step; coefficients are staged in chunks of a multiple of NS steps.
-template <int NS, int T, int G, bool PERIODIC>
+template <int NS, int T, int G>
 __global__ __launch_bounds__(T * G) void k_dm_forward_lds(Job J, DmNoise nz, uint32_t flags) {
   constexpr int H = 1 << NS;
   constexpr int HQ = H / 2;
@@ -1158,7 +1139,7 @@ __global__ __launch_bounds__(T * G) void k_dm_forward_lds(Job J, DmNoise nz, uin
       stage_coeffs<T>(gb_s, steps, ang, J.angle_stride_a, k0, n, nz.gamma, tid);
       __syncthreads();
     }
-    dm_lds_block<NS, T, PERIODIC>(r, steps, gb_s, k0, c0, n, tid,
+    dm_lds_block<NS, T>(r, steps, gb_s, k0, c0, n, tid,
                                   std::make_integer_sequence<int, NS>{});
   }
   // noise of every output qubit
@@ -3401,8 +3382,8 @@ hipError_t launch_dm(const Job& J, const DmNoise& nz, uint32_t flags, bool perio
                      hipStream_t st) {
   const int threads = 256;
   const int64_t blocks = (J.total + threads - 1) / threads;
-  if (periodic)
-    hipLaunchKernelGGL((k_dm_forward<NS, true>), dim3(blocks), dim3(threads), 0, st, J, nz, flags);
+  if (NS == 1 && periodic)   // wider column plans do not come here
+    hipLaunchKernelGGL((k_dm_forward<NS, (NS == 1)>), dim3(blocks), dim3(threads), 0, st, J, nz, flags);
   else
     hipLaunchKernelGGL((k_dm_forward<NS, false>), dim3(blocks), dim3(threads), 0, st, J, nz, flags);
   return hipGetLastError();
@@ -3709,9 +3690,9 @@ hipError_t launch_dm_wave(const Job& J, const DmNoise& nz, uint32_t flags, bool 
   constexpr int SPW = 64 >> (2 * NS);               // simulations per wave
   const int64_t waves = (J.total + SPW - 1) / SPW;
   const int64_t blocks = (waves + 3) / 4;           // 4 waves per workgroup
-  if (periodic)
-    hipLaunchKernelGGL((k_dm_forward_wave<NS, true>), dim3(unsigned(blocks)), dim3(256), 0, st, J,
-                       nz, flags);
+  if (NS == 1 && periodic)   // wider column plans do not come here
+    hipLaunchKernelGGL((k_dm_forward_wave<NS, (NS == 1)>), dim3(unsigned(blocks)), dim3(256), 0, st,
+                       J, nz, flags);
   else
     hipLaunchKernelGGL((k_dm_forward_wave<NS, false>), dim3(unsigned(blocks)), dim3(256), 0, st, J,
                        nz, flags);
@@ -3719,18 +3700,12 @@ hipError_t launch_dm_wave(const Job& J, const DmNoise& nz, uint32_t flags, bool 
 }
 
 template <int NS>
-hipError_t launch_dm_lds(const Job& J, const DmNoise& nz, uint32_t flags, bool periodic,
-                         hipStream_t st) {
+hipError_t launch_dm_lds(const Job& J, const DmNoise& nz, uint32_t flags, hipStream_t st) {
   constexpr int Q = 1 << (2 * (NS - 1));          // quartets per step
   constexpr int T = Q < 256 ? Q : 256;            // threads per simulation
   constexpr int G = T < 64 ? 64 / T : 1;          // simulations per workgroup
   const int64_t blocks = (J.total + G - 1) / G;
-  if (periodic)
-    hipLaunchKernelGGL((k_dm_forward_lds<NS, T, G, true>), dim3(blocks), dim3(T * G), 0, st, J, nz,
-                       flags);
-  else
-    hipLaunchKernelGGL((k_dm_forward_lds<NS, T, G, false>), dim3(blocks), dim3(T * G), 0, st, J, nz,
-                       flags);
+  hipLaunchKernelGGL((k_dm_forward_lds<NS, T, G>), dim3(blocks), dim3(T * G), 0, st, J, nz, flags);
   return hipGetLastError();
 }
 
@@ -3805,6 +3780,10 @@ int dm_forward(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
     e = hipGetLastError();
     return e == hipSuccess ? MBQC_OK : hip_fail(e, "dm_forward launch");
   }
+  if (p->column_steps && p->ns >= 2) {
+    e = launch_dm_pauli(J, nz, p->ns - p->n_in, flags, st);
+    return e == hipSuccess ? MBQC_OK : hip_fail(e, "dm_forward launch");
+  }
   // Small batches of small windows leave the one-simulation-per-lane kernel
   // with a few waves on a few CUs; there the one-entry-per-lane kernel (up to
   // kDmWaveKernelMaxSims[ns] simulations) or the LDS kernel spread the work
@@ -3817,12 +3796,12 @@ int dm_forward(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
     case 2: e = wave ? launch_dm_wave<2>(J, nz, flags, pe, st) : launch_dm<2>(J, nz, flags, pe, st); break;
     case 3:
       e = wave ? launch_dm_wave<3>(J, nz, flags, pe, st)
-               : (small ? launch_dm_lds<3>(J, nz, flags, pe, st) : launch_dm<3>(J, nz, flags, pe, st));
+               : (small ? launch_dm_lds<3>(J, nz, flags, st) : launch_dm<3>(J, nz, flags, pe, st));
       break;
-    case 4: e = launch_dm_lds<4>(J, nz, flags, pe, st); break;
-    case 5: e = launch_dm_lds<5>(J, nz, flags, pe, st); break;
-    case 6: e = launch_dm_lds<6>(J, nz, flags, pe, st); break;
-    case 7: e = launch_dm_lds<7>(J, nz, flags, pe, st); break;
+    case 4: e = launch_dm_lds<4>(J, nz, flags, st); break;
+    case 5: e = launch_dm_lds<5>(J, nz, flags, st); break;
+    case 6: e = launch_dm_lds<6>(J, nz, flags, st); break;
+    case 7: e = launch_dm_lds<7>(J, nz, flags, st); break;
   }
   return e == hipSuccess ? MBQC_OK : hip_fail(e, "dm_forward launch");
 }

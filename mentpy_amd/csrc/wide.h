@@ -51,4 +51,9 @@ hipError_t launch_wide_adj_forward(const Job& J, float2* ckpt, int ck, hipStream
 hipError_t launch_wide_adj_backward(const Job& J, const float2* ckpt, const float2* seed,
                                     const WideAdjoint& A, float* gpart, hipStream_t st);
 
+// Density matrices of column plans with 2..7 slots (wide_dm.hip); pad_slots:
+// slots that start as |+> padding (n_slots - n_inputs).
+hipError_t launch_dm_pauli(const Job& J, const DmNoise& nz, int pad_slots, uint32_t flags,
+                           hipStream_t st);
+
 }  // namespace mbqc

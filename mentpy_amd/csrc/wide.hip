@@ -59,18 +59,6 @@ struct Wide {
   }
 };
 
-// Makes the LDS writes of a simulation's lanes visible to all of them: a
-// barrier where it spans several waves, else only an order within the wave.
-template <int T>
-__device__ __forceinline__ void lanes_sync() {
-  if constexpr (T > 64) {
-    __syncthreads();
-  } else {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  }
-}
-
 __device__ __forceinline__ int padded(int a) { return a + (a >> 4); }
 
 // CZ neighbours of the qubit appended by a step, as a mask over the amplitude
@@ -234,23 +222,6 @@ __device__ __forceinline__ void wide_load(float2 (&t)[1 << R], const Job& J, int
     const int j = (r << (NS - R)) | lane;
     t[r] = flip(psi[in_index[j]], sign[j] ? 0x80000000u : 0u);
   }
-}
-
-// Sum over L neighbouring lanes; `red`: LDS of L / 64 values, used where they
-// span several waves (then the whole workgroup).
-template <int L, typename V>
-__device__ __forceinline__ V lanes_sum(V v, V* red) {
-#pragma unroll
-  for (int m = (L < 64 ? L : 64) / 2; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-  if constexpr (L > 64) {
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    v = red[0];
-#pragma unroll
-    for (int i = 1; i < L / 64; ++i) v += red[i];
-  }
-  return v;
 }
 
 // 1 / norm of the state over the output amplitudes (those with out_pos >= 0).

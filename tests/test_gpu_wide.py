@@ -222,3 +222,43 @@ def test_batched_register_groups_in_one_launch(waves, wg_waves, max_rows, rng):
             assert torch.equal(x, y)
     for (sim, th, st), o in zip(jobs, want):
         assert (sim.run_batch(th, st) - o).abs().max().item() < 1e-6
+
+
+@pytest.mark.parametrize("rows,cols,window,B,S", [
+    (2, 4, None, 1, 1), (2, 30, None, 37, 3), (3, 12, None, 130, 1), (3, 4, None, 1, 2),
+    (4, 6, None, 9, 2), (4, 5, None, 2049, 1), (5, 6, None, 5, 1), (6, 4, None, 3, 1),
+    (7, 3, None, 2, 1), (2, 5, 4, 17, 2), (2, 5, 5, 9, 1), (3, 4, 5, 9, 1), (3, 5, 6, 3, 2),
+    (4, 4, 6, 5, 1), (4, 5, 7, 3, 1), (5, 4, 8, 2, 1), (1, 6, 3, 50, 2)])
+def test_density_matrices_of_column_and_other_plans(rows, cols, window, B, S, rng):
+    """Pauli-vector kernels of column plans (one and two register digits, more
+    steps than a coefficient chunk) and the matrix kernels of the other plans
+    (a window above the grid's own), with and without noise and trace
+    normalisation, against the oracle; nothing stored past the last matrix."""
+    torch = _torch()
+    import mentpy_amd as mp
+    from mentpy_amd.noise import NoiseModel
+    from mentpy_amd.simulators.hip_simulator import dm_forward, _as_angles, _as_states
+    from oracle.vectorized import dm_batch
+    g = mp.templates.linear_cluster(cols) if rows == 1 else mp.templates.grid_cluster(rows, cols)
+    sim = mp.PatternSimulator(g, backend="hip-dm", **({"window_size": window} if window else {}))
+    plan = sim.simulator.plan
+    th = rng.uniform(-7, 7, (B, len(g.trainable_nodes))).astype(np.float32)
+    psi = np.stack([haar_state(rows, rng) for _ in range(S)])
+    dev = torch.device("cuda")
+    a, s = _as_angles(th, plan.info["n_angles"], dev), _as_states(psi, plan.info["n_inputs"], dev)
+    d = 1 << rows
+    at = sorted({0, B // 2, B - 1})
+    for pd, pr in ((0.0, 0.0), (0.03, 0.01)):
+        guard = torch.full((B + 1, S, d, d), 7.0, dtype=torch.complex64, device=dev)
+        out = dm_forward(plan, a, s, p_depol=pd, p_readout=pr, out=guard[:B])
+        raw = dm_forward(plan, a, s, p_depol=pd, p_readout=pr, renormalize=False)
+        torch.cuda.synchronize()
+        assert (guard[B] == 7.0).all()
+        ref = dm_batch(g, th[at].astype(np.float64), psi, p_depol=pd, p_readout=pr)
+        assert np.abs(out[at].cpu().numpy() - ref).max() < 2e-5
+        assert (raw - out).abs().max().item() < 2e-5
+    if window is None:   # the damping channels' population shift on the outputs
+        noise = NoiseModel(amplitude_damping=0.2, gad_gamma=0.1, gad_p=0.7, phase_flip=0.05)
+        got = dm_forward(plan, a, s, noise=noise)
+        gen = dm_forward(plan, a, s, noise=noise, step_probs=True)
+        assert (got - gen).abs().max().item() < 2e-5
