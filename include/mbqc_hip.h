@@ -316,14 +316,16 @@ int mbqc_sv_adjoint_backward_c64(const mbqc_plan* plan, const float* angles, int
  * times as many lanes for 1/n_segments of the steps each (small batches fill
  * the chip).  2 <= n_segments <= min(16, number of blocks).
  *
- * mbqc_sv_segments_auto: the segment count the library picks for B sets
- * (1 means: use the unsegmented entry points).
+ * mbqc_sv_segments_auto: the segment count that fills the chip for B sets
+ * (1 means: use the unsegmented entry points).  mbqc_sv_adjoint_segments: the
+ * same, or 1 where the unsegmented entry points are faster for this plan.
  * Forward: out[B][2^n_inputs][2^n_outputs] = T_b (column c = image of input
  * basis state c).  Backward: seed in the same layout (dL = Re sum conj(seed)
  * d(out)); writes grad[B][n_angles] (entries of non-trainable angles are left
  * untouched).  The backward needs the workspace of the forward of the same
  * angles. */
 int32_t mbqc_sv_segments_auto(const mbqc_plan* plan, int64_t B);
+int32_t mbqc_sv_adjoint_segments(const mbqc_plan* plan, int64_t B);
 size_t mbqc_sv_segmented_workspace_bytes(const mbqc_plan* plan, int64_t B, int32_t n_segments);
 int mbqc_sv_segmented_forward_c64(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
                                   int64_t angle_stride_a, void* out, int64_t B, int32_t n_segments,

@@ -161,6 +161,17 @@ struct Job {
   int64_t S, total;
 };
 
+// Plan tables as constant memory, for loads at uniform addresses: they become
+// scalar loads, also in kernels whose memory fences (the lanes' LDS exchanges)
+// keep the compiler from proving that nothing writes the tables.  A per-lane load
+// in their place costs every wave its full latency.
+template <typename T>
+using Constant = const __attribute__((address_space(4))) T*;
+template <typename T>
+__device__ __forceinline__ Constant<T> constant(const T* p) {
+  return (Constant<T>)p;
+}
+
 // Angle vector and input of simulation g: g / S and g % S, in 32 bits where the
 // batch allows it (a 64-bit division is over a hundred instructions).
 __device__ __forceinline__ void split_sim(const Job& J, int64_t g, int64_t* bi, int64_t* si) {
@@ -222,8 +233,8 @@ __device__ __forceinline__ uint32_t draw32(uint64_t seed, uint64_t sim, uint64_t
 struct SampleMod {
   uint32_t fx = 0, fz = 0;
   uint64_t seed = 0, sim = 0;
-  const uint64_t* xm;
-  const uint64_t* zm;
+  Constant<uint64_t> xm;
+  Constant<uint64_t> zm;
   int32_t* out_words;   // this simulation's outcome words (null for inactive lanes)
   int n;
   uint32_t rbits = 0, word = 0;

@@ -747,8 +747,8 @@ __global__ __launch_bounds__(256) void k_sv_sample(Job J, const uint64_t* __rest
   SampleMod mod;
   mod.seed = seed;
   mod.sim = uint64_t(gg);
-  mod.xm = xm;
-  mod.zm = zm;
+  mod.xm = constant(xm);
+  mod.zm = constant(zm);
   mod.n = J.n_steps;
   int32_t* row = outcomes + gg * (words + 2);
   mod.out_words = active ? row : nullptr;
@@ -1015,8 +1015,8 @@ __device__ __forceinline__ void sample_run(const Job& J, const uint64_t* __restr
   SampleMod mod;
   mod.seed = seed;
   mod.sim = uint64_t(g);
-  mod.xm = xm;
-  mod.zm = zm;
+  mod.xm = constant(xm);
+  mod.zm = constant(zm);
   mod.n = J.n_steps;
   mod.out_words = tid == 0 ? row : nullptr;
   for (int k = 0; k < J.n_steps; ++k) {
@@ -3401,11 +3401,18 @@ inline int32_t adj_reduced_columns(int64_t C) {
   return (C <= 64 && (C & (C - 1)) == 0) ? int32_t(C) : (C % 64 == 0 ? 64 : 1);
 }
 
-// Column plans of 6..14 slots run the register-blocked sweeps (the checkpoints
-// of the two kinds differ, so the choice depends on the plan and C only).
-bool wide_adjoint(const Plan* p, int64_t C) {
-  return p->ns > kMaxAdjSlots && p->column_steps &&
-         wide_adjoint_fits(p->ns, adj_reduced_columns(C), p->n_angles);
+// Column plans of 6..14 slots run the register-blocked sweeps, those of 4 and 5
+// slots up to a number of columns: a simulation takes 4 or 8 lanes there and a
+// quarter of the time, which pays until the lanes are all taken.  4x16 grid,
+// 16 columns per set, forward and backward in us, one lane per simulation -> spread:
+// 16 sets 46.7 -> 26.4, 1024 sets 53.3 -> 36.2, 2048 sets 57.6 -> 47.0, 4096 sets
+// 64.7 -> 70.0.  5x10 grid, 32 columns: 16 sets 61.5 -> 23.5, 1024 sets
+// 74.9 -> 57.2, 1500 sets 81.8 -> 74.9, 2048 sets 88.0 -> 93.5.  (2 and 3 slots:
+// no gain at any size, 2x12 and 3x12 grids.)  The checkpoints of the two kinds
+// differ, so the choice depends on the plan, B and C only.
+bool wide_adjoint(const Plan* p, int64_t B, int64_t C) {
+  if (!p->column_steps || !wide_adjoint_fits(p->ns, adj_reduced_columns(C), p->n_angles)) return false;
+  return p->ns > kMaxAdjSlots || B * C <= (p->ns == 5 ? 49152 : 32768);
 }
 
 // Adjoint sweeps above kMaxAdjLdsSlots slots refuse stream capture whichever
@@ -4306,6 +4313,21 @@ int32_t mbqc_sv_segments_auto(const mbqc_plan* plan, int64_t B) {
   return int32_t(std::max<int64_t>(n, 1));
 }
 
+int32_t mbqc_sv_adjoint_segments(const mbqc_plan* plan, int64_t B) {
+  const int32_t n = mbqc_sv_segments_auto(plan, B);
+  if (n <= 1) return n;
+  const Plan* p = reinterpret_cast<const Plan*>(plan);
+  // Windows of 4 and 5 slots: the sweep over all blocks, several lanes per
+  // column, takes less than the segments and their chain (whole step in us,
+  // segments -> one sweep; 4x16 grid: 16 sets 54.2 -> 37.7, 1024 sets
+  // 63.1 -> 51.5, 4096 sets 128 -> 110; 5x10 grid: 147.8 -> 80.4, 466.8 -> 371.1,
+  // 2048 sets 799 -> 698; 5x40 grid: 211.2 -> 131.0, 569.7 -> 511.0).  The chain
+  // of 4-slot steps is the longer one from about 130 steps (16 sets, 124
+  // steps: 60.8 -> 58.5, 156 steps: 61.3 -> 69.0).
+  if (p->column_steps && (p->ns == 5 || (p->ns == 4 && p->n_steps <= 128))) return 1;
+  return n;
+}
+
 size_t mbqc_sv_segmented_workspace_bytes(const mbqc_plan* plan, int64_t B, int32_t n_segments) {
   if (!plan) return 0;
   return seg_layout(*reinterpret_cast<const Plan*>(plan), B, n_segments, nullptr);
@@ -4386,7 +4408,7 @@ int mbqc_sv_adjoint_forward_c64(const mbqc_plan* plan, const float* angles, int6
   hipStream_t st = static_cast<hipStream_t>(stream);
   float2* ck = static_cast<float2*>(ckpt);
   hipError_t e = hipSuccess;
-  if (wide_adjoint(p, C)) {
+  if (wide_adjoint(p, B, C)) {
     e = refuse_capture(p, st);
     if (e == hipSuccess) e = launch_wide_adj_forward(J, ck, adj_ckpt_blocks(B * C), st);
     return e == hipSuccess ? MBQC_OK : global_fail(e, "adjoint forward launch");
@@ -4446,7 +4468,7 @@ int mbqc_sv_adjoint_backward_c64(const mbqc_plan* plan, const float* angles, int
   const float2* ck = static_cast<const float2*>(ckpt);
   const float2* sd = static_cast<const float2*>(seed);
   hipError_t e = hipSuccess;
-  if (wide_adjoint(p, C)) {
+  if (wide_adjoint(p, B, C)) {
     e = refuse_capture(p, st);
     if (e == hipSuccess)
       e = launch_wide_adj_backward(J, ck, sd, WideAdjoint{A.C, A.P, A.red, A.ck, A.n_angles}, A.gpart,

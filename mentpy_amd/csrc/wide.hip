@@ -100,7 +100,10 @@ __device__ __forceinline__ void wide_step(float2 (&t)[1 << R], float2 b, const m
       }
     }
   } else {
-    const mbqc_step st = steps[k];
+    const Constant<uint32_t> row = constant(reinterpret_cast<const uint32_t*>(steps + k));
+    mbqc_step st{};
+    st.flags = row[1];
+    st.nmask = row[2];
     const float s = (st.flags & 2u) ? -1.0f : 1.0f;
     const float app = (st.flags & 1u) ? 1.0f : 0.0f;
     // the neighbour mask in the phase's amplitude order (rotated by FIRST)
@@ -127,7 +130,6 @@ __device__ __forceinline__ void wide_step(float2 (&t)[1 << R], float2 b, const m
 template <int NS, int R, int M, int T>
 __device__ __forceinline__ void wide_rotate(float2 (&t)[1 << R], float2* buf, int lane) {
   constexpr int NR = 1 << R;
-  if constexpr (R == NS) return;   // one lane: rotated by all its bits, back in place
   lanes_sync<T>();   // earlier reads of the buffer are done
 #pragma unroll
   for (int r = 0; r < NR; ++r) {
@@ -167,14 +169,14 @@ __device__ __forceinline__ void wide_block(float2 (&t)[1 << R], float2* buf, con
 }
 
 // e^{-i theta} of the chunk of steps [k0, k0 + CS), one step per lane.
-// (cl: the lane's place among the CL coefficient lanes.)  POLY: from the float
-// polynomials of the one-simulation-per-lane kernels, bit for bit.
-template <int NS, int R, bool REF, int M = NS, int SPARE = 0, bool POLY = false>
+// (cl: the lane's place among the `clanes` lanes that evaluate them.)  POLY: from
+// the float polynomials of the one-simulation-per-lane kernels, bit for bit.
+template <int CS, bool REF, bool POLY = false>
 __device__ __forceinline__ void wide_coeffs(float2* bs, const mbqc_step* steps, const float* ang,
-                                            int64_t sa, int k0, int n, int cl, RefPhase* ph) {
-  using W = Wide<NS, R, M, SPARE>;
+                                            int64_t sa, int k0, int n, int cl, int clanes,
+                                            RefPhase* ph) {
 #pragma unroll 1
-  for (int i = cl; i < W::CS; i += W::CL) {
+  for (int i = cl; i < CS; i += clanes) {
     const int k = k0 + i;
     if (k < n) {
       const float th = step_angle(steps[k], ang, sa);
@@ -185,19 +187,18 @@ __device__ __forceinline__ void wide_coeffs(float2* bs, const mbqc_step* steps, 
 }
 
 // All steps of one simulation; `on_end(blk, t)` runs after every block.
-template <int NS, int R, bool REF, bool COLUMN, int SPARE = 0, bool POLY = false, typename OnEnd,
-          typename Mod>
+template <int NS, int R, bool REF, bool COLUMN, bool POLY = false, typename OnEnd, typename Mod>
 __device__ __forceinline__ void wide_run(float2 (&t)[1 << R], const Job& J, const float* ang,
-                                         float2* buf, float2* bs, int cl, RefPhase* ph,
-                                         OnEnd on_end, Mod&& mod) {
-  using W = Wide<NS, R, NS, SPARE>;
+                                         float2* buf, float2* bs, int cl, int clanes,
+                                         RefPhase* ph, OnEnd on_end, Mod&& mod) {
+  using W = Wide<NS, R>;
   const int lane = cl & (W::TL - 1);
   const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
-  const int32_t* resc = J.tab + J.off_svres;
+  const Constant<int32_t> resc = constant(J.tab + J.off_svres);
   const int n = J.n_steps;
   for (int kc = 0; kc < n; kc += W::CS) {
     // the previous chunk's last read came before its last exchange
-    wide_coeffs<NS, R, REF, NS, SPARE, POLY>(bs, steps, ang, J.angle_stride_a, kc, n, cl, ph);
+    wide_coeffs<W::CS, REF, POLY>(bs, steps, ang, J.angle_stride_a, kc, n, cl, clanes, ph);
     lanes_sync<W::T>();
     const int ke = kc + W::CS < n ? kc + W::CS : n;
     for (int k0 = kc; k0 < ke; k0 += NS) {
@@ -274,8 +275,8 @@ __device__ __forceinline__ void wide_sim(const Job& J, int64_t g, bool active, u
   wide_load<NS, R>(t, J, si, lane);
   RefPhase rp;
   constexpr bool kLaneKernelToo = NS <= 6;   // then equal to it bit for bit
-  wide_run<NS, R, REF, COLUMN, SPARE, kLaneKernelToo>(
-      t, J, J.angles + bi * J.angle_stride, buf, bs, cl, &rp, [](int, const float2 (&)[W::NR]) {},
+  wide_run<NS, R, REF, COLUMN, kLaneKernelToo>(
+      t, J, J.angles + bi * J.angle_stride, buf, bs, cl, W::CL, &rp, [](int, const float2 (&)[W::NR]) {},
       NoModify());
   if constexpr (REF) {
     rp.m_sum = lanes_sum<W::CL>(rp.m_sum, reinterpret_cast<int32_t*>(bs));
@@ -332,12 +333,12 @@ __global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_sample(
   SampleMod mod;
   mod.seed = seed;
   mod.sim = uint64_t(gg);
-  mod.xm = xm;
-  mod.zm = zm;
+  mod.xm = constant(xm);
+  mod.zm = constant(zm);
   mod.n = J.n_steps;
   mod.out_words = active && lane == 0 ? row : nullptr;
   RefPhase ph;
-  wide_run<NS, R, false, COLUMN>(t, J, J.angles + bi * J.angle_stride, buf, bs, lane, &ph,
+  wide_run<NS, R, false, COLUMN>(t, J, J.angles + bi * J.angle_stride, buf, bs, lane, W::TL, &ph,
                                  [](int, const float2 (&)[W::NR]) {}, mod);
   uint32_t xo = 0, zo = 0;
   for (int m = 0; m < J.n_out; ++m) {
@@ -409,14 +410,31 @@ __global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_batch(
 // and the measured halves in LDS and a barrier per step, forward 22.7 -> 14.2.
 // Gradient error against 64 bits 3.6e-7 -> 3.0e-7 (the running back costs
 // about 8%, the correctly rounded coefficients gain more).
+// Columns of one parameter set have the same angles: groups of `clanes` lanes
+// (TL times a power of two of columns, at most a wave) evaluate one set of
+// coefficients for their simulations.
+template <int NS, int R>
+struct AdjWide {
+  using W = Wide<NS, R>;
+  // float2 of LDS for `groups` simulations: `states` exchange buffers each, then
+  // the coefficients
+  __host__ __device__ static constexpr int lds(int groups, int states, int clanes) {
+    return groups * states * W::BUF + (groups * W::TL + clanes - 1) / clanes * W::CS;
+  }
+  static int clanes(int64_t columns) {
+    int c = W::TL;
+    for (; c < 64 && columns % 2 == 0; columns /= 2) c *= 2;
+    return c;
+  }
+};
+
 template <int NS, int R>
 __global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_adj_forward(Job J,
                                                                        float2* __restrict__ ckpt,
-                                                                       int ck) {
+                                                                       int ck, int clanes) {
   using W = Wide<NS, R>;
-  __shared__ float2 lds[W::G * W::SIM];
+  extern __shared__ float2 lds[];
   const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
-  float2* buf = lds + sub * W::SIM;
   const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
   const bool active = g < J.total;
   const int64_t gg = active ? g : J.total - 1;
@@ -427,11 +445,12 @@ __global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_adj_forward(Job J,
   const int nblk = (J.n_steps + NS - 1) / NS;
   RefPhase ph;
   wide_run<NS, R, false, true>(
-      t, J, J.angles + bi * J.angle_stride, buf, buf + W::BUF, lane, &ph,
+      t, J, J.angles + bi * J.angle_stride, lds + sub * W::BUF,
+      lds + W::G * W::BUF + int(threadIdx.x) / clanes * W::CS, int(threadIdx.x) % clanes, clanes, &ph,
       [&](int blk, const float2 (&tt)[W::NR]) {
-        if ((blk + 1) % ck != 0 && blk + 1 != nblk) return;
+        if (((blk + 1) & (ck - 1)) != 0 && blk + 1 != nblk) return;   // ck: 1 or 2
         // inactive groups repeat the last simulation's stores
-        float2* cp = ckpt + ((int64_t(blk / ck) * J.total + gg) << NS) + lane;
+        float2* cp = ckpt + ((int64_t(blk >> (ck - 1)) * J.total + gg) << NS) + lane;
 #pragma unroll
         for (int r = 0; r < W::NR; ++r) cp[r << (NS - R)] = tt[r];
       },
@@ -447,18 +466,42 @@ __global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_adj_forward(Job J,
   }
 }
 
-// The inverse exchange: v -> rotate-right(v, M).
-template <int NS, int R, int M, int TL>
-__device__ __forceinline__ void wide_unrotate(float2 (&t)[1 << R], float2* buf, int lane) {
-  constexpr int NR = 1 << R;
-  lanes_sync<TL>();
+// The inverse exchange: v -> rotate-right(v, M), of the state and the cotangent.
+// Up to 9 slots they have a buffer each and exchange at once; above, where a
+// buffer is 8 KB and more, one after the other.
+constexpr bool adj_two_buffers(int ns) { return ns <= 9; }
+
+template <int NS, int R>
+__device__ __forceinline__ void put_rows(const float2 (&t)[1 << R], float2* buf, int lane) {
 #pragma unroll
-  for (int r = 0; r < NR; ++r) buf[padded((r << (NS - R)) | lane)] = t[r];
-  lanes_sync<TL>();
+  for (int r = 0; r < (1 << R); ++r) buf[padded((r << (NS - R)) | lane)] = t[r];
+}
+template <int NS, int R, int M>
+__device__ __forceinline__ void get_rotated(float2 (&t)[1 << R], const float2* buf, int lane) {
 #pragma unroll
-  for (int r = 0; r < NR; ++r) {
+  for (int r = 0; r < (1 << R); ++r) {
     const int top = r >> (R - M), low = r & ((1 << (R - M)) - 1);
     t[r] = buf[padded((low << (NS - R + M)) | (lane << M) | top)];
+  }
+}
+template <int NS, int R, int M, int TL>
+__device__ __forceinline__ void wide_unrotate(float2 (&t)[1 << R], float2 (&lam)[1 << R], float2* buf,
+                                              int lane) {
+  lanes_sync<TL>();
+  put_rows<NS, R>(t, buf, lane);
+  if constexpr (adj_two_buffers(NS)) {
+    float2* second = buf + Wide<NS, R>::BUF;
+    put_rows<NS, R>(lam, second, lane);
+    lanes_sync<TL>();
+    get_rotated<NS, R, M>(t, buf, lane);
+    get_rotated<NS, R, M>(lam, second, lane);
+  } else {
+    lanes_sync<TL>();
+    get_rotated<NS, R, M>(t, buf, lane);
+    lanes_sync<TL>();
+    put_rows<NS, R>(lam, buf, lane);
+    lanes_sync<TL>();
+    get_rotated<NS, R, M>(lam, buf, lane);
   }
 }
 
@@ -512,36 +555,46 @@ struct GradSlot {
 
 template <int NS, int R, int P, int... SS>
 __device__ __forceinline__ void wide_unphase(float2 (&t)[1 << R], float2 (&lam)[1 << R], float2* buf,
-                                             const float2* bs, const mbqc_step* steps, int k0,
-                                             int lane, const GradSlot& slot,
+                                             const float2 (&b)[NS], float (&d)[NS], int lane,
                                              std::integer_sequence<int, SS...>) {
   using W = Wide<NS, R>;
   constexpr int F = W::first(P), M = W::len(P);
-  wide_unrotate<NS, R, M, W::TL>(t, buf, lane);
-  wide_unrotate<NS, R, M, W::TL>(lam, buf, lane);
-  auto one = [&](auto sc) {
-    constexpr int S = M - 1 - decltype(sc)::value, SUB = F + S;
-    float d = wide_unstep<NS, R, F, S>(t, lam, bs[SUB], lane);
-    const int ai = steps[k0 + SUB].angle_index;
-    if (ai >= 0) {
-      d = last_lane_sum<(W::TL < 64 ? W::TL : 64)>(d);
-      // the state has been doubled by the NS - 1 - SUB steps after this one
-      d *= 1.0f / float(1 << (NS - SUB));
-      if (slot.writer) slot.acc[ai] = slot.first ? d : slot.acc[ai] + d;
-    }
-  };
-  (one(std::integral_constant<int, SS>{}), ...);
+  wide_unrotate<NS, R, M, W::TL>(t, lam, buf, lane);
+  ((d[F + M - 1 - SS] = wide_unstep<NS, R, F, M - 1 - SS>(t, lam, b[F + M - 1 - SS], lane)), ...);
 }
 
+// A block backwards.  Its coefficients are read at the start and its gradient
+// entries written at the end, so that the steps between have no LDS latency or
+// branch of their own.  With few simulations the sweep is its chain of steps
+// (16 sets of a 4x16 grid, 60 steps: 16.5 us, 29.4 us with one lane per
+// simulation), with many the LDS exchanges and the adds across lanes (4096 sets:
+// 40 us, one lane 41 us).
 template <int NS, int R, int... PS>
 __device__ __forceinline__ void wide_unblock(float2 (&t)[1 << R], float2 (&lam)[1 << R], float2* buf,
-                                             const float2* bs, const mbqc_step* steps, int k0,
-                                             int lane, const GradSlot& slot,
+                                             const float2* bs, Constant<int32_t> aidx, int lane,
+                                             const GradSlot& slot,
                                              std::integer_sequence<int, PS...>) {
   using W = Wide<NS, R>;
-  (wide_unphase<NS, R, W::P - 1 - PS>(t, lam, buf, bs, steps, k0, lane, slot,
+  float2 b[NS];
+  float d[NS];
+  int ai[NS];
+#pragma unroll
+  for (int k = 0; k < NS; ++k) {
+    b[k] = bs[k];
+    ai[k] = aidx[k];
+  }
+  (wide_unphase<NS, R, W::P - 1 - PS>(t, lam, buf, b, d, lane,
                                       std::make_integer_sequence<int, W::len(W::P - 1 - PS)>{}),
    ...);
+  // the state was doubled by each of the steps after step k
+#pragma unroll
+  for (int k = 0; k < NS; ++k)
+    d[k] = last_lane_sum<(W::TL < 64 ? W::TL : 64)>(d[k]) * (1.0f / float(1 << (NS - k)));
+  if (slot.writer) {
+#pragma unroll
+    for (int k = 0; k < NS; ++k)
+      if (ai[k] >= 0) slot.acc[ai[k]] = slot.first ? d[k] : slot.acc[ai[k]] + d[k];
+  }
 }
 
 // Backward sweep of a column plan: a workgroup holds N = blockDim / TL
@@ -552,16 +605,19 @@ __device__ __forceinline__ void wide_unblock(float2 (&t)[1 << R], float2 (&lam)[
 template <int NS, int R>
 __global__ __launch_bounds__((Wide<NS, R>::TL > 256 ? Wide<NS, R>::TL : 256)) void k_wide_adj_backward(
     Job J, const float2* __restrict__ ckpt, const float2* __restrict__ seed, WideAdjoint A,
-    float* __restrict__ gpart) {
+    int clanes, float* __restrict__ gpart) {
   using W = Wide<NS, R>;
+  using AW = AdjWide<NS, R>;
   constexpr int TL = W::TL;
   constexpr int WV = TL > 64 ? TL / 64 : 1;       // waves of one simulation
   extern __shared__ float2 dyn[];
   const int N = blockDim.x / TL;
   const int sub = threadIdx.x / TL, lane = threadIdx.x % TL;
-  float2* buf = dyn + sub * (W::BUF + NS);
-  float2* bs = buf + W::BUF;
-  float* accs = reinterpret_cast<float*>(dyn + N * (W::BUF + NS));
+  constexpr int BUFS = adj_two_buffers(NS) ? 2 : 1;
+  float2* buf = dyn + sub * BUFS * W::BUF;
+  float2* bs = dyn + N * BUFS * W::BUF + int(threadIdx.x) / clanes * W::CS;
+  const int cl = int(threadIdx.x) % clanes;
+  float* accs = reinterpret_cast<float*>(dyn + AW::lds(N, BUFS, clanes));
   const int wave = TL > 64 ? lane >> 6 : 0;
   const int per = A.red < N ? A.red : N;          // columns of a row held at once
   const int rows = N / per;                       // rows of this workgroup
@@ -573,10 +629,11 @@ __global__ __launch_bounds__((Wide<NS, R>::TL > 256 ? Wide<NS, R>::TL : 256)) vo
   const int64_t bi = rr / A.P, r0 = rr - bi * A.P;
   const float* ang = J.angles + bi * J.angle_stride;
   const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
-  const int32_t* resc = J.tab + J.off_svres;
+  const Constant<int32_t> resc = constant(J.tab + J.off_svres);
   const int32_t* out_pos = J.tab + J.off_out;
+  const Constant<int32_t> aidx = constant(J.tab + J.off_aidx);
   const float scale = sv_final_scale(J.e_sv);
-  const int nblk = J.n_steps / NS;
+  const int n = J.n_steps, nblk = n / NS;
   for (int a = threadIdx.x; a < N * WV * A.n_angles; a += blockDim.x) accs[a] = 0.0f;
   __syncthreads();
   GradSlot slot;
@@ -592,29 +649,43 @@ __global__ __launch_bounds__((Wide<NS, R>::TL > 256 ? Wide<NS, R>::TL : 256)) vo
       const int p = out_pos[(r << (NS - R)) | lane];
       lam[r] = cscale(sd[p >= 0 ? p : 0], p >= 0 ? scale : 0.0f);
     }
-    // the angle of the next block this lane evaluates, one block ahead
-    float th = 0.0f;
-    if (lane < NS) th = step_angle(steps[(nblk - 1) * NS + lane], ang, J.angle_stride_a);
-    for (int blk = nblk - 1; blk >= 0; --blk) {
-      if (blk + 1 == nblk || (blk + 1) % A.ck == 0) {
-        const float2* cp = ckpt + ((int64_t(blk / A.ck) * J.total + g) << NS) + lane;
+    // the next checkpoint is on its way while a block runs (a load at the block's
+    // start left every block waiting for it)
+    constexpr bool kPrefetch = R <= 3;
+    float2 ahead[kPrefetch ? W::NR : 1];
+    auto load_ckpt = [&](int blk, auto& to) {
+      const float2* cp = ckpt + ((int64_t(blk >> (A.ck - 1)) * J.total + g) << NS) + lane;
 #pragma unroll
-        for (int r = 0; r < W::NR; ++r) t[r] = cp[r << (NS - R)];
-      }
+      for (int r = 0; r < W::NR; ++r) to[r] = cp[r << (NS - R)];
+    };
+    if constexpr (kPrefetch) load_ckpt(nblk - 1, ahead);
+    for (int kc = ((n - 1) / W::CS) * W::CS; kc >= 0; kc -= W::CS) {
+      lanes_sync<TL>();   // the previous chunk's reads are done
+      wide_coeffs<W::CS, false>(bs, steps, ang, J.angle_stride_a, kc, n, cl, clanes, nullptr);
       lanes_sync<TL>();
-      if (lane < NS) bs[lane] = exp_minus_i(th);
-      if (lane < NS && blk > 0) th = step_angle(steps[(blk - 1) * NS + lane], ang, J.angle_stride_a);
-      lanes_sync<TL>();
-      wide_unblock<NS, R>(t, lam, buf, bs, steps, blk * NS, lane, slot,
-                          std::make_integer_sequence<int, W::P>{});
-      // the block's doublings and rescale undone; the cotangent takes the rescale
-      const bool rs = resc[blk] != 0;
-      const float f = (rs ? 0x1p32f : 1.0f) / float(1 << NS);
+      const int ke = kc + W::CS < n ? kc + W::CS : n;
+      for (int blk = ke / NS - 1; blk * NS >= kc; --blk) {
+        const bool at_ckpt = blk + 1 == nblk || ((blk + 1) & (A.ck - 1)) == 0;   // ck: 1 or 2
+        if constexpr (kPrefetch) {
+          if (at_ckpt) {
 #pragma unroll
-      for (int r = 0; r < W::NR; ++r) t[r] = cscale(t[r], f);
-      if (rs) {
+            for (int r = 0; r < W::NR; ++r) t[r] = ahead[r];
+          }
+          if (blk > 0 && (blk & (A.ck - 1)) == 0) load_ckpt(blk - 1, ahead);
+        } else if (at_ckpt) {
+          load_ckpt(blk, t);
+        }
+        wide_unblock<NS, R>(t, lam, buf, bs + (blk * NS - kc), aidx + blk * NS, lane, slot,
+                            std::make_integer_sequence<int, W::P>{});
+        // the block's doublings and rescale undone; the cotangent takes the rescale
+        const bool rs = resc[blk] != 0;
+        const float f = (rs ? 0x1p32f : 1.0f) / float(1 << NS);
 #pragma unroll
-        for (int r = 0; r < W::NR; ++r) lam[r] = cscale(lam[r], 0x1p-32f);
+        for (int r = 0; r < W::NR; ++r) t[r] = cscale(t[r], f);
+        if (rs) {
+#pragma unroll
+          for (int r = 0; r < W::NR; ++r) lam[r] = cscale(lam[r], 0x1p-32f);
+        }
       }
     }
   }
@@ -627,48 +698,64 @@ __global__ __launch_bounds__((Wide<NS, R>::TL > 256 ? Wide<NS, R>::TL : 256)) vo
   }
 }
 
+// Register bits of the adjoint sweeps (two states).
+constexpr int adj_reg_bits(int ns) { return ns <= 5 ? 2 : wide_reg_bits(ns); }
+
+// Simulations per workgroup of the backward sweep: a row's columns together, up
+// to 256 threads, in whole waves, as far as the LDS allows.  The LDS is taken
+// for unshared coefficients, so that the choice depends on the plan and the
+// columns per row only.
 template <int NS>
-size_t adj_backward_lds(int N, int n_angles) {
-  using W = Wide<NS, wide_reg_bits(NS)>;
-  const int WV = W::TL > 64 ? W::TL / 64 : 1;
-  return size_t(N) * (W::BUF + NS) * sizeof(float2) + size_t(N) * WV * n_angles * sizeof(float);
+size_t adj_backward_lds(int N, int n_angles, int clanes) {
+  using A = AdjWide<NS, adj_reg_bits(NS)>;
+  const int WV = A::W::TL > 64 ? A::W::TL / 64 : 1;
+  return size_t(A::lds(N, adj_two_buffers(NS) ? 2 : 1, clanes)) * sizeof(float2) +
+         size_t(N) * WV * n_angles * sizeof(float);
+}
+
+template <int NS>
+int adj_backward_groups(int red, int n_angles) {
+  constexpr int TL = Wide<NS, adj_reg_bits(NS)>::TL;
+  int N = TL >= 256 ? 1 : std::min(256 / TL, red);
+  if (N * TL < 64) N = 64 / TL;
+  while (N > 1 && N * TL > 64 && adj_backward_lds<NS>(N, n_angles, TL) > kWideMaxLds / 2) N /= 2;
+  return N;
 }
 
 template <int NS>
 hipError_t adj_forward_launch(const Job& J, float2* ckpt, int ck, hipStream_t st) {
-  constexpr int R = wide_reg_bits(NS);
+  constexpr int R = adj_reg_bits(NS);
   using W = Wide<NS, R>;
+  const int clanes = AdjWide<NS, R>::clanes(J.S);
+  const size_t lds = size_t(AdjWide<NS, R>::lds(W::G, 1, clanes)) * sizeof(float2);
+  const void* kern = reinterpret_cast<const void*>(&k_wide_adj_forward<NS, R>);
+  if (lds > 65536) {
+    hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    if (e != hipSuccess) return e;
+  }
   hipLaunchKernelGGL((k_wide_adj_forward<NS, R>), dim3(unsigned((J.total + W::G - 1) / W::G)),
-                     dim3(W::T), 0, st, J, ckpt, ck);
+                     dim3(W::T), lds, st, J, ckpt, ck, clanes);
   return hipGetLastError();
-}
-
-// Threads per workgroup of the backward sweep: a row's columns together, up to
-// 256 threads, in whole waves, as far as the LDS allows.
-template <int NS>
-int adj_backward_groups(int red, int n_angles) {
-  constexpr int TL = Wide<NS, wide_reg_bits(NS)>::TL;
-  int N = TL >= 256 ? 1 : std::min(256 / TL, red);
-  if (N * TL < 64) N = 64 / TL;
-  while (N > 1 && N * TL > 64 && adj_backward_lds<NS>(N, n_angles) > kWideMaxLds / 2) N /= 2;
-  return N;
 }
 
 template <int NS>
 hipError_t adj_backward_launch(const Job& J, const float2* ckpt, const float2* seed,
                                const WideAdjoint& A, float* gpart, hipStream_t st) {
-  constexpr int R = wide_reg_bits(NS);
+  constexpr int R = adj_reg_bits(NS);
+  constexpr int TL = Wide<NS, R>::TL;
   const int N = adj_backward_groups<NS>(A.red, A.n_angles);
-  const size_t lds = adj_backward_lds<NS>(N, A.n_angles);
+  // neighbouring groups are columns of one row as far as the row goes
+  const int clanes = AdjWide<NS, R>::clanes(std::min(A.red, N));
+  const size_t lds = adj_backward_lds<NS>(N, A.n_angles, clanes);
+  const void* kern = reinterpret_cast<const void*>(&k_wide_adj_backward<NS, R>);
   if (lds > 65536) {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&k_wide_adj_backward<NS, R>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
+    hipError_t e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds));
     if (e != hipSuccess) return e;
   }
   const int rows = N / std::min(A.red, N);
   const int64_t n_rows = (J.total / A.C) * A.P;
   hipLaunchKernelGGL((k_wide_adj_backward<NS, R>), dim3(unsigned((n_rows + rows - 1) / rows)),
-                     dim3(unsigned(N * Wide<NS, R>::TL)), lds, st, J, ckpt, seed, A, gpart);
+                     dim3(unsigned(N * TL)), lds, st, J, ckpt, seed, A, clanes, gpart);
   return hipGetLastError();
 }
 
@@ -720,7 +807,7 @@ __global__ __launch_bounds__((Wide<kTileBits, kTileRegBits>::T)) void k_tile_pas
   const int64_t l = int64_t(blockIdx.x) >> tile_bits;          // simulation of this launch
   const uint32_t mid = blockIdx.x & ((1u << tile_bits) - 1);
   const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
-  const int32_t* resc = J.tab + J.off_svres;
+  const Constant<int32_t> resc = constant(J.tab + J.off_svres);
   int64_t bi, si;
   split_sim(J, g0 + l, &bi, &si);
   float2 t[W::NR];
@@ -737,8 +824,8 @@ __global__ __launch_bounds__((Wide<kTileBits, kTileRegBits>::T)) void k_tile_pas
       t[r] = flip(J.psi[si * J.in_stride + in_index[v]], sign[v] ? 0x80000000u : 0u);
     }
   }
-  wide_coeffs<kTileBits, kTileRegBits, false, M>(bs, steps, J.angles + bi * J.angle_stride,
-                                                 J.angle_stride_a, k0, J.n_steps, lane, nullptr);
+  wide_coeffs<M, false>(bs, steps, J.angles + bi * J.angle_stride, J.angle_stride_a, k0, J.n_steps,
+                        lane, W::T, nullptr);
   __syncthreads();
   if (sub == 0 && resc[k0 / J.ns]) {
 #pragma unroll
@@ -954,7 +1041,6 @@ hipError_t batch_launch(bool column, int64_t waves, const Job* jobs, const Batch
 
 #define MBQC_WIDE_SWITCH(ns, CALL)        \
   switch (ns) {                           \
-    case 6: return CALL(6);               \
     case 7: return CALL(7);               \
     case 8: return CALL(8);               \
     case 9: return CALL(9);               \
@@ -1055,8 +1141,12 @@ hipError_t launch_wide_batch(int ns, bool column, int64_t waves, const Job* jobs
 }
 
 bool wide_adjoint_fits(int ns, int red, int n_angles) {
-#define MBQC_CALL(NS) adj_backward_lds<NS>(adj_backward_groups<NS>(red, n_angles), n_angles) <= kWideMaxLds
+#define MBQC_CALL(NS)                                                                          \
+  adj_backward_lds<NS>(adj_backward_groups<NS>(red, n_angles), n_angles,                       \
+                       Wide<NS, adj_reg_bits(NS)>::TL) <= kWideMaxLds
   switch (ns) {
+    case 4: return MBQC_CALL(4);
+    case 5: return MBQC_CALL(5);
     case 6: return MBQC_CALL(6);
     case 7: return MBQC_CALL(7);
     case 8: return MBQC_CALL(8);
@@ -1071,16 +1161,32 @@ bool wide_adjoint_fits(int ns, int red, int n_angles) {
 #undef MBQC_CALL
 }
 
+#define MBQC_ADJ_SWITCH(ns, CALL)         \
+  switch (ns) {                           \
+    case 4: return CALL(4);               \
+    case 5: return CALL(5);               \
+    case 6: return CALL(6);               \
+    case 7: return CALL(7);               \
+    case 8: return CALL(8);               \
+    case 9: return CALL(9);               \
+    case 10: return CALL(10);             \
+    case 11: return CALL(11);             \
+    case 12: return CALL(12);             \
+    case 13: return CALL(13);             \
+    case 14: return CALL(14);             \
+    default: return hipErrorInvalidValue; \
+  }
+
 hipError_t launch_wide_adj_forward(const Job& J, float2* ckpt, int ck, hipStream_t st) {
 #define MBQC_CALL(NS) adj_forward_launch<NS>(J, ckpt, ck, st)
-  MBQC_WIDE_SWITCH(J.ns, MBQC_CALL)
+  MBQC_ADJ_SWITCH(J.ns, MBQC_CALL)
 #undef MBQC_CALL
 }
 
 hipError_t launch_wide_adj_backward(const Job& J, const float2* ckpt, const float2* seed,
                                     const WideAdjoint& A, float* gpart, hipStream_t st) {
 #define MBQC_CALL(NS) adj_backward_launch<NS>(J, ckpt, seed, A, gpart, st)
-  MBQC_WIDE_SWITCH(J.ns, MBQC_CALL)
+  MBQC_ADJ_SWITCH(J.ns, MBQC_CALL)
 #undef MBQC_CALL
 }
 

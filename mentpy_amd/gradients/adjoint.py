@@ -228,7 +228,7 @@ class MBQMLStep:
         if mode == "direct":
             segments = 1
         elif segments == "auto":
-            segments = int(L.mbqc_sv_segments_auto(eng.plan.handle, self.B))
+            segments = int(L.mbqc_sv_adjoint_segments(eng.plan.handle, self.B))
         self.segments = int(segments)
         if self.segments > 1:
             self._need = int(L.mbqc_sv_segmented_workspace_bytes(eng.plan.handle, self.B, self.segments))

@@ -56,12 +56,18 @@ def test_wide_windows_match_oracle(rows, cols, window, B, S, rng):
 
 @pytest.mark.parametrize("rows,cols,C,B", [(6, 14, 4, 5), (6, 14, 128, 512), (7, 12, 3, 2), (8, 4, 16, 3),
                                            (9, 4, 1, 3), (10, 4, 2, 1), (11, 3, 4, 1), (12, 3, 2, 1),
-                                           (13, 3, 2, 1), (14, 3, 1, 1)])
+                                           (13, 3, 2, 1), (14, 3, 1, 1),
+                                           (4, 5, 1, 1), (4, 20, 16, 5), (4, 19, 12, 3), (4, 6, 128, 3),
+                                           (4, 5, 16, 2048), (4, 5, 16, 2049), (5, 4, 1, 1),
+                                           (5, 15, 32, 7), (5, 16, 3, 2), (5, 5, 24, 2048),
+                                           (5, 5, 24, 2049)])
 def test_wide_adjoint_matches_complex128(rows, cols, C, B, rng):
     """Outputs and angle gradients of the register-blocked adjoint sweeps
     against torch autograd on the complex128 grid steps: one and several
     simulations per wave and per row, rows of 64 columns, checkpoint pairs
-    (65,536 columns), a rescale (more than 64 steps)."""
+    (65,536 columns), a rescale (more than 64 steps), shared and unshared
+    coefficients, the last and the first column count on either side of the
+    4- and 5-slot limits."""
     torch = _torch()
     import mentpy_amd as mp
     from mentpy_amd.gradients.adjoint import pattern_sv
