@@ -306,6 +306,19 @@ int mbqc_sv_adjoint_backward_c64(const mbqc_plan* plan, const float* angles, int
                                  const void* ckpt, size_t ckpt_bytes, float* grad_partial,
                                  void* stream);
 
+/* Angle gradients from outputs and seed alone, without checkpoints, for plans
+ * whose steps are one unitary grid step each (column order, 2 to 5 live qubits, all of
+ * them outputs; mbqc_sv_has_outputs_gradient).  out[B][C][2^n_outputs] are the outputs
+ * of mbqc_sv_forward_c64 in the raw phase frame (flags 0) for the same angles,
+ * seed in the same layout as for mbqc_sv_adjoint_backward_c64.  Writes
+ * grad[B][n_angles] (entries of non-trainable angles are left untouched).  The work
+ * per set grows as 4^n_outputs per step whatever C is, so it is meant for C of about
+ * 2^n_outputs and more (the transfer matrix). */
+int32_t mbqc_sv_has_outputs_gradient(const mbqc_plan* plan);
+int mbqc_sv_outputs_gradient_c64(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
+                                 int64_t angle_stride_a, const void* out, const void* seed, int64_t B,
+                                 int64_t C, float* grad, void* stream);
+
 /* Time-segmented transfer-matrix adjoint (no reference counterpart: the
  * reference differentiates by finite differences, mentpy/gradients/
  * _finite_difference.py:9-24).  The columns are the 2^n_inputs input basis
@@ -316,16 +329,14 @@ int mbqc_sv_adjoint_backward_c64(const mbqc_plan* plan, const float* angles, int
  * times as many lanes for 1/n_segments of the steps each (small batches fill
  * the chip).  2 <= n_segments <= min(16, number of blocks).
  *
- * mbqc_sv_segments_auto: the segment count that fills the chip for B sets
- * (1 means: use the unsegmented entry points).  mbqc_sv_adjoint_segments: the
- * same, or 1 where the unsegmented entry points are faster for this plan.
+ * mbqc_sv_segments_auto: the segment count the library picks for B sets
+ * (1 means: use the unsegmented entry points).
  * Forward: out[B][2^n_inputs][2^n_outputs] = T_b (column c = image of input
  * basis state c).  Backward: seed in the same layout (dL = Re sum conj(seed)
  * d(out)); writes grad[B][n_angles] (entries of non-trainable angles are left
  * untouched).  The backward needs the workspace of the forward of the same
  * angles. */
 int32_t mbqc_sv_segments_auto(const mbqc_plan* plan, int64_t B);
-int32_t mbqc_sv_adjoint_segments(const mbqc_plan* plan, int64_t B);
 size_t mbqc_sv_segmented_workspace_bytes(const mbqc_plan* plan, int64_t B, int32_t n_segments);
 int mbqc_sv_segmented_forward_c64(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
                                   int64_t angle_stride_a, void* out, int64_t B, int32_t n_segments,

@@ -47,7 +47,7 @@ EXPORTED_SYMBOLS = (
     "mbqc_overlap_loss_seed_c64",
     "mbqc_sv_adjoint_workspace_bytes", "mbqc_sv_adjoint_forward_c64",
     "mbqc_sv_adjoint_partials", "mbqc_sv_adjoint_backward_c64", "mbqc_sv_segments_auto",
-    "mbqc_sv_adjoint_segments",
+    "mbqc_sv_has_outputs_gradient", "mbqc_sv_outputs_gradient_c64",
     "mbqc_sv_segmented_workspace_bytes", "mbqc_sv_segmented_forward_c64",
     "mbqc_sv_segmented_backward_c64", "mbqc_batch_create",
     "mbqc_batch_destroy", "mbqc_batch_items", "mbqc_batch_launch", "mbqc_batch_group_items",
@@ -164,8 +164,10 @@ def lib() -> C.CDLL:
     L.mbqc_overlap_loss_seed_c64.restype = C.c_int
     L.mbqc_sv_segments_auto.argtypes = [vp, i64]
     L.mbqc_sv_segments_auto.restype = i32
-    L.mbqc_sv_adjoint_segments.argtypes = [vp, i64]
-    L.mbqc_sv_adjoint_segments.restype = i32
+    L.mbqc_sv_has_outputs_gradient.argtypes = [vp]
+    L.mbqc_sv_has_outputs_gradient.restype = i32
+    L.mbqc_sv_outputs_gradient_c64.argtypes = [vp, vp, i64, i64, vp, vp, i64, i64, vp, vp]
+    L.mbqc_sv_outputs_gradient_c64.restype = i32
     L.mbqc_sv_segmented_workspace_bytes.argtypes = [vp, i64, i32]
     L.mbqc_sv_segmented_workspace_bytes.restype = sz
     L.mbqc_sv_segmented_forward_c64.argtypes = [vp, vp, i64, i64, vp, i64, i32, vp, sz, vp]

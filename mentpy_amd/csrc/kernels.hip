@@ -4313,21 +4313,6 @@ int32_t mbqc_sv_segments_auto(const mbqc_plan* plan, int64_t B) {
   return int32_t(std::max<int64_t>(n, 1));
 }
 
-int32_t mbqc_sv_adjoint_segments(const mbqc_plan* plan, int64_t B) {
-  const int32_t n = mbqc_sv_segments_auto(plan, B);
-  if (n <= 1) return n;
-  const Plan* p = reinterpret_cast<const Plan*>(plan);
-  // Windows of 4 and 5 slots: the sweep over all blocks, several lanes per
-  // column, takes less than the segments and their chain (whole step in us,
-  // segments -> one sweep; 4x16 grid: 16 sets 54.2 -> 37.7, 1024 sets
-  // 63.1 -> 51.5, 4096 sets 128 -> 110; 5x10 grid: 147.8 -> 80.4, 466.8 -> 371.1,
-  // 2048 sets 799 -> 698; 5x40 grid: 211.2 -> 131.0, 569.7 -> 511.0).  The chain
-  // of 4-slot steps is the longer one from about 130 steps (16 sets, 124
-  // steps: 60.8 -> 58.5, 156 steps: 61.3 -> 69.0).
-  if (p->column_steps && (p->ns == 5 || (p->ns == 4 && p->n_steps <= 128))) return 1;
-  return n;
-}
-
 size_t mbqc_sv_segmented_workspace_bytes(const mbqc_plan* plan, int64_t B, int32_t n_segments) {
   if (!plan) return 0;
   return seg_layout(*reinterpret_cast<const Plan*>(plan), B, n_segments, nullptr);
@@ -4494,6 +4479,38 @@ int mbqc_sv_adjoint_backward_c64(const mbqc_plan* plan, const float* angles, int
     case 16: e = launch_adj_bwd_global<16>(J, ck, sd, A, st); break;
   }
   return e == hipSuccess ? MBQC_OK : global_fail(e, "adjoint backward launch");
+}
+
+// Plans whose angle gradients follow from the outputs alone.
+static bool outputs_gradient(const Plan* p) {
+  return p->column_steps && p->ns >= 2 && p->ns <= kMaxAdjSlots && p->n_out == p->ns &&
+         check_adjoint_plan(p) == MBQC_OK;
+}
+
+int32_t mbqc_sv_has_outputs_gradient(const mbqc_plan* plan) {
+  return plan && outputs_gradient(reinterpret_cast<const Plan*>(plan)) ? 1 : 0;
+}
+
+int mbqc_sv_outputs_gradient_c64(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
+                                 int64_t angle_stride_a, const void* out, const void* seed, int64_t B,
+                                 int64_t C, float* grad, void* stream) {
+  if (!plan) return fail(MBQC_ERR_VALUE, "null plan");
+  Plan* p = const_cast<Plan*>(reinterpret_cast<const Plan*>(plan));
+  int rc = check_adjoint_plan(p);
+  if (rc != MBQC_OK) return rc;
+  if (!outputs_gradient(p))
+    return fail(MBQC_ERR_NOT_IMPLEMENTED,
+                "gradients from the outputs alone need a grid plan of 2 to 5 live qubits, all outputs");
+  if (!out || !seed || !grad) return fail(MBQC_ERR_VALUE, "null output, seed or gradient pointer");
+  Job J;
+  rc = make_job(p, angles, angle_stride, angle_stride_a, out, 0, const_cast<void*>(out), B, C, &J);
+  if (rc != MBQC_OK) return rc;
+  if (B > 0x7fffffff || C > 0x7fffff) return fail(MBQC_ERR_VALUE, "too many simulations for one launch");
+  if (J.total == 0) return MBQC_OK;
+  hipError_t e = launch_pauli_gradient(J, static_cast<const float2*>(out),
+                                       static_cast<const float2*>(seed), B, C, p->n_angles, grad,
+                                       static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? MBQC_OK : hip_fail(e, "outputs gradient launch");
 }
 
 int mbqc_batch_create(const mbqc_batch_job* jobs, int32_t n_jobs, int32_t sims_per_item,

@@ -51,6 +51,11 @@ hipError_t launch_wide_adj_forward(const Job& J, float2* ckpt, int ck, hipStream
 hipError_t launch_wide_adj_backward(const Job& J, const float2* ckpt, const float2* seed,
                                     const WideAdjoint& A, float* gpart, hipStream_t st);
 
+// Angle gradients of a column plan of 2..5 slots whose slots are all outputs, from
+// outputs and seed [B][C][2^ns] alone, into grad[B][n_angles].
+hipError_t launch_pauli_gradient(const Job& J, const float2* out, const float2* seed, int64_t B,
+                                 int64_t C, int n_angles, float* grad, hipStream_t st);
+
 // Density matrices of column plans with 2..7 slots (wide_dm.hip); pad_slots:
 // slots that start as |+> padding (n_slots - n_inputs).
 hipError_t launch_dm_pauli(const Job& J, const DmNoise& nz, int pad_slots, uint32_t flags,

@@ -333,6 +333,201 @@ __global__ __launch_bounds__((Pauli<NS, K>::T)) void k_dm_pauli(Job J, DmNoise n
                    std::make_integer_sequence<int, W::P>{});
 }
 
+// ------------------------------------------------------------ angle gradients
+//
+// The steps of a column plan are unitary up to their scale, so the gradient needs
+// neither the states nor the cotangents of the steps in between, only
+//   G = sum over columns of |out><seed|   (2^NS x 2^NS),
+// taken backwards through the steps, G -> U^-1 G U: with outputs
+// out_c = U_n ... U_1 in_c and dL = Re sum conj(seed) d(out) the derivative by the
+// angle of step k is Im Tr(P1 G_k), P1 = (1 - Z) / 2 on the measured qubit and
+// G_k before the step's butterfly.  The imaginary parts of Tr(G P) are 4^NS real
+// numbers that evolve among themselves, so a step backwards is the transpose of a
+// density matrix step: per parameter set 4^NS multiply-adds where the sweep of
+// states and cotangents takes 9 C 2^NS for C columns, no checkpoints, and the
+// derivative of a step is two coefficients, (I - Z) / 2.
+
+// The inverse of pauli_rotate.
+template <int NS, int K, int M, bool CZ>
+__device__ __forceinline__ void pauli_unrotate(float (&t)[1 << (2 * K)], float* buf, int lane) {
+  using W = Pauli<NS, K>;
+  if constexpr (K == NS) return;
+  lanes_sync<W::TL>();
+#pragma unroll
+  for (int r = 0; r < W::N; ++r) buf[pad_real((r << (2 * W::LD)) | lane)] = t[r];
+  lanes_sync<W::TL>();
+  constexpr int LOW = 2 * (K - M);
+  const int xq = CZ ? (lane >> 1) & 1 : 0, zq = CZ ? lane & 1 : 0;
+  const uint32_t neg0 = uint32_t(xq & zq) << 31, neg1 = uint32_t(xq & ~zq) << 31;
+#pragma unroll
+  for (int r = 0; r < W::N; ++r) {
+    if ((r >> LOW) & 3) continue;
+    float v[4];
+    if constexpr (CZ && M == 1) {
+      const float2 a = *reinterpret_cast<const float2*>(buf + pad_real(rotated<NS, K, M>(r, lane)));
+      const float2 b =
+          *reinterpret_cast<const float2*>(buf + pad_real(rotated<NS, K, M>(r, lane ^ 1)) + 2);
+      v[0] = xq ? a.y : a.x;
+      v[1] = xq ? a.x : a.y;
+      v[2] = __uint_as_float(__float_as_uint(xq ? b.y : b.x) ^ neg0);
+      v[3] = __uint_as_float(__float_as_uint(xq ? b.x : b.y) ^ neg1);
+    } else {
+      int at = pad_real(rotated<NS, K, M>(r, lane));
+      uint32_t sg = 0;
+      if constexpr (CZ) {
+        constexpr int ZB = 2 * (K - 1), D = 1 << (2 * (M - 1));
+        const int z0 = (r >> ZB) & 1, x0 = (r >> (ZB + 1)) & 1;
+        if (x0) {
+          at = pad_real(rotated<NS, K, M>(r, lane ^ 1));
+          sg = z0 ? neg1 : neg0;
+        }
+        at += (z0 ? -xq : xq) * D;
+      }
+      const float4 u = *reinterpret_cast<const float4*>(buf + at);
+      const float w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+      for (int d = 0; d < 4; ++d) v[d] = __uint_as_float(__float_as_uint(w[d]) ^ sg);
+    }
+#pragma unroll
+    for (int d = 0; d < 4; ++d) t[r | (d << LOW)] = v[d];
+  }
+}
+
+// The inverse of pauli_step (gamma = 1); returns the Z coefficient of the digit
+// alone (lane 0's), which the phase before it leaves as it is.
+template <int K, int S>
+__device__ __forceinline__ float pauli_unstep(float (&t)[1 << (2 * K)], float c, float s) {
+  constexpr int N = 1 << (2 * K), SH = 2 * (K - 1 - S);
+  float n[N];
+#pragma unroll
+  for (int b = 0; b < N; ++b) {
+    if ((b >> SH) & 3) continue;
+    float v[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      int to = b | (d << SH);
+      bool neg = false;
+      if constexpr (S > 0) {
+        const int x = d >> 1, z = d & 1, q = (b >> (SH + 2)) & 3, xq = q >> 1, zq = q & 1;
+        to ^= (xq << SH) | (x << (SH + 2));
+        neg = x && xq && (z ^ zq);
+      }
+      v[d] = neg ? -t[to] : t[to];
+    }
+    n[b] = v[0];
+    n[b | (1 << SH)] = v[2];
+    n[b | (2 << SH)] = fmaf(s, v[3], c * v[1]);
+    n[b | (3 << SH)] = fmaf(-c, v[3], s * v[1]);
+  }
+#pragma unroll
+  for (int b = 0; b < N; ++b) t[b] = n[b];
+  return t[1 << SH];
+}
+
+template <int NS, int K, int P, int... SS>
+__device__ __forceinline__ void unstep_phase(float (&t)[1 << (2 * K)], float* buf, const float2* bs,
+                                             float (&z)[NS], int lane,
+                                             std::integer_sequence<int, SS...>) {
+  using W = Pauli<NS, K>;
+  constexpr int F = W::first(P), M = W::len(P);
+  pauli_unrotate<NS, K, M, (P > 0)>(t, buf, lane);
+  ((z[F + M - 1 - SS] = pauli_unstep<K, M - 1 - SS>(t, bs[F + M - 1 - SS].x, -bs[F + M - 1 - SS].y)),
+   ...);
+}
+
+// m += a conj(b)
+__device__ __forceinline__ void cmul_conj_add(float2& m, float2 a, float2 b) {
+  m.x = fmaf(a.x, b.x, fmaf(a.y, b.y, m.x));
+  m.y = fmaf(a.y, b.x, fmaf(-a.x, b.y, m.y));
+}
+
+template <int NS, int K, int... PS>
+__device__ __forceinline__ void pauli_gradient(const Job& J, const float2* out, const float2* seed,
+                                               int64_t bi, bool active, int C, int n_angles,
+                                               float* grad, float2* buf, float2* bs, int lane,
+                                               std::integer_sequence<int, PS...>) {
+  using W = Pauli<NS, K>;
+  const float* ang = J.angles + bi * J.angle_stride;
+  const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
+  const Constant<int32_t> aidx = constant(J.tab + J.off_aidx);
+  const int32_t* out_pos = J.tab + J.off_out;
+  const int n = J.n_steps;
+  float t[W::N];
+  {
+    float2 m[W::N];
+    const int la = every_second_bit(lane >> 1), lb = every_second_bit(lane);
+    const float2* pa[1 << K];
+    const float2* pb[1 << K];
+#pragma unroll
+    for (int i = 0; i < (1 << K); ++i) {
+      pa[i] = out + ((bi * C) << NS) + out_pos[(i << W::LD) | la];
+      pb[i] = seed + ((bi * C) << NS) + out_pos[(i << W::LD) | lb];
+    }
+#pragma unroll
+    for (int r = 0; r < W::N; ++r) m[r] = make_float2(0.0f, 0.0f);
+#pragma unroll 8
+    for (int c = 0; c < C; ++c) {
+      float2 va[1 << K], vb[1 << K];
+#pragma unroll
+      for (int i = 0; i < (1 << K); ++i) {
+        va[i] = pa[i][int64_t(c) << NS];
+        vb[i] = pb[i][int64_t(c) << NS];
+      }
+#pragma unroll
+      for (int r = 0; r < W::N; ++r)
+        cmul_conj_add(m[r], va[every_second_bit(r >> 1)], vb[every_second_bit(r)]);
+    }
+    (in_phase<NS, K, PS>(m, buf, lane, std::make_integer_sequence<int, W::len(PS)>{}), ...);
+#pragma unroll
+    for (int r = 0; r < W::N; ++r) t[r] = m[r].y;
+  }
+  const float all = t[0];     // of lane 0: the coefficient of I...I, constant from here on
+  const bool writer = active && lane == 0;
+  float* gp = grad + bi * n_angles;
+  for (int kc = ((n - 1) / W::CS) * W::CS; kc >= 0; kc -= W::CS) {
+    lanes_sync<W::TL>();      // the previous chunk's reads are done
+#pragma unroll 1
+    for (int i = lane; i < W::CS; i += W::TL) {
+      const int k = kc + i;
+      if (k < n) bs[i] = exp_minus_i(step_angle(steps[k], ang, J.angle_stride_a));
+    }
+    lanes_sync<W::TL>();
+    const int ke = kc + W::CS < n ? kc + W::CS : n;
+    for (int k0 = ke - NS; k0 >= kc; k0 -= NS) {
+      float2 b[NS];
+      float z[NS];
+      int ai[NS];
+#pragma unroll
+      for (int k = 0; k < NS; ++k) {
+        b[k] = bs[k0 - kc + k];
+        ai[k] = aidx[k0 + k];
+      }
+      (unstep_phase<NS, K, W::P - 1 - PS>(t, reinterpret_cast<float*>(buf), b, z, lane,
+                                          std::make_integer_sequence<int, W::len(W::P - 1 - PS)>{}),
+       ...);
+      if (writer) {
+#pragma unroll
+        for (int k = 0; k < NS; ++k)
+          if (ai[k] >= 0) gp[ai[k]] = 0.5f * (all - z[k]);
+      }
+    }
+  }
+}
+
+template <int NS, int K>
+__global__ __launch_bounds__((Pauli<NS, K>::T)) void k_pauli_gradient(
+    Job J, const float2* __restrict__ out, const float2* __restrict__ seed, int64_t B, int C,
+    int n_angles, float* __restrict__ grad) {
+  using W = Pauli<NS, K>;
+  __shared__ __align__(16) float2 lds[W::G * W::SIM];
+  const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
+  float2* buf = lds + sub * W::SIM;
+  const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
+  const bool active = g < B;
+  pauli_gradient<NS, K>(J, out, seed, active ? g : B - 1, active, C, n_angles, grad, buf,
+                        buf + W::BUF, lane, std::make_integer_sequence<int, W::P>{});
+}
+
 // Register digits K: one keeps many lanes on a simulation and the chain of a step
 // short, two halve the exchanges.  Measured (us per replayed launch, the matrix
 // kernels before / K = 1 / K = 2): 3 slots (12 columns) 1,024 sims 10.2 / 6.7 /
@@ -352,7 +547,33 @@ hipError_t dm_launch(const Job& J, const DmNoise& nz, int pad_slots, uint32_t fl
   return hipGetLastError();
 }
 
+template <int NS, int K>
+hipError_t gradient_launch(const Job& J, const float2* out, const float2* seed, int64_t B, int64_t C,
+                           int n_angles, float* grad, hipStream_t st) {
+  using W = Pauli<NS, K>;
+  hipLaunchKernelGGL((k_pauli_gradient<NS, K>), dim3(unsigned((B + W::G - 1) / W::G)), dim3(W::T), 0,
+                     st, J, out, seed, B, int(C), n_angles, grad);
+  return hipGetLastError();
+}
+
 }  // namespace
+
+// Register digits, us per replayed launch with the transfer matrix's columns, K = 1 /
+// K = 2: 2x12 grid, 16,384 sets 8.6 / 12.9; 3x12 grid, 16 sets 7.3 / 12.4, 16,384
+// 14.6 / 18.3; 4x16 grid, 1,024 sets 12.0 / 14.9, 4,096 22.4 / 18.1; 5x10 grid,
+// 1,024 sets 29.0 / 19.9.
+hipError_t launch_pauli_gradient(const Job& J, const float2* out, const float2* seed, int64_t B,
+                                 int64_t C, int n_angles, float* grad, hipStream_t st) {
+  switch (J.ns) {
+    case 2: return gradient_launch<2, 1>(J, out, seed, B, C, n_angles, grad, st);
+    case 3: return gradient_launch<3, 1>(J, out, seed, B, C, n_angles, grad, st);
+    case 4:
+      return B <= kDm4OneDigitMaxSims ? gradient_launch<4, 1>(J, out, seed, B, C, n_angles, grad, st)
+                                      : gradient_launch<4, 2>(J, out, seed, B, C, n_angles, grad, st);
+    case 5: return gradient_launch<5, 2>(J, out, seed, B, C, n_angles, grad, st);
+    default: return hipErrorInvalidValue;
+  }
+}
 
 hipError_t launch_dm_pauli(const Job& J, const DmNoise& nz, int pad_slots, uint32_t flags,
                            hipStream_t st) {

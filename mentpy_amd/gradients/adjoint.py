@@ -171,10 +171,12 @@ class MBQMLStep:
     * ``"transfer"``: transfer matrix, then ``T X`` and ``(Phi f) X^H`` GEMMs.
     * ``"direct"``: the inputs themselves are the propagated columns.
 
-    In the transfer-matrix modes the steps can be cut in time
+    In the transfer-matrix modes of a grid pattern of 2 to 5 rows the gradient
+    is taken from the outputs and the seed alone.  For other patterns the steps can be cut in time
     (``segments``): the segments' transfer matrices are computed
     concurrently and chained per parameter set, which fills the chip when
-    ``B`` is small.  ``"auto"`` lets the library pick (1 = no cut).
+    ``B`` is small.  ``"auto"`` lets the library pick (1 = no cut); a number
+    above 1 cuts grid patterns too.
 
     All buffers are allocated once, so a step can be captured in a HIP graph
     (``capture``); write new angles into ``self.angles`` before each replay.
@@ -225,17 +227,21 @@ class MBQMLStep:
             nbytes = int(nat.lib().mbqc_gram_workspace_bytes(self.B, K))
             self._gws = torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device=dev)
         L = nat.lib()
-        if mode == "direct":
+        # the whole transfer matrix of a grid pattern: gradients from the outputs
+        # alone, whatever the steps between
+        self._from_outputs = (mode != "direct" and segments in ("auto", 1) and
+                              bool(L.mbqc_sv_has_outputs_gradient(eng.plan.handle)))
+        if mode == "direct" or self._from_outputs:
             segments = 1
         elif segments == "auto":
-            segments = int(L.mbqc_sv_adjoint_segments(eng.plan.handle, self.B))
+            segments = int(L.mbqc_sv_segments_auto(eng.plan.handle, self.B))
         self.segments = int(segments)
         if self.segments > 1:
             self._need = int(L.mbqc_sv_segmented_workspace_bytes(eng.plan.handle, self.B, self.segments))
             if self._need == 0:
                 raise ValueError(f"segments={self.segments} is out of range for this pattern")
             self._ws = torch.empty(self._need, dtype=torch.uint8, device=dev)
-        else:
+        elif not self._from_outputs:
             self._need = eng.workspace_bytes(self.B * C_)
             self._ws = torch.empty(max(self._need, 8), dtype=torch.uint8, device=dev)
 
@@ -269,6 +275,11 @@ class MBQMLStep:
                        self.angles.data_ptr(), sb, sa, self.out.data_ptr(), self.B, self.segments,
                        self._ws.data_ptr(), self._need)
             return
+        if self._from_outputs:
+            nat.launch(eng.device, nat.lib().mbqc_sv_forward_c64, eng.plan.handle,
+                       self.angles.data_ptr(), sb, sa, self.cols.data_ptr(), self.cols.shape[1],
+                       self.out.data_ptr(), None, self.B, self.cols.shape[0], 0)
+            return
         nat.launch(eng.device, nat.lib().mbqc_sv_adjoint_forward_c64, eng.plan.handle,
                    self.angles.data_ptr(), sb, sa, self.cols.data_ptr(), self.cols.shape[1],
                    self.out.data_ptr(), self.B, self.cols.shape[0], self._ws.data_ptr(), self._need)
@@ -280,6 +291,11 @@ class MBQMLStep:
             nat.launch(eng.device, nat.lib().mbqc_sv_segmented_backward_c64, eng.plan.handle,
                        self.angles.data_ptr(), sb, sa, self.seed.data_ptr(), self.B, self.segments,
                        self._ws.data_ptr(), self._need, self.part.data_ptr())
+            return
+        if self._from_outputs:   # P = 1: 2^n columns
+            nat.launch(eng.device, nat.lib().mbqc_sv_outputs_gradient_c64, eng.plan.handle,
+                       self.angles.data_ptr(), sb, sa, self.out.data_ptr(), self.seed.data_ptr(),
+                       self.B, self.cols.shape[0], self.part.data_ptr())
             return
         nat.launch(eng.device, nat.lib().mbqc_sv_adjoint_backward_c64, eng.plan.handle,
                    self.angles.data_ptr(), sb, sa, self.seed.data_ptr(), self.B, self.cols.shape[0],

@@ -54,6 +54,28 @@ def test_wide_windows_match_oracle(rows, cols, window, B, S, rng):
     assert err < 2e-5, f"amplitude error {err}"
 
 
+def _grid_outputs(a, x, rows, cols):
+    """Raw-phase outputs of a grid pattern, differentiable in complex128: angles
+    a [B, n], inputs x [C, 2^rows]."""
+    torch = _torch()
+    B, C, d = a.shape[0], x.shape[0], 1 << rows
+    j = torch.arange(d, device="cuda")
+    bit = [((j >> (rows - 1 - i)) & 1).double() for i in range(rows)]
+    t = x.to(torch.complex128)
+    for i in range(rows - 1):
+        t = t * (1 - 2 * bit[i] * bit[i + 1])
+    t = t[None].expand(B, -1, -1)
+    for k in range(rows * (cols - 1)):
+        i, col = k % rows, k // rows
+        ph = torch.polar(torch.ones_like(a[:, 0]), -a[:, i * (cols - 1) + col])
+        v = t.reshape(B, C, 1 << i, 2, -1)
+        p, q = v[:, :, :, 0], v[:, :, :, 1] * ph[:, None, None, None]
+        t = (torch.stack([p + q, p - q], 3) * 0.5 ** 0.5).reshape(B, C, d)
+        if i:
+            t = t * (1 - 2 * bit[i - 1] * bit[i])
+    return t
+
+
 @pytest.mark.parametrize("rows,cols,C,B", [(6, 14, 4, 5), (6, 14, 128, 512), (7, 12, 3, 2), (8, 4, 16, 3),
                                            (9, 4, 1, 3), (10, 4, 2, 1), (11, 3, 4, 1), (12, 3, 2, 1),
                                            (13, 3, 2, 1), (14, 3, 1, 1),
@@ -83,20 +105,7 @@ def test_wide_adjoint_matches_complex128(rows, cols, C, B, rng):
     grad, = torch.autograd.grad(out, th, cot)
     bs = list(range(B)) if B < 8 else [0, B // 2, B - 1]
     a = th.detach()[bs].double().requires_grad_(True)
-    j = torch.arange(d, device="cuda")
-    bit = [((j >> (rows - 1 - i)) & 1).double() for i in range(rows)]
-    t = x.to(torch.complex128)
-    for i in range(rows - 1):
-        t = t * (1 - 2 * bit[i] * bit[i + 1])
-    t = t[None].expand(len(bs), -1, -1)
-    for k in range(rows * (cols - 1)):
-        i, col = k % rows, k // rows
-        ph = torch.polar(torch.ones_like(a[:, 0]), -a[:, i * (cols - 1) + col])
-        v = t.reshape(len(bs), C, 1 << i, 2, -1)
-        p, q = v[:, :, :, 0], v[:, :, :, 1] * ph[:, None, None, None]
-        t = (torch.stack([p + q, p - q], 3) * 0.5 ** 0.5).reshape(len(bs), C, d)
-        if i:
-            t = t * (1 - 2 * bit[i - 1] * bit[i])
+    t = _grid_outputs(a, x, rows, cols)
     want, = torch.autograd.grad(t, a, cot[bs].to(torch.complex128))
     oerr = (out.detach()[bs] - t.detach()).abs().max().item()
     scale = want.abs().max().item()
@@ -105,6 +114,56 @@ def test_wide_adjoint_matches_complex128(rows, cols, C, B, rng):
     # sqrt(2 C): far below 2e-5 of the largest entry
     assert oerr < 2e-5, f"output error {oerr}"
     assert gerr < 2e-5 * max(scale, 1.0), f"gradient error {gerr} of {scale}"
+
+
+@pytest.mark.parametrize("rows,cols,C,B", [(2, 4, 4, 1), (2, 34, 4, 67), (3, 5, 3, 4), (3, 24, 8, 5),
+                                           (4, 3, 16, 1), (4, 18, 16, 6), (4, 6, 17, 2048),
+                                           (4, 6, 1, 2049), (4, 18, 16, 2051), (5, 4, 32, 1),
+                                           (5, 14, 33, 3)])
+def test_gradient_from_outputs_matches_complex128(rows, cols, C, B, rng):
+    """Angle gradients from outputs and cotangents alone against torch autograd on
+    the complex128 grid steps: every window, one and two register digits on
+    either side of their limit, partly filled last workgroups, several
+    coefficient chunks, fewer, as many and more columns than the transfer matrix."""
+    torch = _torch()
+    import mentpy_amd as mp
+    from mentpy_amd import _native as nat
+    g = mp.templates.grid_cluster(rows, cols)
+    sim = mp.PatternSimulator(g, backend="hip-sv")
+    plan = sim.simulator.plan
+    assert nat.lib().mbqc_sv_has_outputs_gradient(plan.handle) == 1
+    n, d = len(g.trainable_nodes), 1 << rows
+    gen = torch.Generator().manual_seed(rows * cols)
+    th = (torch.rand((B, n), generator=gen) * 6.2).cuda()
+    x = torch.randn((C, d), generator=gen, dtype=torch.complex64).cuda()
+    x = x / torch.linalg.vector_norm(x, dim=1, keepdim=True)
+    cot = torch.randn((B, C, d), generator=gen, dtype=torch.complex64).cuda() / d ** 0.5
+    bs = list(range(B)) if B < 8 else [0, B // 2, B - 1]
+    a = th[bs].double().requires_grad_(True)
+    t = _grid_outputs(a, x, rows, cols)
+    want, = torch.autograd.grad(t, a, cot[bs].to(torch.complex128))
+    out = torch.empty((B, C, d), dtype=torch.complex64, device="cuda")
+    grad = torch.full((B, n), float("nan"), device="cuda")
+    nat.launch(out.device, nat.lib().mbqc_sv_forward_c64, plan.handle, th.data_ptr(), n, 1,
+               x.data_ptr(), d, out.data_ptr(), None, B, C, 0)
+    nat.launch(out.device, nat.lib().mbqc_sv_outputs_gradient_c64, plan.handle, th.data_ptr(), n, 1,
+               out.data_ptr(), cot.data_ptr(), B, C, grad.data_ptr())
+    assert torch.isfinite(grad).all()
+    # one rounding (6e-8) per step on coefficients of norm about sqrt(2 C): far
+    # below 2e-5 of the largest entry
+    gerr = (grad[bs] - want).abs().max().item()
+    scale = want.abs().max().item()
+    assert gerr < 2e-5 * max(scale, 1.0), f"gradient error {gerr} of {scale}"
+
+
+def test_gradient_from_outputs_refuses_other_plans():
+    """Six rows, and a window with spare slots."""
+    _torch()
+    import mentpy_amd as mp
+    from mentpy_amd import _native as nat
+    for rows, kw in ((6, {}), (3, {"window_size": 5})):
+        sim = mp.PatternSimulator(mp.templates.grid_cluster(rows, 4), backend="hip-sv", **kw)
+        assert nat.lib().mbqc_sv_has_outputs_gradient(sim.simulator.plan.handle) == 0
 
 
 @pytest.mark.parametrize("rows,cols,window,B,S", [
