@@ -311,13 +311,15 @@ int mbqc_sv_adjoint_backward_c64(const mbqc_plan* plan, const float* angles, int
  * them outputs; mbqc_sv_has_outputs_gradient).  out[B][C][2^n_outputs] are the outputs
  * of mbqc_sv_forward_c64 in the raw phase frame (flags 0) for the same angles,
  * seed in the same layout as for mbqc_sv_adjoint_backward_c64.  Writes
- * grad[B][n_angles] (entries of non-trainable angles are left untouched).  The work
+ * grad[B][n_angles] (entries of non-trainable angles are left untouched) and, if
+ * loss is not null, loss[B] = 1 + Re sum conj(seed) out / 2, which is the loss itself
+ * for losses 1 - q(out) with q quadratic (the MB-QML infidelity).  The work
  * per set grows as 4^n_outputs per step whatever C is, so it is meant for C of about
  * 2^n_outputs and more (the transfer matrix). */
 int32_t mbqc_sv_has_outputs_gradient(const mbqc_plan* plan);
 int mbqc_sv_outputs_gradient_c64(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
                                  int64_t angle_stride_a, const void* out, const void* seed, int64_t B,
-                                 int64_t C, float* grad, void* stream);
+                                 int64_t C, float* loss, float* grad, void* stream);
 
 /* Time-segmented transfer-matrix adjoint (no reference counterpart: the
  * reference differentiates by finite differences, mentpy/gradients/
@@ -417,6 +419,20 @@ int mbqc_gram_loss_seed_c64(const void* t, const void* MT, int64_t B, int32_t K,
  * race. */
 int mbqc_gram_loss_seed_c64_noalloc(const void* t, const void* MT, int64_t B, int32_t K,
                                     int32_t S, float* loss, void* seed, void* stream);
+
+/* The seed alone (the gradient launch gives the loss, mbqc_sv_outputs_gradient_c64);
+ * any K. */
+int mbqc_gram_seed_c64(const void* t, const void* MT, int64_t B, int32_t K, int32_t S, void* seed,
+                       void* stream);
+
+/* The same loss and seed through the data themselves, for few of them: with
+ * D[s][k] = psi_s[c] conj(phi_s[o]) (k = (c, o)), f_b = D t_b, loss[b] = 1 -
+ * |f_b|^2 / S and seed[b] = -2 D^H f_b / S.  DT is [K][S] = D transposed, DC [S][K] =
+ * conj(D); seed and DC may be null (loss only), or loss may (seed only).  workspace:
+ * mbqc_transfer_workspace_bytes(B, S) bytes of device memory.  Any K and S. */
+size_t mbqc_transfer_workspace_bytes(int64_t B, int32_t S);
+int mbqc_transfer_loss_seed_c64(const void* t, const void* DT, const void* DC, int64_t B, int32_t K,
+                                int32_t S, float* loss, void* seed, void* workspace, void* stream);
 
 /* MB-QML infidelity loss from propagated inputs (no reference counterpart as
  * one kernel: the reference evaluates calculator.fidelity per pair,

@@ -43,7 +43,7 @@ EXPORTED_SYMBOLS = (
     "mbqc_dm_forward_outcomes_c64",
     "mbqc_plan_window_qubits", "mbqc_sv_window_c64", "mbqc_dm_window_c64",
     "mbqc_gram_workspace_bytes", "mbqc_gram_loss_seed_c64", "mbqc_gram_loss_seed_c64_noalloc",
-    "mbqc_gram_finish_c64",
+    "mbqc_gram_finish_c64", "mbqc_gram_seed_c64", "mbqc_transfer_workspace_bytes", "mbqc_transfer_loss_seed_c64",
     "mbqc_overlap_loss_seed_c64",
     "mbqc_sv_adjoint_workspace_bytes", "mbqc_sv_adjoint_forward_c64",
     "mbqc_sv_adjoint_partials", "mbqc_sv_adjoint_backward_c64", "mbqc_sv_segments_auto",
@@ -132,6 +132,12 @@ def lib() -> C.CDLL:
     L.mbqc_gram_workspace_bytes.restype = sz
     L.mbqc_gram_loss_seed_c64.argtypes = [vp, vp, i64, i32, i32, vp, vp, vp, vp]
     L.mbqc_gram_loss_seed_c64.restype = C.c_int
+    L.mbqc_gram_seed_c64.argtypes = [vp, vp, i64, i32, i32, vp, vp]
+    L.mbqc_gram_seed_c64.restype = C.c_int
+    L.mbqc_transfer_workspace_bytes.argtypes = [i64, i32]
+    L.mbqc_transfer_workspace_bytes.restype = sz
+    L.mbqc_transfer_loss_seed_c64.argtypes = [vp, vp, vp, i64, i32, i32, vp, vp, vp, vp]
+    L.mbqc_transfer_loss_seed_c64.restype = C.c_int
     L.mbqc_gram_loss_seed_c64_noalloc.argtypes = [vp, vp, i64, i32, i32, vp, vp, vp]
     L.mbqc_gram_loss_seed_c64_noalloc.restype = C.c_int
     L.mbqc_plan_window_qubits.argtypes = [vp, i32]
@@ -166,7 +172,7 @@ def lib() -> C.CDLL:
     L.mbqc_sv_segments_auto.restype = i32
     L.mbqc_sv_has_outputs_gradient.argtypes = [vp]
     L.mbqc_sv_has_outputs_gradient.restype = i32
-    L.mbqc_sv_outputs_gradient_c64.argtypes = [vp, vp, i64, i64, vp, vp, i64, i64, vp, vp]
+    L.mbqc_sv_outputs_gradient_c64.argtypes = [vp, vp, i64, i64, vp, vp, i64, i64, vp, vp, vp]
     L.mbqc_sv_outputs_gradient_c64.restype = i32
     L.mbqc_sv_segmented_workspace_bytes.argtypes = [vp, i64, i32]
     L.mbqc_sv_segmented_workspace_bytes.restype = sz

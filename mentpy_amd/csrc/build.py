@@ -27,7 +27,7 @@ ROOT = PKG.parent
 LIB_DIR = PKG / "lib"
 LIB = LIB_DIR / "libmbqc_hip.so"
 SANITIZE_LIB = LIB_DIR / "libmbqc_hip_sanitize.so"
-SOURCES = [HERE / "kernels.hip", HERE / "wide.hip", HERE / "wide_dm.hip",
+SOURCES = [HERE / "kernels.hip", HERE / "wide.hip", HERE / "wide_dm.hip", HERE / "gram.hip",
            HERE / "plan.cpp", HERE / "flow.cpp"]
 ARCH = os.environ.get("MBQC_OFFLOAD_ARCH", "gfx950")
 SANITIZE_FLAGS = ["-Xarch_host", "-fsanitize=address", "-Xarch_host", "-fsanitize=undefined",

@@ -390,4 +390,20 @@ __device__ __forceinline__ Job load_job(const Job* jobs, int i) {
 // group counters live kCounterStride ints apart (separate cache lines)
 constexpr int kCounterStride = 64;
 
+// Sum over the TL lanes of a group, in its last lane at least.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float add_dpp(float v) {
+  return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xf, false));
+}
+template <int TL>
+__device__ __forceinline__ float last_lane_sum(float v) {
+  if constexpr (TL > 1) v = add_dpp<0xB1, 0xf>(v);     // quad_perm [1,0,3,2]
+  if constexpr (TL > 2) v = add_dpp<0x4E, 0xf>(v);     // quad_perm [2,3,0,1]
+  if constexpr (TL > 4) v = add_dpp<0x141, 0xf>(v);    // row_half_mirror
+  if constexpr (TL > 8) v = add_dpp<0x140, 0xf>(v);    // row_mirror
+  if constexpr (TL > 16) v = add_dpp<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+  if constexpr (TL > 32) v = add_dpp<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
 }  // namespace mbqc

@@ -21,6 +21,7 @@
 
 #include "device.h"
 #include "plan.h"
+#include "gram.h"
 #include "wide.h"
 
 namespace mbqc {
@@ -2228,87 +2229,6 @@ __global__ __launch_bounds__(256) void k_gram_seed(const float2* __restrict__ t,
   }
 }
 
-// The same on the matrix cores, for K a multiple of 16: one wave per 16 x 16
-// tile of Z (16 parameter sets x 16 indices n), complex products as four real
-// v_mfma_f32_16x16x4f32 per k-chunk of 4 (Zr += Tr Mr' - Ti Mi', Zi += Tr Mi' +
-// Ti Mr').  Operand layout of the 16x16x4 f32 MFMA: lane l holds A[l%16][l/16]
-// and B[l/16][l%16]; the accumulator holds D[4(l/16)+r][l%16], r = 0..3.
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
-__global__ __launch_bounds__(64) void k_gram_seed_mfma(const float2* __restrict__ t,
-                                                       const float2* __restrict__ MT, int64_t B,
-                                                       int K, float inv_S,
-                                                       float2* __restrict__ seed,
-                                                       float* __restrict__ lpart) {
-  const int l = threadIdx.x;
-  const int li = l & 15, lk = l >> 4;
-  const int n0 = blockIdx.x * 16;
-  const int64_t b0 = int64_t(blockIdx.y) * 16;
-  const int64_t ba = b0 + li;                        // A row of this lane
-  const bool arow = ba < B;
-  const float2* ta = t + (arow ? ba : 0) * K + lk;
-  const float2* mb = MT + int64_t(lk) * K + n0 + li;
-  // Two accumulator pairs (even / odd k-chunks) keep consecutive MFMAs
-  // independent; the next U chunks are loaded while the current ones run
-  // (one wave per SIMD at the usual sizes, so nothing else hides the loads).
-  f32x4 zr0 = {0.f, 0.f, 0.f, 0.f}, zi0 = {0.f, 0.f, 0.f, 0.f};
-  f32x4 zr1 = {0.f, 0.f, 0.f, 0.f}, zi1 = {0.f, 0.f, 0.f, 0.f};
-  constexpr int U = 8;                               // k-chunks of 4 loaded together
-  float2 an[U], bn[U];
-  auto fetch = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + 4 * u;
-      const bool in = k < K;
-      an[u] = (in && arow) ? ta[k] : make_float2(0.f, 0.f);
-      bn[u] = in ? mb[int64_t(k) * K] : make_float2(0.f, 0.f);
-    }
-  };
-  fetch(0);
-  for (int k0 = 0; k0 < K; k0 += 4 * U) {
-    float2 a[U], b[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      a[u] = an[u];
-      b[u] = bn[u];
-    }
-    if (k0 + 4 * U < K) fetch(k0 + 4 * U);
-#pragma unroll
-    for (int u = 0; u < U; u += 2) {
-      zr0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, b[u].x, zr0, 0, 0, 0);
-      zi0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].x, b[u].y, zi0, 0, 0, 0);
-      zr1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u + 1].x, b[u + 1].x, zr1, 0, 0, 0);
-      zi1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u + 1].x, b[u + 1].y, zi1, 0, 0, 0);
-      zr0 = __builtin_amdgcn_mfma_f32_16x16x4f32(-a[u].y, b[u].y, zr0, 0, 0, 0);
-      zi0 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u].y, b[u].x, zi0, 0, 0, 0);
-      zr1 = __builtin_amdgcn_mfma_f32_16x16x4f32(-a[u + 1].y, b[u + 1].y, zr1, 0, 0, 0);
-      zi1 = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u + 1].y, b[u + 1].x, zi1, 0, 0, 0);
-    }
-  }
-  f32x4 zr, zi;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    zr[r] = zr0[r] + zr1[r];
-    zi[r] = zi0[r] + zi1[r];
-  }
-  const float sc = -2.0f * inv_S;
-  const int n = n0 + li;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int64_t b = b0 + 4 * lk + r;              // uniform within each 16-lane group
-    float part = 0.0f;
-    if (b < B) {
-      const float2 z = make_float2(zr[r], zi[r]);
-      seed[b * K + n] = cscale(z, sc);
-      const float2 x = t[b * K + n];
-      part = fmaf(x.x, z.x, x.y * z.y);
-    }
-    // sum over the 16 lanes (indices n) of this row
-    for (int m = 8; m >= 1; m >>= 1) part += __shfl_xor(part, m, 64);
-    if (li == 0 && b < B) lpart[b * gridDim.x + blockIdx.x] = part;
-  }
-}
-
 // Loss and seed from t and a precomputed z = M t (library GEMM path): one
 // workgroup per parameter set, loss = 1 - Re(t^H z) / S, seed = -2 z / S.
 __global__ __launch_bounds__(256) void k_gram_finish(const float2* __restrict__ t,
@@ -2393,6 +2313,8 @@ __global__ void k_gram_loss(const float* __restrict__ lpart, int64_t B, int nblk
 constexpr int kChainLd = 17;
 
 // acc += A * B for one k-chunk; a = A[row][kk], b = B[kk][col] of this lane
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
 __device__ __forceinline__ void cmfma_chunk(f32x4& dr, f32x4& di, float2 a, float2 b) {
   dr = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.x, dr, 0, 0, 0);
   di = __builtin_amdgcn_mfma_f32_16x16x4f32(a.x, b.y, di, 0, 0, 0);
@@ -3830,10 +3752,11 @@ int gram_loss_seed(const void* t, const void* MT, int64_t B, int32_t K, int32_t 
   const float inv_S = 1.0f / float(S);
   int nblk;
   if (K % 16 == 0) {
-    nblk = K / 16;
-    hipLaunchKernelGGL(k_gram_seed_mfma, dim3(nblk, unsigned((B + 15) / 16)), dim3(64), 0, st,
-                       static_cast<const float2*>(t), static_cast<const float2*>(MT), B, K, inv_S,
-                       static_cast<float2*>(seed), workspace);
+    nblk = K / product_tile(B, K) + (K % product_tile(B, K) != 0);
+    hipError_t e = launch_product(Product::kGram, static_cast<const float2*>(t),
+                                  static_cast<const float2*>(MT), static_cast<float2*>(seed), B, K, K,
+                                  -2.0f * inv_S, workspace, st);
+    if (e != hipSuccess) return hip_fail(e, "gram loss launch");
   } else {
     nblk = (K + 63) / 64;
     const size_t lds = size_t(kGramSets) * K * sizeof(float2);
@@ -4493,7 +4416,7 @@ int32_t mbqc_sv_has_outputs_gradient(const mbqc_plan* plan) {
 
 int mbqc_sv_outputs_gradient_c64(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
                                  int64_t angle_stride_a, const void* out, const void* seed, int64_t B,
-                                 int64_t C, float* grad, void* stream) {
+                                 int64_t C, float* loss, float* grad, void* stream) {
   if (!plan) return fail(MBQC_ERR_VALUE, "null plan");
   Plan* p = const_cast<Plan*>(reinterpret_cast<const Plan*>(plan));
   int rc = check_adjoint_plan(p);
@@ -4508,7 +4431,7 @@ int mbqc_sv_outputs_gradient_c64(const mbqc_plan* plan, const float* angles, int
   if (B > 0x7fffffff || C > 0x7fffff) return fail(MBQC_ERR_VALUE, "too many simulations for one launch");
   if (J.total == 0) return MBQC_OK;
   hipError_t e = launch_pauli_gradient(J, static_cast<const float2*>(out),
-                                       static_cast<const float2*>(seed), B, C, p->n_angles, grad,
+                                       static_cast<const float2*>(seed), B, C, p->n_angles, loss, grad,
                                        static_cast<hipStream_t>(stream));
   return e == hipSuccess ? MBQC_OK : hip_fail(e, "outputs gradient launch");
 }
@@ -4701,6 +4624,50 @@ int mbqc_gram_loss_seed_c64_noalloc(const void* t, const void* MT, int64_t B, in
   int rc = scratch_ptr(&ws);
   if (rc != MBQC_OK) return rc;
   return gram_loss_seed(t, MT, B, K, S, loss, seed, ws, stream);
+}
+
+int mbqc_gram_seed_c64(const void* t, const void* MT, int64_t B, int32_t K, int32_t S, void* seed,
+                       void* stream) {
+  if (!t || !MT || !seed) return fail(MBQC_ERR_VALUE, "null pointer");
+  if (B < 0 || K <= 0 || S <= 0) return fail(MBQC_ERR_VALUE, "sizes must be B >= 0, K >= 1, S >= 1");
+  if (B == 0) return MBQC_OK;
+  if ((B + 15) / 16 * ((K + 15) / 16) > 0x7fffffff)
+    return fail(MBQC_ERR_VALUE, "too many parameter sets");
+  hipError_t e = launch_product(Product::kScaled, static_cast<const float2*>(t),
+                                static_cast<const float2*>(MT), static_cast<float2*>(seed), B, K, K,
+                                -2.0f / float(S), nullptr, static_cast<hipStream_t>(stream));
+  return e == hipSuccess ? MBQC_OK : hip_fail(e, "gram seed launch");
+}
+
+size_t mbqc_transfer_workspace_bytes(int64_t B, int32_t S) {
+  if (B < 0 || S <= 0) return 0;
+  return size_t(B) * (size_t(S) * sizeof(float2) + size_t((S + 15) / 16) * sizeof(float));
+}
+
+int mbqc_transfer_loss_seed_c64(const void* t, const void* DT, const void* DC, int64_t B, int32_t K,
+                                int32_t S, float* loss, void* seed, void* workspace, void* stream) {
+  if (!t || !DT || !workspace || (seed && !DC) || (!loss && !seed)) return fail(MBQC_ERR_VALUE, "null pointer");
+  if (B < 0 || K <= 0 || S <= 0) return fail(MBQC_ERR_VALUE, "sizes must be B >= 0, K >= 1, S >= 1");
+  if (B == 0) return MBQC_OK;
+  if ((B + 15) / 16 * ((std::max(K, S) + 15) / 16) > 0x7fffffff)
+    return fail(MBQC_ERR_VALUE, "too many parameter sets");
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  float2* f = static_cast<float2*>(workspace);
+  float* part = reinterpret_cast<float*>(f + B * S);
+  const float inv_S = 1.0f / float(S);
+  const int tile = product_tile(B, S);
+  hipError_t e = launch_product(Product::kOverlap, static_cast<const float2*>(t),
+                                static_cast<const float2*>(DT), seed ? f : nullptr, B, S, K, 1.0f, part,
+                                st);
+  if (e == hipSuccess && loss) {
+    hipLaunchKernelGGL(k_gram_loss, dim3(unsigned((B + 255) / 256)), dim3(256), 0, st, part, B,
+                       (S + tile - 1) / tile, inv_S, loss);
+    e = hipGetLastError();
+  }
+  if (e == hipSuccess && seed)
+    e = launch_product(Product::kScaled, f, static_cast<const float2*>(DC), static_cast<float2*>(seed), B,
+                       K, S, -2.0f * inv_S, nullptr, st);
+  return e == hipSuccess ? MBQC_OK : hip_fail(e, "transfer loss launch");
 }
 
 int mbqc_adam_step_f32(float* x, const float* grad, float* m, float* v, int64_t n, float lr, float b1,

@@ -52,9 +52,11 @@ hipError_t launch_wide_adj_backward(const Job& J, const float2* ckpt, const floa
                                     const WideAdjoint& A, float* gpart, hipStream_t st);
 
 // Angle gradients of a column plan of 2..5 slots whose slots are all outputs, from
-// outputs and seed [B][C][2^ns] alone, into grad[B][n_angles].
+// outputs and seed [B][C][2^ns] alone, into grad[B][n_angles]; with `loss`, also loss[B] =
+// 1 + Re sum conj(seed) out / 2.
 hipError_t launch_pauli_gradient(const Job& J, const float2* out, const float2* seed, int64_t B,
-                                 int64_t C, int n_angles, float* grad, hipStream_t st);
+                                 int64_t C, int n_angles, float* loss, float* grad,
+                                 hipStream_t st);
 
 // Density matrices of column plans with 2..7 slots (wide_dm.hip); pad_slots:
 // slots that start as |+> padding (n_slots - n_inputs).

@@ -443,7 +443,7 @@ __device__ __forceinline__ void cmul_conj_add(float2& m, float2 a, float2 b) {
 
 template <int NS, int K, int... PS>
 __device__ __forceinline__ void pauli_gradient(const Job& J, const float2* out, const float2* seed,
-                                               int64_t bi, bool active, int C, int n_angles,
+                                               int64_t bi, bool active, int C, int n_angles, float* loss,
                                                float* grad, float2* buf, float2* bs, int lane,
                                                std::integer_sequence<int, PS...>) {
   using W = Pauli<NS, K>;
@@ -480,6 +480,7 @@ __device__ __forceinline__ void pauli_gradient(const Job& J, const float2* out, 
     (in_phase<NS, K, PS>(m, buf, lane, std::make_integer_sequence<int, W::len(PS)>{}), ...);
 #pragma unroll
     for (int r = 0; r < W::N; ++r) t[r] = m[r].y;
+    if (loss && active && lane == 0) loss[bi] = fmaf(0.5f, m[0].x, 1.0f);
   }
   const float all = t[0];     // of lane 0: the coefficient of I...I, constant from here on
   const bool writer = active && lane == 0;
@@ -517,14 +518,14 @@ __device__ __forceinline__ void pauli_gradient(const Job& J, const float2* out, 
 template <int NS, int K>
 __global__ __launch_bounds__((Pauli<NS, K>::T)) void k_pauli_gradient(
     Job J, const float2* __restrict__ out, const float2* __restrict__ seed, int64_t B, int C,
-    int n_angles, float* __restrict__ grad) {
+    int n_angles, float* __restrict__ loss, float* __restrict__ grad) {
   using W = Pauli<NS, K>;
   __shared__ __align__(16) float2 lds[W::G * W::SIM];
   const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
   float2* buf = lds + sub * W::SIM;
   const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
   const bool active = g < B;
-  pauli_gradient<NS, K>(J, out, seed, active ? g : B - 1, active, C, n_angles, grad, buf,
+  pauli_gradient<NS, K>(J, out, seed, active ? g : B - 1, active, C, n_angles, loss, grad, buf,
                         buf + W::BUF, lane, std::make_integer_sequence<int, W::P>{});
 }
 
@@ -549,10 +550,10 @@ hipError_t dm_launch(const Job& J, const DmNoise& nz, int pad_slots, uint32_t fl
 
 template <int NS, int K>
 hipError_t gradient_launch(const Job& J, const float2* out, const float2* seed, int64_t B, int64_t C,
-                           int n_angles, float* grad, hipStream_t st) {
+                           int n_angles, float* loss, float* grad, hipStream_t st) {
   using W = Pauli<NS, K>;
   hipLaunchKernelGGL((k_pauli_gradient<NS, K>), dim3(unsigned((B + W::G - 1) / W::G)), dim3(W::T), 0,
-                     st, J, out, seed, B, int(C), n_angles, grad);
+                     st, J, out, seed, B, int(C), n_angles, loss, grad);
   return hipGetLastError();
 }
 
@@ -563,14 +564,16 @@ hipError_t gradient_launch(const Job& J, const float2* out, const float2* seed, 
 // 14.6 / 18.3; 4x16 grid, 1,024 sets 12.0 / 14.9, 4,096 22.4 / 18.1; 5x10 grid,
 // 1,024 sets 29.0 / 19.9.
 hipError_t launch_pauli_gradient(const Job& J, const float2* out, const float2* seed, int64_t B,
-                                 int64_t C, int n_angles, float* grad, hipStream_t st) {
+                                 int64_t C, int n_angles, float* loss, float* grad,
+                                 hipStream_t st) {
   switch (J.ns) {
-    case 2: return gradient_launch<2, 1>(J, out, seed, B, C, n_angles, grad, st);
-    case 3: return gradient_launch<3, 1>(J, out, seed, B, C, n_angles, grad, st);
+    case 2: return gradient_launch<2, 1>(J, out, seed, B, C, n_angles, loss, grad, st);
+    case 3: return gradient_launch<3, 1>(J, out, seed, B, C, n_angles, loss, grad, st);
     case 4:
-      return B <= kDm4OneDigitMaxSims ? gradient_launch<4, 1>(J, out, seed, B, C, n_angles, grad, st)
-                                      : gradient_launch<4, 2>(J, out, seed, B, C, n_angles, grad, st);
-    case 5: return gradient_launch<5, 2>(J, out, seed, B, C, n_angles, grad, st);
+      return B <= kDm4OneDigitMaxSims
+                 ? gradient_launch<4, 1>(J, out, seed, B, C, n_angles, loss, grad, st)
+                 : gradient_launch<4, 2>(J, out, seed, B, C, n_angles, loss, grad, st);
+    case 5: return gradient_launch<5, 2>(J, out, seed, B, C, n_angles, loss, grad, st);
     default: return hipErrorInvalidValue;
   }
 }

@@ -150,9 +150,18 @@ def _basis(n_in, device):
     return torch.eye(1 << n_in, dtype=torch.complex64, device=device)
 
 
-# Parameter-set counts up to which the fused VALU Gram kernel is used (above
-# it the library GEMM has enough tiles to fill the chip).
+# Parameter-set counts up to which the fused Gram kernels are used; above it the
+# library GEMM has enough tiles to fill the chip (whole step in us, library / fused:
+# 4 rows, 8,192 sets 111 / 96, 16,384 sets 184 / 187).
 _FUSED_GRAM_MAX_SETS = 8192
+# The same for transfer matrices of at most 64 entries, where the library's passes over
+# the product outweigh it (2 rows, 65,536 sets 81 / 38; 3 rows 146 / 101).
+_FUSED_GRAM_SMALL = 64
+_FUSED_GRAM_SMALL_MAX_SETS = 65535 * 16
+
+# Data matrices [S, K] up to this many entries (8 MB: they stay in the caches) are kept
+# whole for the "transfer" mode.
+_MAX_DATA_MATRIX = 1 << 20
 
 
 class MBQMLStep:
@@ -168,7 +177,9 @@ class MBQMLStep:
       ``M = D^H D``, ``D[s, (c, o)] = psi_s[c] conj(phi_s[o])`` (computed once
       per data set), and the backward seed is ``-2 M t_b / S``: one dense
       complex GEMM ``[B, K] x [K, K]`` per step.
-    * ``"transfer"``: transfer matrix, then ``T X`` and ``(Phi f) X^H`` GEMMs.
+    * ``"transfer"``: transfer matrix, then ``f_b = D t_b``, ``L_b = 1 - |f_b|^2 / S``
+      and the seed ``-2 D^H f_b / S`` (large data sets without the matrix ``D``: ``T X``
+      and ``(Phi f) X^H`` GEMMs).
     * ``"direct"``: the inputs themselves are the propagated columns.
 
     In the transfer-matrix modes of a grid pattern of 2 to 5 rows the gradient
@@ -213,24 +224,37 @@ class MBQMLStep:
         self.P = int(nat.lib().mbqc_sv_adjoint_partials(C_))
         self.part = torch.zeros((self.B, self.P, info["n_angles"]), dtype=torch.float32, device=dev)
         self.loss = torch.empty(self.B, dtype=torch.float32, device=dev)
-        if mode == "gram":
-            self.MT = torch.empty((K, K), dtype=torch.complex64, device=dev)
-            self._gram_matrix()
-            self.Z = torch.empty((self.B, K), dtype=torch.complex64, device=dev)
-            if gram_kernel == "auto":
-                gram_kernel = "fused" if (K <= 512 and self.B <= _FUSED_GRAM_MAX_SETS) else "blas"
-            if gram_kernel not in ("fused", "blas"):
-                raise ValueError("gram_kernel must be 'auto', 'fused' or 'blas'")
-            if gram_kernel == "fused" and K > 512:
-                raise NotImplementedError("the fused Gram kernel supports K <= 512")
-            self.gram_kernel = gram_kernel
-            nbytes = int(nat.lib().mbqc_gram_workspace_bytes(self.B, K))
-            self._gws = torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device=dev)
         L = nat.lib()
         # the whole transfer matrix of a grid pattern: gradients from the outputs
         # alone, whatever the steps between
         self._from_outputs = (mode != "direct" and segments in ("auto", 1) and
                               bool(L.mbqc_sv_has_outputs_gradient(eng.plan.handle)))
+        if mode == "gram":
+            self.MT = torch.empty((K, K), dtype=torch.complex64, device=dev)
+            self._gram_matrix()
+            if gram_kernel == "auto":
+                most = (_FUSED_GRAM_SMALL_MAX_SETS if self._from_outputs and K <= _FUSED_GRAM_SMALL
+                        else _FUSED_GRAM_MAX_SETS)
+                gram_kernel = "fused" if (K <= 512 and self.B <= most) else "blas"
+            if gram_kernel not in ("fused", "blas"):
+                raise ValueError("gram_kernel must be 'auto', 'fused' or 'blas'")
+            if gram_kernel == "fused" and K > 512:
+                raise NotImplementedError("the fused Gram kernel supports K <= 512")
+            self.gram_kernel = gram_kernel
+            if gram_kernel == "blas":
+                self.Z = torch.empty((self.B, K), dtype=torch.complex64, device=dev)
+            nbytes = int(nat.lib().mbqc_gram_workspace_bytes(self.B, K))
+            self._gws = torch.empty(max(nbytes // 4, 1), dtype=torch.float32, device=dev)
+        self._data_matrix = mode == "transfer" and S * K <= _MAX_DATA_MATRIX
+        if self._data_matrix:
+            self.DT = torch.empty((K, S), dtype=torch.complex64, device=dev)
+            self.DC = torch.empty((S, K), dtype=torch.complex64, device=dev)
+            self._data_rows()
+            nbytes = int(nat.lib().mbqc_transfer_workspace_bytes(self.B, S))
+            self._tws = torch.empty(max(nbytes, 8), dtype=torch.uint8, device=dev)
+        # then the gradient launch can give the loss too
+        self._late_loss = self._from_outputs and (
+            self._data_matrix or (mode == "gram" and self.gram_kernel == "fused"))
         if mode == "direct" or self._from_outputs:
             segments = 1
         elif segments == "auto":
@@ -252,6 +276,12 @@ class MBQMLStep:
         M = torch.matmul(D.conj().transpose(0, 1).contiguous(), D)
         self.MT.copy_(M.transpose(0, 1))
 
+    def _data_rows(self):
+        """D of the current data, transposed and conjugated."""
+        D = (self.X.unsqueeze(2) * self.Y.conj().unsqueeze(1)).reshape(self.S, self.K)
+        self.DT.copy_(D.transpose(0, 1))
+        self.DC.copy_(D.conj())
+
     def set_data(self, inputs, targets):
         """Replace the data set (same shapes) in place, recomputing the Gram
         matrix; a captured graph of this step then uses the new data."""
@@ -266,6 +296,8 @@ class MBQMLStep:
         self.Y.copy_(Y)
         if self.mode == "gram":
             self._gram_matrix()
+        elif self._data_matrix:
+            self._data_rows()
 
     def _launch_forward(self):
         eng = self.engine
@@ -295,7 +327,8 @@ class MBQMLStep:
         if self._from_outputs:   # P = 1: 2^n columns
             nat.launch(eng.device, nat.lib().mbqc_sv_outputs_gradient_c64, eng.plan.handle,
                        self.angles.data_ptr(), sb, sa, self.out.data_ptr(), self.seed.data_ptr(),
-                       self.B, self.cols.shape[0], self.part.data_ptr())
+                       self.B, self.cols.shape[0], self.loss.data_ptr() if self._late_loss else None,
+                       self.part.data_ptr())
             return
         nat.launch(eng.device, nat.lib().mbqc_sv_adjoint_backward_c64, eng.plan.handle,
                    self.angles.data_ptr(), sb, sa, self.seed.data_ptr(), self.B, self.cols.shape[0],
@@ -321,7 +354,10 @@ class MBQMLStep:
         torch = _torch()
         S = self.S
         dev = self.engine.device
-        if self.mode == "gram" and self.gram_kernel == "fused":
+        if grad and self._late_loss and self.mode == "gram":
+            nat.launch(dev, nat.lib().mbqc_gram_seed_c64, self.out.data_ptr(), self.MT.data_ptr(),
+                       self.B, self.K, S, self.seed.data_ptr())
+        elif self.mode == "gram" and self.gram_kernel == "fused":
             nat.launch(dev, nat.lib().mbqc_gram_loss_seed_c64, self.out.data_ptr(),
                        self.MT.data_ptr(), self.B, self.K, S, self.loss.data_ptr(),
                        self.seed.data_ptr(), self._gws.data_ptr())
@@ -330,6 +366,11 @@ class MBQMLStep:
             torch.matmul(t, self.MT, out=self.Z)
             nat.launch(dev, nat.lib().mbqc_gram_finish_c64, t.data_ptr(), self.Z.data_ptr(), self.B,
                        self.K, S, self.loss.data_ptr(), self.seed.data_ptr())
+        elif self._data_matrix:
+            nat.launch(dev, nat.lib().mbqc_transfer_loss_seed_c64, self.out.data_ptr(),
+                       self.DT.data_ptr(), self.DC.data_ptr(), self.B, self.K, S,
+                       None if grad and self._late_loss else self.loss.data_ptr(),
+                       self.seed.data_ptr() if grad else None, self._tws.data_ptr())
         elif self.mode == "transfer":
             Tm = self.out.transpose(1, 2)                                # [B, dout, din]
             outs = torch.matmul(Tm, self.X.transpose(0, 1))             # [B, dout, S]

@@ -144,16 +144,55 @@ def test_gradient_from_outputs_matches_complex128(rows, cols, C, B, rng):
     want, = torch.autograd.grad(t, a, cot[bs].to(torch.complex128))
     out = torch.empty((B, C, d), dtype=torch.complex64, device="cuda")
     grad = torch.full((B, n), float("nan"), device="cuda")
+    loss = torch.full((B,), float("nan"), device="cuda")
     nat.launch(out.device, nat.lib().mbqc_sv_forward_c64, plan.handle, th.data_ptr(), n, 1,
                x.data_ptr(), d, out.data_ptr(), None, B, C, 0)
     nat.launch(out.device, nat.lib().mbqc_sv_outputs_gradient_c64, plan.handle, th.data_ptr(), n, 1,
-               out.data_ptr(), cot.data_ptr(), B, C, grad.data_ptr())
+               out.data_ptr(), cot.data_ptr(), B, C, loss.data_ptr(), grad.data_ptr())
     assert torch.isfinite(grad).all()
     # one rounding (6e-8) per step on coefficients of norm about sqrt(2 C): far
     # below 2e-5 of the largest entry
     gerr = (grad[bs] - want).abs().max().item()
     scale = want.abs().max().item()
     assert gerr < 2e-5 * max(scale, 1.0), f"gradient error {gerr} of {scale}"
+    wl = 1 + 0.5 * (t.detach() * cot[bs].to(torch.complex128).conj()).real.sum((1, 2))
+    assert (loss[bs] - wl).abs().max().item() < 2e-5 * C ** 0.5
+
+
+@pytest.mark.parametrize("B,K,S", [(1, 16, 1), (15, 20, 16), (17, 64, 33), (33, 1024, 100), (2049, 256, 37),
+                                   (1030, 1024, 65), (16400, 64, 257), (4097, 256, 256)])
+def test_transfer_products_match_complex128(B, K, S, rng):
+    """Loss and seed through the data matrix, both tilings: partly filled tiles of
+    rows and columns, a contraction length with a remainder, loss alone and
+    seed alone; the Gram seed of the same data."""
+    torch = _torch()
+    from mentpy_amd import _native as nat
+    L = nat.lib()
+    gen = torch.Generator().manual_seed(B + K + S)
+    t = torch.randn((B, K), generator=gen, dtype=torch.complex64).cuda() / K ** 0.5
+    D = torch.randn((S, K), generator=gen, dtype=torch.complex64).cuda()
+    DT, DC = D.t().contiguous(), D.conj().resolve_conj().contiguous()
+    ws = torch.empty(int(L.mbqc_transfer_workspace_bytes(B, S)), dtype=torch.uint8, device="cuda")
+    dev = t.device
+
+    def both(loss, seed):
+        nat.launch(dev, L.mbqc_transfer_loss_seed_c64, t.data_ptr(), DT.data_ptr(), DC.data_ptr(), B, K, S,
+                   loss, seed, ws.data_ptr())
+    l0, l1 = (torch.full((B,), float("nan"), device="cuda") for _ in range(2))
+    s0, s1, s2 = (torch.full((B, K), float("nan"), dtype=torch.complex64, device="cuda") for _ in range(3))
+    both(l0.data_ptr(), s0.data_ptr())
+    both(l1.data_ptr(), None)
+    both(None, s1.data_ptr())
+    assert torch.equal(l0, l1) and torch.equal(s0, s1)
+    MT = (D.to(torch.complex128).conj().t() @ D.to(torch.complex128)).t().to(torch.complex64).contiguous()
+    nat.launch(dev, L.mbqc_gram_seed_c64, t.data_ptr(), MT.data_ptr(), B, K, S, s2.data_ptr())
+    f = t.to(torch.complex128) @ D.to(torch.complex128).t()
+    want_loss = 1 - (f.abs() ** 2).mean(1)
+    want = -2.0 / S * (f @ D.to(torch.complex128).conj())
+    # sums of K (S) products of size 1/K (1) and one rounding (6e-8) each
+    assert (l0 - want_loss).abs().max().item() < 1e-5 * want_loss.abs().max().item()
+    for s in (s0, s2):
+        assert (s - want).abs().max().item() < 1e-5 * want.abs().max().item()
 
 
 def test_gradient_from_outputs_refuses_other_plans():
