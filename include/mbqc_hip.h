@@ -445,6 +445,13 @@ int mbqc_transfer_loss_seed_c64(const void* t, const void* DT, const void* DC, i
 int mbqc_overlap_loss_seed_c64(const void* out, const void* targets, int64_t B, int32_t S,
                                int32_t O, float* loss, void* seed, void* stream);
 
+/* Angle vectors [B][n] (row stride angle_stride, unit stride within) to
+ * angle-major order, out[a * out_stride + b]: the layout whose loads are contiguous in
+ * launches with one simulation per lane (angle_stride 1, angle_stride_a
+ * out_stride there).  out_stride >= B. */
+int mbqc_angle_major_f32(const float* angles, int64_t angle_stride, float* out, int64_t out_stride,
+                         int64_t B, int32_t n, void* stream);
+
 /* Device-resident optimizer steps on n float32 parameters (all pointers device
  * memory, updated in place), replacing the host updates of
  * AdamOptimizer.step (mentpy/optimizers/adam.py:54-66) and SGDOptimizer.step

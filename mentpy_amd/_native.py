@@ -43,6 +43,7 @@ EXPORTED_SYMBOLS = (
     "mbqc_dm_forward_outcomes_c64",
     "mbqc_plan_window_qubits", "mbqc_sv_window_c64", "mbqc_dm_window_c64",
     "mbqc_gram_workspace_bytes", "mbqc_gram_loss_seed_c64", "mbqc_gram_loss_seed_c64_noalloc",
+    "mbqc_angle_major_f32",
     "mbqc_gram_finish_c64", "mbqc_gram_seed_c64", "mbqc_transfer_workspace_bytes", "mbqc_transfer_loss_seed_c64",
     "mbqc_overlap_loss_seed_c64",
     "mbqc_sv_adjoint_workspace_bytes", "mbqc_sv_adjoint_forward_c64",
@@ -132,6 +133,8 @@ def lib() -> C.CDLL:
     L.mbqc_gram_workspace_bytes.restype = sz
     L.mbqc_gram_loss_seed_c64.argtypes = [vp, vp, i64, i32, i32, vp, vp, vp, vp]
     L.mbqc_gram_loss_seed_c64.restype = C.c_int
+    L.mbqc_angle_major_f32.argtypes = [vp, i64, vp, i64, i64, i32, vp]
+    L.mbqc_angle_major_f32.restype = C.c_int
     L.mbqc_gram_seed_c64.argtypes = [vp, vp, i64, i32, i32, vp, vp]
     L.mbqc_gram_seed_c64.restype = C.c_int
     L.mbqc_transfer_workspace_bytes.argtypes = [i64, i32]

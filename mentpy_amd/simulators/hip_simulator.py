@@ -201,6 +201,35 @@ def _angle_strides(a):
     return (a.stride(0) if a.shape[0] > 1 else 0), max(a.stride(1), 1)
 
 
+# Launches with one simulation per lane read a row of angles 128 bytes at a time and
+# 4 of them per step; past this many bytes, in rows of this many angles, the lines
+# leave the caches before their next use and a pass to angle-major order first is
+# faster (launch in us, rows / pass and launch: 4x20 grid, 131,072 sets 66 / 47, 65,536
+# sets 25 / 32; 4x19, 116,509 sets 39 / 41; 4x40, 65,536 sets 82 / 56, 524,288 sets
+# 1485 / 310; 3x40, 131,072 sets 116 / 56; rows of 36 angles, 524,288 sets 57 / 82; with
+# 3 inputs per set the lines are shared: 4x20, 524,288 sets 256 / 302; 2 slots, 78
+# angles, 131,072 sets 36 / 38).
+_ANGLE_PASS_BYTES = 9 << 22
+_ANGLE_PASS_MIN_ANGLES = 72
+
+
+def _lane_angles(plan, a, S: int):
+    """``a [B, n]`` as the statevector launches read it best: itself, or an
+    angle-major copy; ``(tensor, stride over sets, stride over angles)``."""
+    B, n = a.shape
+    sb, sa = _angle_strides(a)
+    if (S != 1 or not 3 <= plan.info["n_slots"] <= 6 or sa != 1 or sb < n
+            or n < _ANGLE_PASS_MIN_ANGLES or 4 * B * n < _ANGLE_PASS_BYTES):
+        return a, sb, sa
+    torch = _torch()
+    try:
+        t = torch.empty((n, (B + 63) // 64 * 64), dtype=torch.float32, device=a.device)
+    except torch.cuda.OutOfMemoryError:
+        return a, sb, sa
+    nat.launch(a.device, nat.lib().mbqc_angle_major_f32, a.data_ptr(), sb, t.data_ptr(), t.stride(0), B, n)
+    return t, 1, t.stride(0)
+
+
 def _as_states(states, n_qubits: int, device):
     torch = _torch()
     s = torch.as_tensor(states, device=device)
@@ -245,7 +274,7 @@ def sv_forward(plan: nat.NativePlan, angles, states, *, ref_phase: bool = True,
     flags = ((nat.FLAG_REF_PHASE if ref_phase else 0) | (nat.FLAG_RENORMALIZE if renormalize else 0)
              | (nat.FLAG_WRITE_PHASE if want_phase else 0)
              | (nat.FLAG_TABLE_STEPS if table_steps else 0))
-    sb, sa = _angle_strides(angles)
+    angles, sb, sa = _lane_angles(plan, angles, S)
     nat.launch(device, nat.lib().mbqc_sv_forward_c64, plan.handle, angles.data_ptr(), sb, sa,
                states.data_ptr(), states.shape[1], out.data_ptr(),
                phase.data_ptr() if phase is not None else 0, B, S, flags)
@@ -271,7 +300,7 @@ def sv_sample(plan: nat.NativePlan, angles, states, seed: int, *, out=None, outc
         out = torch.empty((B, S, 1 << info["n_outputs"]), dtype=torch.complex64, device=device)
     if outcomes is None:
         outcomes = torch.empty((B, S, W + 2), dtype=torch.int32, device=device)
-    sb, sa = _angle_strides(angles)
+    angles, sb, sa = _lane_angles(plan, angles, S)
     nat.launch(device, nat.lib().mbqc_sv_sample_c64, plan.handle, angles.data_ptr(), sb, sa,
                states.data_ptr(), states.shape[1], out.data_ptr(), outcomes.data_ptr(), B, S,
                int(seed) & (2 ** 64 - 1))

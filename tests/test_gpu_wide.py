@@ -366,3 +366,35 @@ def test_density_matrices_of_column_and_other_plans(rows, cols, window, B, S, rn
         got = dm_forward(plan, a, s, noise=noise)
         gen = dm_forward(plan, a, s, noise=noise, step_probs=True)
         assert (got - gen).abs().max().item() < 2e-5
+
+
+@pytest.mark.parametrize("rows,cols,B,pad", [(4, 19, 131073, 0), (4, 19, 131071, 0), (3, 25, 131073, 5),
+                                             (6, 40, 40331, 0), (5, 40, 65536, 1)])
+def test_row_major_angles_equal_angle_major(rows, cols, B, pad, rng):
+    """Large batches of row-major angles (on either side of the copy's byte limit,
+    odd batches, padded rows) against angle-major ones, run and sampled, bit for
+    bit, and inside a captured graph."""
+    torch = _torch()
+    import mentpy_amd as mp
+    g = mp.templates.grid_cluster(rows, cols)
+    n = len(g.trainable_nodes)
+    sim = mp.PatternSimulator(g, backend="hip-sv")
+    gen = torch.Generator(device="cuda").manual_seed(rows)
+    a = torch.rand((B, n + pad), generator=gen, device="cuda")[:, :n]
+    am = a.t().contiguous().t()
+    psi = haar_state(rows, rng)
+    want = sim.run_batch(am, psi)
+    assert torch.equal(sim.run_batch(a, psi), want)
+    out = [mp.PatternSimulator(g, backend="hip-sv", force0=False, seed=3).run_batch(x, psi) for x in (a, am)]
+    assert torch.equal(out[0], out[1])
+    x = torch.as_tensor(psi, device="cuda").to(torch.complex64)
+    sim.run_batch(a, x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = sim.run_batch(a, x)
+    for _ in range(3):
+        got.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
