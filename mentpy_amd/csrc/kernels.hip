@@ -4038,7 +4038,7 @@ int mbqc_sv_forward_c64(const mbqc_plan* plan, const float* angles, int64_t angl
     }
     return e == hipSuccess ? MBQC_OK : hip_fail(e, "sv_forward launch");
   }
-  if (narrow_sv(J)) {
+  if (narrow_sv(J, flags)) {
     e = launch_narrow_sv(J, periodic, flags, st);
     return e == hipSuccess ? MBQC_OK : hip_fail(e, "sv_forward launch");
   }

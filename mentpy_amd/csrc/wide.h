@@ -11,7 +11,7 @@ namespace mbqc {
 hipError_t launch_wide_sv(const Job& J, bool column, uint32_t flags, hipStream_t st);
 // The same for windows of 2..6 slots, where narrow_sv says that the batch is
 // too small for one simulation per lane.
-bool narrow_sv(const Job& J);
+bool narrow_sv(const Job& J, uint32_t flags);
 hipError_t launch_narrow_sv(const Job& J, bool column, uint32_t flags, hipStream_t st);
 // One simulation of a window of 1..6 slots, its input state (2^n_in amplitudes,
 // from word 0) and angles (from word first_angle) passed by value.

@@ -262,10 +262,12 @@ __device__ __forceinline__ float wide_inv_norm_in_order(const float2 (&t)[1 << R
 }
 
 // Simulation g of job J on the lanes of one group (inactive groups run the
-// last simulation and store nothing).
+// last simulation and store nothing).  cl: the lane's place among the `clanes`
+// lanes that share coefficients.
 template <int NS, int R, bool REF, bool COLUMN, int SPARE = 0>
 __device__ __forceinline__ void wide_sim(const Job& J, int64_t g, bool active, uint32_t flags,
-                                         float2* buf, float2* bs, int cl) {
+                                         float2* buf, float2* bs, int cl,
+                                         int clanes = Wide<NS, R, NS, SPARE>::CL) {
   using W = Wide<NS, R, NS, SPARE>;
   const int lane = cl & (W::TL - 1);
   const int64_t gg = active ? g : J.total - 1;
@@ -276,7 +278,7 @@ __device__ __forceinline__ void wide_sim(const Job& J, int64_t g, bool active, u
   RefPhase rp;
   constexpr bool kLaneKernelToo = NS <= 6;   // then equal to it bit for bit
   wide_run<NS, R, REF, COLUMN, kLaneKernelToo>(
-      t, J, J.angles + bi * J.angle_stride, buf, bs, cl, W::CL, &rp, [](int, const float2 (&)[W::NR]) {},
+      t, J, J.angles + bi * J.angle_stride, buf, bs, cl, clanes, &rp, [](int, const float2 (&)[W::NR]) {},
       NoModify());
   if constexpr (REF) {
     rp.m_sum = lanes_sum<W::CL>(rp.m_sum, reinterpret_cast<int32_t*>(bs));
@@ -289,7 +291,7 @@ __device__ __forceinline__ void wide_sim(const Job& J, int64_t g, bool active, u
   else if constexpr (kLaneKernelToo) scale = wide_inv_norm_in_order<NS, R>(t, out_pos, buf, lane);
   else scale = wide_inv_norm<NS, R>(t, out_pos, lane, bs);
   const float2 f = cscale(ph, scale);
-  if (active && cl < W::TL) {
+  if (active && (SPARE == 0 || cl < W::TL)) {
     float2* o = J.out + g * (int64_t(1) << J.n_out);
 #pragma unroll
     for (int r = 0; r < W::NR; ++r) {
@@ -308,6 +310,29 @@ __global__ __launch_bounds__((Wide<NS, R, NS, SPARE>::T)) void k_wide_sv(Job J, 
   float2* buf = lds + sub * W::SIM;
   const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
   wide_sim<NS, R, REF, COLUMN, SPARE>(J, g, g < J.total, flags, buf, buf + W::BUF, cl);
+}
+
+// Lanes that evaluate one set of coefficients for simulations of `lanes` lanes,
+// `same` of which in a row have the same angles: at most a wave.
+inline int shared_lanes(int lanes, int64_t same) {
+  for (; lanes < 64 && same % 2 == 0; same /= 2) lanes *= 2;
+  return lanes;
+}
+
+// The same without the reference phase (whose sums stay with a simulation) for
+// simulations that share their angles in groups of clanes / TL, at least 4 of them:
+// no lanes are spent on coefficients alone.
+template <int NS, int R, bool COLUMN>
+__global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_sv_shared(Job J, uint32_t flags,
+                                                                     int clanes) {
+  using W = Wide<NS, R>;
+  constexpr int SETS = (W::T + 63) / 64 * (W::TL >= 16 ? 1 : 64 / (4 * W::TL));
+  __shared__ float2 lds[W::G * W::BUF + SETS * W::CS];
+  const int sub = threadIdx.x / W::TL;
+  const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
+  wide_sim<NS, R, false, COLUMN>(J, g, g < J.total, flags, lds + sub * W::BUF,
+                                 lds + W::G * W::BUF + int(threadIdx.x) / clanes * W::CS,
+                                 int(threadIdx.x) % clanes, clanes);
 }
 
 // Sampled outcomes: the frame and draws of SampleMod, evaluated identically by
@@ -421,11 +446,7 @@ struct AdjWide {
   __host__ __device__ static constexpr int lds(int groups, int states, int clanes) {
     return groups * states * W::BUF + (groups * W::TL + clanes - 1) / clanes * W::CS;
   }
-  static int clanes(int64_t columns) {
-    int c = W::TL;
-    for (; c < 64 && columns % 2 == 0; columns /= 2) c *= 2;
-    return c;
-  }
+  static int clanes(int64_t columns) { return shared_lanes(W::TL, columns); }
 };
 
 template <int NS, int R>
@@ -941,6 +962,19 @@ hipError_t narrow_launch(const Job& J, bool column, uint32_t flags, hipStream_t 
 }
 
 template <int NS>
+hipError_t shared_launch(const Job& J, bool column, uint32_t flags, hipStream_t st) {
+  constexpr int R = narrow_reg_bits(NS);
+  using W = Wide<NS, R>;
+  const dim3 grid(unsigned((J.total + W::G - 1) / W::G)), block(W::T);
+  const int clanes = shared_lanes(W::TL, J.S);
+  if (column)
+    hipLaunchKernelGGL((k_wide_sv_shared<NS, R, true>), grid, block, 0, st, J, flags, clanes);
+  else
+    hipLaunchKernelGGL((k_wide_sv_shared<NS, R, false>), grid, block, 0, st, J, flags, clanes);
+  return hipGetLastError();
+}
+
+template <int NS>
 hipError_t narrow_launch(const Job& J, bool column, uint32_t flags, hipStream_t st) {
   constexpr int lane_bits = NS - narrow_reg_bits(NS);
   if (J.total <= 1024) return narrow_launch<NS, 6 - lane_bits>(J, column, flags, st);
@@ -1049,9 +1083,28 @@ hipError_t launch_run_one(const Job& J, const HostInputs& in, bool column, uint3
   }
 }
 
-bool narrow_sv(const Job& J) { return J.ns <= 6 && J.total <= kNarrowMaxSims[J.ns]; }
+// Most simulations that run with their angles' coefficients shared (raw phase, inputs a
+// multiple of 4).  Replayed graphs, us (as without sharing / shared): 4x16 grid, 16
+// inputs, 2,048 sims 9.6 / 8.1, 16,384 14.2 / 11.1, 32,768 17.2 / 14.7, 65,536
+// 18.1 / 25.9; 5x10, 32 inputs, 2,048 8.4 / 7.2, 16,384 13.2 / 11.8, 32,768
+// 26.4 / 18.7, 65,536 28.3 / 33.0; 6x12, 64 inputs, 16,384 20.3 / 18.7, 131,072
+// 119.9 / 96.3.
+constexpr int64_t kSharedMaxSims[7] = {0, 0, 0, 0, 32768, 32768, 131072};
+
+static int64_t shared_max(const Job& J, uint32_t flags) {
+  return J.S % 4 == 0 && !(flags & MBQC_FLAG_REF_PHASE) ? kSharedMaxSims[J.ns] : 0;
+}
+
+bool narrow_sv(const Job& J, uint32_t flags) {
+  return J.ns <= 6 && J.total <= std::max(kNarrowMaxSims[J.ns], shared_max(J, flags));
+}
 
 hipError_t launch_narrow_sv(const Job& J, bool column, uint32_t flags, hipStream_t st) {
+  if (J.total > 1024 && J.total <= shared_max(J, flags)) {
+    if (J.ns == 4) return shared_launch<4>(J, column, flags, st);
+    if (J.ns == 5) return shared_launch<5>(J, column, flags, st);
+    return shared_launch<6>(J, column, flags, st);
+  }
   switch (J.ns) {
     case 2: return narrow_launch<2>(J, column, flags, st);
     case 3: return narrow_launch<3>(J, column, flags, st);

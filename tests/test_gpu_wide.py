@@ -238,6 +238,30 @@ def test_narrow_windows_small_batches(rows, cols, window, B, S, rng):
     assert (raw * phase[..., None] - out).abs().max().item() < 2e-5
 
 
+@pytest.mark.parametrize("rows,cols,window,B,S", [
+    (4, 5, None, 257, 4), (4, 19, None, 129, 16), (4, 7, None, 2731, 12), (4, 7, None, 2732, 12),
+    (5, 16, None, 100, 32), (5, 6, None, 8193, 4), (6, 13, None, 41, 64), (6, 5, None, 32769, 4),
+    (4, 6, 7, 300, 8)])
+def test_shared_coefficients_equal_single_inputs(rows, cols, window, B, S, rng):
+    """Raw-phase launches whose inputs share their angles' coefficients (4, 8, 16
+    and more in a row, either side of the largest batches, general plans) equal
+    the launches of one input each bit for bit."""
+    torch = _torch()
+    import mentpy_amd as mp
+    from mentpy_amd.simulators.hip_simulator import sv_forward
+    g = mp.templates.grid_cluster(rows, cols)
+    sim = mp.PatternSimulator(g, backend="hip-sv", **({"window_size": window} if window else {}))
+    plan = sim.simulator.plan
+    gen = torch.Generator().manual_seed(rows * cols)
+    th = (torch.rand((B, len(g.trainable_nodes)), generator=gen) * 12 - 6).cuda()
+    x = torch.randn((S, 1 << rows), generator=gen, dtype=torch.complex64).cuda()
+    for renorm in (False, True):
+        got = sv_forward(plan, th, x, ref_phase=False, renormalize=renorm)
+        for i in range(0, S, max(1, S // 4)):
+            one = sv_forward(plan, th, x[i:i + 1], ref_phase=False, renormalize=renorm)
+            assert torch.equal(got[:, i], one[:, 0])
+
+
 @pytest.mark.parametrize("rows,B", [(2, 4097), (3, 2049), (4, 16385), (5, 16385), (6, 32769)])
 def test_narrow_windows_lane_kernel_above_the_threshold(rows, B, rng):
     """The first batch above the threshold (one simulation per lane) against
