@@ -304,10 +304,10 @@ def config_batched(args, dev, stream):
             "max_amp_err_vs_c128": max(errs),
             "roofline": {"bound": "valu", "achieved": round(achieved, 3), "peak": FP32_PEAK_TFLOPS,
                          "unit": "TFLOP/s", "frac": round(achieved / FP32_PEAK_TFLOPS, 4),
-                         "traffic": profiled_traffic("k_batch", BATCHED_PROFILE, per="launch"),
-                         "traffic_note": "HBM bytes per graph replay (the four window-size "
-                                         "kernels), rocprof counters in " + _rel(BATCHED_PROFILE),
-                         "kernel": "k_batch"}}
+                         "traffic": profiled_traffic("k_batch_mixed", BATCHED_PROFILE, per="launch"),
+                         "traffic_note": "HBM bytes per graph replay (one kernel over the "
+                                         "window sizes), rocprof counters in " + _rel(BATCHED_PROFILE),
+                         "kernel": "k_batch_mixed"}}
 
 
 def config_dm(args, dev, stream):
@@ -349,7 +349,7 @@ def config_dm(args, dev, stream):
     td = 0.5 * np.abs(np.linalg.eigvalsh(out[:k, 0].cpu().numpy() - ref)).sum(-1)
     f_sim = plan.info["n_steps"] * 20 * 4 ** (plan.info["window"] - 1)
     achieved = f_sim * B / (ms / 1e3) / 1e12
-    dm_kernel = "k_dm_forward<3,true>" if B >= 32768 else "k_dm_forward_lds<3,16,4,true>"
+    dm_kernel = "k_dm_pauli<3,1>"
     bps = profiled_traffic(dm_kernel, DM_PROFILE)
     dm_traffic = None if bps is None else round(bps * B)
     return {"metric": "density-matrix pattern sims/s, 3x12 grid, noisy, trace distance vs c128",
@@ -428,15 +428,13 @@ def config_mbqml(args, dev, stream):
     graph = step.capture()
     secs = time_launches(graph.replay, args.steps, args.warmup, stream)
     ms = secs / args.steps * 1e3
-    # roofline of the largest part of the step, the segmented forward (the
-    # segment sweeps and the chain products), timed alone with HIP events
+    # roofline of the forward launch (the transfer matrices), timed alone with
+    # HIP events
     fwd_s = time_each_launch(step._launch_forward, args.steps, args.warmup, stream)
     info = sim.simulator.plan.info
     n_cols = step.cols.shape[0]
-    f_sweep = B * n_cols * flops_per_sim(info["n_steps"], info["window"])
-    f_chain = B * (step.segments - 1) * n_cols ** 3 * 8
-    fwd_flops = f_sweep + f_chain
-    fwd_kernel = "k_sv_seg_forward<4,true>+k_seg_chain_forward_mfma"
+    fwd_flops = B * n_cols * flops_per_sim(info["n_steps"], info["window"])
+    fwd_kernel = "k_wide_sv_shared<4,2,true>"
     fwd_tflops = fwd_flops / fwd_s / 1e12
     fd_secs = time_launches(lambda: fd_loop_infidelity_grad(sim, th, step.X, step.Y, h=1e-3), 1, 1, stream)
     _, gr = step.run(th)
