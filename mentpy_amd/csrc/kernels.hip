@@ -2164,7 +2164,8 @@ __global__ __launch_bounds__(64) void k_sv_seg_backward(Job J, SegInfo G, const 
 // docs/tutorials/intro-to-mbqml.rst:35-54):
 //   z_b = M t_b,  loss_b = 1 - Re(t_b^H z_b) / S,  seed_b = -2 z_b / S,
 // with t_b = vec(T_b) (K = 2^(|I|+|O|) entries) and the data Gram matrix M
-// given transposed (MT[k][n] = M[n][k]).  A workgroup covers kGramSets
+// given transposed (MT[k][n] = M[n][k]).  For K a multiple of 16 the products are
+// those of gram.hip; this is the form for the others.  A workgroup covers kGramSets
 // parameter sets x 64 output indices n; its 256 threads are 64 n x 4 groups
 // of kGramSets/4 sets; the sets' t rows are staged in LDS, MT is read
 // coalesced along n.  Loss partial sums go through LDS and one atomic-free

@@ -346,6 +346,11 @@ __global__ __launch_bounds__((Pauli<NS, K>::T)) void k_dm_pauli(Job J, DmNoise n
 // density matrix step: per parameter set 4^NS multiply-adds where the sweep of
 // states and cotangents takes 9 C 2^NS for C columns, no checkpoints, and the
 // derivative of a step is two coefficients, (I - Z) / 2.
+//
+// Bound by the digit exchanges through LDS (many sets: about half of the issue slots)
+// or by the chain of steps and exchanges (few).  The transfer matrix's columns,
+// against the sweeps with checkpoints: 4x20 grid, 16,384 sets 131 -> 54 us, 4x16
+// grid, 1,024 sets 20.4 -> 11.7 us, 5x10 grid, 4,096 sets 101 -> 49 us.
 
 // The inverse of pauli_rotate.
 template <int NS, int K, int M, bool CZ>
