@@ -210,11 +210,91 @@ __global__ __launch_bounds__(256, 4) void k_product_small(Operands g) {
   }
 }
 
+// In between: a workgroup takes 32 x 32, its four waves a quarter of the k's each
+// (16 at a time, whole lines of A): half the operand bytes of k_product_small.
+template <Product W>
+__global__ __launch_bounds__(256, 2) void k_product_mid(Operands g) {
+  __shared__ float2 red[4 * 32 * 33];
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int li = l & 31, h = l >> 5;
+  const int tiles = (g.N + 31) / 32;
+  const int tile = xcd_block(blockIdx.x, gridDim.x);
+  const int64_t m0 = int64_t(tile / tiles) * 32;
+  const int n0 = (tile % tiles) * 32;
+  const int64_t row = m0 + li < g.M ? m0 + li : g.M - 1;
+  const int col = n0 + li < g.N ? n0 + li : g.N - 1;
+  const float2* pa = g.A + row * g.K;
+  const float2* pb = g.B + col;
+  f32x16 zr, zi;
+#pragma unroll
+  for (int r = 0; r < 16; ++r) zr[r] = zi[r] = 0.0f;
+  float2 an[8], bn[8];
+  auto fetch = [&](int k0) {
+    const int k1 = k0 + 8 * h;
+    if (k0 + 16 <= g.K) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        an[j] = pa[k1 + j];
+        bn[j] = pb[int64_t(k1 + j) * g.N];
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const bool in = k1 + j < g.K;
+        an[j] = in ? pa[k1 + j] : make_float2(0.0f, 0.0f);
+        bn[j] = in ? pb[int64_t(k1 + j) * g.N] : make_float2(0.0f, 0.0f);
+      }
+    }
+  };
+  if (16 * w < g.K) fetch(16 * w);
+  for (int k0 = 16 * w; k0 < g.K; k0 += 64) {
+    float2 a[8], b[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      a[j] = an[j];
+      b[j] = bn[j];
+    }
+    if (k0 + 64 < g.K) fetch(k0 + 64);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      zr = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j].x, b[j].x, zr, 0, 0, 0);
+      zi = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j].x, b[j].y, zi, 0, 0, 0);
+      zr = __builtin_amdgcn_mfma_f32_32x32x2f32(-a[j].y, b[j].y, zr, 0, 0, 0);
+      zi = __builtin_amdgcn_mfma_f32_32x32x2f32(a[j].y, b[j].x, zi, 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 16; ++r)
+    red[(w * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * 33 + li] = make_float2(zr[r], zi[r]);
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int r = (threadIdx.x >> 5) + 8 * i, c = threadIdx.x & 31;
+    float2 z = red[r * 33 + c];
+#pragma unroll
+    for (int q = 1; q < 4; ++q) z = cadd(z, red[(q * 32 + r) * 33 + c]);
+    float p = 0.0f;
+    if (m0 + r < g.M && n0 + c < g.N) p = finish<W>(g, m0 + r, n0 + c, z);
+    if constexpr (W != Product::kScaled) {
+      p = last_lane_sum<32>(p);
+      if (c == 31 && m0 + r < g.M) g.part[(m0 + r) * tiles + n0 / 32] = p;
+    }
+  }
+}
+
 // From 2^20 results on every SIMD has a 32 x 32 wave.  Loss and seed of the Gram form
 // (K = N = 256, us, small / large): 1,024 rows 11.1 / 22, 2,048 18.9 / 23, 4,096
 // 34 / 24.5, 8,192 60 / 44.5 (the one-wave 16 x 16 tiles and loss pass before: 1,024
 // rows 18.0, 8,192 rows 80).
 bool large(int64_t M, int N) { return M * N >= (int64_t(1) << 20); }
+
+// From 2^18 results on a quarter of the CUs' waves is enough for 32 x 32 (seed alone, us,
+// small / mid: K = N = 256, 512 rows 7.3 / 9.9, 1,024 11.1 / 10.4, 2,048 19.5 / 16.7, 3,000
+// 25.7 / 22.7; K = N = 64, 12,000 rows 12.6 / 9.2; K = N = 16, 16,384 rows 6.9 / 7.9).  Not
+// for K above 256: a wave's sums would be longer than the 64 k of the others.
+bool mid(int64_t M, int N, int K) {
+  return M * N >= (int64_t(1) << 18) && K >= 64 && K <= 256;
+}
 
 template <Product W>
 hipError_t product_launch(const Operands& g, hipStream_t st) {
@@ -223,6 +303,9 @@ hipError_t product_launch(const Operands& g, hipStream_t st) {
     hipLaunchKernelGGL((k_product_large<W, true>), grid, dim3(256), 0, st, g);
   else if (large(g.M, g.N))
     hipLaunchKernelGGL((k_product_large<W, false>), grid, dim3(256), 0, st, g);
+  else if (mid(g.M, g.N, g.K))
+    hipLaunchKernelGGL((k_product_mid<W>), dim3(unsigned(((g.M + 31) / 32) * ((g.N + 31) / 32))),
+                       dim3(256), 0, st, g);
   else
     hipLaunchKernelGGL((k_product_small<W>), dim3(unsigned(((g.M + 15) / 16) * ((g.N + 15) / 16))),
                        dim3(256), 0, st, g);
@@ -231,7 +314,7 @@ hipError_t product_launch(const Operands& g, hipStream_t st) {
 
 }  // namespace
 
-int product_tile(int64_t M, int N) { return large(M, N) ? 32 : 16; }
+int product_tile(int64_t M, int N, int K) { return large(M, N) || mid(M, N, K) ? 32 : 16; }
 
 hipError_t launch_product(Product what, const float2* A, const float2* B, float2* C, int64_t M, int N,
                           int K, float scale, float* part, hipStream_t st) {

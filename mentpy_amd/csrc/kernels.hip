@@ -3778,7 +3778,8 @@ int gram_loss_seed(const void* t, const void* MT, int64_t B, int32_t K, int32_t 
   const float inv_S = 1.0f / float(S);
   int nblk;
   if (K % 16 == 0) {
-    nblk = K / product_tile(B, K) + (K % product_tile(B, K) != 0);
+    const int tile = product_tile(B, K, K);
+    nblk = (K + tile - 1) / tile;
     hipError_t e = launch_product(Product::kGram, static_cast<const float2*>(t),
                                   static_cast<const float2*>(MT), static_cast<float2*>(seed), B, K, K,
                                   -2.0f * inv_S, workspace, st);
@@ -4681,7 +4682,7 @@ int mbqc_transfer_loss_seed_c64(const void* t, const void* DT, const void* DC, i
   float2* f = static_cast<float2*>(workspace);
   float* part = reinterpret_cast<float*>(f + B * S);
   const float inv_S = 1.0f / float(S);
-  const int tile = product_tile(B, S);
+  const int tile = product_tile(B, S, K);
   hipError_t e = launch_product(Product::kOverlap, static_cast<const float2*>(t),
                                 static_cast<const float2*>(DT), seed ? f : nullptr, B, S, K, 1.0f, part,
                                 st);

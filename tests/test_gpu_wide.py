@@ -160,9 +160,10 @@ def test_gradient_from_outputs_matches_complex128(rows, cols, C, B, rng):
 
 
 @pytest.mark.parametrize("B,K,S", [(1, 16, 1), (15, 20, 16), (17, 64, 33), (33, 1024, 100), (2049, 256, 37),
-                                   (1030, 1024, 65), (16400, 64, 257), (4097, 256, 256)])
+                                   (1030, 1024, 65), (16400, 64, 257), (4097, 256, 256),
+                                   (1031, 256, 257), (4097, 64, 100)])
 def test_transfer_products_match_complex128(B, K, S, rng):
-    """Loss and seed through the data matrix, both tilings: partly filled tiles of
+    """Loss and seed through the data matrix, every tiling: partly filled tiles of
     rows and columns, a contraction length with a remainder, loss alone and
     seed alone; the Gram seed of the same data."""
     torch = _torch()
