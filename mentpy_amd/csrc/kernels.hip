@@ -2947,7 +2947,7 @@ __device__ __forceinline__ void batch_item(const Job& J, const BatchItem& I, int
 // grids of 2..5 rows x 1,024 x 16, 16,384 items of 64 simulations, all window sizes
 // in one launch: 440 us with one counter, 192 with 32).  Items are
 // sorted by decreasing cost, so the lists carry the same work and long items
-// start first.  The host gives every list at least one wave.
+// start first.  The host makes no more lists than the launch has waves (item_lists).
 // (The item list stays a __restrict__ kernel argument: from a struct its loads, and
 // with them the whole job, would be per-lane vector loads.)
 struct ItemLists {
@@ -3829,6 +3829,11 @@ constexpr int64_t kBatchGlobalSims = 128;
 // per window size, set 0 for the launch over all register groups.
 constexpr int kItemLists = 32;
 constexpr int kBatchCounters = (kMaxBatchSlots + 1) * kItemLists;
+// No more lists than the launch has waves (whole workgroups of them), so that every
+// list is drained.
+static int32_t item_lists(int blocks, int wg_waves) {
+  return int32_t(std::min<int64_t>(int64_t(blocks) * wg_waves, kItemLists));
+}
 
 struct mbqc_batch {
   int max_ns = 1;
@@ -3909,7 +3914,7 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
     const BatchItem* items = bt->d_items + bt->group_begin[ns];
     int* counter = bt->d_counter + ns * kItemLists * kCounterStride;
     const BatchGroupLaunch L{dim3(blocks), dim3(threads), gs, bt->d_jobs,
-                             items, {n, counter, int32_t(std::min<int64_t>(wv, kItemLists))}, flags};
+                             items, {n, counter, item_lists(blocks, wg_waves)}, flags};
     const bool sh = bt->share[ns];
     const bool pe = bt->periodic[ns] && !(flags & MBQC_FLAG_TABLE_STEPS);
     switch (ns) {
@@ -3950,11 +3955,10 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
       periodic = periodic && bt->periodic[ns];
     }
     waves = std::min<int64_t>(waves, ((bt->n_mixed + wg_waves - 1) / wg_waves) * wg_waves);
-    const BatchGroupLaunch L{dim3(unsigned(waves / wg_waves)), dim3(threads), st, bt->d_jobs,
+    const int blocks = int(waves / wg_waves);
+    const BatchGroupLaunch L{dim3(blocks), dim3(threads), st, bt->d_jobs,
                              bt->d_items + bt->items.size(),
-                             {bt->n_mixed, bt->d_counter,
-                              int32_t(std::min<int64_t>(waves, kItemLists))},
-                             flags};
+                             {bt->n_mixed, bt->d_counter, item_lists(blocks, wg_waves)}, flags};
     if (bt->mixed_max == 6) launch_batch_mixed<6>(L, ref, periodic, share);
     else launch_batch_mixed<5>(L, ref, periodic, share);
     e = hipGetLastError();
