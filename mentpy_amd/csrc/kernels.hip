@@ -22,6 +22,7 @@
 #include "device.h"
 #include "plan.h"
 #include "gram.h"
+#include "side_streams.h"
 #include "wide.h"
 
 namespace mbqc {
@@ -3866,6 +3867,15 @@ struct mbqc_batch {
   int64_t gws_sims[kMaxBatchSlots + 1] = {};
 };
 
+struct HipStreams {
+  using Stream = hipStream_t;
+  using Event = hipEvent_t;
+  using Error = hipError_t;
+  static constexpr Error kOk = hipSuccess;
+  static Error record(Event ev, Stream st) { return hipEventRecord(ev, st); }
+  static Error wait(Stream st, Event ev) { return hipStreamWaitEvent(st, ev, 0); }
+};
+
 // One launch of a batch: the counter reset, then one persistent kernel per
 // live-window size ns with group_waves[ns] > 0 resident wavefronts (capped at
 // the group's item count); with several groups all but one run on side streams
@@ -3874,7 +3884,6 @@ struct mbqc_batch {
 // (their outputs are not written).
 static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_waves,
                         uint32_t flags, bool mixed, void* stream) {
-  bool joined[kMaxBatchSlots + 1] = {};
   if (wg_waves < 1 || wg_waves > 4) return fail(MBQC_ERR_VALUE, "wg_waves must be 1..4");
   int launched = 0;
   for (int ns = 1; ns <= kMaxBatchSlots; ++ns) {
@@ -3893,8 +3902,9 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
   const int first_single = mixed ? kMaxSvSlots + 1 : 1;
   if (mixed) launched -= bt->mixed_groups - 1;
   const bool concurrent = bt->fork != nullptr && launched > 1;
+  SideStreams<HipStreams, kMaxBatchSlots + 1> branches(st, bt->fork, bt->side, bt->join);
   hipError_t e = hipGetLastError();
-  if (e == hipSuccess && concurrent) e = hipEventRecord(bt->fork, st);
+  if (e == hipSuccess && concurrent) e = branches.fork();
   // largest windows first; the last launch stays on the caller's stream
   int left = launched;
   for (int ns = kMaxBatchSlots; ns >= first_single && e == hipSuccess; --ns) {
@@ -3904,7 +3914,7 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
     const bool side = concurrent && --left > 0;
     if (side) {
       gs = bt->side[ns];
-      e = hipStreamWaitEvent(gs, bt->fork, 0);
+      e = branches.begin(ns);
       if (e != hipSuccess) break;
     }
     // no more resident waves than the group has items
@@ -3941,8 +3951,6 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
         break;
     }
     if (e == hipSuccess) e = hipGetLastError();
-    if (e == hipSuccess && side) e = hipEventRecord(bt->join[ns], gs);
-    joined[ns] = side;
   }
   if (e == hipSuccess && mixed) {
     int64_t waves = 0;
@@ -3963,8 +3971,8 @@ static int batch_launch(mbqc_batch* bt, const int32_t* group_waves, int32_t wg_w
     else launch_batch_mixed<5>(L, ref, periodic, share);
     e = hipGetLastError();
   }
-  for (int ns = 1; ns <= kMaxBatchSlots && e == hipSuccess; ++ns)
-    if (joined[ns]) e = hipStreamWaitEvent(st, bt->join[ns], 0);
+  const hipError_t ej = branches.join();
+  if (e == hipSuccess) e = ej;
   return e == hipSuccess ? MBQC_OK : hip_fail(e, "batch launch");
 }
 
