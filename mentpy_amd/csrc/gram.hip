@@ -143,8 +143,11 @@ __global__ __launch_bounds__(256, 4) void k_product_large(Operands g) {
 // Few rows: a workgroup takes 16 x 16, its four waves a quarter of the k's each,
 // so that four times the waves hide each other's loads.  MFMA 16x16x4: lane l
 // holds A[l % 16][l / 16] and B[l / 16][l % 16], the accumulator
-// D[4 (l / 16) + r][l % 16], r = 0..3.
-template <Product W>
+// D[4 (l / 16) + r][l % 16], r = 0..3.  A sum has K / 8 of the k's; LONG (K > 512):
+// partial sums of 64 k are added up, as in k_product_large.  (Gradients of 2,000 sets
+// of a 5x4 grid with 64 inputs, K = 1,024, against 64 bits: 1.57e-9 with library
+// products, 1.66e-9 in one sum, 1.49e-9 so; times level.)
+template <Product W, bool LONG>
 __global__ __launch_bounds__(256, 4) void k_product_small(Operands g) {
   __shared__ float2 red[4 * 16 * 17];
   const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -158,11 +161,24 @@ __global__ __launch_bounds__(256, 4) void k_product_small(Operands g) {
   const float2* pa = g.A + row * g.K;
   const float2* pb = g.B + col;
   // two accumulators per part: shorter sums, and no product waits for the last one
-  f32x4 zr[2], zi[2];
+  f32x4 zr[2], zi[2], sr, si;
+  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-  for (int i = 0; i < 2; ++i) zr[i] = zi[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int i = 0; i < 2; ++i) zr[i] = zi[i] = zero;
+  sr = si = zero;
   constexpr int U = 2;                       // chunks of 16 k loaded together
+  [[maybe_unused]] int terms = 0;            // k's of each accumulator
   for (int k0 = 16 * w; k0 < g.K; k0 += 64 * U) {
+    if constexpr (LONG) {
+      if (terms == 64) {
+        sr += zr[0] + zr[1];
+        si += zi[0] + zi[1];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) zr[i] = zi[i] = zero;
+        terms = 0;
+      }
+      terms += 8 * U;
+    }
     float2 a[4 * U], b[4 * U];
     if (k0 + 64 * (U - 1) + 16 <= g.K) {
 #pragma unroll
@@ -194,9 +210,15 @@ __global__ __launch_bounds__(256, 4) void k_product_small(Operands g) {
       zi[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].y, b[i].x, zi[q], 0, 0, 0);
     }
   }
+  zr[0] += zr[1];
+  zi[0] += zi[1];
+  if constexpr (LONG) {
+    zr[0] += sr;
+    zi[0] += si;
+  }
 #pragma unroll
   for (int r = 0; r < 4; ++r)
-    red[(w * 16 + 4 * h + r) * 17 + li] = make_float2(zr[0][r] + zr[1][r], zi[0][r] + zi[1][r]);
+    red[(w * 16 + 4 * h + r) * 17 + li] = make_float2(zr[0][r], zi[0][r]);
   __syncthreads();
   const int r = threadIdx.x >> 4, c = threadIdx.x & 15;
   float2 z = red[r * 17 + c];
@@ -291,7 +313,8 @@ bool large(int64_t M, int N) { return M * N >= (int64_t(1) << 20); }
 // From 2^18 results on a quarter of the CUs' waves is enough for 32 x 32 (seed alone, us,
 // small / mid: K = N = 256, 512 rows 7.3 / 9.9, 1,024 11.1 / 10.4, 2,048 19.5 / 16.7, 3,000
 // 25.7 / 22.7; K = N = 64, 12,000 rows 12.6 / 9.2; K = N = 16, 16,384 rows 6.9 / 7.9).  Not
-// for K above 256: a wave's sums would be longer than the 64 k of the others.
+// for K above 256: a wave takes a quarter of the k's in one sum, which would be longer
+// than the 64 k that the other kernels add up in one.
 bool mid(int64_t M, int N, int K) {
   return M * N >= (int64_t(1) << 18) && K >= 64 && K <= 256;
 }
@@ -306,8 +329,11 @@ hipError_t product_launch(const Operands& g, hipStream_t st) {
   else if (mid(g.M, g.N, g.K))
     hipLaunchKernelGGL((k_product_mid<W>), dim3(unsigned(((g.M + 31) / 32) * ((g.N + 31) / 32))),
                        dim3(256), 0, st, g);
+  else if (g.K > 512)
+    hipLaunchKernelGGL((k_product_small<W, true>), dim3(unsigned(((g.M + 15) / 16) * ((g.N + 15) / 16))),
+                       dim3(256), 0, st, g);
   else
-    hipLaunchKernelGGL((k_product_small<W>), dim3(unsigned(((g.M + 15) / 16) * ((g.N + 15) / 16))),
+    hipLaunchKernelGGL((k_product_small<W, false>), dim3(unsigned(((g.M + 15) / 16) * ((g.N + 15) / 16))),
                        dim3(256), 0, st, g);
   return hipGetLastError();
 }
