@@ -27,6 +27,12 @@ hipError_t launch_run_one(const Job& J, const HostInputs& in, bool column, uint3
 size_t wide_tile_bytes(int ns);
 hipError_t launch_wide_tiles(const Job& J, bool column, uint32_t flags, void* ws, int64_t g0,
                              int64_t n, hipStream_t st);
+// The same for n <= 65,535 simulations of several jobs of window size ns, named by
+// (job, first) of `sims` in order of decreasing steps: active[b] of them have steps
+// in block b of `blocks`; max_out: most output qubits of their jobs.
+hipError_t launch_wide_tiles_jobs(int ns, bool column, uint32_t flags, const Job* jobs,
+                                  const BatchItem* sims, int64_t n, const int64_t* active, int blocks,
+                                  int max_out, void* ws, hipStream_t st);
 hipError_t launch_wide_sample(const Job& J, bool column, const uint64_t* xm, const uint64_t* zm,
                               const int32_t* out_off, int32_t* outcomes, int32_t words,
                               uint64_t seed, hipStream_t st);

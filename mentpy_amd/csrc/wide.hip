@@ -795,26 +795,24 @@ struct TileSigns {
   }
 };
 
-// One pass: steps [k0, k0 + M) of simulations g0 + blockIdx / tiles; `sub`: the
-// rotation before it (k0 % ns).  in == nullptr: the first pass (the input
-// state); `last`: the output and its partial norms.
+// One pass: steps [k0, k0 + M) of simulation g of J, whose state is the l-th of the
+// buffers; `sub`: the rotation before it (k0 % ns).  in == nullptr: the first pass
+// (the input state); `last`: the output and its partial norms.
 template <int M, bool COLUMN>
-__global__ __launch_bounds__((Wide<kTileBits, kTileRegBits>::T)) void k_tile_pass(
-    Job J, const float2* __restrict__ in, float2* __restrict__ out, float* __restrict__ norms,
-    int64_t g0, int k0, int sub, int last) {
+__device__ __forceinline__ void tile_pass(const Job& J, int64_t g, int64_t l,
+                                          const float2* __restrict__ in, float2* __restrict__ out,
+                                          float* __restrict__ norms, int k0, int sub, bool last) {
   using W = Wide<kTileBits, kTileRegBits, M>;
   constexpr int C = kTileBits - M;
   __shared__ float2 buf[W::BUF];
   __shared__ float2 bs[M];
   __shared__ float red[W::T / 64];
   const int lane = threadIdx.x;
-  const int tile_bits = J.ns - kTileBits;
-  const int64_t l = int64_t(blockIdx.x) >> tile_bits;          // simulation of this launch
-  const uint32_t mid = blockIdx.x & ((1u << tile_bits) - 1);
+  const uint32_t mid = blockIdx.x & ((1u << (J.ns - kTileBits)) - 1);
   const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
   const Constant<int32_t> resc = constant(J.tab + J.off_svres);
   int64_t bi, si;
-  split_sim(J, g0 + l, &bi, &si);
+  split_sim(J, g, &bi, &si);
   float2 t[W::NR];
   const int64_t state = l << J.ns;
 #pragma unroll
@@ -847,7 +845,7 @@ __global__ __launch_bounds__((Wide<kTileBits, kTileRegBits>::T)) void k_tile_pas
     return;
   }
   const int32_t* out_pos = J.tab + J.off_out;
-  float2* o = J.out + (g0 + l) * (int64_t(1) << J.n_out);
+  float2* o = J.out + g * (int64_t(1) << J.n_out);
   float n2 = 0.0f;
 #pragma unroll
   for (int r = 0; r < W::NR; ++r) {
@@ -861,16 +859,41 @@ __global__ __launch_bounds__((Wide<kTileBits, kTileRegBits>::T)) void k_tile_pas
   if (lane == 0) norms[blockIdx.x] = n2;
 }
 
+// Workgroup b runs tile b % tiles of simulation b / tiles: simulations g0, g0 + 1, ...
+// of one job, or (batches) those that a list names, of several jobs.
+template <int M, bool COLUMN>
+__global__ __launch_bounds__((Wide<kTileBits, kTileRegBits>::T)) void k_tile_pass(
+    Job J, const float2* __restrict__ in, float2* __restrict__ out, float* __restrict__ norms,
+    int64_t g0, int k0, int sub, int last) {
+  const int64_t l = int64_t(blockIdx.x) >> (J.ns - kTileBits);
+  tile_pass<M, COLUMN>(J, g0 + l, l, in, out, norms, k0, sub, last);
+}
+
+template <int M, bool COLUMN>
+__global__ __launch_bounds__((Wide<kTileBits, kTileRegBits>::T)) void k_tile_pass_jobs(
+    const Job* __restrict__ jobs, const BatchItem* __restrict__ sims, int ns,
+    const float2* __restrict__ in, float2* __restrict__ out, float* __restrict__ norms, int k0,
+    int sub, int block_end) {
+  const int64_t l = int64_t(blockIdx.x) >> (ns - kTileBits);
+  const BatchItem I = sims[l];
+  const Job J = load_job(jobs, I.job);
+  // a job is done with the block that holds its last step
+  const bool last = block_end && k0 - sub + ns >= J.n_steps;
+  tile_pass<M, COLUMN>(J, I.first, l, in, out, norms, k0, sub, last);
+}
+
 // Phase and scale of the outputs a last pass left: workgroup (x, y) takes
-// 1,024 amplitudes of simulation g0 + y.
-__global__ __launch_bounds__(256) void k_tile_finish(Job J, const float* __restrict__ norms,
-                                                     int64_t g0, uint32_t flags) {
+// 1,024 amplitudes of the y-th simulation.
+__device__ __forceinline__ void tile_finish(const Job& J, int64_t g, int64_t l,
+                                            const float* __restrict__ norms, uint32_t flags) {
   __shared__ float red_f[4];
   __shared__ double red_d[4];
   __shared__ int32_t red_i[4];
+  const int64_t dout = int64_t(1) << J.n_out;
+  const int64_t e0 = int64_t(blockIdx.x) * 1024;
+  if (e0 >= dout) return;
   const int tid = threadIdx.x;
   const int tiles = 1 << (J.ns - kTileBits);
-  const int64_t l = blockIdx.y, g = g0 + l;
   const mbqc_step* steps = reinterpret_cast<const mbqc_step*>(J.tab);
   float2 ph = make_float2(1.0f, 0.0f);
   if (flags & MBQC_FLAG_REF_PHASE) {
@@ -890,25 +913,48 @@ __global__ __launch_bounds__(256) void k_tile_finish(Job J, const float* __restr
     scale = 1.0f / sqrtf(lanes_sum<256>(n2, red_f));
   }
   const float2 f = cscale(ph, scale);
-  const int64_t dout = int64_t(1) << J.n_out;
   float2* o = J.out + g * dout;
-  const int64_t e0 = int64_t(blockIdx.x) * 1024;
   for (int64_t e = e0 + tid; e < e0 + 1024 && e < dout; e += 256) o[e] = cmul(o[e], f);
   if (blockIdx.x == 0 && tid == 0 && (flags & MBQC_FLAG_WRITE_PHASE) && J.phase_out)
     J.phase_out[g] = ph;
 }
 
-template <int M>
-void tile_pass(const Job& J, bool column, const float2* in, float2* out, float* norms, int64_t g0,
-               int64_t n, int k0, int sub, int last, hipStream_t st) {
-  const dim3 grid(unsigned(n << (J.ns - kTileBits)));
-  const dim3 block(Wide<kTileBits, kTileRegBits>::T);
-  if (column)
-    hipLaunchKernelGGL((k_tile_pass<M, true>), grid, block, 0, st, J, in, out, norms, g0, k0, sub,
-                       last);
-  else
-    hipLaunchKernelGGL((k_tile_pass<M, false>), grid, block, 0, st, J, in, out, norms, g0, k0, sub,
-                       last);
+__global__ __launch_bounds__(256) void k_tile_finish(Job J, const float* __restrict__ norms,
+                                                     int64_t g0, uint32_t flags) {
+  tile_finish(J, g0 + blockIdx.y, blockIdx.y, norms, flags);
+}
+
+__global__ __launch_bounds__(256) void k_tile_finish_jobs(const Job* __restrict__ jobs,
+                                                          const BatchItem* __restrict__ sims,
+                                                          const float* __restrict__ norms,
+                                                          uint32_t flags) {
+  const BatchItem I = sims[blockIdx.y];
+  tile_finish(load_job(jobs, I.job), I.first, blockIdx.y, norms, flags);
+}
+
+// The passes of patterns of up to `blocks` blocks: at most 8 steps each, of near equal
+// length within a block.  pass(std::integral_constant<int, M>, block, k0, sub,
+// block_end): after a block's last pass the rotation is back at slot order.
+template <typename Pass>
+hipError_t tile_passes(int ns, int blocks, Pass&& pass) {
+  const int per = (ns + 7) / 8;
+  for (int blk = 0; blk < blocks; ++blk) {
+    int sub = 0;
+    for (int p = 0; p < per; ++p) {
+      const int m = ns / per + (p < ns % per ? 1 : 0);
+      const int k0 = blk * ns + sub;
+      const bool end = p + 1 == per;
+      switch (m) {
+        case 5: pass(std::integral_constant<int, 5>{}, blk, k0, sub, end); break;
+        case 6: pass(std::integral_constant<int, 6>{}, blk, k0, sub, end); break;
+        case 7: pass(std::integral_constant<int, 7>{}, blk, k0, sub, end); break;
+        case 8: pass(std::integral_constant<int, 8>{}, blk, k0, sub, end); break;
+        default: return hipErrorInvalidValue;
+      }
+      sub += m;
+    }
+  }
+  return hipSuccess;
 }
 
 template <int NS>
@@ -1130,34 +1176,55 @@ hipError_t launch_wide_tiles(const Job& J, bool column, uint32_t flags, void* ws
   float2* a = static_cast<float2*>(ws);
   float2* b = a + (n << J.ns);
   float* norms = reinterpret_cast<float*>(b + (n << J.ns));
-  // passes of at most 8 steps, of near equal length within a block
-  const int per = (J.ns + 7) / 8;
   const float2* in = nullptr;
-  for (int blk = 0; blk * J.ns < J.n_steps; ++blk) {
-    int sub = 0;
-    for (int p = 0; p < per; ++p) {
-      const int m = J.ns / per + (p < J.ns % per ? 1 : 0);
-      const int k0 = blk * J.ns + sub;
-      // after the last block's last pass the rotation is back at slot order
-      const int last = p + 1 == per && (blk + 1) * J.ns >= J.n_steps;
-      float2* out = in == a ? b : a;
-      switch (m) {
-        case 5: tile_pass<5>(J, column, in, out, norms, g0, n, k0, sub, last, st); break;
-        case 6: tile_pass<6>(J, column, in, out, norms, g0, n, k0, sub, last, st); break;
-        case 7: tile_pass<7>(J, column, in, out, norms, g0, n, k0, sub, last, st); break;
-        case 8: tile_pass<8>(J, column, in, out, norms, g0, n, k0, sub, last, st); break;
-        default: return hipErrorInvalidValue;
-      }
-      in = out;
-      sub += m;
-    }
-  }
+  const dim3 grid(unsigned(n << (J.ns - kTileBits))), block(Wide<kTileBits, kTileRegBits>::T);
+  const int blocks = (J.n_steps + J.ns - 1) / J.ns;
+  const hipError_t e = tile_passes(J.ns, blocks, [&](auto m, int blk, int k0, int sub, bool end) {
+    constexpr int M = decltype(m)::value;
+    const int last = end && blk + 1 == blocks;
+    float2* out = in == a ? b : a;
+    if (column)
+      hipLaunchKernelGGL((k_tile_pass<M, true>), grid, block, 0, st, J, in, out, norms, g0, k0, sub,
+                         last);
+    else
+      hipLaunchKernelGGL((k_tile_pass<M, false>), grid, block, 0, st, J, in, out, norms, g0, k0, sub,
+                         last);
+    in = out;
+  });
+  if (e != hipSuccess) return e;
   const unsigned chunks = unsigned(((int64_t(1) << J.n_out) + 1023) / 1024);
   for (int64_t y = 0; y < n; y += 65535) {   // grid rows are limited to 65,535
     const unsigned ny = unsigned(std::min<int64_t>(n - y, 65535));
     hipLaunchKernelGGL(k_tile_finish, dim3(chunks, ny), dim3(256), 0, st, J,
                        norms + (y << (J.ns - kTileBits)), g0 + y, flags);
   }
+  return hipGetLastError();
+}
+
+hipError_t launch_wide_tiles_jobs(int ns, bool column, uint32_t flags, const Job* jobs,
+                                  const BatchItem* sims, int64_t n, const int64_t* active, int blocks,
+                                  int max_out, void* ws, hipStream_t st) {
+  float2* a = static_cast<float2*>(ws);
+  float2* b = a + (n << ns);
+  float* norms = reinterpret_cast<float*>(b + (n << ns));
+  const float2* in = nullptr;
+  const dim3 block(Wide<kTileBits, kTileRegBits>::T);
+  const hipError_t e = tile_passes(ns, blocks, [&](auto m, int blk, int k0, int sub, bool end) {
+    constexpr int M = decltype(m)::value;
+    const dim3 grid(unsigned(active[blk] << (ns - kTileBits)));
+    float2* out = in == a ? b : a;
+    if (column)
+      hipLaunchKernelGGL((k_tile_pass_jobs<M, true>), grid, block, 0, st, jobs, sims, ns, in, out,
+                         norms, k0, sub, int(end));
+    else
+      hipLaunchKernelGGL((k_tile_pass_jobs<M, false>), grid, block, 0, st, jobs, sims, ns, in, out,
+                         norms, k0, sub, int(end));
+    in = out;
+  });
+  if (e != hipSuccess) return e;
+  const unsigned chunks = unsigned(((int64_t(1) << max_out) + 1023) / 1024);
+  hipLaunchKernelGGL(k_tile_finish_jobs, dim3(chunks, unsigned(n)), dim3(256), 0, st, jobs, sims, norms,
+                     flags);
   return hipGetLastError();
 }
 
