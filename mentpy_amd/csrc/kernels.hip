@@ -132,7 +132,13 @@ __device__ __forceinline__ void shared_block_coeffs(const float (&th)[NS], float
   const int j = int(threadIdx.x) & (G - 1);
   float mine = th[0];
 #pragma unroll
-  for (int sub = 1; sub < NS; ++sub) mine = (j == sub) ? th[sub] : mine;
+  for (int sub = 1; sub < NS; ++sub) {
+    // (loaded outside the choice: as one of its arms the load kept th in LDS or scratch
+    // memory in the batched kernels; 64 grids of 2..6 rows x 1,024 x 16: 554 -> 309 us,
+    // occupancy of k_batch_mixed 1 -> 2 up to 6 slots; 2..5 rows 181 -> 170 us)
+    const float v = th[sub];
+    mine = (j == sub) ? v : mine;
+  }
   float sn, cs;
   sincos_poly(mine, &sn, &cs);
   if constexpr (REF) ph->add_if(mine, j < NS && k0 + j < n_steps);
@@ -213,7 +219,10 @@ __device__ __forceinline__ void sv_fetched_blocks(float2 (&t)[1 << NS], const mb
   const int j = int(threadIdx.x) & 15;
   float mine = th[0];
 #pragma unroll
-  for (int m = 1; m < K * NS; ++m) mine = (j == m) ? th[m] : mine;
+  for (int m = 1; m < K * NS; ++m) {
+    const float v = th[m];
+    mine = (j == m) ? v : mine;
+  }
   float sn, cs;
   sincos_poly(mine, &sn, &cs);
   if constexpr (REF) ph->add_if(mine, j < K * NS);
@@ -2990,10 +2999,11 @@ __global__ __launch_bounds__(256) void k_batch(const Job* __restrict__ jobs,
 // launch instead of a kernel per size forked to and joined from side streams.
 // The chip's few hardware queues run some of those one after the other, and each
 // fork and join costs the host and the device several us.  It runs at the
-// register footprint of the largest window size, which costs less than that
-// (call by call, us per launch, a kernel per size / this: 64 grids x 1,024 x 16
-// 221 / 192, 405 before with one counter and every kernel on a side stream;
-// 40 grids x 100 x 3 90 / 48; 8 grids x 16 76 / 24).
+// register footprint of the largest window size (occupancy 3 up to 5 slots, 2 up to
+// 6), which costs less than that (call by call, us per launch, the best of two wave
+// counts with a kernel per size / this: 64 grids of 2..5 rows x 1,024 x 16 216 / 170,
+// 40 x 100 x 3 83 / 47; 64 of 2..6 rows x 1,024 x 16 368 / 310, x 256 x 3 179 / 107; 64
+// of 5 and 6 rows x 1,024 x 16 650 / 594; 63 of 2..5 rows and one of 6 257 / 200).
 // share: bit ns set where the lanes of that group share coefficients.
 template <bool REF, bool PERIODIC, int MAXNS>
 __global__ __launch_bounds__(256) void k_batch_mixed(const Job* __restrict__ jobs,
