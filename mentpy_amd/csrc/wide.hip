@@ -977,16 +977,18 @@ hipError_t sv_launch(const Job& J, bool column, uint32_t flags, hipStream_t st) 
 // lane, where a launch takes as long as one lane's chain of steps: here the
 // lanes of a group share a simulation's coefficients (one step per lane) and,
 // from 4 slots on, its amplitudes, 4 per lane.  A group is a whole wave up to
-// 1,024 simulations (one wave per SIMD), else at least 8 lanes.
+// 1,024 simulations (one wave per SIMD), else 8 lanes (6 slots: 16).
 constexpr int narrow_reg_bits(int ns) { return ns <= 3 ? ns : 2; }
 
-// Most simulations that run so.  Measured in replayed graphs, 30-column grids,
-// us per launch (one lane per simulation / this): 2 slots 64 sims 8.1 / 6.4,
-// 4,096 9.7 / 9.4, 8,192 9.9 / 10.0; 3 slots 64 13.3 / 9.8, 1,024 14.0 / 11.9,
-// 4,096 14.3 / 14.6; 4 slots 64 22.4 / 11.2, 8,192 23.6 / 20.4, 16,384
+// Most simulations that run so.  Measured in replayed graphs, us per launch (one lane
+// per simulation / this), angle-major angles: 2 slots, 40 columns, 16 sims 9.7 / 8.9,
+// 512 10.1 / 9.7, 768 10.1 / 10.6, 4,096 10.3 / 13.0; 3 slots, 40 columns, 16 sims
+// 16.5 / 14.5, 512 17.1 / 15.1, 640 17.0 / 17.6, 2,048 17.1 / 19.0 (rows of angles: 2
+// slots, 2,048 sims 11.6 / 11.4, 3 slots 17.5 / 18.5; 4 and 80 columns cross at the
+// same sizes).  30-column grids: 4 slots 64 22.4 / 11.2, 8,192 23.6 / 20.4, 16,384
 // 24.0 / 23.8, 32,768 24.8 / 38.5; 5 slots 64 45.5 / 14.1, 16,384 48.0 / 32.4,
 // 32,768 49.9 / 54.2; 6 slots 64 86 / 14.7, 32,768 94.7 / 75.6.  One slot: no gain.
-constexpr int64_t kNarrowMaxSims[7] = {0, 0, 4096, 2048, 16384, 16384, 32768};
+constexpr int64_t kNarrowMaxSims[7] = {0, 0, 512, 512, 16384, 16384, 32768};
 
 template <int NS, int SPARE>
 hipError_t narrow_launch(const Job& J, bool column, uint32_t flags, hipStream_t st) {
@@ -1023,8 +1025,9 @@ hipError_t shared_launch(const Job& J, bool column, uint32_t flags, hipStream_t 
 template <int NS>
 hipError_t narrow_launch(const Job& J, bool column, uint32_t flags, hipStream_t st) {
   constexpr int lane_bits = NS - narrow_reg_bits(NS);
-  if (J.total <= 1024) return narrow_launch<NS, 6 - lane_bits>(J, column, flags, st);
-  return narrow_launch<NS, (lane_bits < 3 ? 3 - lane_bits : 0)>(J, column, flags, st);
+  if constexpr (kNarrowMaxSims[NS] <= 1024) return narrow_launch<NS, 6 - lane_bits>(J, column, flags, st);
+  else if (J.total <= 1024) return narrow_launch<NS, 6 - lane_bits>(J, column, flags, st);
+  else return narrow_launch<NS, (lane_bits < 3 ? 3 - lane_bits : 0)>(J, column, flags, st);
 }
 
 // One simulation whose angles and input come with the kernel's arguments and
