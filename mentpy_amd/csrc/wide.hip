@@ -1133,15 +1133,23 @@ hipError_t launch_run_one(const Job& J, const HostInputs& in, bool column, uint3
 }
 
 // Most simulations that run with their angles' coefficients shared (raw phase, inputs a
-// multiple of 4).  Replayed graphs, us (as without sharing / shared): 4x16 grid, 16
-// inputs, 2,048 sims 9.6 / 8.1, 16,384 14.2 / 11.1, 32,768 17.2 / 14.7, 65,536
-// 18.1 / 25.9; 5x10, 32 inputs, 2,048 8.4 / 7.2, 16,384 13.2 / 11.8, 32,768
-// 26.4 / 18.7, 65,536 28.3 / 33.0; 6x12, 64 inputs, 16,384 20.3 / 18.7, 131,072
-// 119.9 / 96.3.
-constexpr int64_t kSharedMaxSims[7] = {0, 0, 0, 0, 32768, 32768, 131072};
-
+// multiple of 4).  Both forms take time in proportion to the steps, but the one with
+// one simulation per lane waits for the same memory latencies whatever the steps, so
+// that the line lies higher for short patterns.  Replayed graphs, us (one simulation
+// per lane / shared), 4 inputs: 4 slots, 33 columns, 32,768 sims 27.2 / 26.7; 80
+// columns, 28,672 sims 55.2 / 54.1, 32,768 55.1 / 57.4; 5 slots, 26 columns, 32,768 sims
+// 44.7 / 41.7; 80 columns, 28,672 sims 105.4 / 103.6, 32,768 105.5 / 115.6; 6 slots, 13
+// columns, 131,072 sims 110 / 98; 20 columns, 49,152 sims 74.6 / 61.5, 131,072 112 / 150;
+// 41 columns, 49,152 sims 127.7 / 122.5, 65,536 131 / 159; 80 columns, 40,960 sims
+// 219 / 199, 49,152 (16 inputs) 218 / 236.
 static int64_t shared_max(const Job& J, uint32_t flags) {
-  return J.S % 4 == 0 && !(flags & MBQC_FLAG_REF_PHASE) ? kSharedMaxSims[J.ns] : 0;
+  if (J.S % 4 != 0 || (flags & MBQC_FLAG_REF_PHASE)) return 0;
+  switch (J.ns) {
+    case 4:
+    case 5: return J.n_steps <= 128 ? 32768 : 28672;
+    case 6: return J.n_steps <= 72 ? 131072 : J.n_steps <= 240 ? 49152 : 40960;
+    default: return 0;
+  }
 }
 
 bool narrow_sv(const Job& J, uint32_t flags) {

@@ -38,3 +38,27 @@ def test_two_and_three_slots_either_side_of_512(rows, cols, window, B, rng):
         assert torch.equal(full[part], sim.run_batch(th[part].contiguous(), psi))
     ref = sv_batch(g, th[-8:].double().cpu().numpy(), psi[None])
     assert np.abs(full[-8:].cpu().numpy() - ref).max() < 2e-5
+
+
+# (rows, cols, B, S): the raw-phase batches where the longest patterns of 4, 5 and 6 slots
+# stop sharing coefficients between inputs, and where shorter ones still do
+@pytest.mark.parametrize("rows,cols,B,S", [
+    (4, 34, 7168, 4), (4, 34, 7169, 4), (4, 33, 8192, 4), (4, 33, 8193, 4),
+    (5, 27, 3584, 8), (5, 27, 3585, 8), (5, 26, 4096, 8),
+    (6, 13, 8192, 16), (6, 14, 3072, 16), (6, 14, 3073, 16), (6, 42, 2560, 16), (6, 42, 2561, 16)])
+def test_shared_coefficients_by_steps(rows, cols, B, S):
+    """Either side of the largest shared batches of short, longer and long patterns: equal
+    to the launches of one input each."""
+    torch = _torch()
+    from mentpy_amd.simulators.hip_simulator import sv_forward
+    g, sim = _sim(rows, cols)
+    plan = sim.simulator.plan
+    gen = torch.Generator().manual_seed(rows * cols)
+    th = (torch.rand((B, len(g.trainable_nodes)), generator=gen) * 12 - 6).cuda()
+    x = torch.randn((S, 1 << rows), generator=gen, dtype=torch.complex64).cuda()
+    got = sv_forward(plan, th, x, ref_phase=False, renormalize=False)
+    for i in (0, S - 1):
+        one = sv_forward(plan, th[-64:], x[i:i + 1], ref_phase=False, renormalize=False)
+        assert torch.equal(got[-64:, i], one[:, 0])
+        one = sv_forward(plan, th[:64], x[i:i + 1], ref_phase=False, renormalize=False)
+        assert torch.equal(got[:64, i], one[:, 0])
