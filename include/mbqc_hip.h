@@ -285,7 +285,8 @@ int mbqc_dm_forward_outcomes_c64(const mbqc_plan* plan, const float* angles, int
  * and every angle-vector entry used by at most one measured node
  * (angle_index values unique).  These two take live windows of up to 16
  * qubits.  Plans in column order (grids) spread a simulation's state over lanes
- * from 4 slots (up to 32,768 columns; 5 slots: 49,152; from 6 any number) to 14; other
+ * from 4 slots (4 and 5 up to a measured number of columns in all, 16,384 to 45,056
+ * by slots, steps and columns per set; from 6 any number) to 14; other
  * plans hold it in registers up to 5 slots, with one workgroup per
  * simulation (forward) or partial-sum row (backward) in LDS from 6 to 10
  * (the backward pass keeps n_angles floats of per-angle sums in LDS too, so

@@ -3362,16 +3362,24 @@ inline int32_t adj_reduced_columns(int64_t C) {
 
 // Column plans of 6..14 slots run the register-blocked sweeps, those of 4 and 5
 // slots up to a number of columns: a simulation takes 4 or 8 lanes there and a
-// quarter of the time, which pays until the lanes are all taken.  4x16 grid,
-// 16 columns per set, forward and backward in us, one lane per simulation -> spread:
-// 16 sets 46.7 -> 26.4, 1024 sets 53.3 -> 36.2, 2048 sets 57.6 -> 47.0, 4096 sets
-// 64.7 -> 70.0.  5x10 grid, 32 columns: 16 sets 61.5 -> 23.5, 1024 sets
-// 74.9 -> 57.2, 1500 sets 81.8 -> 74.9, 2048 sets 88.0 -> 93.5.  (2 and 3 slots:
-// no gain at any size, 2x12 and 3x12 grids.)  The checkpoints of the two kinds
-// differ, so the choice depends on the plan, B and C only.
+// quarter of the time, which pays until the lanes are all taken.  That is earlier where
+// the columns of a row are few, so that they share no coefficients, and in long
+// patterns, whose per-angle sums take LDS.  Replayed graphs, forward and backward in
+// us, one lane per simulation / spread: 4x16 grid, 16 columns, 1,024 sets 53.3 / 36.2,
+// 2,048 sets 57.6 / 47.0, 4,096 sets 64.7 / 70.0; 4x40, 24,576 columns of 3 143.6 / 135.9,
+// 32,768 174.6 / 202.0, of 16 126.2 / 99.4; 4x80, 16,384 columns of 3 256.8 / 237.8,
+// 20,480 278.4 / 365.7; 5x30, 45,056 columns of 3 305.0 / 253.7, of 16 209.7 / 215.8,
+// 40,960 of 16 205.4 / 199.1; 5x60, 36,864 columns of 16 422 / 372, of 64 421 / 450.
+// (2 and 3 slots: no gain at any size, 2x12 and 3x12 grids.)  The checkpoints of the
+// two kinds differ, so the choice depends on the plan, B and C only.
 bool wide_adjoint(const Plan* p, int64_t B, int64_t C) {
   if (!p->column_steps || !wide_adjoint_fits(p->ns, adj_reduced_columns(C), p->n_angles)) return false;
-  return p->ns > kMaxAdjSlots || B * C <= (p->ns == 5 ? 49152 : 32768);
+  if (p->ns > kMaxAdjSlots) return true;
+  const int32_t red = adj_reduced_columns(C);
+  const bool lng = p->n_steps > 160;
+  const int64_t most = p->ns == 4 ? (red > 1 ? 32768 : lng ? 16384 : 24576)
+                                  : (red < 16 ? 45056 : red == 64 && lng ? 32768 : 40960);
+  return B * C <= most;
 }
 
 // Adjoint sweeps above kMaxAdjLdsSlots slots refuse stream capture whichever

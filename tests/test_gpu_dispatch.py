@@ -62,3 +62,32 @@ def test_shared_coefficients_by_steps(rows, cols, B, S):
         assert torch.equal(got[-64:, i], one[:, 0])
         one = sv_forward(plan, th[:64], x[i:i + 1], ref_phase=False, renormalize=False)
         assert torch.equal(got[:64, i], one[:, 0])
+
+
+# (rows, cols, columns per set, sets): the last batch of the sweeps that spread a
+# simulation over lanes and the first one above it
+@pytest.mark.parametrize("rows,cols,C,B", [
+    (4, 6, 3, 8192), (4, 6, 3, 8193), (4, 42, 1, 16384), (4, 42, 1, 16385), (4, 6, 16, 2048),
+    (4, 6, 16, 2049), (5, 5, 3, 15018), (5, 5, 3, 15019), (5, 5, 16, 2560), (5, 5, 16, 2561),
+    (5, 34, 64, 512), (5, 34, 64, 513)])
+def test_adjoint_either_side_of_its_limits(rows, cols, C, B):
+    """Outputs and gradients of sets at the ends of the batch against those of a few sets
+    alone.  Both are float32 sweeps of the same steps: within 2e-5 of the largest
+    gradient, the bound that the sweeps meet against complex128."""
+    torch = _torch()
+    from mentpy_amd.gradients.adjoint import AdjointEngine
+    g, sim = _sim(rows, cols)
+    eng = AdjointEngine(sim.simulator.plan)
+    gen = torch.Generator().manual_seed(rows * cols)
+    th = (torch.rand((B, len(g.trainable_nodes)), generator=gen) * 6.2).cuda()
+    x = torch.randn((C, 1 << rows), generator=gen, dtype=torch.complex64).cuda()
+    x = x / torch.linalg.vector_norm(x, dim=1, keepdim=True)
+    seed = torch.randn((B, C, 1 << rows), generator=gen, dtype=torch.complex64).cuda() * 2.0 ** (-rows / 2)
+    out, state = eng.forward(th, x)
+    grad = eng.backward(state, seed)
+    assert torch.isfinite(grad).all()
+    for part in (slice(0, 3), slice(B - 3, B)):
+        o, st = eng.forward(th[part].contiguous(), x)
+        gr = eng.backward(st, seed[part].contiguous())
+        assert (out[part] - o).abs().max().item() < 2e-5
+        assert (grad[part] - gr).abs().max().item() < 2e-5 * max(1.0, gr.abs().max().item())
