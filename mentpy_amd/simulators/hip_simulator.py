@@ -202,24 +202,38 @@ def _angle_strides(a):
 
 
 # Launches with one simulation per lane read a row of angles 128 bytes at a time and
-# 4 of them per step; past this many bytes, in rows of this many angles, the lines
-# leave the caches before their next use and a pass to angle-major order first is
-# faster (launch in us, rows / pass and launch: 4x20 grid, 131,072 sets 66 / 47, 65,536
-# sets 25 / 32; 4x19, 116,509 sets 39 / 41; 4x40, 65,536 sets 82 / 56, 524,288 sets
-# 1485 / 310; 3x40, 131,072 sets 116 / 56; rows of 36 angles, 524,288 sets 57 / 82; with
-# 3 inputs per set the lines are shared: 4x20, 524,288 sets 256 / 302; 2 slots, 78
-# angles, 131,072 sets 36 / 38).
-_ANGLE_PASS_BYTES = 9 << 22
+# 4 of them per step.  Past this many bytes in rows of this many angles the lines leave
+# the caches before their next use, and a pass to angle-major order first is faster, if
+# there are sets enough in flight to crowd them out.  It pays later where a step takes
+# longer (6 slots, sampled outcomes).  Launch in us, rows / pass and launch: 4x20 grid,
+# 131,072 sets 66 / 47, 65,536 sets 25 / 32; 4x40, 62,000 sets 69 / 52, 524,288 sets
+# 1485 / 310; 5x40, 49,000 sets 101 / 82; 5x80, 40,506 sets 132 / 144; 6 slots, 16 columns,
+# 106,000 sets (38 MB) 87 / 110, 40 columns, 41,000 sets (38 MB) 120 / 139, 25 columns,
+# 111,111 sets (64 MB) 198 / 135, 80 columns, 33,755 sets (64 MB) 217 / 249, 52,742 sets
+# (100 MB) 367 / 267; 3 slots, 80 columns, 60,000 sets 61 / 63, 67,510 sets 123 / 67.
+# Sampled: 5x20, 100,000 sets (38 MB) 74 / 83; 4x60, 60,000 sets 96 / 103; 5x80, 63,291
+# sets 373 / 215; 4x40, 72,115 sets (45 MB) 116 / 75; 3x80, 60,000 sets 67 / 92.  Rows of 36 angles, 524,288 sets
+# 57 / 82; with 3 inputs per set the lines are shared: 4x20, 524,288 sets 256 / 302; 2
+# slots, 78 angles, 131,072 sets 36 / 38.
 _ANGLE_PASS_MIN_ANGLES = 72
 
 
-def _lane_angles(plan, a, S: int):
+def _angle_pass(n_slots: int, B: int, n: int, S: int, sampled: bool) -> bool:
+    """Whether ``B`` rows of ``n`` angles are worth the pass."""
+    if S != 1 or not 3 <= n_slots <= 6 or n < _ANGLE_PASS_MIN_ANGLES:
+        return False
+    if sampled:
+        return B >= 62000 and 4 * B * n >= 42 << 20
+    return (B >= (62000 if n_slots == 3 else 49000)
+            and 4 * B * n >= (42 << 20 if n_slots == 6 else 36 << 20))
+
+
+def _lane_angles(plan, a, S: int, sampled: bool):
     """``a [B, n]`` as the statevector launches read it best: itself, or an
     angle-major copy; ``(tensor, stride over sets, stride over angles)``."""
     B, n = a.shape
     sb, sa = _angle_strides(a)
-    if (S != 1 or not 3 <= plan.info["n_slots"] <= 6 or sa != 1 or sb < n
-            or n < _ANGLE_PASS_MIN_ANGLES or 4 * B * n < _ANGLE_PASS_BYTES):
+    if sa != 1 or sb < n or not _angle_pass(plan.info["n_slots"], B, n, S, sampled):
         return a, sb, sa
     torch = _torch()
     try:
@@ -274,7 +288,7 @@ def sv_forward(plan: nat.NativePlan, angles, states, *, ref_phase: bool = True,
     flags = ((nat.FLAG_REF_PHASE if ref_phase else 0) | (nat.FLAG_RENORMALIZE if renormalize else 0)
              | (nat.FLAG_WRITE_PHASE if want_phase else 0)
              | (nat.FLAG_TABLE_STEPS if table_steps else 0))
-    angles, sb, sa = _lane_angles(plan, angles, S)
+    angles, sb, sa = _lane_angles(plan, angles, S, False)
     nat.launch(device, nat.lib().mbqc_sv_forward_c64, plan.handle, angles.data_ptr(), sb, sa,
                states.data_ptr(), states.shape[1], out.data_ptr(),
                phase.data_ptr() if phase is not None else 0, B, S, flags)
@@ -300,7 +314,7 @@ def sv_sample(plan: nat.NativePlan, angles, states, seed: int, *, out=None, outc
         out = torch.empty((B, S, 1 << info["n_outputs"]), dtype=torch.complex64, device=device)
     if outcomes is None:
         outcomes = torch.empty((B, S, W + 2), dtype=torch.int32, device=device)
-    angles, sb, sa = _lane_angles(plan, angles, S)
+    angles, sb, sa = _lane_angles(plan, angles, S, True)
     nat.launch(device, nat.lib().mbqc_sv_sample_c64, plan.handle, angles.data_ptr(), sb, sa,
                states.data_ptr(), states.shape[1], out.data_ptr(), outcomes.data_ptr(), B, S,
                int(seed) & (2 ** 64 - 1))
