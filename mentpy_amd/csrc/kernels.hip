@@ -22,6 +22,7 @@
 #include "device.h"
 #include "plan.h"
 #include "gram.h"
+#include "grids.h"
 #include "side_streams.h"
 #include "wide.h"
 
@@ -4757,11 +4758,17 @@ int mbqc_angle_major_f32(const float* angles, int64_t angle_stride, float* out, 
     return fail(MBQC_ERR_VALUE, "sizes must be B >= 0, n >= 0, angle_stride >= 0, out_stride >= B");
   if (B == 0 || n == 0) return MBQC_OK;
   if (!angles || !out) return fail(MBQC_ERR_VALUE, "null pointer");
-  const int64_t blocks = (B + 63) / 64 * ((n + 31) / 32);
-  if (blocks > 0x7fffffff) return fail(MBQC_ERR_VALUE, "too many angles for one launch");
-  hipLaunchKernelGGL(k_angle_major, dim3(unsigned(blocks)), dim3(256), 0,
-                     static_cast<hipStream_t>(stream), angles, angle_stride, out, out_stride, B, n);
-  hipError_t e = hipGetLastError();
+  // whole rows of tiles per launch (64 angle vectors, n_tiles workgroups each)
+  const int64_t n_tiles = (n + 31) / 32;
+  if (n_tiles > 0xffffff) return fail(MBQC_ERR_VALUE, "too many angles for one launch");
+  const hipError_t e = in_grids((B + 63) / 64, n_tiles * 256, hipSuccess,
+                                [&](int64_t first, int64_t count) {
+    const int64_t b0 = first * 64;
+    hipLaunchKernelGGL(k_angle_major, dim3(unsigned(count * n_tiles)), dim3(256), 0,
+                       static_cast<hipStream_t>(stream), angles + b0 * angle_stride, angle_stride,
+                       out + b0, out_stride, B - b0, n);
+    return hipGetLastError();
+  });
   return e == hipSuccess ? MBQC_OK : hip_fail(e, "angle transpose launch");
 }
 

@@ -20,6 +20,7 @@
 // Bound by LDS bandwidth and VALU issue about equally: a block of the 9-slot
 // loop is 232 VALU and 41 LDS instructions per wave.  9x10 grid, 4,099
 // simulations: 103.6 us with one LDS pass and one barrier per step, 28.4 us so.
+#include "grids.h"
 #include "wide.h"
 
 #include <algorithm>
@@ -303,12 +304,13 @@ __device__ __forceinline__ void wide_sim(const Job& J, int64_t g, bool active, u
 }
 
 template <int NS, int R, bool REF, bool COLUMN, int SPARE = 0>
-__global__ __launch_bounds__((Wide<NS, R, NS, SPARE>::T)) void k_wide_sv(Job J, uint32_t flags) {
+__global__ __launch_bounds__((Wide<NS, R, NS, SPARE>::T)) void k_wide_sv(Job J, int64_t g0,
+                                                                       uint32_t flags) {
   using W = Wide<NS, R, NS, SPARE>;
   __shared__ float2 lds[W::G * W::SIM];
   const int sub = threadIdx.x / W::CL, cl = threadIdx.x % W::CL;
   float2* buf = lds + sub * W::SIM;
-  const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
+  const int64_t g = g0 + int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
   wide_sim<NS, R, REF, COLUMN, SPARE>(J, g, g < J.total, flags, buf, buf + W::BUF, cl);
 }
 
@@ -341,13 +343,13 @@ template <int NS, int R, bool COLUMN>
 __global__ __launch_bounds__((Wide<NS, R>::T)) void k_wide_sample(
     Job J, const uint64_t* __restrict__ xm, const uint64_t* __restrict__ zm,
     const int32_t* __restrict__ out_off, int32_t* __restrict__ outcomes, int32_t words,
-    uint64_t seed) {
+    uint64_t seed, int64_t g0) {
   using W = Wide<NS, R>;
   __shared__ float2 lds[W::G * W::SIM];
   const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
   float2* buf = lds + sub * W::SIM;
   float2* bs = buf + W::BUF;
-  const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
+  const int64_t g = g0 + int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
   const bool active = g < J.total;
   const int64_t gg = active ? g : J.total - 1;
   int64_t bi, si;
@@ -957,20 +959,31 @@ hipError_t tile_passes(int ns, int blocks, Pass&& pass) {
   return hipSuccess;
 }
 
+// launch(grid, g0) over all simulations.  (13 and 14 slots take 512 and 1,024 threads per
+// simulation: 8,388,608 and 4,194,304 of them are more than one launch has.)
+template <typename W, typename Launch>
+hipError_t in_sim_grids(int64_t total, Launch&& launch) {
+  return in_grids((total + W::G - 1) / W::G, W::T, hipSuccess, [&](int64_t first, int64_t count) {
+    launch(dim3(unsigned(count)), first * W::G);
+    return hipGetLastError();
+  });
+}
+
 template <int NS>
 hipError_t sv_launch(const Job& J, bool column, uint32_t flags, hipStream_t st) {
   constexpr int R = wide_reg_bits(NS);
   using W = Wide<NS, R>;
-  const dim3 grid(unsigned((J.total + W::G - 1) / W::G)), block(W::T);
   const bool ref = flags & MBQC_FLAG_REF_PHASE;
-  if (column) {
-    if (ref) hipLaunchKernelGGL((k_wide_sv<NS, R, true, true>), grid, block, 0, st, J, flags);
-    else hipLaunchKernelGGL((k_wide_sv<NS, R, false, true>), grid, block, 0, st, J, flags);
-  } else {
-    if (ref) hipLaunchKernelGGL((k_wide_sv<NS, R, true, false>), grid, block, 0, st, J, flags);
-    else hipLaunchKernelGGL((k_wide_sv<NS, R, false, false>), grid, block, 0, st, J, flags);
-  }
-  return hipGetLastError();
+  return in_sim_grids<W>(J.total, [&](dim3 grid, int64_t g0) {
+    const dim3 block(W::T);
+    if (column) {
+      if (ref) hipLaunchKernelGGL((k_wide_sv<NS, R, true, true>), grid, block, 0, st, J, g0, flags);
+      else hipLaunchKernelGGL((k_wide_sv<NS, R, false, true>), grid, block, 0, st, J, g0, flags);
+    } else {
+      if (ref) hipLaunchKernelGGL((k_wide_sv<NS, R, true, false>), grid, block, 0, st, J, g0, flags);
+      else hipLaunchKernelGGL((k_wide_sv<NS, R, false, false>), grid, block, 0, st, J, g0, flags);
+    }
+  });
 }
 
 // Windows of 1..6 slots with too few simulations to fill the chip at one per
@@ -997,7 +1010,7 @@ hipError_t narrow_launch(const Job& J, bool column, uint32_t flags, hipStream_t 
   const dim3 grid(unsigned((J.total + W::G - 1) / W::G)), block(W::T);
   const bool ref = flags & MBQC_FLAG_REF_PHASE;
 #define MBQC_NARROW(REF, COL) \
-  hipLaunchKernelGGL((k_wide_sv<NS, R, REF, COL, SPARE>), grid, block, 0, st, J, flags)
+  hipLaunchKernelGGL((k_wide_sv<NS, R, REF, COL, SPARE>), grid, block, 0, st, J, int64_t(0), flags)
   if (column) {
     if (ref) MBQC_NARROW(true, true);
     else MBQC_NARROW(false, true);
@@ -1072,14 +1085,15 @@ hipError_t sample_launch(const Job& J, bool column, const uint64_t* xm, const ui
                          hipStream_t st) {
   constexpr int R = wide_reg_bits(NS);
   using W = Wide<NS, R>;
-  const dim3 grid(unsigned((J.total + W::G - 1) / W::G)), block(W::T);
-  if (column)
-    hipLaunchKernelGGL((k_wide_sample<NS, R, true>), grid, block, 0, st, J, xm, zm, out_off, outcomes,
-                       words, seed);
-  else
-    hipLaunchKernelGGL((k_wide_sample<NS, R, false>), grid, block, 0, st, J, xm, zm, out_off,
-                       outcomes, words, seed);
-  return hipGetLastError();
+  return in_sim_grids<W>(J.total, [&](dim3 grid, int64_t g0) {
+    const dim3 block(W::T);
+    if (column)
+      hipLaunchKernelGGL((k_wide_sample<NS, R, true>), grid, block, 0, st, J, xm, zm, out_off, outcomes,
+                         words, seed, g0);
+    else
+      hipLaunchKernelGGL((k_wide_sample<NS, R, false>), grid, block, 0, st, J, xm, zm, out_off,
+                         outcomes, words, seed, g0);
+  });
 }
 
 template <int NS>

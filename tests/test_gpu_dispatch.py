@@ -91,3 +91,32 @@ def test_adjoint_either_side_of_its_limits(rows, cols, C, B):
         gr = eng.backward(st, seed[part].contiguous())
         assert (out[part] - o).abs().max().item() < 2e-5
         assert (grad[part] - gr).abs().max().item() < 2e-5 * max(1.0, gr.abs().max().item())
+
+
+@pytest.mark.parametrize("sampled", [False, True])
+def test_more_threads_than_one_launch_takes(sampled, rng):
+    """14 slots take 1,024 threads per simulation: 4,194,304 simulations are 2^32 threads,
+    more than one launch has.  The last ones (in the second launch) and those around
+    the end of the first equal small launches; sampled, they meet their own draws."""
+    torch = _torch()
+    import mentpy_amd as mp
+    g = mp.templates.linear_cluster(16)
+    kw = {"force0": False, "seed": 4} if sampled else {}
+    sim = mp.PatternSimulator(g, backend="hip-sv", window_size=15, **kw)
+    assert sim.simulator.plan.info["n_slots"] == 14
+    B = (1 << 22) + 3
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    th = torch.rand((B, len(g.trainable_nodes)), generator=gen, device="cuda") * 6.2
+    psi = haar_state(1, rng)
+    out = sim.run_batch(th, psi)
+    torch.cuda.synchronize()
+    norm = torch.linalg.vector_norm(out, dim=-1)
+    assert (norm - 1).abs().max().item() < 1e-5      # every row written
+    post = mp.PatternSimulator(g, backend="hip-sv", window_size=15)
+    for part in (slice(0, 2), slice((1 << 22) - 3, B)):
+        want = post.run_batch(th[part].contiguous(), psi)
+        if sampled:   # equal up to a global phase
+            overlap = (want.conj() * out[part]).sum(-1).abs()
+            assert (overlap - 1).abs().max().item() < 1e-5
+        else:
+            assert torch.equal(out[part], want)
