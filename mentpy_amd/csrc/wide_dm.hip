@@ -28,6 +28,7 @@
 #include "grids.h"
 #include "wide.h"
 
+#include <algorithm>
 #include <utility>
 
 namespace mbqc {
@@ -323,13 +324,13 @@ __device__ __forceinline__ void pauli_sim(const Job& J, int64_t g, bool active, 
 }
 
 template <int NS, int K>
-__global__ __launch_bounds__((Pauli<NS, K>::T)) void k_dm_pauli(Job J, int64_t g0, DmNoise nz,
-                                                               int pad_slots, uint32_t flags) {
+__global__ __launch_bounds__((Pauli<NS, K>::T)) void k_dm_pauli(Job J, DmNoise nz, int pad_slots,
+                                                               uint32_t flags) {
   using W = Pauli<NS, K>;
   __shared__ __align__(16) float2 lds[W::G * W::SIM];
   const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
   float2* buf = lds + sub * W::SIM;
-  const int64_t g = g0 + int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
+  const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
   pauli_sim<NS, K>(J, g, g < J.total, nz, pad_slots, flags, buf, buf + W::BUF, lane,
                    std::make_integer_sequence<int, W::P>{});
 }
@@ -523,13 +524,13 @@ __device__ __forceinline__ void pauli_gradient(const Job& J, const float2* out, 
 
 template <int NS, int K>
 __global__ __launch_bounds__((Pauli<NS, K>::T)) void k_pauli_gradient(
-    Job J, int64_t g0, const float2* __restrict__ out, const float2* __restrict__ seed, int64_t B,
-    int C, int n_angles, float* __restrict__ loss, float* __restrict__ grad) {
+    Job J, const float2* __restrict__ out, const float2* __restrict__ seed, int64_t B, int C,
+    int n_angles, float* __restrict__ loss, float* __restrict__ grad) {
   using W = Pauli<NS, K>;
   __shared__ __align__(16) float2 lds[W::G * W::SIM];
   const int sub = threadIdx.x / W::TL, lane = threadIdx.x % W::TL;
   float2* buf = lds + sub * W::SIM;
-  const int64_t g = g0 + int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
+  const int64_t g = int64_t(xcd_block(blockIdx.x, gridDim.x)) * W::G + sub;
   const bool active = g < B;
   pauli_gradient<NS, K>(J, out, seed, active ? g : B - 1, active, C, n_angles, loss, grad, buf,
                         buf + W::BUF, lane, std::make_integer_sequence<int, W::P>{});
@@ -549,9 +550,16 @@ template <int NS, int K>
 hipError_t dm_launch(const Job& J, const DmNoise& nz, int pad_slots, uint32_t flags,
                      hipStream_t st) {
   using W = Pauli<NS, K>;
-  return in_grids((J.total + W::G - 1) / W::G, W::T, hipSuccess, [&](int64_t first, int64_t count) {
-    hipLaunchKernelGGL((k_dm_pauli<NS, K>), dim3(unsigned(count)), dim3(W::T), 0, st, J, first * W::G,
-                       nz, pad_slots, flags);
+  return in_parts(J.total / J.S, J.S, max_grid(W::T) * W::G, hipSuccess,
+                  [&](int64_t b, int64_t sets, int64_t s, int64_t inputs) {
+    Job part = J;
+    part.angles = J.angles + b * J.angle_stride;
+    part.psi = J.psi + s * J.in_stride;
+    part.out = J.out + ((b * J.S + s) << (2 * J.n_out));
+    part.S = inputs;
+    part.total = sets * inputs;
+    hipLaunchKernelGGL((k_dm_pauli<NS, K>), dim3(unsigned((part.total + W::G - 1) / W::G)), dim3(W::T),
+                       0, st, part, nz, pad_slots, flags);
     return hipGetLastError();
   });
 }
@@ -561,8 +569,12 @@ hipError_t gradient_launch(const Job& J, const float2* out, const float2* seed, 
                            int n_angles, float* loss, float* grad, hipStream_t st) {
   using W = Pauli<NS, K>;
   return in_grids((B + W::G - 1) / W::G, W::T, hipSuccess, [&](int64_t first, int64_t count) {
-    hipLaunchKernelGGL((k_pauli_gradient<NS, K>), dim3(unsigned(count)), dim3(W::T), 0, st, J,
-                       first * W::G, out, seed, B, int(C), n_angles, loss, grad);
+    const int64_t b = first * W::G, rows = (b * C) << NS;
+    Job part = J;
+    part.angles = J.angles + b * J.angle_stride;
+    hipLaunchKernelGGL((k_pauli_gradient<NS, K>), dim3(unsigned(count)), dim3(W::T), 0, st, part,
+                       out + rows, seed + rows, std::min(B - b, count * W::G), int(C), n_angles,
+                       loss ? loss + b : nullptr, grad + b * n_angles);
     return hipGetLastError();
   });
 }
