@@ -84,6 +84,8 @@ class AdjointEngine:
         torch = _torch()
         info = self.plan.info
         B, C_ = state.B, state.C
+        if seed.is_conj():   # autograd hands on lazily conjugated views; the launch reads memory
+            seed = seed.resolve_conj()
         seed = seed.to(torch.complex64).contiguous()
         if tuple(seed.shape) != (B, C_, 1 << info["n_outputs"]):
             raise ValueError(f"seed must have shape {(B, C_, 1 << info['n_outputs'])}")
@@ -125,7 +127,8 @@ class PatternSVFunction:
                     # a private copy: a later in-place change of the caller's
                     # angles must not reach this call's backward pass
                     a = angles.detach().to(torch.float32).contiguous().clone()
-                    out, state = engine.forward(a, cols.detach().to(torch.complex64).contiguous())
+                    x = cols.detach().resolve_conj() if cols.is_conj() else cols.detach()
+                    out, state = engine.forward(a, x.to(torch.complex64).contiguous())
                     ctx.engine = engine
                     ctx.state = state
                     return out

@@ -186,6 +186,8 @@ def _as_angles(angles, n_angles: int, device):
     ``[n, B]`` tensor passed as ``.t()`` gives coalesced loads)."""
     torch = _torch()
     a = torch.as_tensor(angles, dtype=torch.float32, device=device)
+    if a.is_neg():   # a lazily negated view: the launches read memory
+        a = a.resolve_neg()
     if a.dim() == 2 and a.shape[1] == n_angles and a.stride(1) != 0:
         return a
     if a.dim() == 1:
@@ -247,6 +249,8 @@ def _lane_angles(plan, a, S: int, sampled: bool):
 def _as_states(states, n_qubits: int, device):
     torch = _torch()
     s = torch.as_tensor(states, device=device)
+    if s.is_conj():   # a lazily conjugated view: the launches read memory
+        s = s.resolve_conj()
     if (s.dtype == torch.complex64 and s.dim() == 2 and s.shape[1] == (1 << n_qubits)
             and s.is_contiguous()):
         return s
