@@ -121,25 +121,37 @@ __device__ __forceinline__ float group_bcast(float v) {
   }
 }
 
+// th[j] of the lane (th[0] for j past the end).  VALUES: all elements are loaded and
+// chosen among; else the choice has loads as its arms, for which the compiler keeps th
+// in LDS: 1% faster in the single-pattern kernels of 2 slots, but in the batched ones it
+// went to scratch memory (k_batch_mixed: 64 grids of 2..6 rows x 1,024 x 16 554 -> 309 us
+// with VALUES, occupancy 1 -> 2 up to 6 slots; 2..5 rows 181 -> 170 us).
+template <bool VALUES, int M>
+__device__ __forceinline__ float pick(const float (&th)[M], int j) {
+  float mine = th[0];
+#pragma unroll
+  for (int m = 1; m < M; ++m) {
+    if constexpr (VALUES) {
+      const float v = th[m];
+      mine = (j == m) ? v : mine;
+    } else {
+      mine = (j == m) ? th[m] : mine;
+    }
+  }
+  return mine;
+}
+
 // Block [k0, k0 + NS): lane j of the group evaluates step j (and, with REF,
 // adds its reference phase: the group's lanes hold disjoint parts of the sum,
 // reduced by group_reduce_phase at the end).
-template <int NS, bool REF, int... SUBS>
+template <int NS, bool REF, bool VALUES, int... SUBS>
 __device__ __forceinline__ void shared_block_coeffs(const float (&th)[NS], float2 (&bb)[NS],
                                                     RefPhase* ph, int k0, int n_steps,
                                                     std::integer_sequence<int, SUBS...>) {
   constexpr int G = kShareGroup<NS>;
   static_assert(NS >= 2 && NS <= G, "one step per lane of the group");
   const int j = int(threadIdx.x) & (G - 1);
-  float mine = th[0];
-#pragma unroll
-  for (int sub = 1; sub < NS; ++sub) {
-    // (loaded outside the choice: as one of its arms the load kept th in LDS or scratch
-    // memory in the batched kernels; 64 grids of 2..6 rows x 1,024 x 16: 554 -> 309 us,
-    // occupancy of k_batch_mixed 1 -> 2 up to 6 slots; 2..5 rows 181 -> 170 us)
-    const float v = th[sub];
-    mine = (j == sub) ? v : mine;
-  }
+  const float mine = pick<VALUES>(th, j);
   float sn, cs;
   sincos_poly(mine, &sn, &cs);
   if constexpr (REF) ph->add_if(mine, j < NS && k0 + j < n_steps);
@@ -176,14 +188,14 @@ __device__ __forceinline__ void sv_sub(float2 (&t)[1 << NS], const mbqc_step* st
   }
 }
 
-template <int NS, bool REF, bool FULL, bool PER_STEP, bool SH, bool PERIODIC, typename Mod,
-          int... SUBS>
+template <int NS, bool REF, bool FULL, bool PER_STEP, bool SH, bool PERIODIC, bool VALUES,
+          typename Mod, int... SUBS>
 __device__ __forceinline__ void sv_block(float2 (&t)[1 << NS], const mbqc_step* steps,
                                          const float* coef, int k0, int n_steps,
                                          const float (&th)[NS], RefPhase* ph, Mod& mod,
                                          std::integer_sequence<int, SUBS...> seq) {
   float2 bb[NS];
-  if constexpr (SH) shared_block_coeffs<NS, REF>(th, bb, ph, k0, n_steps, seq);
+  if constexpr (SH) shared_block_coeffs<NS, REF, VALUES>(th, bb, ph, k0, n_steps, seq);
   (sv_sub<NS, REF, FULL, PER_STEP, SH, PERIODIC, SUBS>(t, steps, coef, k0, n_steps, th, bb, ph,
                                                        mod),
    ...);
@@ -209,8 +221,8 @@ __device__ __forceinline__ void sv_fetched_block(float2 (&t)[1 << NS], const mbq
 
 // The K full blocks of one angle fetch, sharing over 16 lanes: lane m of the
 // row evaluates step m of the fetch (and adds its reference phase).
-template <int NS, int K, bool REF, bool PER_STEP, bool PERIODIC, typename OnBlock, typename Mod,
-          int... BS>
+template <int NS, int K, bool REF, bool PER_STEP, bool PERIODIC, bool VALUES, typename OnBlock,
+          typename Mod, int... BS>
 __device__ __forceinline__ void sv_fetched_blocks(float2 (&t)[1 << NS], const mbqc_step* steps,
                                                   const float* coef, int blk, int n_steps,
                                                   const float (&th)[K * NS], RefPhase* ph,
@@ -218,12 +230,7 @@ __device__ __forceinline__ void sv_fetched_blocks(float2 (&t)[1 << NS], const mb
                                                   std::integer_sequence<int, BS...>) {
   static_assert(K * NS <= 16, "one step per lane of the row");
   const int j = int(threadIdx.x) & 15;
-  float mine = th[0];
-#pragma unroll
-  for (int m = 1; m < K * NS; ++m) {
-    const float v = th[m];
-    mine = (j == m) ? v : mine;
-  }
+  const float mine = pick<VALUES>(th, j);
   float sn, cs;
   sincos_poly(mine, &sn, &cs);
   if constexpr (REF) ph->add_if(mine, j < K * NS);
@@ -333,7 +340,7 @@ __device__ __forceinline__ void sv_run_blocks(float2 (&t)[1 << NS], const Job& J
       for (int m = 0; m < K * NS; ++m) th[m] = th_next[m];
       fetch_step_angles<K * NS>(steps, aidx, (blk + K) * NS, n, ang, sa, fast, th_next);
       if constexpr (SH && kShareGroup<NS> == 16) {
-        sv_fetched_blocks<NS, K, REF, PER_STEP, PERIODIC>(t, steps, coef, blk, n, th, ph, on_block,
+        sv_fetched_blocks<NS, K, REF, PER_STEP, PERIODIC, !SETTLE>(t, steps, coef, blk, n, th, ph, on_block,
                                                           mod, std::make_integer_sequence<int, K>{});
       } else {
 #pragma unroll
@@ -342,7 +349,7 @@ __device__ __forceinline__ void sv_run_blocks(float2 (&t)[1 << NS], const Job& J
 #pragma unroll
           for (int s2 = 0; s2 < NS; ++s2) tb[s2] = th[b * NS + s2];
           on_block(blk + b, t);
-          sv_block<NS, REF, true, PER_STEP, SH, PERIODIC>(t, steps, coef, (blk + b) * NS, n, tb,
+          sv_block<NS, REF, true, PER_STEP, SH, PERIODIC, !SETTLE>(t, steps, coef, (blk + b) * NS, n, tb,
                                                           ph, mod, Seq{});
         }
       }
@@ -358,7 +365,7 @@ __device__ __forceinline__ void sv_run_blocks(float2 (&t)[1 << NS], const Job& J
 #pragma unroll
             for (int s2 = 0; s2 < NS; ++s2) tb[s2] = th_next[b * NS + s2];
             on_block(blk + b, t);
-            sv_block<NS, REF, true, PER_STEP, SH, PERIODIC>(t, steps, coef, (blk + b) * NS, n, tb,
+            sv_block<NS, REF, true, PER_STEP, SH, PERIODIC, !SETTLE>(t, steps, coef, (blk + b) * NS, n, tb,
                                                             ph, mod, Seq{});
           }
         }
@@ -377,7 +384,7 @@ __device__ __forceinline__ void sv_run_blocks(float2 (&t)[1 << NS], const Job& J
 #pragma unroll
     for (int s2 = 0; s2 < NS; ++s2) tb[s2] = th_next[s2];
     on_block(blk, t);
-    sv_block<NS, REF, false, PER_STEP, SH, false>(t, steps, coef, blk * NS, n, tb, ph, mod, Seq{});
+    sv_block<NS, REF, false, PER_STEP, SH, false, !SETTLE>(t, steps, coef, blk * NS, n, tb, ph, mod, Seq{});
   }
 }
 
@@ -1620,7 +1627,7 @@ __global__ __launch_bounds__(64) void k_sv_adj_backward(Job J, const float2* __r
       for (int j = 0; j < H; ++j) t[j] = s0[j];
       RefPhase ph;
       NoModify nomod;
-      sv_block<NS, false, true, false, false, PERIODIC>(t, steps, coef, b0 * NS, n, th0, &ph,
+      sv_block<NS, false, true, false, false, PERIODIC, false>(t, steps, coef, b0 * NS, n, th0, &ph,
                                                         nomod, std::make_integer_sequence<int, NS>{});
       if (resc[b0 + 1]) {
 #pragma unroll
