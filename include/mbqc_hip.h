@@ -224,8 +224,8 @@ int mbqc_sv_run_host_c64(const mbqc_plan* plan, const float* angles, const void*
  * frame applied to the output (bit n_outputs-1-m = output node m).  Draws are
  * a counter-based hash of (seed, simulation, step).  Needs the flow in the
  * pattern description, no dropped edges and n_slots <= 20 (else
- * MBQC_ERR_NOT_IMPLEMENTED with the reason); windows of 7..14 slots run one
- * workgroup per simulation with the state in LDS, 15..20 the same with the
+ * MBQC_ERR_NOT_IMPLEMENTED with the reason); windows of 7..14 slots spread a
+ * simulation's state over lanes, 15..20 run one workgroup per simulation with the
  * state in a workspace allocated and freed in stream order. */
 int mbqc_sv_sample_c64(const mbqc_plan* plan, const float* angles, int64_t angle_stride,
                        int64_t angle_stride_a, const void* psi_in, int64_t in_stride, void* out,
@@ -369,28 +369,30 @@ int mbqc_batch_create(const mbqc_batch_job* jobs, int32_t n_jobs, int32_t sims_p
                       mbqc_batch** out);
 void mbqc_batch_destroy(mbqc_batch* batch);
 int64_t mbqc_batch_items(const mbqc_batch* batch);
-/* Launch the persistent kernel: `waves` resident wavefronts pull work items
- * from a device counter (reset by a kernel, so the launch pair can be captured
- * in a hipGraph), `wg_waves` wavefronts per workgroup. */
+/* One launch of every job.  The groups of live windows up to 6 slots run together as one
+ * persistent kernel: `waves` resident wavefronts per group, in whole workgroups of
+ * `wg_waves` (1..4, waves >= wg_waves), take work items from up to 32 lists with a
+ * device counter each (reset by a kernel, so that the launch can be captured in a
+ * hipGraph).  Wider groups run as mbqc_batch_group_items says. */
 int mbqc_batch_launch(mbqc_batch* batch, int32_t waves, int32_t wg_waves, uint32_t flags,
                       void* stream);
 /* Work items of the group of live-window size n_slots (0..20; -1 for a null
- * batch or n_slots out of range).  Each non-empty group runs its own
- * persistent kernel, concurrently with the others: up to 6 slots one
- * simulation per lane, 7..14 slots one simulation at a time per workgroup
- * with the state in LDS (2^(n_slots-1) threads, at most 256; its resident
- * waves make waves / (threads / 64) workgroups), 15..20 the same with the
- * states in a workspace that mbqc_batch_create allocates with the batch
- * (256 threads, at most 256 resident workgroups per group: up to 256 * 2^n_slots
- * complex64, 2 GiB for a 20-slot group), so every batch launch allocates
- * nothing and can be captured.  Launches of one batch must not overlap (they
- * share its counters and workspaces). */
+ * batch or n_slots out of range).  Up to 6 slots run one simulation per lane; 7..14
+ * slots a persistent kernel per group whose workgroups of 64 to 1,024 threads spread a
+ * simulation over lanes (its resident waves make waves / (threads / 64)
+ * workgroups, at least one); 15..20 slots passes over tiles of the states, which take the
+ * simulations of all the group's jobs together, as many at a time as fit a workspace that
+ * mbqc_batch_create allocates with the batch (2 x 2^n_slots complex64 for up to 128
+ * simulations, 2 GiB for a 20-slot group): there a wave count above 0 only says that
+ * the group runs.  Groups above 6 slots run on side streams joined into `stream`, beside
+ * the others.  A launch allocates nothing and can be captured.  Launches of one batch
+ * must not overlap (they share its counters and workspaces). */
 int64_t mbqc_batch_group_items(const mbqc_batch* batch, int32_t n_slots);
-/* mbqc_batch_launch with the resident wavefront count chosen per group:
- * group_waves[ns] (n_entries <= 21 entries, indexed by live-window size) for
- * the group of size ns; 0 skips the group (its outputs are not written), a
- * positive count must be at least wg_waves.  Sizing the groups by their
- * work makes the concurrent kernels finish together. */
+/* The same with a persistent kernel per group, also up to 6 slots, and the resident
+ * wavefront count chosen for each: group_waves[ns] (n_entries <= 21 entries, indexed
+ * by live-window size) for the group of size ns; 0 skips the group (its outputs are
+ * not written), a positive count must be at least wg_waves.  Sizing the groups by
+ * their work makes the concurrent kernels finish together. */
 int mbqc_batch_launch_groups(mbqc_batch* batch, const int32_t* group_waves, int32_t n_entries,
                              int32_t wg_waves, uint32_t flags, void* stream);
 

@@ -114,8 +114,10 @@ class BatchedForward:
         return hashlib.sha1(repr(parts).encode()).hexdigest()[:16]
 
     def groups(self) -> dict:
-        """Work items per live-window size (the groups that run as separate,
-        concurrent persistent kernels)."""
+        """Work items per live-window size.  The groups up to 6 slots run as one
+        persistent kernel (or, with ``group_waves``, as one each), the wider ones
+        as one each beside it; from 15 slots on a group runs as passes over the
+        states of all its simulations, where a wave count only says that it runs."""
         L = nat.lib()
         out = {}
         for ns in range(MAX_GROUPS):

@@ -227,9 +227,8 @@ __device__ __forceinline__ uint32_t draw32(uint64_t seed, uint64_t sim, uint64_t
 // (-1)^x theta, the drawn projection m' (probability 1/2 each) is onto
 // |+/- theta'>, and the physical outcome is m' xor z.  An outcome 1 flips the
 // frames of the flow successor and of its later neighbours (xmask/zmask).
-// Frames are 32-bit: a plan that samples applies every CZ edge within its
-// window of at most 7 positions, so every offset is below 14 (the host
-// checks < 32).
+// Frames are 32-bit: a plan that samples has every offset below 32 (the plan
+// compiler checks it).
 struct SampleMod {
   uint32_t fx = 0, fz = 0;
   uint64_t seed = 0, sim = 0;

@@ -42,7 +42,7 @@ hipError_t launch_wide_batch(int ns, bool column, int64_t waves, const Job* jobs
                              const BatchItem* items, int64_t n_items, int* counter, uint32_t flags,
                              hipStream_t st);
 
-// Adjoint sweeps of column plans with 6..14 slots.  Checkpoints: the state after
+// Adjoint sweeps of column plans with 4..14 slots.  Checkpoints: the state after
 // every ck-th block and after the last, ckpt[(block / ck) * total + g] each
 // 2^ns amplitudes.
 struct WideAdjoint {

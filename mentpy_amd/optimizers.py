@@ -189,8 +189,9 @@ class MBQMLTrainer:
     def capture(self):
         """Capture one iteration in a HIP graph (the parameters advance by one
         optimizer step during capture warm-up; use a fresh trainer to time).
-        Live windows of 11..16 qubits allocate the adjoint's workspace on every
-        call, which graph capture refuses (NotImplementedError): run those
+        Adjoint sweeps of live windows of 11..16 qubits refuse capture
+        (NotImplementedError), whichever kernels run them: those that allocate a
+        workspace on every call must, and the rule is the window alone.  Run those
         without a graph."""
         import torch
         self._iteration()
