@@ -5,8 +5,9 @@ expressivity sweep loops over them (`docs/tutorials/intro-to-mbqml.rst:43-54`,
 `docs/tutorials/intro-to-mbqml-parallel.rst:43-47`).  ``BatchedForward`` packs
 jobs (pattern, angles ``[B, n]``, inputs ``[S, 2^|I|]``) of uneven sizes into
 one work list, sorted longest first, and runs them with one persistent kernel
-whose wavefronts pull work items from a device counter.  The launch (counter
-reset kernel + persistent kernel) can be captured in a HIP graph and replayed.
+whose wavefronts pull work items from lists with a device counter each (windows of
+more than 6 slots: kernels of their own beside it).  The launch (counter reset
+kernel and the others) can be captured in a HIP graph and replayed.
 
 ``autotune`` picks the resident wavefront count, wavefronts per workgroup and
 simulations per work item by timing graph replays of candidate launches with
